@@ -11,15 +11,18 @@ Run ``python -m cpw2000_amd.build``.
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "libcpwgpu.so")
 FLIB = os.path.join(PKG, "libcpwgpu_fortran.so")
+OBJ = os.path.join(ROOT, "build")
 PLIB = os.path.join(PKG, "libcpwprobe.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -27,7 +30,7 @@ FLANG = os.environ.get("FLANG", shutil.which("flang") or "/opt/rocm/lib/llvm/bin
 ARCH = os.environ.get("CPWGPU_ARCH", "gfx950")
 
 HIP_FLAGS = [
-    "-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared",
+    "-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC",
     # no packed FP32 instructions anywhere in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
@@ -39,19 +42,42 @@ def _run(cmd):
     subprocess.run(cmd, check=True)
 
 
+def mesh_lengths():
+    """The specialised mesh lengths (CPW_FAST_SIZES of csrc/mesh.hpp)."""
+    with open(os.path.join(CSRC, "mesh.hpp")) as f:
+        line = next(t for t in f if t.startswith("#define CPW_FAST_SIZES"))
+    return [int(n) for n in re.findall(r"X\((\d+)\)", line)]
+
+
 def build_hip():
-    srcs = [os.path.join(CSRC, "cpwgpu.hip")]
+    # one object per specialised mesh length (csrc/mesh.hip), side by side, and
+    # the rest (csrc/cpwgpu.hip); the longest compiles first
+    os.makedirs(OBJ, exist_ok=True)
+    jobs = [("cpwgpu.hip", "cpwgpu.o", [])]
+    jobs += [("mesh.hip", f"mesh{n}.o", [f"-DCPW_N={n}"]) for n in sorted(mesh_lengths(), reverse=True)]
+    objs = [os.path.join(OBJ, o) for _, o, _ in jobs]
+
+    def compile_one(job):
+        src, obj, defs = job
+        _run([HIPCC, *HIP_FLAGS, "-c", *defs, "-I", os.path.join(ROOT, "include"), "-o", os.path.join(OBJ, obj),
+              os.path.join(CSRC, src)])
+
+    with ThreadPoolExecutor(max_workers=int(os.environ.get("MAX_JOBS", 0)) or os.cpu_count() or 1) as pool:
+        for done in [pool.submit(compile_one, j) for j in jobs]:
+            done.result()
     tmp = LIB + ".tmp"
     # rocSOLVER (zheevd, zpotrf) and rocBLAS (ztrsm) for the small dense
-    # eigenproblems of the iterative diagonalisation
-    _run([HIPCC, *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), "-o", tmp, *srcs,
-          "-lrocsolver", "-lrocblas"])
+    # eigenproblems of the iterative diagonalisation.  The first device bundle
+    # of the library is the one that offload tools read: length 72, which has
+    # every kind of line transform.
+    objs.sort(key=lambda o: not o.endswith("mesh72.o"))
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-o", tmp, *objs, "-lrocsolver", "-lrocblas"])
     os.replace(tmp, LIB)
 
 
 def build_probe():
     tmp = PLIB + ".tmp"
-    _run([HIPCC, *HIP_FLAGS, "-o", tmp, os.path.join(CSRC, "issue_rates.hip")])
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, os.path.join(CSRC, "issue_rates.hip")])
     os.replace(tmp, PLIB)
 
 

@@ -20,12 +20,8 @@
 #include <string>
 #include <vector>
 
-#include "../../include/cpwgpu.h"
-#include "fft_fast.hpp"
-#include "fft_local.hpp"
-#include "fft_reg.hpp"
-#include "fft_wave.hpp"
-#include "fft_col_reg.hpp"
+#include "host.hpp"
+#include "mesh.hpp"
 #include "nl_gemm.hpp"
 #include "subspace.hpp"
 #include "forces.hpp"
@@ -33,64 +29,7 @@
 #include "spin.hpp"
 #include "proj_kb.hpp"
 
-using namespace cpwgpu;
-
 namespace {
-
-thread_local std::string g_err;
-std::mutex g_mu;
-int g_device = 0;
-int g_prec = CPWGPU_PREC_FP64;
-int g_ditsp_method = CPWGPU_DITSP_CHEB;
-int g_overlap = 1;
-hipStream_t g_stream = nullptr;
-
-int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
-int fail(int code, const char *fmt, ...) {
-    char buf[512];
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(buf, sizeof buf, fmt, ap);
-    va_end(ap);
-    g_err = buf;
-    return code;
-}
-
-#define HIPCHK(x)                                                                          \
-    do {                                                                                   \
-        hipError_t e_ = (x);                                                               \
-        if (e_ != hipSuccess)                                                              \
-            return fail(e_ == hipErrorOutOfMemory ? CPWGPU_ERR_NOMEM : CPWGPU_ERR_HIP,     \
-                        "%s: %s (%s:%d)", #x, hipGetErrorString(e_), __FILE__, __LINE__);  \
-    } while (0)
-
-int ensure_stream() {
-    if (!g_stream) {
-        HIPCHK(hipSetDevice(g_device));
-        HIPCHK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
-    }
-    return CPWGPU_OK;
-}
-
-// grow-only device buffer
-struct DevBuf {
-    void *p = nullptr;
-    size_t n = 0;
-    int reserve(size_t bytes) {
-        if (bytes <= n) return CPWGPU_OK;
-        if (p) hipFree(p);
-        p = nullptr;
-        n = 0;
-        HIPCHK(hipMalloc(&p, std::max<size_t>(bytes, 256)));
-        n = bytes;
-        return CPWGPU_OK;
-    }
-    void release() {
-        if (p) hipFree(p);
-        p = nullptr;
-        n = 0;
-    }
-};
 
 // Src/ALFA/size_fft.f90:53-76
 void size_fft(const int *km, int *ns, int *mfft, int *mwrk) {
@@ -132,113 +71,9 @@ int min_radix(const int *rad, int nrad) {
     return r;
 }
 
-// ---- per-kernel event timing (measurement hook) ----------------------------
-struct Prof {
-    bool on = false;
-    unsigned mask = 0;
-    struct Rec { int k; hipEvent_t a, b; };
-    std::vector<Rec> recs;
-    std::vector<hipEvent_t> pool;
-    hipEvent_t get() {
-        if (!pool.empty()) { hipEvent_t e = pool.back(); pool.pop_back(); return e; }
-        // timing only (read after the whole stream has finished): no
-        // system-scope fence, so recording them does not write back and
-        // invalidate the caches in the middle of the work they time
-        hipEvent_t e = nullptr;
-        if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) return nullptr;
-        return e;
-    }
-} g_prof;
-
-// Launches kernel f on stream s.  With the measurement hook on for kernel id
-// k, the start and stop events travel with the dispatch itself (the kernel's
-// own timestamps, hipExtLaunchKernelGGL) instead of as marker packets
-// recorded around it, which would idle the stream between the kernels.
-template <typename... Args, typename F = void (*)(Args...)>
-void launch_timed(int k, F f, dim3 grid, dim3 block, size_t shmem, hipStream_t s, Args... args) {
-    if (g_prof.on && (g_prof.mask >> k & 1u)) {
-        hipEvent_t a = g_prof.get(), b = a ? g_prof.get() : nullptr;
-        if (a && b) {
-            hipExtLaunchKernelGGL(f, grid, block, (std::uint32_t)shmem, s, a, b, 0u, args...);
-            g_prof.recs.push_back({k, a, b});
-            return;
-        }
-        if (a) g_prof.pool.push_back(a);
-    }
-    hipLaunchKernelGGL(f, grid, block, shmem, s, args...);
-}
-
 constexpr int COL_CT = 16;   // z-columns per block of the column kernels
 constexpr int KMAX = 8;      // butterflies per thread per FFT stage
 
-}  // namespace
-
-struct cpwgpu_plan_s {
-    FftGeom g{};
-    int mtxd = 0, ng = 0, nanl = 0;
-    int kdmax[3] = {0, 0, 0};
-    double inv_n = 1.0;
-    size_t ntot = 0;          // id*n2*n3
-    int mwrk = 0;
-    // host copies used to recognise an unchanged k-point in the drop-in
-    std::vector<long> key_pts;
-    std::vector<double> h_ekpg;
-    // device arrays
-    DevBuf col_ptr, col_uy, ent_i, ent_cz, ekpg, tw[3];
-    DevBuf zmap;              // [col][z] -> psi row or -1 (register column kernels)
-    DevBuf v64, v32;          // V(r) in FP64 and FP32
-    double v0 = 0.0;          // mean of V(r) over the mesh = V(G=0), the local part of diag(H)
-    DevBuf anl64, anl32, xnl; // projectors
-    long lda = 0;             // leading dimension of anl64
-    long lda32 = 0;           // of anl32: lda rounded up to even (16-byte aligned rows)
-    bool anl32_valid = false;
-    // plane-stage kernel per precision (index 0 FP64, 1 FP32): -1 = default for
-    // the mesh, else a variant number (set by the tuner or by the caller)
-    int plane_var[2] = {-1, -1};
-    // column kernels: 0 LDS lines, 1 register lines; -1 default
-    int col_var[2] = {-1, -1};
-    // stream schedule of the two-stream apply: 0 (default) the whole
-    // non-local term beside the local one, the gather adding to it; 1 the
-    // projection beside the local term, the back-projection after the gather
-    int sched_var[2] = {-1, -1};
-    // split-K target blocks of the projection GEMM per precision (-1 = 256)
-    int splitk[2] = {-1, -1};
-    // projection GEMM kernel per precision: 0 LDS-staged k_proj, 1 k_proj_direct
-    // (-1 = default)
-    int proj_var[2] = {-1, -1};
-    // back-projection GEMM kernel per precision: 0 LDS-staged k_back, 1
-    // k_back_direct (-1 = default)
-    int back_var[2] = {-1, -1};
-    // where the kinetic term ekpg*psi is added when the non-local term is on:
-    // 0 the back-projection epilogue, 1 the gather of the forward column kernel
-    // (-1 = default, 0)
-    int kin_var[2] = {-1, -1};
-    // plane kernel of the coupled two-component case (nsp = 4): 0 LDS
-    // two-pass, 1 register lines (-1 = default)
-    int spin_var[2] = {-1, -1};
-    // workspaces
-    DevBuf colbuf, part, dhd;
-    DevBuf gw;                // g_j of each plane wave as doubles [3][mtxd] (force projections)
-    // spinor path (hk_psi_spin_c16): potential components in the layout of
-    // k_spin_potential, projectors on the 2*mtxd interleaved rows, split bands
-    int nsp = 0;
-    DevBuf vsp64, vsp32;
-    DevBuf sanl64, sanl32, sxnl;
-    long slda = 0, slda32 = 0;
-    int snanl = 0;
-    bool sanl32_valid = false;
-    DevBuf spsi, shpsi;
-    ~cpwgpu_plan_s() {
-        col_ptr.release(); col_uy.release(); ent_i.release(); ent_cz.release(); ekpg.release();
-        for (auto &t : tw) t.release();
-        v64.release(); v32.release(); anl64.release(); anl32.release(); xnl.release();
-        colbuf.release(); part.release(); dhd.release(); gw.release();
-        vsp64.release(); vsp32.release(); sanl64.release(); sanl32.release(); sxnl.release();
-        spsi.release(); shpsi.release();
-    }
-};
-
-namespace {
 
 // lines of the G list of each plane wave, wrapped into the mesh
 // (Src/hk_psi/reference/hk_psi_c16.f90:143-158)
@@ -372,246 +207,12 @@ int plane_rows(const FftGeom &g, size_t cs, size_t *bytes) {
     return rb;
 }
 
-// ---- specialised kernels: mesh lengths with a two-pass split ---------------
-#define CPW_FAST_SIZES(X) X(24) X(48) X(64) X(72) X(80) X(96) X(108) X(128)
-
-enum LocalStage { ST_COL_BWD, ST_PLANE, ST_COL_FWD };
-
-struct LocalArgs {
-    const double2 *psi;
-    long ldp;
-    double2 *hpsi;
-    long ldh;
-    int nb;
-    int mode;  // COLF_ACC / COLF_KIN: what the gather adds to local/N
-};
-
-template <typename R, int N>
-int launch_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, int stage,
-                hipStream_t s) {
-    const FftGeom &g = p->g;
-    constexpr int CT = col_tile<N>();
-    const int ntiles = (g.ncol + CT - 1) / CT;
-    const dim3 grid(8 * ((a.nb + 7) / 8) * ntiles);
-    if (stage == ST_COL_BWD) {
-        launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, colbuf,
-                           (const int *)p->col_ptr.p, (const int *)p->ent_i.p,
-                           (const int *)p->ent_cz.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb);
-    } else if (stage == ST_COL_FWD) {
-        launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, a.hpsi, a.ldh,
-                           (const cplx<R> *)colbuf, (const int *)p->col_ptr.p,
-                           (const int *)p->ent_i.p, (const int *)p->ent_cz.p,
-                           (const double *)p->ekpg.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb,
-                           p->inv_n, a.mode);
-    } else {
-        const size_t dyn =
-            sizeof(cplx<R>) * ((size_t)N * plane_sub_stride(g.nx) + (size_t)plane_rows_fast<N>() * row_stride<N>());
-        const size_t stat = sizeof(cplx<R>) * 2 * N;
-        if (dyn + stat > 160 * 1024)
-            return fail(CPWGPU_ERR_SIZE, "plane of %d x %d does not fit in LDS", N, N);
-        static bool attr = false;
-        if (!attr) {
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_fast<R, N, N>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)(160 * 1024 - stat)));
-            attr = true;
-        }
-        launch_timed(CPWGPU_K_PLANE, (k_plane_fast<R, N, N>), dim3(g.n[2] * a.nb), dim3(FT), dyn, s, colbuf,
-                           (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p,
-                           (const double2 *)p->tw[1].p, g);
-    }
-    HIPCHK(hipGetLastError());
-    return CPWGPU_OK;
-}
-
-// ---- plane stage variants ---------------------------------------------------
-// 0: k_plane_fast (LDS two-pass lines); 4..6: k_plane_wave (LDS two-pass
-// lines, wave-local exchanges) with 256, 192 and 128 threads per block; the
-// others: k_plane_reg shapes (x lanes GX, y lanes GY, planes per block P,
-// threads T, waves per SIMD W, y lines through the LDS wave transform YW,
-// box pruning PR) per precision.
-struct RegShapeT {
-    int GX, GY, P, T, W;
-    bool YW, PR;
-};
-template <typename R> constexpr RegShapeT reg_shape(int v);
-template <> constexpr RegShapeT reg_shape<float>(int v) {
-    // 1-3 spill-free at 72: 67, 74 and 127 VGPRs
-    return v == 1 ? RegShapeT{8, 8, 1, 256, 5, false, false}
-         : v == 2 ? RegShapeT{8, 8, 2, 256, 4, false, false}
-         : v == 3 ? RegShapeT{4, 4, 1, 256, 3, false, false}
-         : v == 7 ? RegShapeT{8, 8, 1, 256, 5, true, false}
-         : v == 8 ? RegShapeT{2, 2, 1, 256, 3, true, true}
-         : v == 9 ? RegShapeT{4, 4, 1, 256, 4, true, true}
-         : v == 10 ? RegShapeT{8, 8, 1, 256, 5, true, true}
-         : v == 11 ? RegShapeT{2, 4, 1, 256, 3, false, true}
-                   : RegShapeT{0, 0, 0, 0, 0, false, false};
-}
-template <> constexpr RegShapeT reg_shape<double>(int v) {
-    return v == 1 ? RegShapeT{8, 8, 1, 256, 3, false, false}
-         : v == 2 ? RegShapeT{8, 8, 1, 320, 4, false, false}
-         : v == 3 ? RegShapeT{4, 8, 1, 256, 3, false, false}
-         : v == 7 ? RegShapeT{8, 8, 1, 256, 3, true, false}
-         : v == 8 ? RegShapeT{4, 4, 1, 256, 3, true, true}
-         : v == 9 ? RegShapeT{8, 8, 1, 256, 3, true, true}
-         : v == 10 ? RegShapeT{4, 4, 1, 256, 3, false, true}
-         : v == 11 ? RegShapeT{8, 8, 1, 256, 3, false, true}
-                   : RegShapeT{0, 0, 0, 0, 0, false, false};
-}
-constexpr int NPLANE_VAR = 12;
-constexpr int WAVE_T[3] = {256, 192, 128};
-constexpr bool is_reg_variant(int v) { return (v >= 1 && v <= 3) || (v >= 7 && v < NPLANE_VAR); }
 // back-projection kernels: 0 LDS-staged, 1..NBACK_DIRECT direct, NBACK_DIRECT+1 LDS-staged with half chunks
 constexpr int NBACK_VAR = NBACK_DIRECT + 2;
 // projection kernels: 0 LDS-staged, 1..NPROJ_DIRECT direct, NPROJ_DIRECT+1 LDS-staged with half wave tiles
 constexpr int NPROJ_VAR = NPROJ_DIRECT + 2;
 template <typename R> constexpr int proj_half_wm() { return GemmCfg<R>::WM / 2; }
 template <typename R> constexpr int proj_half_wn() { return GemmCfg<R>::WN > 1 ? GemmCfg<R>::WN / 2 : 1; }
-
-// a register shape is built for a mesh length when both splits divide N and a
-// lane holds at most 288 bytes of one line
-template <typename R, int N, int GX, int GY> constexpr bool reg_ok() {
-    return GX > 0 && GY > 0 && N % GX == 0 && N % GY == 0 && first_factor(N / GX) <= 5 &&
-           first_factor(N / GY) <= 5 && 2 * sizeof(R) * (N / GX) <= 288 && 2 * sizeof(R) * (N / GY) <= 288 &&
-           N / GX <= 64 && N / GY <= 64;
-}
-template <typename R, int N> constexpr bool reg_var_ok(int v) {
-#define CPW_RV(V) (v == V && reg_ok<R, N, reg_shape<R>(V).GX, reg_shape<R>(V).GY>())
-    return CPW_RV(1) || CPW_RV(2) || CPW_RV(3) || CPW_RV(7) || CPW_RV(8) || CPW_RV(9) || CPW_RV(10) ||
-           CPW_RV(11);
-#undef CPW_RV
-}
-// a pruned shape needs the sphere box inside |x|, |y| <= N/4 (true on the
-// meshes size_fft chooses for the density, n >= 4 kd + 1)
-inline bool prune_fits(const FftGeom &g) { return 4 * g.kd[0] <= g.n[0] && 4 * g.kd[1] <= g.n[1]; }
-
-// LDS row stride of the register variant's sub-plane for nx box columns
-inline int reg_stride(int nx) { return plane_sub_stride(nx); }
-
-template <typename R, int N, int V>
-int launch_plane_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr,
-                     hipStream_t s) {
-    constexpr RegShapeT SH = reg_shape<R>(V);
-    constexpr int GX = SH.GX, GY = SH.GY, P = SH.P, T = SH.T, W = SH.W;
-    constexpr bool YW = SH.YW, PR = SH.PR;
-    if constexpr (!reg_ok<R, N, GX, GY>()) {
-        return fail(CPWGPU_ERR_MODE, "plane variant %d is not built for N = %d", V, N);
-    } else {
-        const FftGeom &g = p->g;
-        if (PR && !prune_fits(g))
-            return fail(CPWGPU_ERR_MODE, "plane variant %d needs the sphere box inside N/4", V);
-        // pruned shapes use their compile-time row stride (the box has at
-        // most N/2 + 1 columns there)
-        const int S = PR ? pr_sub_stride<N>() : reg_stride(g.nx);
-        if (reg_stride(g.nx) > S)
-            return fail(CPWGPU_ERR_MODE, "plane variant %d: %d box columns exceed its row stride", V, g.nx);
-        const size_t dyn = plane_reg_lds<R, N, P>(S);
-        if (dyn > 160 * 1024)
-            return fail(CPWGPU_ERR_SIZE, "plane variant %d: %zu bytes of LDS", V, dyn);
-        static bool attr = false;
-        if (!attr) {
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            attr = true;
-        }
-        launch_timed(CPWGPU_K_PLANE, k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
-                     dim3(((a.nb + P - 1) / P) * g.n[2]), dim3(T), dyn, s, colbuf,
-                     (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, g, a.nb, S);
-        HIPCHK(hipGetLastError());
-        return CPWGPU_OK;
-    }
-}
-
-template <typename R, int N, int T>
-int launch_plane_wave(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
-    const FftGeom &g = p->g;
-    const size_t dyn = plane_wave_lds<R, N, T>(g.nx);
-    const size_t stat = sizeof(cplx<R>) * 2 * N;
-    if (dyn + stat > 160 * 1024)
-        return fail(CPWGPU_ERR_SIZE, "plane of %d x %d does not fit in LDS with %d threads", N, N, T);
-    static bool attr = false;
-    if (!attr) {
-        HIPCHK(hipFuncSetAttribute((const void *)k_plane_wave<R, N, N, T, 2>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024 - stat)));
-        attr = true;
-    }
-    launch_timed(CPWGPU_K_PLANE, (k_plane_wave<R, N, N, T, 2>), dim3(g.n[2] * a.nb), dim3(T), dyn, s, colbuf,
-                       (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, (const double2 *)p->tw[1].p, g);
-    HIPCHK(hipGetLastError());
-    return CPWGPU_OK;
-}
-
-// ---- register column kernels -------------------------------------------------
-// lanes per z column: 8 where the column fits in registers, else 4
-template <typename R, int N> constexpr int col_reg_g() {
-    return reg_ok<R, N, 8, 8>() ? 8 : reg_ok<R, N, 4, 4>() ? 4 : 0;
-}
-template <typename R, int N> constexpr bool col_reg_built() { return col_reg_g<R, N>() > 0; }
-// the sphere box inside |z| <= N3/4: the pruned register column kernels
-inline bool col_prune_fits(const FftGeom &g) { return 4 * g.kd[2] <= g.n[2]; }
-
-template <typename R, int N>
-int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int stage, hipStream_t s) {
-    constexpr int G = col_reg_g<R, N>();
-    if constexpr (G == 0) {
-        return fail(CPWGPU_ERR_MODE, "register column kernels are not built for N = %d", N);
-    } else {
-        const FftGeom &g = p->g;
-        constexpr int CPB = COLR_T / G;
-        const int ntiles = (g.ncol + CPB - 1) / CPB;
-        const dim3 grid(8 * ((a.nb + 7) / 8) * ntiles);
-        const bool pr = col_prune_fits(g);
-        const double2 *tw3 = (const double2 *)p->tw[2].p;
-        const int *zm = (const int *)p->zmap.p;
-        if (stage == ST_COL_BWD) {
-            if (pr)
-                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
-                                   zm, tw3, g, ntiles, a.nb);
-            else
-                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
-                                   zm, tw3, g, ntiles, a.nb);
-        } else {
-            if (pr)
-                launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
-                                   a.ldh, (const cplx<R> *)colbuf, zm, (const double *)p->ekpg.p, tw3, g, ntiles,
-                                   a.nb, p->inv_n, a.mode);
-            else
-                launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
-                                   a.ldh, (const cplx<R> *)colbuf, zm, (const double *)p->ekpg.p, tw3, g, ntiles,
-                                   a.nb, p->inv_n, a.mode);
-        }
-        HIPCHK(hipGetLastError());
-        return CPWGPU_OK;
-    }
-}
-
-// whether the wave-exchange variant v (4..6) fits in LDS for nx box columns
-template <typename R, int N> bool plane_wave_fits(int v, int nx) {
-    const size_t stat = sizeof(cplx<R>) * 2 * N;
-    const size_t dyn = v == 4 ? plane_wave_lds<R, N, WAVE_T[0]>(nx)
-                       : v == 5 ? plane_wave_lds<R, N, WAVE_T[1]>(nx) : plane_wave_lds<R, N, WAVE_T[2]>(nx);
-    return dyn + stat <= 160 * 1024;
-}
-
-template <typename R, int N> constexpr bool plane_var_ok(int v) {
-    return v == 0 || (v >= 4 && v <= 6) || reg_var_ok<R, N>(v);
-}
-
-// default plane variant of a mesh length
-template <typename R, int N> constexpr int plane_var_default() { return 0; }
-
-template <typename R, int N>
-int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
-    int v = p->plane_var[sizeof(R) == 4 ? 1 : 0];
-    if (v < 0 || !plane_var_ok<R, N>(v)) v = plane_var_default<R, N>();
-#define CPW_LR(V) if (v == V) return launch_plane_reg<R, N, V>(p, a, colbuf, vr, s);
-    CPW_LR(1) CPW_LR(2) CPW_LR(3) CPW_LR(7) CPW_LR(8) CPW_LR(9) CPW_LR(10) CPW_LR(11)
-#undef CPW_LR
-    if (v == 4) return launch_plane_wave<R, N, WAVE_T[0]>(p, a, colbuf, vr, s);
-    if (v == 5) return launch_plane_wave<R, N, WAVE_T[1]>(p, a, colbuf, vr, s);
-    if (v == 6) return launch_plane_wave<R, N, WAVE_T[2]>(p, a, colbuf, vr, s);
-    return launch_fast<R, N>(p, a, colbuf, vr, ST_PLANE, s);
-}
 
 bool fast_sizes(const FftGeom &g) {
     bool col_ok = false, plane_ok = false;
@@ -672,7 +273,7 @@ int local_stage(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *
             const bool reg = col_var_resolve<R>(p, p->col_var[sizeof(R) == 4 ? 1 : 0], nullptr) == 1;
 #define CPW_CO(N)                                                                \
     if (g.n[2] == N)                                                             \
-        st = reg ? launch_col_reg<R, N>(p, a, colbuf, stage, s) : launch_fast<R, N>(p, a, colbuf, vr, stage, s);
+        st = reg ? launch_col_reg<R, N>(p, a, colbuf, stage, s) : launch_col_fast<R, N>(p, a, colbuf, stage, s);
             CPW_FAST_SIZES(CPW_CO)
 #undef CPW_CO
         }
@@ -1308,17 +909,6 @@ int set_projectors_spin_host(cpwgpu_plan_s *p, const double *anlsp, const double
     return st;
 }
 
-// register shape of the coupled two-component plane kernel: (x lanes, y
-// lanes, threads, waves per SIMD); both components' rows live in registers.
-// FP64: the two sub-planes (about 86 KB at 72) allow one block per CU, so the
-// block has 512 threads for 2 waves per SIMD (184 VGPRs fit that budget).
-template <typename R> struct SpinShape;
-template <> struct SpinShape<float> { static constexpr int GX = 8, GY = 8, T = 256, W = 3; };
-template <> struct SpinShape<double> { static constexpr int GX = 8, GY = 8, T = 512, W = 2; };
-template <typename R, int N> constexpr bool spin_reg_ok() {
-    return reg_ok<R, N, SpinShape<R>::GX, SpinShape<R>::GY>();
-}
-
 // whether the register variant of the coupled plane kernel is built for the
 // plan's mesh
 template <typename R> bool spin_reg_built(const cpwgpu_plan_s *p) {
@@ -1337,61 +927,6 @@ template <typename R> int spin_var_resolve(const cpwgpu_plan_s *p) {
     // measured on the 64-atom cell (64 spinor bands): register lines 11-12%
     // faster than the LDS two-pass kernel in both precisions
     return v < 0 ? 1 : v;
-}
-
-template <typename R, int N>
-int launch_plane_spin_reg(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair,
-                          hipStream_t s) {
-    constexpr int GX = SpinShape<R>::GX, GY = SpinShape<R>::GY, T = SpinShape<R>::T, W = SpinShape<R>::W;
-    if constexpr (!spin_reg_ok<R, N>()) {
-        return fail(CPWGPU_ERR_MODE, "register two-component plane kernel is not built for N = %d", N);
-    } else {
-        const FftGeom &g = p->g;
-        // a box inside N/4: the compile-time row stride
-        const bool cs = prune_fits(g);
-        const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
-        const size_t dyn = sizeof(cplx<R>) * ((size_t)N + 2 * (size_t)N * S);
-        if (dyn > 160 * 1024)
-            return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
-        static bool attr = false;
-        if (!attr) {
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, true>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            attr = true;
-        }
-        if (cs)
-            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, true>), dim3(g.n[2] * npair), dim3(T), dyn, s,
-                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
-        else
-            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, false>), dim3(g.n[2] * npair), dim3(T), dyn, s,
-                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
-        HIPCHK(hipGetLastError());
-        return CPWGPU_OK;
-    }
-}
-
-template <typename R, int N>
-int launch_plane_spin(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair, hipStream_t s) {
-    if (spin_var_resolve<R>(p) == 1) return launch_plane_spin_reg<R, N>(p, colbuf, vr, vstride, npair, s);
-    const FftGeom &g = p->g;
-    const size_t dyn = sizeof(cplx<R>) * (2 * (size_t)N * plane_sub_stride(g.nx) +
-                                          (size_t)plane_rows_fast<N>() * row_stride<N>());
-    const size_t stat = sizeof(cplx<R>) * 2 * N;
-    if (dyn + stat > 160 * 1024)
-        return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
-    static bool attr = false;
-    if (!attr) {
-        HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin<R, N, N>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(160 * 1024 - stat)));
-        attr = true;
-    }
-    launch_timed(CPWGPU_K_PLANE, (k_plane_spin<R, N, N>), dim3(g.n[2] * npair), dim3(FT), dyn, s, colbuf,
-                       (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p,
-                       (const double2 *)p->tw[1].p, g, npair);
-    HIPCHK(hipGetLastError());
-    return CPWGPU_OK;
 }
 
 // H psi_sp for neig two-component bands (rows 2i / 2i+1 = up / down of plane
@@ -1461,7 +996,7 @@ int apply_spin(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, double2
             if ((st = columns(ST_COL_BWD, n0, np_, colbuf)) || (st = columns(ST_COL_BWD, neig + n0, np_, cb_dn)))
                 return st;
             st = CPWGPU_ERR_SIZE;
-#define CPW_SPL(N) if (g.n[0] == N) st = launch_plane_spin<R, N>(p, colbuf, vr, ntot, np_, s);
+#define CPW_SPL(N) if (g.n[0] == N) st = launch_plane_spin<R, N>(p, colbuf, vr, ntot, np_, spin_var_resolve<R>(p), s);
             CPW_FAST_SIZES(CPW_SPL)
 #undef CPW_SPL
             if (st) return st;
@@ -2255,71 +1790,6 @@ int plan_ditsp(cpwgpu_plan_s *p, int prec, int icmax, int iguess, double epspsi,
 struct ForceWs {
     DevBuf t2, t2s, rho, qv, fq, rat, species, patom, occ, fl, fnl, enl, p, rhor;
 } g_fw;
-
-// register shape of the density pass: x lanes, y lanes, waves per SIMD
-constexpr int DEN_GX = 8, DEN_GY = 8, DEN_W = 3;
-// threads of the register density pass for line length N: the smallest of 256,
-// 320 and 384 that keeps a lane's row accumulators (rows per x task x N / GX
-// doubles) within 27, for lines of at most 10 values per lane: spill-free at 3
-// waves per SIMD (24-72: 256, 80: 320); 0 = not built (96 and 128 spill, 108 has
-// no 8-lane split: k_density_fast)
-template <int N> constexpr int den_threads() {
-    if (!reg_ok<double, N, DEN_GX, DEN_GY>() || N / DEN_GX > 10) return 0;
-    for (int t : {256, 320, 384})
-        if (((N + t / DEN_GX - 1) / (t / DEN_GX)) * (N / DEN_GX) <= 27) return t;
-    return 0;
-}
-template <int N> constexpr bool den_reg_ok() { return den_threads<N>() > 0; }
-
-template <int N>
-int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg,
-                   int ngrp, int Q1, int Q2, double2 *t2, hipStream_t s, double *rhor = nullptr) {
-    const FftGeom &g = p->g;
-    if constexpr (den_reg_ok<N>()) {
-        if (rhor) {
-            // the density planes alone: register lines, accumulation in registers
-            constexpr int DT = den_threads<N>();
-            // a box inside N/4: the compile-time row stride
-            const bool cs = prune_fits(g);
-            const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
-            const size_t dyn = 16 * ((size_t)N + (size_t)N * S);
-            if (dyn > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
-            static bool attr_r = false;
-            if (!attr_r) {
-                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                attr_r = true;
-            }
-            if (cs)
-                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>), dim3(g.n[2] * ngrp),
-                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
-                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
-            else
-                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>), dim3(g.n[2] * ngrp),
-                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
-                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
-            HIPCHK(hipGetLastError());
-            return CPWGPU_OK;
-        }
-    }
-    constexpr int RB = plane_rows_fast<N>();
-    const size_t dyn = 16 * ((size_t)N * (g.nx | 1) + (size_t)RB * row_stride<N>()) + 8 * (size_t)N * N;
-    const size_t stat = 16 * 2 * (size_t)N;
-    if (dyn + stat > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
-    static bool attr = false;
-    if (!attr) {
-        HIPCHK(hipFuncSetAttribute((const void *)k_density_fast<N, N>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024 - stat)));
-        attr = true;
-    }
-    hipLaunchKernelGGL((k_density_fast<N, N>), dim3(g.n[2] * ngrp), dim3(FT), dyn, s, colbuf,
-                       (const int *)p->col_uy.p, occ, (const double2 *)p->tw[0].p,
-                       (const double2 *)p->tw[1].p, g, nb, bpg, Q1, Q2, t2, rhor);
-    HIPCHK(hipGetLastError());
-    return CPWGPU_OK;
-}
 
 // Electron density on the mesh, the band loop of Src/omp/charge_by_fft.f90:170-197:
 // rho(r) = sum_n occ_n |psi_n(r)|^2, psi_n(r) the unnormalised G -> r transform.

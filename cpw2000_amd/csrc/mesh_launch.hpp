@@ -1,0 +1,260 @@
+// Bodies of the per-length launchers declared in mesh.hpp.
+#pragma once
+
+#include "mesh.hpp"
+#include "density.hpp"
+#include "spin_plane.hpp"
+
+namespace cpwgpu {
+
+template <typename R, int N>
+int launch_col_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int stage, hipStream_t s) {
+    const FftGeom &g = p->g;
+    constexpr int CT = col_tile<N>();
+    const int ntiles = (g.ncol + CT - 1) / CT;
+    const dim3 grid(8 * ((a.nb + 7) / 8) * ntiles);
+    if (stage == ST_COL_BWD) {
+        launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, colbuf,
+                           (const int *)p->col_ptr.p, (const int *)p->ent_i.p,
+                           (const int *)p->ent_cz.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb);
+    } else {
+        launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, a.hpsi, a.ldh,
+                           (const cplx<R> *)colbuf, (const int *)p->col_ptr.p,
+                           (const int *)p->ent_i.p, (const int *)p->ent_cz.p,
+                           (const double *)p->ekpg.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb,
+                           p->inv_n, a.mode);
+    }
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+template <typename R, int N>
+int launch_plane_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
+    const FftGeom &g = p->g;
+    const size_t dyn =
+        sizeof(cplx<R>) * ((size_t)N * plane_sub_stride(g.nx) + (size_t)plane_rows_fast<N>() * row_stride<N>());
+    const size_t stat = sizeof(cplx<R>) * 2 * N;
+    if (dyn + stat > 160 * 1024)
+        return fail(CPWGPU_ERR_SIZE, "plane of %d x %d does not fit in LDS", N, N);
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_plane_fast<R, N, N>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)(160 * 1024 - stat)));
+        attr = true;
+    }
+    launch_timed(CPWGPU_K_PLANE, (k_plane_fast<R, N, N>), dim3(g.n[2] * a.nb), dim3(FT), dyn, s, colbuf,
+                       (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p,
+                       (const double2 *)p->tw[1].p, g);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+template <typename R, int N, int V>
+int launch_plane_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr,
+                     hipStream_t s) {
+    constexpr RegShapeT SH = reg_shape<R>(V);
+    constexpr int GX = SH.GX, GY = SH.GY, P = SH.P, T = SH.T, W = SH.W;
+    constexpr bool YW = SH.YW, PR = SH.PR;
+    if constexpr (!reg_ok<R, N, GX, GY>()) {
+        return fail(CPWGPU_ERR_MODE, "plane variant %d is not built for N = %d", V, N);
+    } else {
+        const FftGeom &g = p->g;
+        if (PR && !prune_fits(g))
+            return fail(CPWGPU_ERR_MODE, "plane variant %d needs the sphere box inside N/4", V);
+        // pruned shapes use their compile-time row stride (the box has at
+        // most N/2 + 1 columns there)
+        const int S = PR ? pr_sub_stride<N>() : reg_stride(g.nx);
+        if (reg_stride(g.nx) > S)
+            return fail(CPWGPU_ERR_MODE, "plane variant %d: %d box columns exceed its row stride", V, g.nx);
+        const size_t dyn = plane_reg_lds<R, N, P>(S);
+        if (dyn > 160 * 1024)
+            return fail(CPWGPU_ERR_SIZE, "plane variant %d: %zu bytes of LDS", V, dyn);
+        static bool attr = false;
+        if (!attr) {
+            HIPCHK(hipFuncSetAttribute((const void *)k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            attr = true;
+        }
+        launch_timed(CPWGPU_K_PLANE, k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
+                     dim3(((a.nb + P - 1) / P) * g.n[2]), dim3(T), dyn, s, colbuf,
+                     (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, g, a.nb, S);
+        HIPCHK(hipGetLastError());
+        return CPWGPU_OK;
+    }
+}
+
+template <typename R, int N, int T>
+int launch_plane_wave(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
+    const FftGeom &g = p->g;
+    const size_t dyn = plane_wave_lds<R, N, T>(g.nx);
+    const size_t stat = sizeof(cplx<R>) * 2 * N;
+    if (dyn + stat > 160 * 1024)
+        return fail(CPWGPU_ERR_SIZE, "plane of %d x %d does not fit in LDS with %d threads", N, N, T);
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_plane_wave<R, N, N, T, 2>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024 - stat)));
+        attr = true;
+    }
+    launch_timed(CPWGPU_K_PLANE, (k_plane_wave<R, N, N, T, 2>), dim3(g.n[2] * a.nb), dim3(T), dyn, s, colbuf,
+                       (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, (const double2 *)p->tw[1].p, g);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+template <typename R, int N>
+int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int stage, hipStream_t s) {
+    constexpr int G = col_reg_g<R, N>();
+    if constexpr (G == 0) {
+        return fail(CPWGPU_ERR_MODE, "register column kernels are not built for N = %d", N);
+    } else {
+        const FftGeom &g = p->g;
+        constexpr int CPB = COLR_T / G;
+        const int ntiles = (g.ncol + CPB - 1) / CPB;
+        const dim3 grid(8 * ((a.nb + 7) / 8) * ntiles);
+        const bool pr = col_prune_fits(g);
+        const double2 *tw3 = (const double2 *)p->tw[2].p;
+        const int *zm = (const int *)p->zmap.p;
+        if (stage == ST_COL_BWD) {
+            if (pr)
+                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
+                                   zm, tw3, g, ntiles, a.nb);
+            else
+                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
+                                   zm, tw3, g, ntiles, a.nb);
+        } else {
+            if (pr)
+                launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
+                                   a.ldh, (const cplx<R> *)colbuf, zm, (const double *)p->ekpg.p, tw3, g, ntiles,
+                                   a.nb, p->inv_n, a.mode);
+            else
+                launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
+                                   a.ldh, (const cplx<R> *)colbuf, zm, (const double *)p->ekpg.p, tw3, g, ntiles,
+                                   a.nb, p->inv_n, a.mode);
+        }
+        HIPCHK(hipGetLastError());
+        return CPWGPU_OK;
+    }
+}
+
+template <typename R, int N>
+int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
+    int v = p->plane_var[sizeof(R) == 4 ? 1 : 0];
+    if (v < 0 || !plane_var_ok<R, N>(v)) v = plane_var_default<R, N>();
+#define CPW_LR(V) if (v == V) return launch_plane_reg<R, N, V>(p, a, colbuf, vr, s);
+    CPW_LR(1) CPW_LR(2) CPW_LR(3) CPW_LR(7) CPW_LR(8) CPW_LR(9) CPW_LR(10) CPW_LR(11)
+#undef CPW_LR
+    if (v == 4) return launch_plane_wave<R, N, WAVE_T[0]>(p, a, colbuf, vr, s);
+    if (v == 5) return launch_plane_wave<R, N, WAVE_T[1]>(p, a, colbuf, vr, s);
+    if (v == 6) return launch_plane_wave<R, N, WAVE_T[2]>(p, a, colbuf, vr, s);
+    return launch_plane_fast<R, N>(p, a, colbuf, vr, s);
+}
+
+template <typename R, int N>
+int launch_plane_spin_reg(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair,
+                          hipStream_t s) {
+    constexpr int GX = SpinShape<R>::GX, GY = SpinShape<R>::GY, T = SpinShape<R>::T, W = SpinShape<R>::W;
+    if constexpr (!spin_reg_ok<R, N>()) {
+        return fail(CPWGPU_ERR_MODE, "register two-component plane kernel is not built for N = %d", N);
+    } else {
+        const FftGeom &g = p->g;
+        // a box inside N/4: the compile-time row stride
+        const bool cs = prune_fits(g);
+        const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
+        const size_t dyn = sizeof(cplx<R>) * ((size_t)N + 2 * (size_t)N * S);
+        if (dyn > 160 * 1024)
+            return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
+        static bool attr = false;
+        if (!attr) {
+            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, false>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, true>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            attr = true;
+        }
+        if (cs)
+            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, true>), dim3(g.n[2] * npair), dim3(T), dyn, s,
+                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
+        else
+            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, false>), dim3(g.n[2] * npair), dim3(T), dyn, s,
+                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
+        HIPCHK(hipGetLastError());
+        return CPWGPU_OK;
+    }
+}
+
+template <typename R, int N>
+int launch_plane_spin(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair, int var,
+                      hipStream_t s) {
+    if (var == 1) return launch_plane_spin_reg<R, N>(p, colbuf, vr, vstride, npair, s);
+    const FftGeom &g = p->g;
+    const size_t dyn = sizeof(cplx<R>) * (2 * (size_t)N * plane_sub_stride(g.nx) +
+                                          (size_t)plane_rows_fast<N>() * row_stride<N>());
+    const size_t stat = sizeof(cplx<R>) * 2 * N;
+    if (dyn + stat > 160 * 1024)
+        return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin<R, N, N>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)(160 * 1024 - stat)));
+        attr = true;
+    }
+    launch_timed(CPWGPU_K_PLANE, (k_plane_spin<R, N, N>), dim3(g.n[2] * npair), dim3(FT), dyn, s, colbuf,
+                       (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p,
+                       (const double2 *)p->tw[1].p, g, npair);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+template <int N>
+int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg,
+                   int ngrp, int Q1, int Q2, double2 *t2, hipStream_t s, double *rhor) {
+    const FftGeom &g = p->g;
+    if constexpr (den_reg_ok<N>()) {
+        if (rhor) {
+            // the density planes alone: register lines, accumulation in registers
+            constexpr int DT = den_threads<N>();
+            // a box inside N/4: the compile-time row stride
+            const bool cs = prune_fits(g);
+            const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
+            const size_t dyn = 16 * ((size_t)N + (size_t)N * S);
+            if (dyn > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
+            static bool attr_r = false;
+            if (!attr_r) {
+                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                attr_r = true;
+            }
+            if (cs)
+                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>), dim3(g.n[2] * ngrp),
+                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
+                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
+            else
+                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>), dim3(g.n[2] * ngrp),
+                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
+                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
+            HIPCHK(hipGetLastError());
+            return CPWGPU_OK;
+        }
+    }
+    constexpr int RB = plane_rows_fast<N>();
+    const size_t dyn = 16 * ((size_t)N * (g.nx | 1) + (size_t)RB * row_stride<N>()) + 8 * (size_t)N * N;
+    const size_t stat = 16 * 2 * (size_t)N;
+    if (dyn + stat > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_density_fast<N, N>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024 - stat)));
+        attr = true;
+    }
+    hipLaunchKernelGGL((k_density_fast<N, N>), dim3(g.n[2] * ngrp), dim3(FT), dyn, s, colbuf,
+                       (const int *)p->col_uy.p, occ, (const double2 *)p->tw[0].p,
+                       (const double2 *)p->tw[1].p, g, nb, bpg, Q1, Q2, t2, rhor);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+}  // namespace cpwgpu
