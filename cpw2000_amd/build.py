@@ -42,10 +42,10 @@ def _run(cmd):
     subprocess.run(cmd, check=True)
 
 
-def mesh_lengths():
-    """The specialised mesh lengths (CPW_FAST_SIZES of csrc/mesh.hpp)."""
+def mesh_lengths(which="CPW_FAST_SIZES"):
+    """The specialised mesh lengths (CPW_FAST_SIZES or CPW_FULL_SIZES of csrc/mesh.hpp)."""
     with open(os.path.join(CSRC, "mesh.hpp")) as f:
-        line = next(t for t in f if t.startswith("#define CPW_FAST_SIZES"))
+        line = next(t for t in f if t.startswith("#define " + which))
     return [int(n) for n in re.findall(r"X\((\d+)\)", line)]
 
 
@@ -54,7 +54,9 @@ def build_hip():
     # the rest (csrc/cpwgpu.hip); the longest compiles first
     os.makedirs(OBJ, exist_ok=True)
     jobs = [("cpwgpu.hip", "cpwgpu.o", [])]
-    jobs += [("mesh.hip", f"mesh{n}.o", [f"-DCPW_N={n}"]) for n in sorted(mesh_lengths(), reverse=True)]
+    full = mesh_lengths("CPW_FULL_SIZES")
+    jobs += [("mesh.hip", f"mesh{n}.o", [f"-DCPW_N={n}", f"-DCPW_N_FULL={int(n in full)}"])
+             for n in sorted(mesh_lengths(), key=lambda n: (n in full, n), reverse=True)]
     objs = [os.path.join(OBJ, o) for _, o, _ in jobs]
 
     def compile_one(job):

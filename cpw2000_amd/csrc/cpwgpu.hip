@@ -11,6 +11,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdarg>
 #include <cmath>
 #include <cstdio>
@@ -214,45 +215,66 @@ constexpr int NPROJ_VAR = NPROJ_DIRECT + 2;
 template <typename R> constexpr int proj_half_wm() { return GemmCfg<R>::WM / 2; }
 template <typename R> constexpr int proj_half_wn() { return GemmCfg<R>::WN > 1 ? GemmCfg<R>::WN / 2 : 1; }
 
-bool fast_sizes(const FftGeom &g) {
-    bool col_ok = false, plane_ok = false;
-#define CPW_HAS(N) col_ok |= g.n[2] == N; plane_ok |= (g.n[0] == N && g.n[1] == N);
+// column kernels specialised for n3
+bool col_fast(const FftGeom &g) {
+    bool ok = false;
+#define CPW_HAS(N) ok |= g.n[2] == N;
     CPW_FAST_SIZES(CPW_HAS)
 #undef CPW_HAS
-    return col_ok && plane_ok;
+    return ok;
+}
+// every kernel family specialised for the mesh
+bool full_sizes(const FftGeom &g) { return g.n[0] == g.n[1] && full_length(g.n[0]) && full_length(g.n[2]); }
+// Plane kernels specialised for n1 = n2.  Outside the fully specialised meshes
+// only the pruned register shapes are used, whose LDS holds any box inside N/4;
+// a wider box goes to the generic kernel, which fits larger ones.
+bool plane_fast(const FftGeom &g) {
+    if (full_sizes(g)) return true;
+    if (g.n[0] != g.n[1] || !prune_fits(g)) return false;
+    bool ok = false;
+#define CPW_HAS(N) ok |= g.n[0] == N;
+    CPW_FAST_SIZES(CPW_HAS)
+#undef CPW_HAS
+    return ok;
 }
 
 // plane variant the next apply uses (defaults resolved), and whether v is
-// built for the plan's mesh
+// built for the plan's mesh.  0 is the generic kernel where the mesh is not
+// fully specialised.
 template <typename R> int plane_var_resolve(const cpwgpu_plan_s *p, int v, bool *ok) {
     const FftGeom &g = p->g;
     *ok = v == 0 || v == -1;
-    if (!fast_sizes(g)) return 0;
+    if (!plane_fast(g)) return 0;
+    const bool full = full_sizes(g);
     int def = 0;
 #define CPW_PV(N)                                      \
     if (g.n[0] == N) {                                 \
-        def = plane_var_default<R, N>();               \
+        def = prune_fits(g) ? plane_var_default<R, N>() : 0; \
         if (v > 0)                                     \
-            *ok = v < NPLANE_VAR && plane_var_ok<R, N>(v) && (v < 4 || v > 6 || plane_wave_fits<R, N>(v, g.nx)) && \
-                  (!is_reg_variant(v) || !reg_shape<R>(v).PR || prune_fits(g)); \
+            *ok = v < NPLANE_VAR && plane_var_ok<R, N>(v) && \
+                  (v < 4 || v > 6 || (full && plane_wave_fits<R, N>(v, g.nx))) && \
+                  (!is_reg_variant(v) || !reg_shape<R, N>(v).PR || prune_fits(g)); \
     }
     CPW_FAST_SIZES(CPW_PV)
 #undef CPW_PV
     return v < 0 || !*ok ? def : v;
 }
 
-// column kernel the next apply uses (default resolved: 0, the LDS lines,
-// which measured as fast as the register lines in FP64 and faster in FP32 at
-// 72^3); *ok: whether v is usable (1 needs the register kernels built for n3)
-template <typename R> int col_var_resolve(const cpwgpu_plan_s *p, int v, bool *ok) {
+// Column kernel the next apply uses; *ok: whether v is usable (1, the register
+// lines, needs them built for n3).  Default: LDS lines in FP32 (inverse + forward
+// at 72, 128 bands: 24 + 50 us against 35 + 61); in FP64 register lines for the
+// forward columns (72: 62 against 65, 32x32x128, 72 bands: 15 against 19, 36, 20
+// bands: 5 against 8), for the inverse ones only up to 40 (36: 6.5 against 7.1;
+// 72: 38 against 37).  Choice 0 or 1 holds for both directions; the default is
+// reported for the forward one.
+template <typename R> int col_var_resolve(const cpwgpu_plan_s *p, int v, bool *ok, int stage = ST_COL_FWD) {
     const FftGeom &g = p->g;
     bool built = false;
-    if (fast_sizes(g)) {
 #define CPW_CB(N) if (g.n[2] == N) built = col_reg_built<R, N>();
-        CPW_FAST_SIZES(CPW_CB)
+    CPW_FAST_SIZES(CPW_CB)
 #undef CPW_CB
-    }
     if (ok) *ok = v <= 0 || (v == 1 && built);
+    if (v < 0) return built && sizeof(R) == 8 && (stage == ST_COL_FWD || g.n[2] <= 40) ? 1 : 0;
     return v == 1 && built ? 1 : 0;
 }
 
@@ -263,20 +285,24 @@ int local_stage(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *
                 hipStream_t s) {
     const FftGeom &g = p->g;
     const size_t cs = sizeof(cplx<R>);
-    if (fast_sizes(g)) {
-        int st = CPWGPU_OK;
-        if (stage == ST_PLANE) {
-#define CPW_PL(N) if (g.n[0] == N) st = launch_plane<R, N>(p, a, colbuf, vr, s);
+    if (stage == ST_PLANE) {
+        bool ok;
+        const int v = plane_var_resolve<R>(p, p->plane_var[sizeof(R) == 4 ? 1 : 0], &ok);
+        if (full_sizes(g) || v > 0) {
+            int st = CPWGPU_OK;
+#define CPW_PL(N) if (g.n[0] == N) st = launch_plane<R, N>(p, a, colbuf, vr, v, s);
             CPW_FAST_SIZES(CPW_PL)
 #undef CPW_PL
-        } else {
-            const bool reg = col_var_resolve<R>(p, p->col_var[sizeof(R) == 4 ? 1 : 0], nullptr) == 1;
+            return st;
+        }
+    } else if (col_fast(g)) {
+        int st = CPWGPU_OK;
+        const bool reg = col_var_resolve<R>(p, p->col_var[sizeof(R) == 4 ? 1 : 0], nullptr, stage) == 1;
 #define CPW_CO(N)                                                                \
     if (g.n[2] == N)                                                             \
         st = reg ? launch_col_reg<R, N>(p, a, colbuf, stage, s) : launch_col_fast<R, N>(p, a, colbuf, stage, s);
-            CPW_FAST_SIZES(CPW_CO)
+        CPW_FAST_SIZES(CPW_CO)
 #undef CPW_CO
-        }
         return st;
     }
     const int ntiles = (g.ncol + COL_CT - 1) / COL_CT;
@@ -350,6 +376,7 @@ struct Work {
     size_t part_n = 0;
     void *dhd = nullptr;
     size_t dhd_n = 0;
+    bool lean = false;  // split-K partials of one round of blocks only (splitk_shape)
 };
 
 // Block tile (BM x BN) and K granule of the projection kernel variant pv.
@@ -366,24 +393,76 @@ template <typename R> void proj_tile(int pv, int *BM, int *BN, int *BK) {
 #undef CPW_PD
 }
 
-// projection kernel variant of the plan for precision R
-template <typename R> int proj_variant(const cpwgpu_plan_s *p) {
+// Projection kernel of the plan for precision R and nanl projectors x neig
+// bands.  Default: the direct kernel with 64 x 64 (FP32 128 x 64) tiles per
+// block, and in FP64 with at most 32 bands a shape 32 bands wide, whose tiles
+// are not half padding.  us, LDS-staged k_proj / default: FP64 23,928 plane waves
+// x 256 projectors x 128 bands 161 / 92, x 24 bands 79 / 31 (64-wide: 41),
+// 80,852 x 864 x 256 4021 / 2072; FP32 23,928 x 256 x 128 75 / 49, x 64 66 / 28.
+template <typename R> int proj_variant(const cpwgpu_plan_s *p, int nanl, int neig) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
-    return p->proj_var[ix] >= 1 && p->proj_var[ix] < NPROJ_VAR ? p->proj_var[ix] : 0;
+    if (p->proj_var[ix] >= 0) return p->proj_var[ix] < NPROJ_VAR ? p->proj_var[ix] : 0;
+    if (sizeof(R) == 4 || neig > 32) return 1;
+    return nanl >= 256 ? 3 : 4;
+}
+
+// Back-projection kernel for rows plane waves and neig bands.  FP32: LDS-staged
+// with half chunks (54 us against 62-82 of the others at 23,928 x 256 x 128, 33
+// against 34-47 at 24 bands).  FP64: direct with 128 plane waves x 32 bands per
+// block; where that makes fewer than 2 blocks per CU, 64 x 32 (96 / 114 us at 128
+// bands, 59 / 57 at 64, 20 / 14 at 7,550 x 128 x 20; LDS-staged 141 / 91 / 23).
+template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int neig) {
+    const int ix = sizeof(R) == 4 ? 1 : 0;
+    if (p->back_var[ix] >= 0) return p->back_var[ix] < NBACK_VAR ? p->back_var[ix] : 0;
+    if (sizeof(R) == 4) return NBACK_DIRECT + 1;
+    const long blocks = (long)((rows + back_bi<double, 2>() - 1) / back_bi<double, 2>()) *
+                        ((neig + back_bn<double, 2>() - 1) / back_bn<double, 2>());
+    return blocks < 512 ? 3 : 2;
 }
 
 // Split-K shape of the projection GEMM over rows plane waves: number of K
 // slices and rows per slice (whole LDS stages of k_proj / whole chunks of
-// k_proj_direct), for nanl projectors and neig bands.
+// k_proj_direct), for nanl projectors and neig bands.  A target set by the
+// caller is the number of blocks; the default counts rounds: the tiles of one
+// slice run one block per CU at a time on the matrix cores' clock, so the slices
+// are chosen among those that just fill 1, 2, ... rounds of the 256 CUs, and
+// each costs its partials (written and read once) and a step of the reduction.
+// FP64 80,852 x 864 x 64 (14 tiles): 19 slices, 266 blocks, 951 us; 10 slices,
+// 140 blocks, 824 us; 18 slices (252 blocks) is what the rule takes.
+// lean: as a target of 256 blocks, the smallest workspace.
 template <typename R> void splitk_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *nsl_out,
-                                        int *kslice_out) {
+                                        int *kslice_out, bool lean = false) {
     int BM, BN, BK;
-    proj_tile<R>(proj_variant<R>(p), &BM, &BN, &BK);
+    proj_tile<R>(proj_variant<R>(p, nanl, neig), &BM, &BN, &BK);
     const int ix = sizeof(R) == 4 ? 1 : 0;
     const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
     const int ksteps = (rows + BK - 1) / BK;
-    const int target = p->splitk[ix] > 0 ? p->splitk[ix] : 256;
-    int nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
+    int nsl;
+    const int target = p->splitk[ix] > 0 ? p->splitk[ix] : lean ? 256 : 0;
+    if (target > 0) {
+        nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
+    } else {
+        constexpr long CUS = 256;
+        const long tiles = (long)tm * tn;
+        // us of one K step on one CU (6 of the 8 flops of a complex product, at
+        // 0.7 of the matrix peak) and of one slice's partials
+        const double step = 6.0 * BM * BN * BK / (sizeof(R) == 8 ? 2.1e5 : 4.2e5);
+        const double per = 0.04 + 2.0 * sizeof(cplx<R>) * nanl * neig / 6e6;
+        nsl = 1;
+        double best = HUGE_VAL;
+        const auto consider = [&](long n) {
+            n = std::max(1L, std::min<long>(n, ksteps));
+            const long len = (ksteps + n - 1) / n;
+            const double cost = (double)((tiles * n + CUS - 1) / CUS) * len * step + n * per;
+            if (cost < best) {
+                best = cost;
+                nsl = (int)n;
+            }
+        };
+        // one round or less: the slice cost against the shortened K loop
+        consider(std::min(CUS / std::max(1L, tiles), (long)std::sqrt(ksteps * step / per) + 1));
+        for (long k = 1; k <= 8; k++) consider(CUS * k / tiles);
+    }
     const int kslice = ((ksteps + nsl - 1) / nsl) * BK;
     *nsl_out = (rows + kslice - 1) / kslice;
     *kslice_out = kslice;
@@ -422,14 +501,13 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         anl = (const cplx<R> *)pv_.anl32->p;
     }
     const long lda = sizeof(R) == 8 ? pv_.lda : *pv_.lda32;
-    const int ix = sizeof(R) == 4 ? 1 : 0;
-    const int pv = proj_variant<R>(p);
+    const int pv = proj_variant<R>(p, nanl, neig);
     // block tile and K granule of the chosen projection kernel
     int BM, BN, BK;
     proj_tile<R>(pv, &BM, &BN, &BK);
     const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
     int nsl, kslice;
-    splitk_shape<R>(p, rows, nanl, neig, &nsl, &kslice);
+    splitk_shape<R>(p, rows, nanl, neig, &nsl, &kslice, w && w->lean);
     cplx<R> *part, *dhd;
     if (w) {
         if (cs * (size_t)nsl * neig * nanl > w->part_n || cs * (size_t)neig * nanl > w->dhd_n)
@@ -470,7 +548,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
                          dim3(RED_OUT * RED_GRP), 0, s, (const cplx<R> *)part, pv_.xnl, dhd, nanl, neig, nsl, 0);
     }
     if (phase != NL_PROJ) {
-        const int bv = p->back_var[ix] >= 1 && p->back_var[ix] <= NBACK_VAR - 1 ? p->back_var[ix] : 0;
+        const int bv = back_variant<R>(p, rows, neig);
         const cplx<R> *dh = dhd;
         double2 *hp = (double2 *)hpsi;
         // the kinetic term ekpg * psi is added here (coalesced), not in the gather
@@ -513,13 +591,12 @@ int ensure_aux() {
     return CPWGPU_OK;
 }
 
-// Local and kinetic terms of one k-point on stream s, in band chunks that keep
-// colbuf below 4 GiB.  acc: the gather adds to the non-local term already in
-// hpsi; join (may be null): event the first gather waits for (that term).
+// Local and kinetic terms of one k-point written into hpsi on stream s, in band
+// chunks that keep colbuf below 4 GiB.  nl: a back-projection adds the non-local
+// term afterwards, and with it the kinetic one unless kin_gather.
 template <typename R>
 int local_part(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hpsi, long ldh,
-               bool acc, hipEvent_t join, hipStream_t s, bool kin_gather = false, const Work *w = nullptr,
-               bool write_nokin = false) {
+               bool nl, hipStream_t s, bool kin_gather = false, const Work *w = nullptr) {
     const FftGeom &g = p->g;
     const size_t cs = sizeof(cplx<R>);
     const R *vr = sizeof(R) == 8 ? (const R *)p->v64.p : (const R *)p->v32.p;
@@ -536,27 +613,16 @@ int local_part(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *
         if ((st = p->colbuf.reserve(per_band * nbc))) return st;
         colbuf = (cplx<R> *)p->colbuf.p;
     }
-    bool joined = join == nullptr;
+    const int mode = !nl || kin_gather ? COLF_KIN : 0;
     for (int b0 = 0; b0 < neig; b0 += nbc) {
         const int nb = std::min(nbc, neig - b0);
-        // with the non-local term the back-projection already wrote it and the
-        // kinetic term into hpsi; without it the gather adds the kinetic term
-        // write_nokin: the gather writes local/N (+ ekpg psi if kin_gather)
-        // and the back-projection adds the rest afterwards
-        const int mode = acc ? (COLF_ACC | (kin_gather ? COLF_KIN : 0))
-                             : write_nokin ? (kin_gather ? COLF_KIN : 0) : COLF_KIN;
         const LocalArgs la{(const double2 *)psi + (long)b0 * ldp, ldp,
                            (double2 *)hpsi + (long)b0 * ldh, ldh, nb, mode};
         if (g.ncol > 0) {
             if ((st = local_stage<R>(p, la, colbuf, vr, ST_COL_BWD, s))) return st;
             if ((st = local_stage<R>(p, la, colbuf, vr, ST_PLANE, s))) return st;
+            if ((st = local_stage<R>(p, la, colbuf, vr, ST_COL_FWD, s))) return st;
         }
-        if (!joined) {
-            // join: the gather adds the local and kinetic terms to the non-local one
-            HIPCHK(hipStreamWaitEvent(s, join, 0));
-            joined = true;
-        }
-        if (g.ncol > 0 && (st = local_stage<R>(p, la, colbuf, vr, ST_COL_FWD, s))) return st;
     }
     return CPWGPU_OK;
 }
@@ -611,15 +677,13 @@ template <typename R>
 int apply_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hpsi, long ldh,
             hipStream_t s, const Work *w = nullptr) {
     const bool nl = p->nanl > 0 && p->g.mtxd > 0;
+    if (!nl) return local_part<R>(p, neig, psi, ldp, hpsi, ldh, false, s, false, w);
+    const int ix = sizeof(R) == 4 ? 1 : 0;
     // kinetic term in the gather (kg) or in the back-projection epilogue
-    const bool kg = p->kin_var[sizeof(R) == 4 ? 1 : 0] == 1;
+    const bool kg = p->kin_var[ix] == 1;
+    const int sched = g_overlap && !(w && !g_aux) ? p->sched_var[ix] : 0;
     int st;
-    if (nl && (!g_overlap || (w && !g_aux))) {
-        // serial: non-local term first (writes hpsi), then the local term adds
-        if ((st = nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 0, !kg, s, w))) return st;
-        return local_part<R>(p, neig, psi, ldp, hpsi, ldh, true, nullptr, s, kg, w);
-    }
-    if (nl && p->sched_var[sizeof(R) == 4 ? 1 : 0] == 1) {
+    if (sched == 1) {
         // fork: projection and D scaling on the second stream, beside the
         // column and plane kernels; the gather writes the local term, then the
         // back-projection adds the non-local one on the caller's stream
@@ -629,11 +693,11 @@ int apply_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hps
         if ((st = nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 1, !kg, g_aux, w, NL_PROJ)))
             return st;
         HIPCHK(hipEventRecord(g_join, g_aux));
-        if ((st = local_part<R>(p, neig, psi, ldp, hpsi, ldh, false, nullptr, s, kg, w, true))) return st;
+        if ((st = local_part<R>(p, neig, psi, ldp, hpsi, ldh, true, s, kg, w))) return st;
         HIPCHK(hipStreamWaitEvent(s, g_join, 0));
         return nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 1, !kg, s, w, NL_BACK);
     }
-    if (nl && p->sched_var[sizeof(R) == 4 ? 1 : 0] == 2) {
+    if (sched == 2) {
         // fork the other way round: the inverse column and plane kernels on
         // the second stream, the non-local term on the caller's stream (written
         // into hpsi), then the gather there once the plane stage is done.  The
@@ -645,16 +709,17 @@ int apply_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hps
         if ((st = nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 0, !kg, s, w))) return st;
         return local_beside<R>(p, neig, psi, ldp, hpsi, ldh, s, g_aux, kg, w);
     }
-    if (nl) {
-        // fork: non-local term on the second stream, written into hpsi
-        if ((st = ensure_aux())) return st;
-        HIPCHK(hipEventRecord(g_fork, s));
-        HIPCHK(hipStreamWaitEvent(g_aux, g_fork, 0));
-        if ((st = nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 0, !kg, g_aux, w))) return st;
-        HIPCHK(hipEventRecord(g_join, g_aux));
-        return local_part<R>(p, neig, psi, ldp, hpsi, ldh, true, g_join, s, kg, w);
-    }
-    return local_part<R>(p, neig, psi, ldp, hpsi, ldh, false, nullptr, s, false, w);
+    // One stream.  The kernels of both terms fill the GPU by themselves, on the
+    // same issue slots (FP64) or close to it (FP32), so that beside each other
+    // they end no sooner than one after the other, and an event between streams
+    // idles its stream 6-11 us.  The gather writes the local term (it would read
+    // hpsi in scattered 16-byte pieces to add to it), the back-projection adds
+    // to it in whole rows.  us, the whole non-local term on a second stream
+    // before / one stream: 24^3, 16 bands 50 / 24; 32x32x128, 72 bands 120 / 108;
+    // 72^3, 128 bands 500 / 474, FP32-mixed 274 / 262.
+    if ((st = nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 1, !kg, s, w, NL_PROJ))) return st;
+    if ((st = local_part<R>(p, neig, psi, ldp, hpsi, ldh, true, s, kg, w))) return st;
+    return nonlocal<R>(p, scalar_proj(p), neig, psi, ldp, hpsi, ldh, 1, !kg, s, w, NL_BACK);
 }
 
 int set_potential(cpwgpu_plan_s *p, const double *vscr, int mxdscr) {
@@ -913,10 +978,10 @@ int set_projectors_spin_host(cpwgpu_plan_s *p, const double *anlsp, const double
 // plan's mesh
 template <typename R> bool spin_reg_built(const cpwgpu_plan_s *p) {
     const FftGeom &g = p->g;
-    if (!fast_sizes(g)) return false;
+    if (!full_sizes(g)) return false;
     bool ok = false;
 #define CPW_SR(N) if (g.n[0] == N) ok = spin_reg_ok<R, N>();
-    CPW_FAST_SIZES(CPW_SR)
+    CPW_FULL_SIZES(CPW_SR)
 #undef CPW_SR
     return ok;
 }
@@ -939,7 +1004,7 @@ int apply_spin(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, double2
     const FftGeom &g = p->g;
     const int mtxd = g.mtxd;
     if (!p->nsp) return fail(CPWGPU_ERR_ARG, "two-component potential not set");
-    if (p->nsp == 4 && g.ncol > 0 && !fast_sizes(g))
+    if (p->nsp == 4 && g.ncol > 0 && !full_sizes(g))
         return fail(CPWGPU_ERR_SIZE, "the non-collinear potential needs one of the specialised meshes");
     if (neig == 0 || mtxd == 0) return CPWGPU_OK;
     int st;
@@ -997,7 +1062,7 @@ int apply_spin(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, double2
                 return st;
             st = CPWGPU_ERR_SIZE;
 #define CPW_SPL(N) if (g.n[0] == N) st = launch_plane_spin<R, N>(p, colbuf, vr, ntot, np_, spin_var_resolve<R>(p), s);
-            CPW_FAST_SIZES(CPW_SPL)
+            CPW_FULL_SIZES(CPW_SPL)
 #undef CPW_SPL
             if (st) return st;
             if ((st = columns(ST_COL_FWD, n0, np_, colbuf)) || (st = columns(ST_COL_FWD, neig + n0, np_, cb_dn)))
@@ -1797,7 +1862,7 @@ struct ForceWs {
 int plan_density(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const double *occ_h, double *rho,
                  hipStream_t s) {
     const FftGeom &g = p->g;
-    if (!fast_sizes(g)) return fail(CPWGPU_ERR_SIZE, "the density needs a mesh with a two-pass split");
+    if (!full_sizes(g)) return fail(CPWGPU_ERR_SIZE, "the density needs a mesh with a two-pass split");
     int rc;
     const int bpg = 8, ngrp = (neig + bpg - 1) / bpg;
     const long nmesh = (long)g.n[0] * g.n[1] * g.n[2];
@@ -1815,7 +1880,7 @@ int plan_density(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const
         return rc;
     rc = CPWGPU_ERR_SIZE;
 #define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, 0, 0, nullptr, s, (double *)g_fw.rhor.p);
-    CPW_FAST_SIZES(CPW_DEN)
+    CPW_FULL_SIZES(CPW_DEN)
 #undef CPW_DEN
     if (rc) return rc;
     const long tot = (long)g.id * g.n[1] * g.n[2];
@@ -1830,7 +1895,7 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
                 const int *qv, int nspec, const int *species, const double *fq, double *force,
                 double *enl, hipStream_t s) {
     const FftGeom &g = p->g;
-    if (!fast_sizes(g)) return fail(CPWGPU_ERR_SIZE, "forces need a mesh with a two-pass split");
+    if (!full_sizes(g)) return fail(CPWGPU_ERR_SIZE, "forces need a mesh with a two-pass split");
     int rc;
     std::vector<double> fcov(3 * (size_t)natom, 0.0);
     // local part ------------------------------------------------------------
@@ -1866,7 +1931,7 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
             return rc;
         bool reg = false;
 #define CPW_DR(N) if (g.n[0] == N) reg = den_reg_ok<N>();
-        CPW_FAST_SIZES(CPW_DR)
+        CPW_FULL_SIZES(CPW_DR)
 #undef CPW_DR
         const int W1 = 2 * Q1 + 1;
         const long nplane = (long)g.n[2] * (2 * Q2 + 1) * W1;
@@ -1881,7 +1946,7 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
             if ((rc = g_fw.rhor.reserve(8 * (size_t)ngrp * nmesh))) return rc;
             rc = CPWGPU_ERR_SIZE;
 #define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, 0, 0, nullptr, s, (double *)g_fw.rhor.p);
-            CPW_FAST_SIZES(CPW_DEN)
+            CPW_FULL_SIZES(CPW_DEN)
 #undef CPW_DEN
             if (rc) return rc;
             static bool attr = false;
@@ -1897,7 +1962,7 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
             // partial transforms per band group inside the density pass, then the
             // band groups summed (fixed order, all of the GPU)
 #define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, Q1, Q2, (double2 *)g_fw.t2.p, s);
-            CPW_FAST_SIZES(CPW_DEN)
+            CPW_FULL_SIZES(CPW_DEN)
 #undef CPW_DEN
             if (rc) return rc;
             hipLaunchKernelGGL(k_t2_sum, dim3((unsigned)((nplane + 255) / 256)), dim3(256), 0, s,
@@ -2273,12 +2338,12 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 // bytes of scratch an apply of nb bands takes: z-column buffer, split-K
 // partials and D<beta|psi>, each 256-byte aligned
-template <typename R> size_t noalloc_need(const cpwgpu_plan_s *p, int nb) {
+template <typename R> size_t noalloc_need(const cpwgpu_plan_s *p, int nb, bool lean) {
     const size_t cs = sizeof(cplx<R>);
     size_t n = align256(cs * (size_t)p->g.n[2] * p->g.ncolp * nb);
     if (p->nanl > 0 && p->g.mtxd > 0) {
         int nsl, kslice;
-        splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice);
+        splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice, lean);
         n += align256(cs * (size_t)nsl * nb * p->nanl) + align256(cs * (size_t)nb * p->nanl);
     }
     return n;
@@ -2292,22 +2357,24 @@ int apply_noalloc_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, dou
     if (sizeof(R) == 4 && nl && !p->anl32_valid)
         return fail(CPWGPU_ERR_ARG, "no FP32 copy of the projectors: it is made by the first FP32 "
                                     "cpwgpu_plan_apply after the projectors are set");
-    if (noalloc_need<R>(p, 1) > NOALLOC_SCRATCH)
+    const auto fits = [&](int nb, bool lean) { return noalloc_need<R>(p, nb, lean) <= NOALLOC_SCRATCH; };
+    if (!fits(1, false) && !fits(1, true))
         return fail(CPWGPU_ERR_SIZE, "one band needs %zu bytes of workspace, more than the %zu of the "
                                      "allocation-free entry point",
-                    noalloc_need<R>(p, 1), NOALLOC_SCRATCH);
+                    noalloc_need<R>(p, 1, true), NOALLOC_SCRATCH);
     int nbc = neig;
-    while (nbc > 1 && noalloc_need<R>(p, nbc) > NOALLOC_SCRATCH) nbc--;
+    while (nbc > 1 && !fits(nbc, false) && !fits(nbc, true)) nbc--;
     for (int b0 = 0; b0 < neig; b0 += nbc) {
         const int nb = std::min(nbc, neig - b0);
         const size_t cs = sizeof(cplx<R>);
         Work w;
+        w.lean = !fits(nb, false);
         w.colbuf = scr;
         w.colbuf_n = cs * (size_t)p->g.n[2] * p->g.ncolp * nb;
         size_t off = align256(w.colbuf_n);
         if (nl) {
             int nsl, kslice;
-            splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice);
+            splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice, w.lean);
             w.part = scr + off;
             w.part_n = cs * (size_t)nsl * nb * p->nanl;
             off += align256(w.part_n);
@@ -2812,11 +2879,11 @@ int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value) 
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_PROJ) {
-        *value = plan->proj_var[ix] >= 1 && plan->proj_var[ix] < NPROJ_VAR ? plan->proj_var[ix] : 0;
+        *value = ix ? proj_variant<float>(plan, plan->nanl, INT_MAX) : proj_variant<double>(plan, plan->nanl, INT_MAX);
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_BACK) {
-        *value = plan->back_var[ix] >= 1 && plan->back_var[ix] < NBACK_VAR ? plan->back_var[ix] : 0;
+        *value = ix ? back_variant<float>(plan, plan->mtxd, 1 << 20) : back_variant<double>(plan, plan->mtxd, 1 << 20);
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_KIN) {

@@ -344,7 +344,7 @@ constexpr u64mask box_slots(int N, int G, int M, int KD) {
 // Split of a line length N into A*B for the two-pass transform (A <= B, both
 // register-sized); 0 if N is not served by the specialised kernels.
 constexpr int split_a(int n) {
-    return n == 24 ? 4 : n == 32 ? 4 : n == 36 ? 6 : n == 40 ? 5 : n == 48 ? 6 : n == 54 ? 6
+    return n == 18 ? 3 : n == 20 ? 4 : n == 24 ? 4 : n == 32 ? 4 : n == 36 ? 6 : n == 40 ? 5 : n == 48 ? 6 : n == 50 ? 5 : n == 54 ? 6
          : n == 60 ? 6 : n == 64 ? 8 : n == 72 ? 8 : n == 80 ? 8 : n == 96 ? 8 : n == 100 ? 10
          : n == 108 ? 9 : n == 120 ? 10 : n == 128 ? 8 : n == 144 ? 12 : 0;
 }

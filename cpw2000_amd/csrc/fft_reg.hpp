@@ -315,13 +315,14 @@ __device__ __forceinline__ void scatter_plane(cplx<R> *__restrict__ cb, const cp
 // register slots that hold only x (y) outside the box on every lane are known
 // zeros of the inverse transforms and unused outputs of the forward ones:
 // they are neither loaded, transformed nor stored.  The box then has at most
-// N/2 + 1 columns, and the sub-plane row stride is the compile-time
-// pr_sub_stride<N>() instead of the argument S: every LDS offset of the y
-// lines and x rows folds into the instructions' immediate offsets.
+// N/2 + 1 columns.
+// SC: the sub-plane row stride at compile time (0: the argument S): every LDS
+// offset of the y lines and x rows folds into the instructions' immediate
+// offsets.
 // ---------------------------------------------------------------------------
 template <int N> constexpr int pr_sub_stride() { return N / 2 + 3; }
 
-template <typename R, int N, int GX, int GY, int P, int T, int W, bool YW = false, bool PR = false>
+template <typename R, int N, int GX, int GY, int P, int T, int W, bool YW = false, bool PR = false, int SC = 0>
 __global__ __launch_bounds__(T, W) void k_plane_reg(cplx<R> *__restrict__ colbuf,
                                                  const int *__restrict__ col_uy,
                                                  const R *__restrict__ vr,
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(T, W) void k_plane_reg(cplx<R> *__restrict__ colbuf
                                                  int nb, int S_arg) {
     static_assert(N % GX == 0 && N % GY == 0 && T % 64 == 0, "bad plane shape");
     constexpr int MX = N / GX, MY = N / GY;
-    const int S = PR ? pr_sub_stride<N>() : S_arg;
+    const int S = SC ? SC : S_arg;
     // slots that can hold box points (all of them unless PR)
     constexpr u64mask XB = PR ? box_slots(N, GX, MX, N / 4) : full_mask(MX);
     constexpr u64mask YB = PR ? box_slots(N, GY, MY, N / 4) : full_mask(MY);

@@ -141,9 +141,8 @@ struct cpwgpu_plan_s {
     int plane_var[2] = {-1, -1};
     // column kernels: 0 LDS lines, 1 register lines; -1 default
     int col_var[2] = {-1, -1};
-    // stream schedule of the two-stream apply: 0 (default) the whole
-    // non-local term beside the local one, the gather adding to it; 1 the
-    // projection beside the local term, the back-projection after the gather
+    // stream schedule: 0 (default) one stream; 1 the projection beside the
+    // local term; 2 the inverse columns and planes beside the non-local term
     int sched_var[2] = {-1, -1};
     // split-K target blocks of the projection GEMM per precision (-1 = 256)
     int splitk[2] = {-1, -1};

@@ -12,7 +12,18 @@
 namespace cpwgpu {
 
 // ---- specialised kernels: mesh lengths with a two-pass split ---------------
-#define CPW_FAST_SIZES(X) X(24) X(48) X(64) X(72) X(80) X(96) X(108) X(128)
+// CPW_FULL_SIZES: every kernel family (all plane variants, density, coupled
+// two-component plane).  CPW_FAST_SIZES adds the lengths of the size table that
+// small and elongated cells take: column kernels and one pruned register plane
+// shape each (with the generic kernels a 36^3 plane stage of 20 bands took 70 us
+// against 10, a 32x32x128 one of 72 bands 442 against 41).
+#define CPW_FULL_SIZES(X) X(24) X(48) X(64) X(72) X(80) X(96) X(108) X(128)
+#define CPW_FAST_SIZES(X) X(18) X(20) X(24) X(32) X(36) X(40) X(48) X(50) X(54) X(64) X(72) X(80) X(96) X(100) X(108) X(128)
+constexpr bool full_length(int n) {
+#define CPW_IS(N) || n == N
+    return false CPW_FULL_SIZES(CPW_IS);
+#undef CPW_IS
+}
 
 enum LocalStage { ST_COL_BWD, ST_PLANE, ST_COL_FWD };
 
@@ -35,43 +46,61 @@ struct RegShapeT {
     int GX, GY, P, T, W;
     bool YW, PR;
 };
-template <typename R> constexpr RegShapeT reg_shape(int v);
-template <> constexpr RegShapeT reg_shape<float>(int v) {
-    // 1-3 spill-free at 72: 67, 74 and 127 VGPRs
-    return v == 1 ? RegShapeT{8, 8, 1, 256, 5, false, false}
-         : v == 2 ? RegShapeT{8, 8, 2, 256, 4, false, false}
-         : v == 3 ? RegShapeT{4, 4, 1, 256, 3, false, false}
-         : v == 7 ? RegShapeT{8, 8, 1, 256, 5, true, false}
-         : v == 8 ? RegShapeT{2, 2, 1, 256, 3, true, true}
-         : v == 9 ? RegShapeT{4, 4, 1, 256, 4, true, true}
-         : v == 10 ? RegShapeT{8, 8, 1, 256, 5, true, true}
-         : v == 11 ? RegShapeT{2, 4, 1, 256, 3, false, true}
-                   : RegShapeT{0, 0, 0, 0, 0, false, false};
-}
-template <> constexpr RegShapeT reg_shape<double>(int v) {
-    return v == 1 ? RegShapeT{8, 8, 1, 256, 3, false, false}
-         : v == 2 ? RegShapeT{8, 8, 1, 320, 4, false, false}
-         : v == 3 ? RegShapeT{4, 8, 1, 256, 3, false, false}
-         : v == 7 ? RegShapeT{8, 8, 1, 256, 3, true, false}
-         : v == 8 ? RegShapeT{4, 4, 1, 256, 3, true, true}
-         : v == 9 ? RegShapeT{8, 8, 1, 256, 3, true, true}
-         : v == 10 ? RegShapeT{4, 4, 1, 256, 3, false, true}
-         : v == 11 ? RegShapeT{8, 8, 1, 256, 3, false, true}
-                   : RegShapeT{0, 0, 0, 0, 0, false, false};
+constexpr RegShapeT NO_SHAPE{0, 0, 0, 0, 0, false, false};
+// Lengths that 8 does not divide go by 4 or 2 lanes with up to 27 values each:
+// FP64 gives them the registers of 2 waves per SIMD, as many as their LDS lets
+// run (108: one block of 512 threads per CU).
+template <typename R, int N> constexpr RegShapeT reg_shape(int v) {
+    if constexpr (!full_length(N)) {
+        // one pruned shape: 9 in FP64, 10 in FP32
+        if (v != (sizeof(R) == 8 ? 9 : 10)) return NO_SHAPE;
+        const int w = sizeof(R) == 8 ? 3 : N % 8 == 0 ? 5 : 4;
+        return N == 18 ? RegShapeT{2, 2, 1, 64, 2, false, true}
+             : N == 20 ? RegShapeT{4, 4, 1, 128, w, false, true}
+             : N == 36 ? RegShapeT{4, 4, 1, 256, w, true, true}
+             : N == 50 || N == 54 ? RegShapeT{2, 2, 1, 128, sizeof(R) == 8 ? 2 : 3, false, true}
+             : N == 100 ? (sizeof(R) == 8 ? RegShapeT{4, 4, 1, 512, 2, false, true} : RegShapeT{4, 4, 1, 256, 4, true, true})
+                        : RegShapeT{8, 8, 1, 256, w, true, true};
+    } else if constexpr (sizeof(R) == 4) {
+        // 1-3 spill-free at 72: 67, 74 and 127 VGPRs
+        return v == 1 ? RegShapeT{8, 8, 1, 256, 5, false, false}
+             : v == 2 ? RegShapeT{8, 8, 2, 256, 4, false, false}
+             : v == 3 ? RegShapeT{4, 4, 1, 256, 3, false, false}
+             : v == 7 ? RegShapeT{8, 8, 1, 256, 5, true, false}
+             : v == 8 ? RegShapeT{2, 2, 1, 256, 3, true, true}
+             : v == 9 ? RegShapeT{4, 4, 1, 256, 4, true, true}
+             : v == 10 ? RegShapeT{8, 8, 1, 256, 5, true, true}
+             : v == 11 ? RegShapeT{2, 4, 1, 256, 3, false, true}
+                       : NO_SHAPE;
+    } else {
+        if (N == 108 && v == 9) return RegShapeT{4, 4, 1, 512, 2, false, true};
+        if (N == 128 && v == 10) return RegShapeT{8, 8, 1, 768, 3, false, true};
+        return v == 1 ? RegShapeT{8, 8, 1, 256, 3, false, false}
+             : v == 2 ? RegShapeT{8, 8, 1, 320, 4, false, false}
+             : v == 3 ? RegShapeT{4, 8, 1, 256, 3, false, false}
+             : v == 7 ? RegShapeT{8, 8, 1, 256, 3, true, false}
+             : v == 8 ? RegShapeT{4, 4, 1, 256, 3, true, true}
+             : v == 9 ? RegShapeT{8, 8, 1, 256, 3, true, true}
+             : v == 10 ? RegShapeT{4, 4, 1, 256, 3, false, true}
+             : v == 11 ? RegShapeT{8, 8, 1, 256, 3, false, true}
+                       : NO_SHAPE;
+    }
 }
 constexpr int NPLANE_VAR = 12;
 constexpr int WAVE_T[3] = {256, 192, 128};
 constexpr bool is_reg_variant(int v) { return (v >= 1 && v <= 3) || (v >= 7 && v < NPLANE_VAR); }
 
 // a register shape is built for a mesh length when both splits divide N and a
-// lane holds at most 288 bytes of one line
-template <typename R, int N, int GX, int GY> constexpr bool reg_ok() {
+// lane holds at most MAXB bytes of one line: 288, or 432 with the registers of
+// 2 waves per SIMD
+template <typename R, int N, int GX, int GY, int MAXB = 288> constexpr bool reg_ok() {
     return GX > 0 && GY > 0 && N % GX == 0 && N % GY == 0 && first_factor(N / GX) <= 5 &&
-           first_factor(N / GY) <= 5 && 2 * sizeof(R) * (N / GX) <= 288 && 2 * sizeof(R) * (N / GY) <= 288 &&
+           first_factor(N / GY) <= 5 && 2 * sizeof(R) * (N / GX) <= MAXB && 2 * sizeof(R) * (N / GY) <= MAXB &&
            N / GX <= 64 && N / GY <= 64;
 }
+template <typename R, int N> constexpr int reg_bytes(int v) { return reg_shape<R, N>(v).W <= 2 ? 432 : 288; }
 template <typename R, int N> constexpr bool reg_var_ok(int v) {
-#define CPW_RV(V) (v == V && reg_ok<R, N, reg_shape<R>(V).GX, reg_shape<R>(V).GY>())
+#define CPW_RV(V) (v == V && reg_ok<R, N, reg_shape<R, N>(V).GX, reg_shape<R, N>(V).GY, reg_bytes<R, N>(V)>())
     return CPW_RV(1) || CPW_RV(2) || CPW_RV(3) || CPW_RV(7) || CPW_RV(8) || CPW_RV(9) || CPW_RV(10) ||
            CPW_RV(11);
 #undef CPW_RV
@@ -82,6 +111,20 @@ inline bool prune_fits(const FftGeom &g) { return 4 * g.kd[0] <= g.n[0] && 4 * g
 
 // LDS row stride of the register variant's sub-plane for nx box columns
 inline int reg_stride(int nx) { return plane_sub_stride(nx); }
+// Compile-time row stride of a pruned shape.  N/2 + 3 holds every box inside
+// N/4; N/2 + 1 (odd) all but the one with kd = N/4 exactly, and is taken where it
+// lets one more block run per CU (80: three FP64 blocks instead of two, 181 ->
+// 150 us for 64 bands; 72, 96 and 128 gain no block and measured up to 10%
+// slower) or where N/2 + 3 is even (18, 50, 54: their box never has kd = N/4).
+template <typename R, int N, int V> constexpr int pr_stride() {
+    constexpr RegShapeT SH = reg_shape<R, N>(V);
+    constexpr int wide = N / 2 + 3, tight = (N / 2 + 1) | 1;
+    if (wide % 2 == 0) return tight;
+    const int cap = sizeof(R) == 8 ? SH.W * 256 / SH.T : 8;
+    const int bw = 160 * 1024 / (2 * (int)sizeof(R) * (N + N * wide));
+    const int bt = 160 * 1024 / (2 * (int)sizeof(R) * (N + N * tight));
+    return (bt < cap ? bt : cap) > (bw < cap ? bw : cap) ? tight : wide;
+}
 
 // ---- register column kernels -------------------------------------------------
 // lanes per z column: 8 where the column fits in registers, else 4
@@ -101,11 +144,18 @@ template <typename R, int N> bool plane_wave_fits(int v, int nx) {
 }
 
 template <typename R, int N> constexpr bool plane_var_ok(int v) {
-    return v == 0 || (v >= 4 && v <= 6) || reg_var_ok<R, N>(v);
+    return v == 0 || (full_length(N) && v >= 4 && v <= 6) || reg_var_ok<R, N>(v);
 }
 
-// default plane variant of a mesh length
-template <typename R, int N> constexpr int plane_var_default() { return 0; }
+// Default plane variant of a mesh length for a box inside N/4: the pruned
+// register shape that measured fastest (64-128 bands, us, LDS two-pass kernel
+// in brackets; FP64 64: 57 [98], 72: 181 [323], 80: 150 [349], 96: 280 [596],
+// 108: 1060 [1757], 128: 704 [1484]; FP32 64: 34 [50], 72: 97 [154], 80: 85 [122],
+// 96: 148 [284], 108: 489 [735], 128: 473 [607]).
+template <typename R, int N> constexpr int plane_var_default() {
+    if (sizeof(R) == 4) return N == 96 || N == 108 ? 9 : 10;
+    return N == 96 ? 11 : N == 128 ? 10 : 9;
+}
 
 // register shape of the coupled two-component plane kernel: (x lanes, y
 // lanes, threads, waves per SIMD); both components' rows live in registers.
@@ -133,13 +183,13 @@ template <int N> constexpr int den_threads() {
 }
 template <int N> constexpr bool den_reg_ok() { return den_threads<N>() > 0; }
 
-// launchers (mesh_launch.hpp)
+// launchers (mesh_launch.hpp); v: the plane variant, resolved for the mesh
 template <typename R, int N>
 int launch_col_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int stage, hipStream_t s);
 template <typename R, int N>
 int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int stage, hipStream_t s);
 template <typename R, int N>
-int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s);
+int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, int v, hipStream_t s);
 // var: the plan's resolved two-component plane kernel
 template <typename R, int N>
 int launch_plane_spin(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair, int var, hipStream_t s);

@@ -53,34 +53,42 @@ int launch_plane_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, con
 template <typename R, int N, int V>
 int launch_plane_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr,
                      hipStream_t s) {
-    constexpr RegShapeT SH = reg_shape<R>(V);
+    constexpr RegShapeT SH = reg_shape<R, N>(V);
     constexpr int GX = SH.GX, GY = SH.GY, P = SH.P, T = SH.T, W = SH.W;
     constexpr bool YW = SH.YW, PR = SH.PR;
-    if constexpr (!reg_ok<R, N, GX, GY>()) {
+    if constexpr (!reg_var_ok<R, N>(V)) {
         return fail(CPWGPU_ERR_MODE, "plane variant %d is not built for N = %d", V, N);
     } else {
         const FftGeom &g = p->g;
         if (PR && !prune_fits(g))
             return fail(CPWGPU_ERR_MODE, "plane variant %d needs the sphere box inside N/4", V);
-        // pruned shapes use their compile-time row stride (the box has at
-        // most N/2 + 1 columns there)
-        const int S = PR ? pr_sub_stride<N>() : reg_stride(g.nx);
-        if (reg_stride(g.nx) > S)
-            return fail(CPWGPU_ERR_MODE, "plane variant %d: %d box columns exceed its row stride", V, g.nx);
-        const size_t dyn = plane_reg_lds<R, N, P>(S);
-        if (dyn > 160 * 1024)
-            return fail(CPWGPU_ERR_SIZE, "plane variant %d: %zu bytes of LDS", V, dyn);
-        static bool attr = false;
-        if (!attr) {
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            attr = true;
+        const auto go = [&](auto kernel, int S, bool &attr) -> int {
+            const size_t dyn = plane_reg_lds<R, N, P>(S);
+            if (dyn > 160 * 1024)
+                return fail(CPWGPU_ERR_SIZE, "plane variant %d: %zu bytes of LDS", V, dyn);
+            if (!attr) {
+                HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                attr = true;
+            }
+            launch_timed(CPWGPU_K_PLANE, kernel, dim3(((a.nb + P - 1) / P) * g.n[2]), dim3(T), dyn, s, colbuf,
+                         (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, g, a.nb, S);
+            HIPCHK(hipGetLastError());
+            return CPWGPU_OK;
+        };
+        const int S = reg_stride(g.nx);
+        static bool attr_rt = false;
+        if constexpr (PR) {
+            constexpr int SC = pr_stride<R, N, V>();
+            static bool attr_ct = false;
+            if (S <= SC) return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, SC>, SC, attr_ct);
+            // kd = N/4 exactly where the stride is N/2 + 1
+            if constexpr (SC >= N / 2 + 3 || N % 4 != 0)
+                return fail(CPWGPU_ERR_MODE, "plane variant %d: %d box columns exceed its row stride", V, g.nx);
+            else
+                return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, S, attr_rt);
+        } else {
+            return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, S, attr_rt);
         }
-        launch_timed(CPWGPU_K_PLANE, k_plane_reg<R, N, GX, GY, P, T, W, YW, PR>,
-                     dim3(((a.nb + P - 1) / P) * g.n[2]), dim3(T), dyn, s, colbuf,
-                     (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, g, a.nb, S);
-        HIPCHK(hipGetLastError());
-        return CPWGPU_OK;
     }
 }
 
@@ -139,16 +147,18 @@ int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int st
 }
 
 template <typename R, int N>
-int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, hipStream_t s) {
-    int v = p->plane_var[sizeof(R) == 4 ? 1 : 0];
-    if (v < 0 || !plane_var_ok<R, N>(v)) v = plane_var_default<R, N>();
+int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R *vr, int v, hipStream_t s) {
 #define CPW_LR(V) if (v == V) return launch_plane_reg<R, N, V>(p, a, colbuf, vr, s);
     CPW_LR(1) CPW_LR(2) CPW_LR(3) CPW_LR(7) CPW_LR(8) CPW_LR(9) CPW_LR(10) CPW_LR(11)
 #undef CPW_LR
-    if (v == 4) return launch_plane_wave<R, N, WAVE_T[0]>(p, a, colbuf, vr, s);
-    if (v == 5) return launch_plane_wave<R, N, WAVE_T[1]>(p, a, colbuf, vr, s);
-    if (v == 6) return launch_plane_wave<R, N, WAVE_T[2]>(p, a, colbuf, vr, s);
-    return launch_plane_fast<R, N>(p, a, colbuf, vr, s);
+    if constexpr (full_length(N)) {
+        if (v == 4) return launch_plane_wave<R, N, WAVE_T[0]>(p, a, colbuf, vr, s);
+        if (v == 5) return launch_plane_wave<R, N, WAVE_T[1]>(p, a, colbuf, vr, s);
+        if (v == 6) return launch_plane_wave<R, N, WAVE_T[2]>(p, a, colbuf, vr, s);
+        return launch_plane_fast<R, N>(p, a, colbuf, vr, s);
+    } else {
+        return fail(CPWGPU_ERR_MODE, "plane variant %d is not built for N = %d", v, N);
+    }
 }
 
 template <typename R, int N>

@@ -215,17 +215,22 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
  *                       shapes that neither load, transform nor store the
  *                       register slots outside the sphere box (where the box
  *                       lies inside |x|, |y| <= N/4); -1 = the default for
- *                       the mesh
+ *                       the mesh (the fastest pruned shape where the box
+ *                       lies inside N/4).  On meshes outside the fully
+ *                       specialised set 0 = the generic kernel
  *   CPWGPU_TUNE_SPLITK  target number of blocks of the split-K projection
- *                       GEMM (64..4096); -1 = default (256)
+ *                       GEMM (64..4096); -1 = default (whole rounds of the
+ *                       compute units; reported as 256)
  *   CPWGPU_TUNE_PROJ    kernel of the projection GEMM: 0 = LDS-staged tiles,
  *                       1..4 = direct register loads in four tile shapes,
  *                       5 = LDS-staged with half the wave tile;
- *                       -1 = default (0)
+ *                       -1 = default (by size; reported for wide blocks of
+ *                       bands)
  *   CPWGPU_TUNE_BACK    kernel of the back-projection GEMM: 0 = LDS-staged D,
  *                       1..3 = direct register loads in three tile shapes,
  *                       4 = LDS-staged with half-size projector chunks;
- *                       -1 = default (0)
+ *                       -1 = default (by size; reported for wide blocks of
+ *                       bands)
  *   CPWGPU_TUNE_KIN     where ekpg*psi is added when projectors are set: 0 = in
  *                       the back-projection epilogue, 1 = in the gather of the
  *                       forward column kernel (moves work between the two
@@ -236,11 +241,11 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
  *                       where built, else 0)
  *   CPWGPU_TUNE_COL     z-column kernels: 0 = LDS two-pass lines, 1 =
  *                       register-resident lines (built where a column fits in
- *                       the registers of 8 or 4 lanes); -1 = default (0)
- *   CPWGPU_TUNE_SCHED   stream schedule with overlap on: 0 = the non-local
- *                       term (projection, D scaling, back-projection) on the
- *                       second stream beside the local term, the gather adding
- *                       the local term to it; 1 = the projection and D scaling
+ *                       the registers of 8 or 4 lanes); -1 = default (FP64 1
+ *                       where built, else 0)
+ *   CPWGPU_TUNE_SCHED   stream schedule: 0 = everything on the caller's stream
+ *                       (projection, D scaling, local term written, back-
+ *                       projection added to it); with overlap on, 1 = the projection and D scaling
  *                       beside the local term, the gather writing H psi, then
  *                       the back-projection adding to it on the caller's
  *                       stream; 2 = the inverse column and plane kernels on
