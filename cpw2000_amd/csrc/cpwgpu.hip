@@ -25,6 +25,7 @@
 #include "mesh.hpp"
 #include "nl_gemm.hpp"
 #include "subspace.hpp"
+#include "small_eig.hpp"
 #include "forces.hpp"
 #include "ditsp.hpp"
 #include "spin.hpp"
@@ -1153,7 +1154,8 @@ namespace {
 
 // ---- FP64 subspace workspace ------------------------------------------------
 struct Subspace {
-    DevBuf s, m, w, v, part, pos, rot, info, eig, res, tmp;
+    DevBuf s, m, w, v, part, pos, info, eig, res, tmp, rec, dinv, jac, ctl;
+    int *stop = nullptr;  // pinned: the Jacobi sweeps are done
 } g_ss;
 
 // The subspace products use the direct-load FP64 GEMM shapes that measured
@@ -1184,6 +1186,123 @@ int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb
     return CPWGPU_OK;
 }
 
+// Eigenvectors (ascending, in V) and eigenvalues (in g_ss.eig) of the average of
+// M and M^H; M and W are overwritten; dsweeps: number of Jacobi sweeps.
+int jacobi(double2 *M, double2 *W, double2 *V, int n, int max_sweeps, double tol, int *dsweeps, hipStream_t st) {
+    int rc;
+    const int np = (n + 1) & ~1, half = np / 2;
+    double *eig = (double *)g_ss.eig.p;
+    int *pos = (int *)g_ss.pos.p;
+    if (n <= SE_FULL_MAX) {
+        if ((rc = g_ss.rec.reserve(sizeof(double4) * (size_t)max_sweeps * (np - 1) * half))) return rc;
+        static bool attr = false;
+        if (!attr) {
+            HIPCHK(hipFuncSetAttribute((const void *)k_jacobi_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       16 * SE_FULL_MAX * SE_FULL_MAX));
+            attr = true;
+        }
+        double4 *rec = (double4 *)g_ss.rec.p;
+        hipLaunchKernelGGL(k_jacobi_lds, dim3(1), dim3(SE_THREADS), 16 * (size_t)n * n, st, (const double2 *)M, rec, eig,
+                           n, max_sweeps, tol, pos, dsweeps);
+        hipLaunchKernelGGL(k_jacobi_vectors, dim3((n + SE_VROWS - 1) / SE_VROWS), dim3(64), 0, st, (const double4 *)rec,
+                           (const int *)dsweeps, (const int *)pos, V, n);
+        HIPCHK(hipGetLastError());
+        return CPWGPU_OK;
+    }
+    // one launch per round, the matrix from one buffer to the other
+    if ((rc = g_ss.jac.reserve(16 * (size_t)n * n)) || (rc = g_ss.ctl.reserve(sizeof(JacobiCtl)))) return rc;
+    if (!g_ss.stop) HIPCHK(hipHostMalloc((void **)&g_ss.stop, sizeof(int), hipHostMallocDefault));
+    JacobiCtl *ctl = (JacobiCtl *)g_ss.ctl.p;
+    double2 *a = W, *b = (double2 *)g_ss.jac.p;
+    const unsigned nn = (unsigned)(((long)n * n + 255) / 256);
+    hipLaunchKernelGGL(k_jacobi_init, dim3(nn), dim3(256), 0, st, (const double2 *)M, a, V, n, ctl);
+    const dim3 grid((half + 63) / 64, 2 * ((half + 3) / 4));
+    hipEvent_t checked;
+    HIPCHK(hipEventCreateWithFlags(&checked, hipEventDisableTiming));
+    hipError_t err = hipSuccess;
+    for (int sweep = 0; sweep < max_sweeps && err == hipSuccess; sweep++) {
+        hipLaunchKernelGGL(k_jacobi_check, dim3(1), dim3(SE_THREADS), 0, st, (const double2 *)a, n, tol, ctl, g_ss.stop);
+        err = hipEventRecord(checked, st);
+        // the first rounds go out before the answer is read, and do nothing if it is to stop
+        const int ahead = std::min(16, np - 1);
+        double2 *x = a, *y = b;
+        for (int r = 0; r < np - 1 && err == hipSuccess; r++) {
+            if (r == ahead) {
+                err = hipEventSynchronize(checked);
+                if (err != hipSuccess || *(volatile int *)g_ss.stop) break;
+            }
+            hipLaunchKernelGGL(k_jacobi_round, grid, dim3(256), 0, st, (const double2 *)x, y, V, n, r,
+                               (const JacobiCtl *)ctl);
+            std::swap(x, y);
+        }
+        if (err == hipSuccess && np - 1 <= ahead) err = hipEventSynchronize(checked);
+        if (err != hipSuccess || *(volatile int *)g_ss.stop) break;
+        a = x;
+        b = y;
+    }
+    (void)hipEventDestroy(checked);
+    HIPCHK(err);
+    hipLaunchKernelGGL(k_jacobi_order, dim3((n + 255) / 256), dim3(256), 0, st, (const double2 *)a, eig, n, pos);
+    hipLaunchKernelGGL(k_jacobi_permute, dim3(nn), dim3(256), 0, st, (const double2 *)V, (const int *)pos, M, n);
+    HIPCHK(hipMemcpyAsync(V, M, 16 * (size_t)n * n, hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipMemcpyAsync(dsweeps, &ctl->sweeps, sizeof(int), hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
+// V = the generalised eigenvectors of (M, S), ascending, and their eigenvalues
+// in g_ss.eig; S, M, W are overwritten; dinfo[0]: failed Cholesky pivot (or 0),
+// dinfo[1]: Jacobi sweeps.
+int small_eig(double2 *S, double2 *M, double2 *W, double2 *V, int n, int max_sweeps, double tol, int *dinfo,
+              hipStream_t st) {
+    int rc;
+    if ((rc = g_ss.dinv.reserve(8 * (size_t)n))) return rc;
+    double *dinv = (double *)g_ss.dinv.p;
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_cholesky_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)se_lds_bytes(SE_TRI_MAX)));
+        HIPCHK(hipFuncSetAttribute((const void *)k_back_cols<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   16 * (SE_BW + 1) * SE_MAX));
+        HIPCHK(hipFuncSetAttribute((const void *)k_back_cols<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   16 * (SE_BW + 1) * 128));
+        attr = true;
+    }
+    if (n <= SE_TRI_MAX) {
+        hipLaunchKernelGGL(k_cholesky_lds, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, (const double2 *)S, S, dinv, n,
+                           dinfo);
+    } else {
+        hipLaunchKernelGGL(k_cholesky, dim3(1), dim3(SS_THREADS), 0, st, S, n, dinfo);
+        hipLaunchKernelGGL(k_factor_dinv, dim3((n + 255) / 256), dim3(256), 0, st, (const double2 *)S, dinv, n);
+    }
+    // W = L^-1 M, then M = L^-1 W^H
+    const auto by_rows_per_lane = [&](auto f) {
+        if (n <= 64) f(std::integral_constant<int, 1>{});
+        else if (n <= 128) f(std::integral_constant<int, 2>{});
+        else f(std::integral_constant<int, 4>{});
+    };
+    const auto solves = [&](auto rows_per_lane) {
+        constexpr int R = decltype(rows_per_lane)::value;
+        hipLaunchKernelGGL((k_solve_cols<R, false>), dim3(n), dim3(64), 0, st, (const double2 *)S, (const double *)dinv,
+                           (const double2 *)M, W, n);
+        hipLaunchKernelGGL((k_solve_cols<R, true>), dim3(n), dim3(64), 0, st, (const double2 *)S, (const double *)dinv,
+                           (const double2 *)W, M, n);
+    };
+    if (n <= SE_MAX) by_rows_per_lane(solves);
+    else hipLaunchKernelGGL(k_to_standard, dim3(1), dim3(SS_THREADS), 0, st, (const double2 *)S, M, W, n);
+    if ((rc = jacobi(M, W, V, n, max_sweeps, tol, dinfo + 1, st))) return rc;
+    if (n <= SE_MAX)
+        by_rows_per_lane([&](auto rows_per_lane) {
+            constexpr int R = decltype(rows_per_lane)::value;
+            hipLaunchKernelGGL(k_back_cols<R>, dim3((n + SE_BW - 1) / SE_BW), dim3(64), 16 * (size_t)(SE_BW * n + 64 * R),
+                               st, (const double2 *)S, (const double *)dinv, V, n);
+        });
+    else
+        hipLaunchKernelGGL(k_back_substitute, dim3(1), dim3(SS_THREADS), 0, st, (const double2 *)S, V, n);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
 int rayleigh_ritz(int mtxd, int nb, double2 *psi, long ldp, double2 *hpsi, long ldh, int rotate,
                   double *eig_h, double *res_h, hipStream_t st) {
     int rc;
@@ -1192,7 +1311,7 @@ int rayleigh_ritz(int mtxd, int nb, double2 *psi, long ldp, double2 *hpsi, long 
         (rc = g_ss.v.reserve(mat)))
         return rc;
     const int np = (nb + 1) & ~1;
-    if ((rc = g_ss.pos.reserve(4 * (size_t)np + 64)) || (rc = g_ss.rot.reserve(8 * (3 * (size_t)np + 8))) ||
+    if ((rc = g_ss.pos.reserve(4 * (size_t)np + 64)) ||
         (rc = g_ss.info.reserve(64)) || (rc = g_ss.eig.reserve(8 * (size_t)nb)) ||
         (rc = g_ss.res.reserve(8 * (size_t)nb)))
         return rc;
@@ -1208,14 +1327,10 @@ int rayleigh_ritz(int mtxd, int nb, double2 *psi, long ldp, double2 *hpsi, long 
                                    (cplx<double> *)(which == 0 ? S : M), nb, nb, nsl, st);
     }
     int *dinfo = (int *)g_ss.info.p;
-    hipLaunchKernelGGL(k_cholesky, dim3(1), dim3(SS_THREADS), 0, st, S, nb, dinfo);
-    hipLaunchKernelGGL(k_to_standard, dim3(1), dim3(SS_THREADS), 0, st, (const double2 *)S, M, W, nb);
     // tol 1e-13: off-diagonal elements below 1e-13 |M| / nb are left, which moves
     // the Ritz values by at most ~1e-13 relative; a tighter tol sits at the
     // rounding-noise level the rotations themselves regenerate
-    hipLaunchKernelGGL(k_jacobi, dim3(1), dim3(SS_THREADS), 0, st, M, V, (double *)g_ss.eig.p, nb, 60,
-                       1e-13, (int *)g_ss.pos.p, (double *)g_ss.rot.p, dinfo + 1);
-    hipLaunchKernelGGL(k_back_substitute, dim3(1), dim3(SS_THREADS), 0, st, (const double2 *)S, V, nb);
+    if ((rc = small_eig(S, M, W, V, nb, 60, 1e-13, dinfo, st))) return rc;
     HIPCHK(hipGetLastError());
     int hinfo[2] = {0, 0};
     HIPCHK(hipMemcpyAsync(hinfo, dinfo, sizeof hinfo, hipMemcpyDeviceToHost, st));

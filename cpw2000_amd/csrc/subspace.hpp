@@ -11,8 +11,9 @@
 //   Src/ditsp/ditsp_error.f90:70-76        residual ||H psi - eps psi||^2
 //
 // The nb x nb matrices are column-major complex128 (element (i,j) at i + j*n).
-// The dense steps run in one workgroup of SS_THREADS threads each (nb is at
-// most a few hundred): no grid-wide synchronisation, deterministic order.
+// The dense steps here run in one workgroup of SS_THREADS threads each, for any
+// nb; small_eig.hpp holds the Jacobi eigensolver and the faster forms for nb up
+// to a few hundred.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -112,14 +113,7 @@ __global__ __launch_bounds__(SS_THREADS) void k_to_standard(const double2 *l, do
     }
 }
 
-// Cyclic two-sided Jacobi for the Hermitian matrix a (destroyed): on exit the
-// eigenvalues ascend in eig and v holds the eigenvectors (columns).  Each
-// round applies n/2 disjoint rotations at once (round-robin pairing); a sweep
-// is n-1 rounds; stops when off(a) <= tol*|a| or after max_sweeps sweeps;
-// elements below tol*|a|/n are not rotated.  Round r pairs the positions
-// (slot k, slot np-1-k) of the rotating schedule: slot 0 holds index 0 and
-// slot i >= 1 holds index 1 + (i - 1 - r) mod (np - 1).  pos is n ints of
-// scratch (the final ordering), rot is unused (kept for the workspace layout).
+// index at slot i in round r of the round-robin schedule of np (even) positions
 __device__ __forceinline__ int rr_slot(int i, int r, int np) {
     if (i == 0) return 0;
     int m = (i - 1 - r) % (np - 1);
@@ -128,143 +122,6 @@ __device__ __forceinline__ int rr_slot(int i, int r, int np) {
 }
 
 constexpr int JAC_MAXPAIR = 1024;  // n <= 2048
-
-__global__ __launch_bounds__(SS_THREADS) void k_jacobi(double2 *a, double2 *v, double *eig, int n,
-                                                       int max_sweeps, double tol, int *pos,
-                                                       double *rot, int *sweeps_out) {
-    (void)rot;
-    __shared__ double red[SS_THREADS];
-    __shared__ int stop;
-    __shared__ double rc[JAC_MAXPAIR], rs[JAC_MAXPAIR];
-    __shared__ double2 ru[JAC_MAXPAIR];
-    __shared__ short rp[JAC_MAXPAIR], rq[JAC_MAXPAIR];
-    const int np = (n + 1) & ~1;  // even number of positions (one dummy if n odd)
-    for (long idx = threadIdx.x; idx < (long)n * n; idx += blockDim.x) {
-        const int i = (int)(idx % n), j = (int)(idx / n);
-        v[idx] = make_double2(i == j ? 1.0 : 0.0, 0.0);
-    }
-    __syncthreads();
-    int sweep = 0;
-    for (; sweep < max_sweeps; sweep++) {
-        // convergence test: off-diagonal vs total Frobenius norm
-        double off = 0.0, tot = 0.0;
-        for (long idx = threadIdx.x; idx < (long)n * n; idx += blockDim.x) {
-            const int i = (int)(idx % n), j = (int)(idx / n);
-            const double2 x = a[idx];
-            const double m = x.x * x.x + x.y * x.y;
-            tot += m;
-            if (i != j) off += m;
-        }
-        red[threadIdx.x] = off;
-        __syncthreads();
-        for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-            if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-            __syncthreads();
-        }
-        const double off_all = red[0];
-        __syncthreads();
-        red[threadIdx.x] = tot;
-        __syncthreads();
-        for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-            if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) stop = off_all <= tol * tol * red[0] || off_all == 0.0;
-        // pairs with |a_pq| below thr are left alone: together they stay below
-        // the stopping bound (n^2 thr^2 = tol^2 |a|^2), and rotating them only
-        // stirs rounding noise that keeps the sweeps from ever meeting it
-        const double thr = fmax(1e-300, tol * sqrt(red[0]) / n);
-        __syncthreads();
-        if (stop) break;
-        for (int round = 0; round < np - 1; round++) {
-            // rotation parameters of the pairs of this round
-            for (int k = threadIdx.x; k < np / 2; k += blockDim.x) {
-                int p = rr_slot(k, round, np), q = rr_slot(np - 1 - k, round, np);
-                if (p > q) { const int t = p; p = q; q = t; }
-                double c = 1.0, sn = 0.0;
-                double2 u = make_double2(1.0, 0.0);
-                if (q < n) {
-                    const double app = a[p + (long)p * n].x, aqq = a[q + (long)q * n].x;
-                    const double2 apq = a[p + (long)q * n];
-                    // |apq| without squaring: once the element has decayed
-                    // below ~1e-154, apq.x^2 + apq.y^2 is denormal and keeps
-                    // only a few digits, |u| drifts from 1 and the phase
-                    // factor would rescale row and column q
-                    const double g = hypot(apq.x, apq.y);
-                    if (g > thr) {
-                        const double zeta = (aqq - app) / (2.0 * g);
-                        const double t = (zeta >= 0.0 ? 1.0 : -1.0) /
-                                         (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-                        if (t != 0.0) {  // a zero angle is the identity: no phase either
-                            u = make_double2(apq.x / g, -apq.y / g);  // exp(-i phi)
-                            c = 1.0 / sqrt(1.0 + t * t);
-                            sn = t * c;
-                        }
-                    }
-                }
-                rc[k] = c;
-                rs[k] = sn;
-                ru[k] = u;
-                rp[k] = (short)p;
-                rq[k] = (short)q;
-            }
-            __syncthreads();
-            // rows: p' = c p - conj(u) s q ; q' = s p + conj(u) c q
-            for (long idx = threadIdx.x; idx < (long)(np / 2) * n; idx += blockDim.x) {
-                const int k = (int)(idx / n), j = (int)(idx % n);
-                const int p = rp[k], q = rq[k];
-                const double s = rs[k];
-                if (q >= n || (s == 0.0 && ru[k].y == 0.0 && ru[k].x == 1.0)) continue;  // identity
-                const double c = rc[k];
-                const double2 uc = zconj(ru[k]);
-                const double2 ap = a[p + (long)j * n], aq = a[q + (long)j * n];
-                const double2 t = zmul(uc, aq);
-                a[p + (long)j * n] = make_double2(c * ap.x - s * t.x, c * ap.y - s * t.y);
-                a[q + (long)j * n] = make_double2(s * ap.x + c * t.x, s * ap.y + c * t.y);
-            }
-            __syncthreads();
-            // columns (of a and v): p' = c p - u s q ; q' = s p + u c q
-            for (long idx = threadIdx.x; idx < (long)(np / 2) * n; idx += blockDim.x) {
-                const int k = (int)(idx / n), i = (int)(idx % n);
-                const int p = rp[k], q = rq[k];
-                const double s = rs[k];
-                if (q >= n || (s == 0.0 && ru[k].y == 0.0 && ru[k].x == 1.0)) continue;  // identity
-                const double c = rc[k];
-                const double2 u = ru[k];
-                double2 ap = a[i + (long)p * n], aq = a[i + (long)q * n];
-                double2 t = zmul(u, aq);
-                a[i + (long)p * n] = make_double2(c * ap.x - s * t.x, c * ap.y - s * t.y);
-                a[i + (long)q * n] = make_double2(s * ap.x + c * t.x, s * ap.y + c * t.y);
-                ap = v[i + (long)p * n];
-                aq = v[i + (long)q * n];
-                t = zmul(u, aq);
-                v[i + (long)p * n] = make_double2(c * ap.x - s * t.x, c * ap.y - s * t.y);
-                v[i + (long)q * n] = make_double2(s * ap.x + c * t.x, s * ap.y + c * t.y);
-            }
-            __syncthreads();
-        }
-    }
-    // eigenvalues in ascending order (rank by value, ties by index), vectors with them
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const double e = a[i + (long)i * n].x;
-        int r = 0;
-        for (int j = 0; j < n; j++) {
-            const double f = a[j + (long)j * n].x;
-            r += (f < e) || (f == e && j < i);
-        }
-        pos[i] = r;
-        eig[r] = e;
-    }
-    __syncthreads();
-    // permute eigenvector columns into a (a is free now): a[:, rank] = v[:, i]
-    for (long idx = threadIdx.x; idx < (long)n * n; idx += blockDim.x) {
-        const int i = (int)(idx % n), j = (int)(idx / n);
-        a[i + (long)pos[j] * n] = v[idx];
-    }
-    __syncthreads();
-    for (long idx = threadIdx.x; idx < (long)n * n; idx += blockDim.x) v[idx] = a[idx];
-    if (threadIdx.x == 0) *sweeps_out = sweep;
-}
 
 // In place on v: v <- L^-H v (backward substitution, one thread per column)
 __global__ __launch_bounds__(SS_THREADS) void k_back_substitute(const double2 *l, double2 *v, int n) {
