@@ -526,20 +526,20 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         const double2 *ps = (const double2 *)psi;
         cplx<R> *pt = part;
         if (pv == 1)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 1>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, nullptr, 0);
+            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 1>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
         else if (pv == 2)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 2>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, nullptr, 0);
+            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 2>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
         else if (pv == 3)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 3>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, nullptr, 0);
+            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 3>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
         else if (pv == 4)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 4>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, nullptr, 0);
+            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 4>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
         else if (pv == NPROJ_DIRECT + 1)
             launch_timed(CPWGPU_K_PROJ, (k_proj<R, proj_half_wm<R>(), proj_half_wn<R>()>), dim3(tm, tn, nsl),
                                dim3(GEMM_THREADS), 0, s, anl, lda, (const double2 *)psi, ldp,
-                               pt, rows, nanl, neig, kslice, nullptr, 0);
+                               pt, rows, nanl, neig, kslice, 0);
         else
             launch_timed(CPWGPU_K_PROJ, k_proj<R>, dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, s, anl, lda,
-                               (const double2 *)psi, ldp, pt, rows, nanl, neig, kslice, nullptr, 0);
+                               (const double2 *)psi, ldp, pt, rows, nanl, neig, kslice, 0);
     }
     if (phase != NL_BACK) {
         // launch_proj_reduce's launch, with the measurement hook
@@ -1164,10 +1164,9 @@ struct Subspace {
 // LDS-staged kernels).
 constexpr int SUB_PROJ_V = 2, SUB_BACK_V = 2;
 
-// split-K partials of a^H W b (na x nbc over mtxd rows, W = diag(wrow) or
-// the identity) into part; returns the number of slices in *nsl
+// split-K partials of a^H b (na x nbc over mtxd rows) into part; returns the number of slices in *nsl
 int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb, int nbc, int mtxd,
-                  DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0, const double *wrow = nullptr) {
+                  DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0) {
     constexpr int BM = direct_bm<double, SUB_PROJ_V>(), BN = direct_bn<double, SUB_PROJ_V>();
     constexpr int BK = direct_bk<double, SUB_PROJ_V>();
     const int tm = (na + BM - 1) / BM, tn = (nbc + BN - 1) / BN;
@@ -1180,7 +1179,7 @@ int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb
     if ((rc = part.reserve(16 * (size_t)nsl * na * nbc))) return rc;
     hipLaunchKernelGGL((k_proj_direct<double, SUB_PROJ_V>), dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, st,
                        (const cplx<double> *)a, lda, b, ldb, (cplx<double> *)part.p, mtxd, na, nbc, kslice,
-                       wrow, lower);
+                       lower);
     HIPCHK(hipGetLastError());
     *nsl_out = nsl;
     return CPWGPU_OK;
@@ -1968,8 +1967,31 @@ int plan_ditsp(cpwgpu_plan_s *p, int prec, int icmax, int iguess, double epspsi,
 
 // ---- atomic forces ------------------------------------------------------------
 struct ForceWs {
-    DevBuf t2, t2s, rho, qv, fq, rat, species, patom, occ, fl, fnl, enl, p, rhor;
+    DevBuf t1, t2, rho, qv, fq, rat, species, patom, occ, out, coef, phi, rhor;
 } g_fw;
+
+// rhor[grp][z][y][x] of the bands (density.hpp) from their z-columns in the
+// plan's column buffer, which this fills; the number of groups in *ngrp.
+int density_planes(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const double *occ, int *ngrp,
+                   hipStream_t s) {
+    const FftGeom &g = p->g;
+    int rc, bpg = 1;
+#define CPW_DB(N) if (g.n[0] == N) bpg = den_bands_per_group<N>(g, neig);
+    CPW_FULL_SIZES(CPW_DB)
+#undef CPW_DB
+    *ngrp = (neig + bpg - 1) / bpg;
+    if ((rc = p->colbuf.reserve(16 * (size_t)g.n[2] * g.ncolp * neig)) ||
+        (rc = g_fw.rhor.reserve(8 * (size_t)*ngrp * g.n[0] * g.n[1] * g.n[2])))
+        return rc;
+    const LocalArgs la{psi, ldp, nullptr, 0, neig, 0};
+    if ((rc = local_stage<double>(p, la, (cplx<double> *)p->colbuf.p, (const double *)p->v64.p, ST_COL_BWD, s)))
+        return rc;
+    rc = CPWGPU_ERR_SIZE;
+#define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, s, (double *)g_fw.rhor.p);
+    CPW_FULL_SIZES(CPW_DEN)
+#undef CPW_DEN
+    return rc;
+}
 
 // Electron density on the mesh, the band loop of Src/omp/charge_by_fft.f90:170-197:
 // rho(r) = sum_n occ_n |psi_n(r)|^2, psi_n(r) the unnormalised G -> r transform.
@@ -1978,26 +2000,14 @@ int plan_density(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const
                  hipStream_t s) {
     const FftGeom &g = p->g;
     if (!full_sizes(g)) return fail(CPWGPU_ERR_SIZE, "the density needs a mesh with a two-pass split");
-    int rc;
-    const int bpg = 8, ngrp = (neig + bpg - 1) / bpg;
-    const long nmesh = (long)g.n[0] * g.n[1] * g.n[2];
-    if ((rc = p->colbuf.reserve(16 * (size_t)g.n[2] * g.ncolp * neig)) ||
-        (rc = g_fw.rhor.reserve(8 * (size_t)ngrp * nmesh)))
-        return rc;
+    int rc, ngrp;
     const double *occ = nullptr;
     if (occ_h) {
         if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
         occ = (const double *)g_fw.occ.p;
         HIPCHK(hipStreamSynchronize(g_stream));  // the upload went through the library stream
     }
-    const LocalArgs la{psi, ldp, nullptr, 0, neig, 0};
-    if ((rc = local_stage<double>(p, la, (cplx<double> *)p->colbuf.p, (const double *)p->v64.p, ST_COL_BWD, s)))
-        return rc;
-    rc = CPWGPU_ERR_SIZE;
-#define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, 0, 0, nullptr, s, (double *)g_fw.rhor.p);
-    CPW_FULL_SIZES(CPW_DEN)
-#undef CPW_DEN
-    if (rc) return rc;
+    if ((rc = density_planes(p, neig, psi, ldp, occ, &ngrp, s))) return rc;
     const long tot = (long)g.id * g.n[1] * g.n[2];
     hipLaunchKernelGGL(k_rho_r_reduce, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
                        (const double *)g_fw.rhor.p, ngrp, g.n[0], g.n[1], g.n[2], g.id, rho);
@@ -2012,128 +2022,90 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
     const FftGeom &g = p->g;
     if (!full_sizes(g)) return fail(CPWGPU_ERR_SIZE, "forces need a mesh with a two-pass split");
     int rc;
-    std::vector<double> fcov(3 * (size_t)natom, 0.0);
-    // local part ------------------------------------------------------------
-    if (nq > 0) {
-        int Q1 = 0, Q2 = 0;
-        for (int k = 0; k < nq; k++) {
-            Q1 = std::max(Q1, std::abs(qv[3 * k]));
-            Q2 = std::max(Q2, std::abs(qv[3 * k + 1]));
-            if (2 * std::abs(qv[3 * k]) >= g.n[0] || 2 * std::abs(qv[3 * k + 1]) >= g.n[1] ||
-                2 * std::abs(qv[3 * k + 2]) >= g.n[2])
-                return fail(CPWGPU_ERR_ARG, "q vector %d outside the mesh", k);
-        }
-        if (2 * Q1 + 1 > (g.nx | 1) || 2 * Q2 + 1 > g.n[1])
-            return fail(CPWGPU_ERR_SIZE, "local potential q box wider than the wave-function box");
-        const int bpg = 8, ngrp = (neig + bpg - 1) / bpg;
-        const size_t per_band = 16 * (size_t)g.n[2] * g.ncolp;
-        if ((rc = p->colbuf.reserve(per_band * neig))) return rc;
-        const size_t t2n = (size_t)ngrp * g.n[2] * (2 * Q2 + 1) * (2 * Q1 + 1);
-        if ((rc = g_fw.t2.reserve(16 * t2n)) || (rc = g_fw.rho.reserve(16 * (size_t)nq)) ||
-            (rc = upload(g_fw.qv, qv, 3 * (size_t)nq)) ||
-            (rc = upload(g_fw.fq, fq, (size_t)nq * nspec)) || (rc = upload(g_fw.rat, rat, 3 * (size_t)natom)) ||
-            (rc = upload(g_fw.species, species, (size_t)natom)) || (rc = g_fw.fl.reserve(24 * (size_t)natom)))
-            return rc;
-        const double *occ = nullptr;
-        if (occ_h) {
-            if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
-            occ = (const double *)g_fw.occ.p;
-        }
-        HIPCHK(hipStreamSynchronize(g_stream));  // uploads went through the library stream
-        const LocalArgs la{psi, ldp, nullptr, 0, neig, 0};
-        if ((rc = local_stage<double>(p, la, (cplx<double> *)p->colbuf.p, (const double *)p->v64.p,
-                                      ST_COL_BWD, s)))
-            return rc;
-        bool reg = false;
-#define CPW_DR(N) if (g.n[0] == N) reg = den_reg_ok<N>();
-        CPW_FULL_SIZES(CPW_DR)
-#undef CPW_DR
-        const int W1 = 2 * Q1 + 1;
-        const long nplane = (long)g.n[2] * (2 * Q2 + 1) * W1;
-        if ((rc = g_fw.t2s.reserve(16 * (size_t)nplane))) return rc;
-        rc = CPWGPU_ERR_SIZE;
-        if (reg) {
-            // density planes per band group (register lines), then per z-plane
-            // the group sum and the partial transforms along x and y
-            const long nmesh = (long)g.n[0] * g.n[1] * g.n[2];
-            const size_t lds = 16 * ((size_t)g.n[0] + g.n[1] + (size_t)g.n[1] * W1) + 8 * (size_t)g.n[0] * g.n[1];
-            if (lds > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane of %d x %d does not fit in LDS", g.n[0], g.n[1]);
-            if ((rc = g_fw.rhor.reserve(8 * (size_t)ngrp * nmesh))) return rc;
-            rc = CPWGPU_ERR_SIZE;
-#define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, 0, 0, nullptr, s, (double *)g_fw.rhor.p);
-            CPW_FULL_SIZES(CPW_DEN)
-#undef CPW_DEN
-            if (rc) return rc;
-            static bool attr = false;
-            if (!attr) {
-                HIPCHK(hipFuncSetAttribute((const void *)k_rho_partial, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           160 * 1024));
-                attr = true;
-            }
-            hipLaunchKernelGGL(k_rho_partial, dim3(g.n[2]), dim3(256), lds, s, (const double *)g_fw.rhor.p, ngrp,
-                               g.n[0], g.n[1], g.n[2], Q1, Q2, (const double2 *)p->tw[0].p,
-                               (const double2 *)p->tw[1].p, (double2 *)g_fw.t2s.p);
-        } else {
-            // partial transforms per band group inside the density pass, then the
-            // band groups summed (fixed order, all of the GPU)
-#define CPW_DEN(N) if (g.n[0] == N) rc = launch_density<N>(p, (const cplx<double> *)p->colbuf.p, occ, neig, bpg, ngrp, Q1, Q2, (double2 *)g_fw.t2.p, s);
-            CPW_FULL_SIZES(CPW_DEN)
-#undef CPW_DEN
-            if (rc) return rc;
-            hipLaunchKernelGGL(k_t2_sum, dim3((unsigned)((nplane + 255) / 256)), dim3(256), 0, s,
-                               (const double2 *)g_fw.t2.p, nplane, ngrp, (double2 *)g_fw.t2s.p);
-        }
-        // per q the z sum
-        hipLaunchKernelGGL(k_rho_q, dim3((nq + 255) / 256), dim3(256), 0, s, (const double2 *)g_fw.t2s.p,
-                           (const int *)g_fw.qv.p, nq, (const double2 *)p->tw[2].p, g.n[2], Q1, Q2, p->inv_n,
-                           (double2 *)g_fw.rho.p);
-        hipLaunchKernelGGL(k_force_local, dim3(natom), dim3(256), 0, s, (const double2 *)g_fw.rho.p,
-                           (const int *)g_fw.qv.p, (const double *)g_fw.fq.p, nq,
-                           (const double *)g_fw.rat.p, (const int *)g_fw.species.p, (double *)g_fw.fl.p);
-        HIPCHK(hipGetLastError());
-        std::vector<double> fl(3 * (size_t)natom);
-        HIPCHK(hipMemcpyAsync(fl.data(), g_fw.fl.p, 24 * (size_t)natom, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        for (size_t k = 0; k < fl.size(); k++) fcov[k] += fl[k];
-    }
-    // non-local part --------------------------------------------------------
-    double e_nl = 0.0;
     const int nanl = p->nanl;
+    int Q1 = 0, Q2 = 0;
+    for (int k = 0; k < nq; k++) {
+        Q1 = std::max(Q1, std::abs(qv[3 * k]));
+        Q2 = std::max(Q2, std::abs(qv[3 * k + 1]));
+        if (2 * std::abs(qv[3 * k]) >= g.n[0] || 2 * std::abs(qv[3 * k + 1]) >= g.n[1] ||
+            2 * std::abs(qv[3 * k + 2]) >= g.n[2])
+            return fail(CPWGPU_ERR_ARG, "q vector %d outside the mesh", k);
+    }
+    if (nq > 0 && (2 * Q1 + 1 > (g.nx | 1) || 2 * Q2 + 1 > g.n[1]))
+        return fail(CPWGPU_ERR_SIZE, "local potential q box wider than the wave-function box");
     if (nanl > 0) {
         if (!proj_atom) return fail(CPWGPU_ERR_ARG, "proj_atom missing");
         for (int a = 0; a < nanl; a++)
             if (proj_atom[a] < 0 || proj_atom[a] >= natom) return fail(CPWGPU_ERR_ARG, "proj_atom[%d] = %d", a, proj_atom[a]);
-        const long mat = (long)nanl * neig;
-        if ((rc = g_fw.p.reserve(16 * 4 * (size_t)mat)) || (rc = upload(g_fw.patom, proj_atom, (size_t)nanl)) ||
-            (rc = g_fw.fnl.reserve(24 * (size_t)natom)) || (rc = g_fw.enl.reserve(8 * (size_t)natom)))
-            return rc;
-        const double *occ = nullptr;
-        if (occ_h) {
-            if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
-            occ = (const double *)g_fw.occ.p;
-        }
-        HIPCHK(hipStreamSynchronize(g_stream));
-        for (int j = 0; j < 4; j++) {
-            // <beta|psi>, then <beta|g_j psi> for the three Cartesian components
-            const double *w = j == 0 ? nullptr : (const double *)p->gw.p + (size_t)(j - 1) * g.mtxd;
-            int nsl;
-            if ((rc = gram_partials((const double2 *)p->anl64.p, p->lda, nanl, psi, ldp, neig, g.mtxd, p->part,
-                                    &nsl, s, 0, w)))
-                return rc;
-            launch_proj_reduce<double>((const cplx<double> *)p->part.p, nullptr,
-                                       (cplx<double> *)g_fw.p.p + (size_t)j * mat, nanl, neig, nsl, s);
-        }
-        hipLaunchKernelGGL(k_force_nl, dim3(natom), dim3(256), 0, s, (const double2 *)g_fw.p.p, nanl,
-                           neig, (const double *)p->xnl.p, occ, (const int *)g_fw.patom.p,
-                           (double *)g_fw.fnl.p, (double *)g_fw.enl.p);
-        HIPCHK(hipGetLastError());
-        std::vector<double> fn(3 * (size_t)natom), en(natom);
-        HIPCHK(hipMemcpyAsync(fn.data(), g_fw.fnl.p, 24 * (size_t)natom, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipMemcpyAsync(en.data(), g_fw.enl.p, 8 * (size_t)natom, hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        for (size_t k = 0; k < fn.size(); k++) fcov[k] += fn[k];
-        for (int a = 0; a < natom; a++) e_nl += en[a];
     }
+    // covariant local forces, non-local forces and non-local energies of the atoms
+    if ((rc = g_fw.out.reserve(56 * (size_t)natom))) return rc;
+    double *floc = (double *)g_fw.out.p, *fnl = floc + 3 * (size_t)natom, *en = fnl + 3 * (size_t)natom;
+    const double *occ = nullptr;
+    if (occ_h && (nq > 0 || nanl > 0)) {
+        if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
+        occ = (const double *)g_fw.occ.p;
+    }
+    // the uploads go through the library stream; the host arrays are read until
+    // the synchronisation at the end
+    // local part ------------------------------------------------------------
+    if (nq > 0) {
+        const int W1 = 2 * Q1 + 1, W2 = 2 * Q2 + 1;
+        if ((rc = g_fw.t1.reserve(16 * (size_t)g.n[2] * g.n[1] * W1)) ||
+            (rc = g_fw.t2.reserve(16 * (size_t)g.n[2] * W2 * W1)) || (rc = g_fw.rho.reserve(16 * (size_t)nq)) ||
+            (rc = upload(g_fw.qv, qv, 3 * (size_t)nq)) || (rc = upload(g_fw.fq, fq, (size_t)nq * nspec)) ||
+            (rc = upload(g_fw.rat, rat, 3 * (size_t)natom)) || (rc = upload(g_fw.species, species, (size_t)natom)))
+            return rc;
+        if (s != g_stream) HIPCHK(hipStreamSynchronize(g_stream));
+        int ngrp;
+        if ((rc = density_planes(p, neig, psi, ldp, occ, &ngrp, s))) return rc;
+        hipLaunchKernelGGL(k_rho_x, dim3(g.n[2], (g.n[1] + RHO_RY - 1) / RHO_RY), dim3(256),
+                           (16 + 8 * RHO_RY) * (size_t)g.n[0], s, (const double *)g_fw.rhor.p, ngrp, g.n[0], g.n[1],
+                           g.n[2], Q1, (const double2 *)p->tw[0].p, (double2 *)g_fw.t1.p);
+        hipLaunchKernelGGL(k_rho_y, dim3(g.n[2], (W1 * W2 + 255) / 256), dim3(256), 16 * (size_t)g.n[1], s,
+                           (const double2 *)g_fw.t1.p, g.n[1], Q1, Q2, (const double2 *)p->tw[1].p,
+                           (double2 *)g_fw.t2.p);
+        hipLaunchKernelGGL(k_rho_q, dim3((unsigned)(((long)nq * RHO_L + 255) / 256)), dim3(256), 0, s,
+                           (const double2 *)g_fw.t2.p, (const int *)g_fw.qv.p, nq, (const double2 *)p->tw[2].p,
+                           g.n[2], Q1, Q2, p->inv_n, (double2 *)g_fw.rho.p);
+        hipLaunchKernelGGL(k_force_local, dim3(natom), dim3(256), 0, s, (const double2 *)g_fw.rho.p,
+                           (const int *)g_fw.qv.p, (const double *)g_fw.fq.p, nq,
+                           (const double *)g_fw.rat.p, (const int *)g_fw.species.p, floc);
+        HIPCHK(hipGetLastError());
+    }
+    // non-local part --------------------------------------------------------
+    if (nanl > 0) {
+        const long mat = (long)nanl * neig;
+        const int nblk = (g.mtxd + PHI_BI - 1) / PHI_BI;
+        if ((rc = g_fw.coef.reserve(16 * (size_t)mat)) || (rc = g_fw.phi.reserve(24 * (size_t)nblk * nanl)) ||
+            (rc = upload(g_fw.patom, proj_atom, (size_t)nanl)))
+            return rc;
+        if (s != g_stream) HIPCHK(hipStreamSynchronize(g_stream));
+        // <beta|psi> without the strengths
+        ProjView pv = scalar_proj(p);
+        pv.xnl = nullptr;
+        if ((rc = nonlocal<double>(p, pv, neig, (const double *)psi, ldp, nullptr, 0, 0, false, s, nullptr, NL_PROJ)))
+            return rc;
+        const double2 *p0 = (const double2 *)p->dhd.p;
+        hipLaunchKernelGGL(k_force_coef, dim3((unsigned)((mat + 255) / 256)), dim3(256), 0, s, p0, nanl, neig, occ,
+                           (cplx<double> *)g_fw.coef.p);
+        hipLaunchKernelGGL(k_force_phi, dim3(nblk, (nanl + PHI_BA - 1) / PHI_BA), dim3(GEMM_THREADS), 0, s,
+                           (const cplx<double> *)psi, ldp, (const cplx<double> *)g_fw.coef.p,
+                           (const cplx<double> *)p->anl64.p, p->lda, (const double *)p->gw.p, g.mtxd, nanl, neig,
+                           (double *)g_fw.phi.p);
+        hipLaunchKernelGGL(k_force_nl, dim3(natom), dim3(FNL_CHUNK), 0, s, (const double *)g_fw.phi.p, nblk, p0, nanl,
+                           neig, (const double *)p->xnl.p, occ, (const int *)g_fw.patom.p, fnl, en);
+        HIPCHK(hipGetLastError());
+    }
+    std::vector<double> out(7 * (size_t)natom, 0.0);
+    if (nq > 0 || nanl > 0)
+        HIPCHK(hipMemcpyAsync(out.data(), floc, 56 * (size_t)natom, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    std::vector<double> fcov(3 * (size_t)natom, 0.0);
+    double e_nl = 0.0;
+    for (size_t k = 0; k < fcov.size(); k++)
+        fcov[k] = (nq > 0 ? out[k] : 0.0) + (nanl > 0 ? out[fcov.size() + k] : 0.0);
+    for (int a = 0; nanl > 0 && a < natom; a++) e_nl += out[6 * (size_t)natom + a];
     // Cartesian: F = inv(avec)^T f_cov  (avec columns are the lattice vectors)
     const double *A = avec;  // A[i + 3 j] = component i of a_j
     const double det = A[0] * (A[4] * A[8] - A[7] * A[5]) - A[3] * (A[1] * A[8] - A[7] * A[2]) +
@@ -2547,7 +2519,7 @@ int cpwgpu_finalize(void) {
     for (DevBuf *b : {&g_dt.xa, &g_dt.hxa, &g_dt.xb, &g_dt.hxb, &g_dt.pb, &g_dt.cpk, &g_dt.hd, &g_dt.m,
                       &g_dt.g, &g_dt.g0,
                       &g_dt.pm, &g_dt.w, &g_dt.e, &g_dt.info, &g_dt.res, &g_dt.act, &g_dt.d, &g_dt.mones,
-                      &g_dt.eall, &g_fw.rhor, &g_fw.t2, &g_fw.t2s})
+                      &g_dt.eall, &g_fw.rhor, &g_fw.t1, &g_fw.t2, &g_fw.coef, &g_fw.phi})
         b->release();
     if (g_aux) {
         HIPCHK(hipStreamSynchronize(g_aux));

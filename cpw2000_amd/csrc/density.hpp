@@ -8,19 +8,16 @@
 
 namespace cpwgpu {
 
-// per (z, band group): rho(x,y) = sum_{bands in group} occ |psi(x,y,z)|^2, then
-// T2[grp][z][q2][q1] = sum_y e^{-2 pi i q2 y/N2} sum_x e^{-2 pi i q1 x/N1} rho(x,y)
-// for |q1| <= Q1, |q2| <= Q2.  LDS: tw1[N1] tw2[N2] static; dynamic
-// sub[N2][nxp] (reused for the x-partial transform), rows[RB][row_stride], acc[N2][N1].
+// per (z, band group): rho(x,y) = sum_{bands in group} occ |psi(x,y,z)|^2 into
+// rhor[grp][z][y][x], for lengths and boxes without a register shape.  LDS:
+// tw1[N1] tw2[N2] static; dynamic sub[N2][nxp], rows[RB][row_stride], acc[N2][N1].
 template <int N1, int N2>
 __global__ __launch_bounds__(FT) void k_density_fast(const cplx<double> *__restrict__ colbuf,
                                                      const int *__restrict__ col_uy,
                                                      const double *__restrict__ occ,
                                                      const double2 *__restrict__ tw1g,
                                                      const double2 *__restrict__ tw2g, FftGeom g,
-                                                     int nb, int bpg, int Q1, int Q2,
-                                                     double2 *__restrict__ t2,
-                                                     double *__restrict__ rhor = nullptr) {
+                                                     int nb, int bpg, double *__restrict__ rhor) {
     typedef double R;
     constexpr int A1 = split_a(N1), B1 = N1 / A1;
     constexpr int RB = FT / B1;
@@ -81,58 +78,27 @@ __global__ __launch_bounds__(FT) void k_density_fast(const cplx<double> *__restr
             __syncthreads();
         }
     }
-    if (rhor) {
-        // rho(x, y) of this plane and band group, for a fixed-order sum over groups
-        __syncthreads();
-        double *o = rhor + ((long)grp * n3 + z) * (N2 * N1);
-        for (int q = threadIdx.x; q < N2 * N1; q += FT) o[q] = acc[q];
-        return;
-    }
-    // partial transform along x into sub: T1[y][q1 + Q1]
-    const int W1 = 2 * Q1 + 1, W2 = 2 * Q2 + 1;
-    for (int idx = threadIdx.x; idx < N2 * W1; idx += FT) {
-        const int y = idx / W1, q1 = idx - y * W1 - Q1;
-        double sr = 0.0, si = 0.0;
-        for (int x = 0; x < N1; x++) {
-            int e = (q1 * x) % N1;
-            if (e < 0) e += N1;
-            const cplx<R> w1 = tw1[e];  // exp(+2 pi i e/N1); use the conjugate
-            const double a = acc[y * N1 + x];
-            sr += a * w1.x;
-            si -= a * w1.y;
-        }
-        sub[idx] = mk<R>(sr, si);
-    }
     __syncthreads();
-    double2 *out = t2 + ((long)grp * n3 + z) * W2 * W1;
-    for (int idx = threadIdx.x; idx < W2 * W1; idx += FT) {
-        const int q2 = idx / W1 - Q2, q1i = idx - (idx / W1) * W1;
-        double sr = 0.0, si = 0.0;
-        for (int y = 0; y < N2; y++) {
-            int e = (q2 * y) % N2;
-            if (e < 0) e += N2;
-            const cplx<R> w2 = tw2[e];
-            const cplx<R> a = sub[y * W1 + q1i];
-            // a * conj(w2)
-            sr += a.x * w2.x + a.y * w2.y;
-            si += a.y * w2.x - a.x * w2.y;
-        }
-        out[idx] = make_double2(sr, si);
-    }
+    double *o = rhor + ((long)grp * n3 + z) * (N2 * N1);
+    for (int q = threadIdx.x; q < N2 * N1; q += FT) o[q] = acc[q];
 }
 
-// Register-line variant of the density pass of k_density_fast (the line
-// layout of k_plane_reg): per (z, band group) each band's y/x-box sub-plane
-// (LDS, S = nx + 2 columns with a zero column) goes through the inverse y and
-// x transforms in registers.  An x-row task keeps the same rows for every band
-// of the group, so occ |psi(x, y)|^2 accumulates in the registers of the lane
-// that holds (x, y) (x = MX k2 + k after the decimation-in-frequency
-// transform), and each block writes its rho(x, y) plane once:
-// rhor[grp][z][y][x], summed over groups in a fixed order afterwards.
+// Register-line variant of the density pass (the line layout of k_plane_reg):
+// per (z, band group) each band's y/x-box sub-plane (LDS, with a zero column)
+// goes through the inverse y and x transforms.  An x-row task keeps the same
+// rows for every band of the group, so occ |psi(x, y)|^2 accumulates in the
+// registers of the lane that holds (x, y) (x = MX k2 + k after the
+// decimation-in-frequency transform), and each block writes its rho(x, y) plane
+// once: rhor[grp][z][y][x], summed over groups in a fixed order afterwards.
 // Grid: n3 * ceil(nb / bpg) blocks of T threads.
-// CS: the sphere box lies inside N/4 (checked by the caller) and the row
-// stride is the compile-time pr_sub_stride<N>() instead of the argument.
-template <int N, int GX, int GY, int T, int W, bool CS = false>
+// PR: the sphere box lies inside N/4 (checked by the caller): row stride at
+// compile time (SC), and the register slots that hold only x (y) outside the box
+// are known zeros (as in k_plane_reg).  YW: y lines by the wave-exchanged LDS
+// transform (GY unused).
+// Bound by FP64 issue of the transforms, so the work of a band is what counts:
+// the z-column map is read once per block and the columns of the next band are
+// loaded while this one is transformed, where the registers allow it.
+template <int N, int GX, int GY, int T, int W, bool YW, bool PR, int SC>
 __global__ __launch_bounds__(T, W) void k_density_reg(const cplx<double> *__restrict__ colbuf,
                                                    const int *__restrict__ col_uy,
                                                    const double *__restrict__ occ,
@@ -140,8 +106,10 @@ __global__ __launch_bounds__(T, W) void k_density_reg(const cplx<double> *__rest
                                                    int bpg, int S_arg, double *__restrict__ rhor) {
     typedef double R;
     static_assert(N % GX == 0 && N % GY == 0 && T % 64 == 0, "bad plane shape");
-    const int S = CS ? pr_sub_stride<N>() : S_arg;
+    const int S = SC ? SC : S_arg;
     constexpr int MX = N / GX, MY = N / GY;
+    constexpr u64mask XB = PR ? box_slots(N, GX, MX, N / 4) : full_mask(MX);
+    constexpr u64mask YB = PR ? box_slots(N, GY, MY, N / 4) : full_mask(MY);
     constexpr int TX = T / GX;                 // x-row tasks per round
     constexpr int RPT = (N + TX - 1) / TX;     // rows per x task
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -152,28 +120,66 @@ __global__ __launch_bounds__(T, W) void k_density_reg(const cplx<double> *__rest
     const int b0 = grp * bpg, b1 = min(nb, b0 + bpg);
     const int nx = g.nx, kd1 = g.kd[0], ushift = N - nx, xhi = N - kd1;
     const int tid = threadIdx.x;
+    // NPRE columns per thread go through registers (clamped: ncol >= 1), the others
+    // through gather_plane; p0..p3: their places in the sub-plane
+    // (named values of a vector type: arrays and structures go to scratch memory)
+    typedef double V2 __attribute__((ext_vector_type(2)));
+    constexpr int NPRE = 4;
+    const long bstep = (long)n3 * g.ncolp;
+    const cplx<R> *cb = colbuf + ((long)b0 * n3 + z) * g.ncolp;
+    const int c0 = min(tid, g.ncol - 1), c1 = min(tid + T, g.ncol - 1), c2 = min(tid + 2 * T, g.ncol - 1),
+              c3 = min(tid + 3 * T, g.ncol - 1);
+    const auto place = [&](int c) {
+        const int uy = col_uy[c];
+        return (uy >> 16) * S + (uy & 0xffff);
+    };
+    const int p0 = place(c0), p1 = place(c1), p2 = place(c2), p3 = place(c3);
+    const auto col = [](const cplx<R> *p) { return *reinterpret_cast<const V2 *>(p); };
+    V2 q0, q1, q2, q3;
+    const auto fetch = [&](const cplx<R> *p) {
+        q0 = col(p + c0);
+        q1 = col(p + c1);
+        q2 = col(p + c2);
+        q3 = col(p + c3);
+    };
+    // one band ahead where the registers last (with 9 and more values per lane
+    // at 3 waves per SIMD they spill: there before the sub-plane is cleared)
+    constexpr bool AHEAD = MX <= 8 || W <= 2;
+    if (AHEAD) fetch(cb);
     load_twiddles(twN, twg, N);
     const Lanes<R, GX> LX;
-    const Lanes<R, GY> LY;
     R racc[RPT][MX];
 #pragma unroll
     for (int r = 0; r < RPT; r++)
 #pragma unroll
         for (int k = 0; k < MX; k++) racc[r][k] = 0.0;
-    for (int b = b0; b < b1; b++) {
+    for (int b = b0; b < b1; b++, cb += bstep) {
+        if (!AHEAD) fetch(cb);
         for (int q = tid; q < N * S; q += T) sub[q] = mk<R>(0, 0);
         __syncthreads();
-        gather_plane<R, T>(sub, colbuf + ((long)b * n3 + z) * g.ncolp, col_uy, g.ncol, S, 0);
+        // (a clamped column is stored again by its own thread with the same value)
+        sub[p0] = mk<R>(q0.x, q0.y);
+        sub[p1] = mk<R>(q1.x, q1.y);
+        sub[p2] = mk<R>(q2.x, q2.y);
+        sub[p3] = mk<R>(q3.x, q3.y);
+        gather_plane<R, T>(sub, cb, col_uy, g.ncol, S, NPRE * T);
         __syncthreads();
+        if (AHEAD) fetch(b + 1 < b1 ? cb + bstep : cb);  // the last band: its own again, unused
         // inverse y on the nx box lines
-        for (int u = tid / GY; u < nx; u += T / GY) {
-            cplx<R> *col = sub + u;
-            cplx<R> v[MY];
+        if constexpr (YW) {
+            line_fft_wave<R, N, +1, T>(sub, nx, 1, S, twN);
+        } else {
+            const Lanes<R, GY> LY;
+            for (int u = tid / GY; u < nx; u += T / GY) {
+                cplx<R> *col = sub + u;
+                cplx<R> v[MY];
 #pragma unroll
-            for (int j = 0; j < MY; j++) v[j] = col[(LY.g + GY * j) * S];
-            line_dif<+1, GY, MY>(v, LY, twN);
+                for (int j = 0; j < MY; j++)
+                    if (has_bit(YB, j)) v[j] = col[(LY.g + GY * j) * S];
+                line_dif<+1, GY, MY, R, YB>(v, LY, twN);
 #pragma unroll
-            for (int k = 0; k < MY; k++) col[(k + MY * LY.k2) * S] = v[k];
+                for (int k = 0; k < MY; k++) col[(k + MY * LY.k2) * S] = v[k];
+            }
         }
         __syncthreads();
         // inverse x per row, occ |psi|^2 into the row's registers
@@ -187,9 +193,9 @@ __global__ __launch_bounds__(T, W) void k_density_reg(const cplx<double> *__rest
 #pragma unroll
                 for (int j = 0; j < MX; j++) {
                     const int x = LX.g + GX * j;
-                    v[j] = row[x <= kd1 ? x : x >= xhi ? x - ushift : nx];
+                    if (has_bit(XB, j)) v[j] = row[x <= kd1 ? x : x >= xhi ? x - ushift : nx];
                 }
-                line_dif<+1, GX, MX>(v, LX, twN);
+                line_dif<+1, GX, MX, R, XB>(v, LX, twN);
 #pragma unroll
                 for (int k = 0; k < MX; k++) racc[r][k] += w * (v[k].x * v[k].x + v[k].y * v[k].y);
             }

@@ -17,8 +17,8 @@ template int launch_plane_spin<float, CPW_N>(cpwgpu_plan_s *, cplx<float> *, con
                                              hipStream_t);
 template int launch_plane_spin<double, CPW_N>(cpwgpu_plan_s *, cplx<double> *, const double *, long, int, int,
                                               hipStream_t);
-template int launch_density<CPW_N>(cpwgpu_plan_s *, const cplx<double> *, const double *, int, int, int, int, int,
-                                   double2 *, hipStream_t, double *);
+template int launch_density<CPW_N>(cpwgpu_plan_s *, const cplx<double> *, const double *, int, int, hipStream_t,
+                                   double *);
 #endif
 
 }  // namespace cpwgpu

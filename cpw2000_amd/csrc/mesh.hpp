@@ -168,20 +168,50 @@ template <typename R, int N> constexpr bool spin_reg_ok() {
     return reg_ok<R, N, SpinShape<R>::GX, SpinShape<R>::GY>();
 }
 
-// register shape of the density pass: x lanes, y lanes, waves per SIMD
-constexpr int DEN_GX = 8, DEN_GY = 8, DEN_W = 3;
-// threads of the register density pass for line length N: the smallest of 256,
-// 320 and 384 that keeps a lane's row accumulators (rows per x task x N / GX
-// doubles) within 27, for lines of at most 10 values per lane: spill-free at 3
-// waves per SIMD (24-72: 256, 80: 320); 0 = not built (96 and 128 spill, 108 has
-// no 8-lane split: k_density_fast)
-template <int N> constexpr int den_threads() {
-    if (!reg_ok<double, N, DEN_GX, DEN_GY>() || N / DEN_GX > 10) return 0;
+// Register shapes of the density pass: 8 lanes per line, den_threads() threads,
+// den_waves() waves per SIMD, row stride den_stride() for a box inside N/4 (0:
+// any box, the stride an argument).  Threads: the smallest of 256, 320 and 384
+// that keeps a lane's row accumulators (rows per x task x N / 8 doubles) within
+// 27, for lines of at most 10 values per lane (24-72: 256, 80: 320).  For a box
+// inside N/4 also 96, at 2 waves per SIMD, and 80 takes 256 threads and the
+// tighter stride: three blocks per CU instead of two (128 bands 306 -> 220 us).
+// 72, 128 bands: 158 us before the pruning and the whole rounds, 128 with them.
+// 108 has no 8-lane split and 128 no room for its accumulators: k_density_fast.
+constexpr int DEN_G = 8;
+template <int N> constexpr int den_threads(bool pr) {
+    if (!reg_ok<double, N, DEN_G, DEN_G>()) return 0;
+    if (pr && (N == 80 || N == 96)) return 256;
+    if (N / DEN_G > 10) return 0;
     for (int t : {256, 320, 384})
-        if (((N + t / DEN_GX - 1) / (t / DEN_GX)) * (N / DEN_GX) <= 27) return t;
+        if (((N + t / DEN_G - 1) / (t / DEN_G)) * (N / DEN_G) <= 27) return t;
     return 0;
 }
-template <int N> constexpr bool den_reg_ok() { return den_threads<N>() > 0; }
+template <int N> constexpr int den_waves() { return N / DEN_G > 10 ? 2 : 3; }
+template <int N> constexpr int den_stride() { return N == 80 ? N / 2 + 1 : pr_sub_stride<N>(); }
+template <int N> bool den_prune_fits(const FftGeom &g) { return prune_fits(g) && reg_stride(g.nx) <= den_stride<N>(); }
+template <int N> constexpr bool den_reg_ok(bool pr) { return den_threads<N>(pr) > 0; }
+// Bands per group of the density pass: a block takes one plane of a group, so
+// the groups are chosen to fill whole rounds of the blocks that fit on the GPU at
+// once (half a band more per round for its start and its plane of output).  72,
+// 128 bands: 10 groups of 13 in one round; groups of 8 took two.
+template <int N> int den_bands_per_group(const FftGeom &g, int nb) {
+    const bool pr = den_prune_fits<N>(g);
+    if (!den_reg_ok<N>(pr)) return 8;
+    const long lds = 16 * ((long)N + (long)N * (pr ? den_stride<N>() : reg_stride(g.nx)));
+    const int wpb = den_threads<N>(pr) / 64;
+    const long slots = 256 * std::max(1L, std::min<long>(160 * 1024 / lds, 4 * den_waves<N>() / wpb));
+    int best = 1;
+    double cost = HUGE_VAL;
+    for (int bpg = std::max(1, nb / 64); bpg <= nb; bpg++) {
+        const long ngrp = (nb + bpg - 1) / bpg;
+        const double c = (double)((g.n[2] * ngrp + slots - 1) / slots) * (bpg + 0.5);
+        if (c < cost) {
+            cost = c;
+            best = bpg;
+        }
+    }
+    return best;
+}
 
 // launchers (mesh_launch.hpp); v: the plane variant, resolved for the mesh
 template <typename R, int N>
@@ -194,7 +224,7 @@ int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R 
 template <typename R, int N>
 int launch_plane_spin(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair, int var, hipStream_t s);
 template <int N>
-int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg,
-                   int ngrp, int Q1, int Q2, double2 *t2, hipStream_t s, double *rhor = nullptr);
+int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg, hipStream_t s,
+                   double *rhor);
 
 }  // namespace cpwgpu

@@ -218,37 +218,34 @@ int launch_plane_spin(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstri
 }
 
 template <int N>
-int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg,
-                   int ngrp, int Q1, int Q2, double2 *t2, hipStream_t s, double *rhor) {
+int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *occ, int nb, int bpg, hipStream_t s,
+                   double *rhor) {
     const FftGeom &g = p->g;
-    if constexpr (den_reg_ok<N>()) {
-        if (rhor) {
-            // the density planes alone: register lines, accumulation in registers
-            constexpr int DT = den_threads<N>();
-            // a box inside N/4: the compile-time row stride
-            const bool cs = prune_fits(g);
-            const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
-            const size_t dyn = 16 * ((size_t)N + (size_t)N * S);
-            if (dyn > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
-            static bool attr_r = false;
-            if (!attr_r) {
-                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                HIPCHK(hipFuncSetAttribute((const void *)k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-                attr_r = true;
-            }
-            if (cs)
-                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, true>), dim3(g.n[2] * ngrp),
-                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
-                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
-            else
-                hipLaunchKernelGGL((k_density_reg<N, DEN_GX, DEN_GY, DT, DEN_W, false>), dim3(g.n[2] * ngrp),
-                                   dim3(DT), dyn, s, colbuf, (const int *)p->col_uy.p, occ,
-                                   (const double2 *)p->tw[0].p, g, nb, bpg, S, rhor);
-            HIPCHK(hipGetLastError());
-            return CPWGPU_OK;
+    const bool pr = den_prune_fits<N>(g);
+    const int ngrp = (nb + bpg - 1) / bpg;
+    const int *uy = (const int *)p->col_uy.p;
+    const double2 *tw = (const double2 *)p->tw[0].p;
+    const auto go = [&](auto kernel, int S, int T, bool &attr) -> int {
+        const size_t dyn = 16 * ((size_t)N + (size_t)N * S);
+        if (dyn > 160 * 1024) return fail(CPWGPU_ERR_SIZE, "density plane %d does not fit in LDS", N);
+        if (!attr) {
+            HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            attr = true;
         }
+        hipLaunchKernelGGL(kernel, dim3(g.n[2] * ngrp), dim3(T), dyn, s, colbuf, uy, occ, tw, g, nb, bpg, S, rhor);
+        HIPCHK(hipGetLastError());
+        return CPWGPU_OK;
+    };
+    constexpr int G = DEN_G;
+    if constexpr (den_reg_ok<N>(true)) {
+        static bool attr_p = false;
+        constexpr int T = den_threads<N>(true), SC = den_stride<N>();
+        if (pr) return go(k_density_reg<N, G, G, T, den_waves<N>(), true, true, SC>, SC, T, attr_p);
+    }
+    if constexpr (den_reg_ok<N>(false)) {
+        static bool attr_u = false;
+        constexpr int T = den_threads<N>(false);
+        return go(k_density_reg<N, G, G, T, den_waves<N>(), false, false, 0>, reg_stride(g.nx), T, attr_u);
     }
     constexpr int RB = plane_rows_fast<N>();
     const size_t dyn = 16 * ((size_t)N * (g.nx | 1) + (size_t)RB * row_stride<N>()) + 8 * (size_t)N * N;
@@ -260,9 +257,8 @@ int launch_density(cpwgpu_plan_s *p, const cplx<double> *colbuf, const double *o
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024 - stat)));
         attr = true;
     }
-    hipLaunchKernelGGL((k_density_fast<N, N>), dim3(g.n[2] * ngrp), dim3(FT), dyn, s, colbuf,
-                       (const int *)p->col_uy.p, occ, (const double2 *)p->tw[0].p,
-                       (const double2 *)p->tw[1].p, g, nb, bpg, Q1, Q2, t2, rhor);
+    hipLaunchKernelGGL((k_density_fast<N, N>), dim3(g.n[2] * ngrp), dim3(FT), dyn, s, colbuf, uy, occ, tw,
+                       (const double2 *)p->tw[1].p, g, nb, bpg, rhor);
     HIPCHK(hipGetLastError());
     return CPWGPU_OK;
 }

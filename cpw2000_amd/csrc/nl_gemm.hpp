@@ -102,8 +102,8 @@ template <typename R> constexpr int proj_bm() { return 2 * GemmCfg<R>::WM * 16; 
 template <typename R> constexpr int proj_bn() { return 2 * GemmCfg<R>::WN * 16; }
 
 // ---------------------------------------------------------------------------
-// k_proj: part[s][n][a] = sum_{i in slice s} w_i conj(anlga[i,a]) psi[i,n]
-// (w_i = 1 without wrow) grid (ceil(nanl/BM), ceil(neig/BN), nslice); 4 waves,
+// k_proj: part[s][n][a] = sum_{i in slice s} conj(anlga[i,a]) psi[i,n]
+// grid (ceil(nanl/BM), ceil(neig/BN), nslice); 4 waves,
 // each WM*16 a x WN*16 n
 // (FP32: block 128 x 128, so a K slice of anlga and psi is read at most
 // twice).  Double-buffered LDS: one barrier per K stage, the next stage's
@@ -115,9 +115,7 @@ template <typename R, int WMX = GemmCfg<R>::WM, int WNX = GemmCfg<R>::WN>
 __global__ __launch_bounds__(GEMM_THREADS) void k_proj(const cplx<R> *__restrict__ anl, long lda,
                                                        const double2 *__restrict__ psi, long ldp,
                                                        cplx<R> *__restrict__ part, int mtxd,
-                                                       int nanl, int neig, int kslice,
-                                                       const double *__restrict__ wrow = nullptr,
-                                                       int lower = 0) {
+                                                       int nanl, int neig, int kslice, int lower = 0) {
     typedef typename MF<R>::v4 v4;
     constexpr int WM = WMX, WN = WNX;
     constexpr int BK = GemmCfg<R>::BK, KP = GemmCfg<R>::KP;
@@ -171,10 +169,6 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_proj(const cplx<R> *__restrict
                 const double2 v = psi[bbase + min(i, mtxd - 1)];
                 rb[q] = make_double2(i < ke ? v.x : 0.0, i < ke ? v.y : 0.0);
             }
-        }
-        if (wrow) {  // per-plane-wave weight on the projector operand
-#pragma unroll
-            for (int q = 0; q < LPA; q++) ra[q] = scale(ra[q], (R)wrow[min(k0 + aoff + q, mtxd - 1)]);
         }
     };
     auto sstore = [&](int buf) {
@@ -328,8 +322,7 @@ __device__ __forceinline__ void load_psi_tail(double2 (&dst)[KPL], const double2
 template <typename R, int V>
 __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_direct(
     const cplx<R> *__restrict__ anl, long lda, const double2 *__restrict__ psi, long ldp,
-    cplx<R> *__restrict__ part, int mtxd, int nanl, int neig, int kslice,
-    const double *__restrict__ wrow = nullptr, int lower = 0) {
+    cplx<R> *__restrict__ part, int mtxd, int nanl, int neig, int kslice, int lower = 0) {
     typedef typename MF<R>::v4 v4;
     constexpr int WM = DirectCfg<R, V>::WM, WN = DirectCfg<R, V>::WN;
     constexpr int KPL = DirectCfg<R, V>::KPL, KC = 4 * KPL;
@@ -381,15 +374,6 @@ __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_dir
 #pragma unroll
             for (int t = 0; t < WN; t++) load_psi_tail<KPL>(rb_[t], bcol[t], i0, ke, mtxd);
         }
-        if (wrow) {
-            // per-plane-wave weight w_i on the projector operand (zeros stay zero)
-#pragma unroll
-            for (int u = 0; u < KPL; u++) {
-                const R w = (R)wrow[min(i0 + u, mtxd - 1)];
-#pragma unroll
-                for (int t = 0; t < WM; t++) ra_[t][u] = scale(ra_[t][u], w);
-            }
-        }
     };
     auto compute = [&](const cplx<R>(&ra_)[WM][KPL], const double2(&rb_)[WN][KPL]) {
 #pragma unroll
@@ -421,7 +405,9 @@ __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_dir
     // c + D - 1 is loaded while chunk c is multiplied, unconditionally (at
     // the last full chunk again when there is none: a valid address whose
     // values go unused), so that the loop body is one straight block and each
-    // chunk's loads have D - 1 chunks of MFMAs to arrive.  Then the partial
+    // chunk's loads have D - 1 chunks of MFMAs to arrive.  The scheduling barrier
+    // keeps the loads above those MFMAs: without it the compiler sinks them to
+    // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122).  Then the partial
     // chunk, if any.  Chunks are accumulated in K order for any D.
     const int nfull = max(0, ke - kb) / KC;
     if (nfull > 0) {
@@ -432,6 +418,7 @@ __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_dir
 #pragma unroll
             for (int j = 0; j < D; j++) {
                 load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
+                __builtin_amdgcn_sched_barrier(0);
                 compute(ra[j], rb[j]);
             }
         }
@@ -776,6 +763,7 @@ __global__ __launch_bounds__(GEMM_THREADS, (BackDirectCfg<R, V>::W)) void k_back
 #pragma unroll
             for (int j = 0; j < D; j++) {
                 load(dv[(j + D - 1) % D], av[(j + D - 1) % D], min(c + j + D - 1, nfull - 1) * KC, false);
+                __builtin_amdgcn_sched_barrier(0);  // as in k_proj_direct
                 compute(dv[j], av[j]);
             }
         }
