@@ -377,7 +377,7 @@ struct Work {
     size_t part_n = 0;
     void *dhd = nullptr;
     size_t dhd_n = 0;
-    bool lean = false;  // split-K partials of one round of blocks only (splitk_shape)
+    bool lean = false;  // split-K partials of one round of blocks only (proj_shape)
 };
 
 // Block tile (BM x BN) and K granule of the projection kernel variant pv.
@@ -391,79 +391,117 @@ template <typename R> void proj_tile(int pv, int *BM, int *BN, int *BK) {
     }
 #define CPW_PD(V) if (pv == V) { *BM = direct_bm<R, V>(); *BN = direct_bn<R, V>(); *BK = direct_bk<R, V>(); }
     CPW_PD(1) CPW_PD(2) CPW_PD(3) CPW_PD(4)
+    CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
 #undef CPW_PD
 }
 
-// Projection kernel of the plan for precision R and nanl projectors x neig
-// bands.  Default: the direct kernel with 64 x 64 (FP32 128 x 64) tiles per
-// block, and in FP64 with at most 32 bands a shape 32 bands wide, whose tiles
-// are not half padding.  us, LDS-staged k_proj / default: FP64 23,928 plane waves
-// x 256 projectors x 128 bands 161 / 92, x 24 bands 79 / 31 (64-wide: 41),
-// 80,852 x 864 x 256 4021 / 2072; FP32 23,928 x 256 x 128 75 / 49, x 64 66 / 28.
-template <typename R> int proj_variant(const cpwgpu_plan_s *p, int nanl, int neig) {
-    const int ix = sizeof(R) == 4 ? 1 : 0;
-    if (p->proj_var[ix] >= 0) return p->proj_var[ix] < NPROJ_VAR ? p->proj_var[ix] : 0;
-    if (sizeof(R) == 4 || neig > 32) return 1;
-    return nanl >= 256 ? 3 : 4;
-}
-
-// Back-projection kernel for rows plane waves and neig bands.  FP32: LDS-staged
-// with half chunks (54 us against 62-82 of the others at 23,928 x 256 x 128, 33
-// against 34-47 at 24 bands).  FP64: direct with 128 plane waves x 32 bands per
-// block; where that makes fewer than 2 blocks per CU, 64 x 32 (96 / 114 us at 128
-// bands, 59 / 57 at 64, 20 / 14 at 7,550 x 128 x 20; LDS-staged 141 / 91 / 23).
+// Back-projection kernel for rows plane waves and neig bands.  FP64: direct with
+// 128 plane waves x 32 bands per block, or 64 x 16 where fewer bands are padded and
+// fewer compute units idle in the last round of blocks: both are counted in whole
+// rounds of the 256 CUs, a quarter of the work and 1.35 times the time per flop
+// for the small one, while the large one makes few rounds (the small one rereads
+// the projectors once per 16 bands).  us, 128 x 32 / 64 x 16: 23,928 plane waves x
+// 256 projectors x 16 bands 30 / 22, x 40 57 / 47, x 72 82 / 75, x 100 84 / 101;
+// 7,550 x 128 x 20 18 / 8, x 100 21 / 23; 80,852 x 864 x 72 656 / 861.
+// FP32: LDS-staged with half chunks, 16, 32 or 48 bands per block: what pads least,
+// 6% per flop against the narrow one where more than 3 tiles of bands are full.
+// us at 64 / 48 / 32 / 16 bands per block: 23,928 x 256 x 16 37 / 29 / 22 / 15, x 72
+// 60 / 43 / 48 / 42, x 128 61 / 68 / 58 / 61, x 144 91 / 67 / 72 / 70.
 template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int neig) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
     if (p->back_var[ix] >= 0) return p->back_var[ix] < NBACK_VAR ? p->back_var[ix] : 0;
-    if (sizeof(R) == 4) return NBACK_DIRECT + 1;
-    const long blocks = (long)((rows + back_bi<double, 2>() - 1) / back_bi<double, 2>()) *
-                        ((neig + back_bn<double, 2>() - 1) / back_bn<double, 2>());
-    return blocks < 512 ? 3 : 2;
+    if (sizeof(R) == 4) {
+        const int t = (neig + 15) / 16;
+        if (t <= 3) return BACK_BANDS + 1;
+        const double c1 = 1.06 * t, c2 = 2.0 * ((t + 1) / 2), c3 = 3.0 * ((t + 2) / 3);
+        return BACK_BANDS + (c1 < c2 && c1 < c3 ? 1 : c3 < c2 ? 3 : 2);
+    }
+    const long big = ((long)(rows + 127) / 128 * ((neig + 31) / 32) + 255) / 256;
+    const long small = ((long)(rows + 63) / 64 * ((neig + 15) / 16) + 255) / 256;
+    return big <= 3 && 0.25 * 1.35 * small < big ? BACK_BANDS + 1 : 2;
 }
 
-// Split-K shape of the projection GEMM over rows plane waves: number of K
+// Projection kernel and split-K shape of the projection GEMM over rows plane
+// waves, nanl projectors and neig bands: the kernel variant, the number of K
 // slices and rows per slice (whole LDS stages of k_proj / whole chunks of
-// k_proj_direct), for nanl projectors and neig bands.  A target set by the
-// caller is the number of blocks; the default counts rounds: the tiles of one
-// slice run one block per CU at a time on the matrix cores' clock, so the slices
-// are chosen among those that just fill 1, 2, ... rounds of the 256 CUs, and
-// each costs its partials (written and read once) and a step of the reduction.
+// k_proj_direct).  A target set by the caller is the number of blocks; the
+// default counts rounds: the tiles of one slice run one block per CU at a time on
+// the matrix cores' clock, so the slices are chosen among those that just fill
+// 1, 2, ... rounds of the 256 CUs, and each costs its partials (written and read
+// once) and a step of the reduction.
 // FP64 80,852 x 864 x 64 (14 tiles): 19 slices, 266 blocks, 951 us; 10 slices,
 // 140 blocks, 824 us; 18 slices (252 blocks) is what the rule takes.
+// Without a kernel set by the caller the same cost chooses it, among the direct
+// kernel with 64 (FP32 128) projectors x 64 bands per block and those 16, 32, 48
+// and 80 bands wide; slow is the time per flop of each relative to the first.  It
+// took the fastest at every size measured but three (within 7%): us, 64 wide /
+// chosen: FP64 23,928 x 256 x 16 41 / 26 (16 wide), x 72 90 / 68 (80), x 128 92 / 92;
+// 7,550 x 128 x 40 18 / 15 (16); 80,852 x 864 x 72 815 / 581 (80), x 144 1213 / 1062
+// (80); FP32 23,928 x 256 x 20 30 / 20 (32), x 72 49 / 43 (80); 7,550 x 128 x 128
+// 22 / 16 (16).
 // lean: as a target of 256 blocks, the smallest workspace.
-template <typename R> void splitk_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *nsl_out,
-                                        int *kslice_out, bool lean = false) {
-    int BM, BN, BK;
-    proj_tile<R>(proj_variant<R>(p, nanl, neig), &BM, &BN, &BK);
+template <typename R> struct ProjShapes;
+template <> struct ProjShapes<double> {
+    static constexpr double slow[5] = {1.0, 1.65, 1.22, 1.39, 1.18};
+};
+template <> struct ProjShapes<float> {
+    static constexpr double slow[5] = {1.0, 1.72, 1.36, 1.13, 1.01};
+};
+constexpr int PROJ_AUTO[5] = {1, PROJ_BANDS + 1, PROJ_BANDS + 2, PROJ_BANDS + 3, PROJ_BANDS + 5};
+
+// estimated us of the projection with block tile BM x BN and K granule BK, and
+// its number of slices
+template <typename R> double proj_cost(int BM, int BN, int BK, double slow, int rows, int nanl, int neig, int *nsl) {
+    constexpr long CUS = 256;
+    const long tiles = (long)((nanl + BM - 1) / BM) * ((neig + BN - 1) / BN);
+    const long ksteps = (rows + BK - 1) / BK;
+    // us of one K step on one CU (6 of the 8 flops of a complex product, at
+    // 0.7 of the matrix peak) and of one slice's partials
+    const double step = slow * 6.0 * BM * BN * BK / (sizeof(R) == 8 ? 2.1e5 : 4.2e5);
+    const double per = 0.04 + 2.0 * sizeof(cplx<R>) * nanl * neig / 6e6;
+    double best = HUGE_VAL;
+    const auto consider = [&](long n) {
+        n = std::max(1L, std::min<long>(n, ksteps));
+        const long len = (ksteps + n - 1) / n;
+        const double cost = (double)((tiles * n + CUS - 1) / CUS) * len * step + n * per;
+        if (cost < best) {
+            best = cost;
+            *nsl = (int)n;
+        }
+    };
+    // one round or less: the slice cost against the shortened K loop
+    consider(std::min(CUS / std::max(1L, tiles), (long)std::sqrt(ksteps * step / per) + 1));
+    for (long k = 1; k <= 8; k++) consider(CUS * k / tiles);
+    return best;
+}
+
+template <typename R> void proj_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *pv, int *nsl_out,
+                                      int *kslice_out, bool lean = false) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
+    const int set = p->proj_var[ix], target = p->splitk[ix] > 0 ? p->splitk[ix] : lean ? 256 : 0;
+    int BM, BN, BK, nsl = 1;
+    if (set >= 0) {
+        *pv = set < NPROJ_VAR ? set : 0;
+        proj_tile<R>(*pv, &BM, &BN, &BK);
+        if (target <= 0) proj_cost<R>(BM, BN, BK, 1.0, rows, nanl, neig, &nsl);
+    } else {
+        double best = HUGE_VAL;
+        *pv = 1;
+        for (int i = 0; i < 5; i++) {
+            int n;
+            proj_tile<R>(PROJ_AUTO[i], &BM, &BN, &BK);
+            const double c = proj_cost<R>(BM, BN, BK, ProjShapes<R>::slow[i], rows, nanl, neig, &n);
+            if (c < best) {
+                best = c;
+                *pv = PROJ_AUTO[i];
+                nsl = n;
+            }
+        }
+        proj_tile<R>(*pv, &BM, &BN, &BK);
+    }
     const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
     const int ksteps = (rows + BK - 1) / BK;
-    int nsl;
-    const int target = p->splitk[ix] > 0 ? p->splitk[ix] : lean ? 256 : 0;
-    if (target > 0) {
-        nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
-    } else {
-        constexpr long CUS = 256;
-        const long tiles = (long)tm * tn;
-        // us of one K step on one CU (6 of the 8 flops of a complex product, at
-        // 0.7 of the matrix peak) and of one slice's partials
-        const double step = 6.0 * BM * BN * BK / (sizeof(R) == 8 ? 2.1e5 : 4.2e5);
-        const double per = 0.04 + 2.0 * sizeof(cplx<R>) * nanl * neig / 6e6;
-        nsl = 1;
-        double best = HUGE_VAL;
-        const auto consider = [&](long n) {
-            n = std::max(1L, std::min<long>(n, ksteps));
-            const long len = (ksteps + n - 1) / n;
-            const double cost = (double)((tiles * n + CUS - 1) / CUS) * len * step + n * per;
-            if (cost < best) {
-                best = cost;
-                nsl = (int)n;
-            }
-        };
-        // one round or less: the slice cost against the shortened K loop
-        consider(std::min(CUS / std::max(1L, tiles), (long)std::sqrt(ksteps * step / per) + 1));
-        for (long k = 1; k <= 8; k++) consider(CUS * k / tiles);
-    }
+    if (target > 0) nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
     const int kslice = ((ksteps + nsl - 1) / nsl) * BK;
     *nsl_out = (rows + kslice - 1) / kslice;
     *kslice_out = kslice;
@@ -502,13 +540,10 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         anl = (const cplx<R> *)pv_.anl32->p;
     }
     const long lda = sizeof(R) == 8 ? pv_.lda : *pv_.lda32;
-    const int pv = proj_variant<R>(p, nanl, neig);
-    // block tile and K granule of the chosen projection kernel
-    int BM, BN, BK;
+    int pv, nsl, kslice, BM, BN, BK;
+    proj_shape<R>(p, rows, nanl, neig, &pv, &nsl, &kslice, w && w->lean);
     proj_tile<R>(pv, &BM, &BN, &BK);
     const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
-    int nsl, kslice;
-    splitk_shape<R>(p, rows, nanl, neig, &nsl, &kslice, w && w->lean);
     cplx<R> *part, *dhd;
     if (w) {
         if (cs * (size_t)nsl * neig * nanl > w->part_n || cs * (size_t)neig * nanl > w->dhd_n)
@@ -525,19 +560,18 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         const dim3 grid(tm, tn, nsl);
         const double2 *ps = (const double2 *)psi;
         cplx<R> *pt = part;
-        if (pv == 1)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 1>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
-        else if (pv == 2)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 2>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
-        else if (pv == 3)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 3>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
-        else if (pv == 4)
-            launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, 4>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
-        else if (pv == NPROJ_DIRECT + 1)
+#define CPW_PD(V)                                                                                                     \
+    if (pv == V)                                                                                                      \
+        launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, V>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, \
+                     nanl, neig, kslice, 0);
+        CPW_PD(1) CPW_PD(2) CPW_PD(3) CPW_PD(4)
+        CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
+#undef CPW_PD
+        if (pv == NPROJ_DIRECT + 1)
             launch_timed(CPWGPU_K_PROJ, (k_proj<R, proj_half_wm<R>(), proj_half_wn<R>()>), dim3(tm, tn, nsl),
                                dim3(GEMM_THREADS), 0, s, anl, lda, (const double2 *)psi, ldp,
                                pt, rows, nanl, neig, kslice, 0);
-        else
+        if (pv == 0)
             launch_timed(CPWGPU_K_PROJ, k_proj<R>, dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, s, anl, lda,
                                (const double2 *)psi, ldp, pt, rows, nanl, neig, kslice, 0);
     }
@@ -563,7 +597,15 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
                            dim3(GEMM_THREADS), 0, s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta, kp,   \
                            ldp, ek);
         CPW_BD(1) CPW_BD(2) CPW_BD(3)
+        if constexpr (sizeof(R) == 8) CPW_BD(BACK_BANDS + 1)
 #undef CPW_BD
+#define CPW_BL(NT)                                                                                            \
+    if (bv == BACK_BANDS + NT)                                                                                \
+        launch_timed(CPWGPU_K_BACK, (k_back<R, GemmCfg<R>::KC / 2, NT>),                                      \
+                     dim3((rows + BP_BI - 1) / BP_BI, (neig + 16 * NT - 1) / (16 * NT)), dim3(GEMM_THREADS), 0, \
+                     s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta, kp, ldp, ek);
+        if constexpr (sizeof(R) == 4) { CPW_BL(1) CPW_BL(2) CPW_BL(3) }
+#undef CPW_BL
         if (bv == 0)
             launch_timed(CPWGPU_K_BACK, k_back<R>, dim3((rows + BP_BI - 1) / BP_BI, (neig + BP_BN - 1) / BP_BN),
                                dim3(GEMM_THREADS), 0, s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta,
@@ -2279,12 +2321,13 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         // projection kernel x split-K target
         const int cand[4] = {128, 256, 512, 1024};
         best = 3.4e38f;
-        for (int jv = 0; jv < NPROJ_VAR; jv++)
+        for (int jv = -1; jv < NPROJ_VAR; jv++)
             for (int c : cand) {
+                if (jv < 0 && c != cand[0]) continue;  // the default chooses its own split
                 p->proj_var[ix] = jv;
-                p->splitk[ix] = c;
+                p->splitk[ix] = jv < 0 ? -1 : c;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
-                if (t < best) { best = t; best_sk = c; best_jv = jv; }
+                if (t < best) { best = t; best_sk = p->splitk[ix]; best_jv = jv; }
             }
     }
     p->proj_var[ix] = best_jv;
@@ -2292,7 +2335,7 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
     int best_bv = 0;
     if (p->nanl > 0) {
         best = 3.4e38f;
-        for (int bv = 0; bv < NBACK_VAR; bv++) {
+        for (int bv = -1; bv < NBACK_VAR; bv++) {
             p->back_var[ix] = bv;
             if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
             if (t < best) { best = t; best_bv = bv; }
@@ -2318,7 +2361,7 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &best))) return st;
         for (int sv = 1; sv <= 2; sv++) {
             p->sched_var[ix] = sv;
-            for (int bv = 0; bv < NBACK_VAR; bv++) {
+            for (int bv = -1; bv < NBACK_VAR; bv++) {
                 p->back_var[ix] = bv;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
                 if (t < best) { best = t; best_sv = sv; best_bv = bv; }
@@ -2370,18 +2413,19 @@ int tune_spin(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         const int cand[4] = {128, 256, 512, 1024};
         int best_jv = 0, best_sk = -1;
         best = 3.4e38f;
-        for (int jv = 0; jv < NPROJ_VAR; jv++)
+        for (int jv = -1; jv < NPROJ_VAR; jv++)
             for (int c : cand) {
+                if (jv < 0 && c != cand[0]) continue;  // the default chooses its own split
                 p->proj_var[ix] = jv;
-                p->splitk[ix] = c;
+                p->splitk[ix] = jv < 0 ? -1 : c;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t, true))) return st;
-                if (t < best) { best = t; best_sk = c; best_jv = jv; }
+                if (t < best) { best = t; best_sk = p->splitk[ix]; best_jv = jv; }
             }
         p->proj_var[ix] = best_jv;
         p->splitk[ix] = best_sk;
         int best_bv = 0;
         best = 3.4e38f;
-        for (int bv = 0; bv < NBACK_VAR; bv++) {
+        for (int bv = -1; bv < NBACK_VAR; bv++) {
             p->back_var[ix] = bv;
             if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t, true))) return st;
             if (t < best) { best = t; best_bv = bv; }
@@ -2429,8 +2473,8 @@ template <typename R> size_t noalloc_need(const cpwgpu_plan_s *p, int nb, bool l
     const size_t cs = sizeof(cplx<R>);
     size_t n = align256(cs * (size_t)p->g.n[2] * p->g.ncolp * nb);
     if (p->nanl > 0 && p->g.mtxd > 0) {
-        int nsl, kslice;
-        splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice, lean);
+        int pv, nsl, kslice;
+        proj_shape<R>(p, p->g.mtxd, p->nanl, nb, &pv, &nsl, &kslice, lean);
         n += align256(cs * (size_t)nsl * nb * p->nanl) + align256(cs * (size_t)nb * p->nanl);
     }
     return n;
@@ -2449,8 +2493,10 @@ int apply_noalloc_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, dou
         return fail(CPWGPU_ERR_SIZE, "one band needs %zu bytes of workspace, more than the %zu of the "
                                      "allocation-free entry point",
                     noalloc_need<R>(p, 1, true), NOALLOC_SCRATCH);
+    // the last chunk has to fit as well: its kernel may cut more slices
+    const auto fits_any = [&](int nb) { return nb == 0 || fits(nb, false) || fits(nb, true); };
     int nbc = neig;
-    while (nbc > 1 && !fits(nbc, false) && !fits(nbc, true)) nbc--;
+    while (nbc > 1 && !(fits_any(nbc) && fits_any(neig % nbc))) nbc--;
     for (int b0 = 0; b0 < neig; b0 += nbc) {
         const int nb = std::min(nbc, neig - b0);
         const size_t cs = sizeof(cplx<R>);
@@ -2460,8 +2506,8 @@ int apply_noalloc_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, dou
         w.colbuf_n = cs * (size_t)p->g.n[2] * p->g.ncolp * nb;
         size_t off = align256(w.colbuf_n);
         if (nl) {
-            int nsl, kslice;
-            splitk_shape<R>(p, p->g.mtxd, p->nanl, nb, &nsl, &kslice, w.lean);
+            int pv, nsl, kslice;
+            proj_shape<R>(p, p->g.mtxd, p->nanl, nb, &pv, &nsl, &kslice, w.lean);
             w.part = scr + off;
             w.part_n = cs * (size_t)nsl * nb * p->nanl;
             off += align256(w.part_n);
@@ -2966,11 +3012,11 @@ int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value) 
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_PROJ) {
-        *value = ix ? proj_variant<float>(plan, plan->nanl, INT_MAX) : proj_variant<double>(plan, plan->nanl, INT_MAX);
+        *value = plan->proj_var[ix] >= 0 ? std::min(plan->proj_var[ix], NPROJ_VAR - 1) : 1;
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_BACK) {
-        *value = ix ? back_variant<float>(plan, plan->mtxd, 1 << 20) : back_variant<double>(plan, plan->mtxd, 1 << 20);
+        *value = plan->back_var[ix] >= 0 ? std::min(plan->back_var[ix], NBACK_VAR - 1) : ix ? NBACK_DIRECT + 1 : 2;
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_KIN) {

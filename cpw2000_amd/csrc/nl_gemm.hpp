@@ -258,18 +258,23 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_proj(const cplx<R> *__restrict
 // buffering; a third buffer measured no faster on gfx950)
 constexpr int DIRECT_D = 2;
 constexpr int NPROJ_DIRECT = 4;
-template <typename R, int V> struct DirectCfg;
+constexpr int PROJ_BANDS = 16;
+// (WM*16) x (WN*16) per wave, GM waves along the projectors and 4 / GM along the
+// bands.  PROJ_BANDS + WN: WN band tiles, four waves along the projectors
+template <typename R, int V> struct DirectCfg {
+    static constexpr int GM = 4, WM = sizeof(R) == 4 ? 2 : 1, WN = V - PROJ_BANDS, KPL = 2, W = 2, D = DIRECT_D;
+};
 // (all compile without register spills on gfx950)
-template <> struct DirectCfg<float, 1> { static constexpr int WM = 4, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<float, 2> { static constexpr int WM = 4, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<float, 3> { static constexpr int WM = 2, WN = 2, KPL = 8, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<float, 4> { static constexpr int WM = 2, WN = 2, KPL = 4, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 1> { static constexpr int WM = 2, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 2> { static constexpr int WM = 2, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<double, 3> { static constexpr int WM = 4, WN = 1, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 4> { static constexpr int WM = 2, WN = 1, KPL = 4, W = 2, D = DIRECT_D; };
-template <typename R, int V> constexpr int direct_bm() { return 2 * DirectCfg<R, V>::WM * 16; }
-template <typename R, int V> constexpr int direct_bn() { return 2 * DirectCfg<R, V>::WN * 16; }
+template <> struct DirectCfg<float, 1> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
+template <> struct DirectCfg<float, 2> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
+template <> struct DirectCfg<float, 3> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 8, W = 1, D = DIRECT_D; };
+template <> struct DirectCfg<float, 4> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 2, D = DIRECT_D; };
+template <> struct DirectCfg<double, 1> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
+template <> struct DirectCfg<double, 2> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
+template <> struct DirectCfg<double, 3> { static constexpr int GM = 2, WM = 4, WN = 1, KPL = 2, W = 2, D = DIRECT_D; };
+template <> struct DirectCfg<double, 4> { static constexpr int GM = 2, WM = 2, WN = 1, KPL = 4, W = 2, D = DIRECT_D; };
+template <typename R, int V> constexpr int direct_bm() { return DirectCfg<R, V>::GM * DirectCfg<R, V>::WM * 16; }
+template <typename R, int V> constexpr int direct_bn() { return 4 / DirectCfg<R, V>::GM * DirectCfg<R, V>::WN * 16; }
 template <typename R, int V> constexpr int direct_bk() { return 4 * DirectCfg<R, V>::KPL; }
 
 // Chunk loads of the direct kernels.  Rows beyond the matrix (projectors
@@ -334,7 +339,8 @@ __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_dir
     if (lower && a0 + BM <= n0) return;
     const int kb = tl.z * kslice, ke = min(mtxd, kb + kslice);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
+    constexpr int GM = DirectCfg<R, V>::GM;
+    const int wm = wave % GM, wn = wave / GM;
     const int lr = lane & 15, lg = lane >> 4;
     const cplx<R> *arow[WM];
 #pragma unroll
@@ -517,7 +523,8 @@ constexpr int BP_BN = 64;  // bands per block
 // ---------------------------------------------------------------------------
 // KCX: projectors per LDS chunk (variant 0 uses GemmCfg<R>::KC; half of it
 // keeps fewer values in flight per lane, for more waves per SIMD)
-template <typename R, int KCX = GemmCfg<R>::KC>
+// NT: tiles of 16 bands per block
+template <typename R, int KCX = GemmCfg<R>::KC, int NT = BP_BN / 16>
 __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict__ anl, long lda,
                                                        const cplx<R> *__restrict__ dhd,
                                                        double2 *__restrict__ hpsi, long ldh,
@@ -530,37 +537,41 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict
     constexpr int KC = KCX, KCP = KCX + 16 / (int)sizeof(R);
     static_assert((KCP * sizeof(R) / 16) % 2 == 1 && KC % 16 == 0, "bad k_back chunk");
     constexpr int KPL = KC / 4;             // projectors per lane group per chunk
-    constexpr int DPT = BP_BN * KC / GEMM_THREADS;  // dhd values a thread stages
-    __shared__ __align__(16) R sD[3][BP_BN][KCP];   // re, im, re+im
+    constexpr int BN = 16 * NT;
+    constexpr int DPT = BN * KC / GEMM_THREADS;  // dhd values a thread stages
+    __shared__ __align__(16) R sD[3][BN][KCP];   // re, im, re+im
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 15, lg = lane >> 4;
     const Tile3 tl = gemm_tile_yfirst();
     const int i = tl.x * BP_BI + wave * 16 + lr;
-    const int n0 = tl.y * BP_BN;
-    v4 P1[4], P2[4], P3[4];
+    const int n0 = tl.y * BN;
+    v4 P1[NT], P2[NT], P3[NT];
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
+    for (int t = 0; t < NT; t++) {
         P1[t] = v4{0, 0, 0, 0};
         P2[t] = v4{0, 0, 0, 0};
         P3[t] = v4{0, 0, 0, 0};
     }
-    // staging of dhd: thread -> band row tid/4, projector offset (tid%4)*DPT
-    const int srow = threadIdx.x >> 2, soff = (threadIdx.x & 3) * DPT;
+    // staging of dhd: value q of a thread is projector tid % KC of band row
+    // tid / KC + q * (256 / KC)
+    constexpr int RPQ = GEMM_THREADS / KC;
+    static_assert(GEMM_THREADS % KC == 0 && BN % RPQ == 0, "bad k_back staging");
+    const int srow = threadIdx.x / KC, soff = threadIdx.x % KC;
     cplx<R> rd[DPT];
     // rows beyond the matrix (bands n >= neig, plane waves i >= mtxd) are
     // read at clamped addresses and only reach outputs that are not stored;
     // full chunks issue plain loads (first used after the current chunk's
     // MFMAs), the projector tail is clamped with dhd zero-masked
-    const long dbase = (long)min(n0 + srow, neig - 1) * nanl;
+    const auto dat = [&](int q, int a) { return (long)min(n0 + srow + q * RPQ, neig - 1) * nanl + a; };
     auto dload = [&](int ka) {
         if (ka + KC <= nanl) {  // the same for the whole block
 #pragma unroll
-            for (int q = 0; q < DPT; q++) rd[q] = dhd[dbase + ka + soff + q];
+            for (int q = 0; q < DPT; q++) rd[q] = dhd[dat(q, ka + soff)];
         } else {
 #pragma unroll
             for (int q = 0; q < DPT; q++) {
-                const int a = ka + soff + q;
-                const cplx<R> v = dhd[dbase + min(a, nanl - 1)];
+                const int a = ka + soff;
+                const cplx<R> v = dhd[dat(q, min(a, nanl - 1))];
                 rd[q] = mk<R>(a < nanl ? v.x : (R)0, a < nanl ? v.y : (R)0);
             }
         }
@@ -581,9 +592,9 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict
     for (int ka = 0; ka < nanl; ka += KC) {
 #pragma unroll
         for (int q = 0; q < DPT; q++) {
-            sD[0][srow][soff + q] = rd[q].x;
-            sD[1][srow][soff + q] = rd[q].y;
-            sD[2][srow][soff + q] = rd[q].x + rd[q].y;
+            sD[0][srow + q * RPQ][soff] = rd[q].x;
+            sD[1][srow + q * RPQ][soff] = rd[q].y;
+            sD[2][srow + q * RPQ][soff] = rd[q].x + rd[q].y;
         }
         __syncthreads();
         R cr[KPL], ci[KPL], cs[KPL];
@@ -598,7 +609,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict
             aload(ka + KC);
         }
 #pragma unroll
-        for (int ni = 0; ni < 4; ni++) {
+        for (int ni = 0; ni < NT; ni++) {
             R dr[KPL], di[KPL], ds[KPL];
 #pragma unroll
             for (int u = 0; u < KPL; u++) {
@@ -621,7 +632,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict
         // a row beyond neig is loaded and not used), then their stores
         const double ek = kpsi ? ekpg[i] : 0.0;
 #pragma unroll
-        for (int ni = 0; ni < 4; ni++) {
+        for (int ni = 0; ni < NT; ni++) {
             double2 kp[4], ho[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
@@ -654,7 +665,11 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict
 // lane per chunk, register budget for W waves per SIMD.  A block is 4 waves
 // along the plane waves: 64*IT plane waves x 16*NT bands.
 constexpr int NBACK_DIRECT = 3;
-template <typename R, int V> struct BackDirectCfg;
+constexpr int BACK_BANDS = 16;
+// BACK_BANDS + NT: NT band tiles, one tile of plane waves per wave
+template <typename R, int V> struct BackDirectCfg {
+    static constexpr int NT = V - BACK_BANDS, IT = 1, KPL = 2, W = V - BACK_BANDS > 3 ? 2 : 3, D = DIRECT_D;
+};
 // (all compile without register spills on gfx950)
 template <> struct BackDirectCfg<float, 1> { static constexpr int NT = 4, IT = 1, KPL = 4, W = 2, D = DIRECT_D; };
 template <> struct BackDirectCfg<float, 2> { static constexpr int NT = 4, IT = 2, KPL = 4, W = 2, D = DIRECT_D; };
