@@ -407,6 +407,11 @@ template <typename R> void proj_tile(int pv, int *BM, int *BN, int *BK) {
 // 6% per flop against the narrow one where more than 3 tiles of bands are full.
 // us at 64 / 48 / 32 / 16 bands per block: 23,928 x 256 x 16 37 / 29 / 22 / 15, x 72
 // 60 / 43 / 48 / 42, x 128 61 / 68 / 58 / 61, x 144 91 / 67 / 72 / 70.
+int back_shape64(int rows, int neig) {
+    const long big = ((long)(rows + 127) / 128 * ((neig + 31) / 32) + 255) / 256;
+    const long small = ((long)(rows + 63) / 64 * ((neig + 15) / 16) + 255) / 256;
+    return big <= 3 && 0.25 * 1.35 * small < big ? BACK_BANDS + 1 : 2;
+}
 template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int neig) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
     if (p->back_var[ix] >= 0) return p->back_var[ix] < NBACK_VAR ? p->back_var[ix] : 0;
@@ -416,9 +421,7 @@ template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int nei
         const double c1 = 1.06 * t, c2 = 2.0 * ((t + 1) / 2), c3 = 3.0 * ((t + 2) / 3);
         return BACK_BANDS + (c1 < c2 && c1 < c3 ? 1 : c3 < c2 ? 3 : 2);
     }
-    const long big = ((long)(rows + 127) / 128 * ((neig + 31) / 32) + 255) / 256;
-    const long small = ((long)(rows + 63) / 64 * ((neig + 15) / 16) + 255) / 256;
-    return big <= 3 && 0.25 * 1.35 * small < big ? BACK_BANDS + 1 : 2;
+    return back_shape64(rows, neig);
 }
 
 // Projection kernel and split-K shape of the projection GEMM over rows plane
@@ -475,6 +478,23 @@ template <typename R> double proj_cost(int BM, int BN, int BK, double slow, int 
     return best;
 }
 
+// the cheapest of PROJ_AUTO and its number of slices
+template <typename R> int proj_auto(int rows, int nanl, int neig, int *nsl) {
+    double best = HUGE_VAL;
+    int pv = 1;
+    for (int i = 0; i < 5; i++) {
+        int BM, BN, BK, n = 1;
+        proj_tile<R>(PROJ_AUTO[i], &BM, &BN, &BK);
+        const double c = proj_cost<R>(BM, BN, BK, ProjShapes<R>::slow[i], rows, nanl, neig, &n);
+        if (c < best) {
+            best = c;
+            pv = PROJ_AUTO[i];
+            *nsl = n;
+        }
+    }
+    return pv;
+}
+
 template <typename R> void proj_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *pv, int *nsl_out,
                                       int *kslice_out, bool lean = false) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
@@ -485,18 +505,7 @@ template <typename R> void proj_shape(const cpwgpu_plan_s *p, int rows, int nanl
         proj_tile<R>(*pv, &BM, &BN, &BK);
         if (target <= 0) proj_cost<R>(BM, BN, BK, 1.0, rows, nanl, neig, &nsl);
     } else {
-        double best = HUGE_VAL;
-        *pv = 1;
-        for (int i = 0; i < 5; i++) {
-            int n;
-            proj_tile<R>(PROJ_AUTO[i], &BM, &BN, &BK);
-            const double c = proj_cost<R>(BM, BN, BK, ProjShapes<R>::slow[i], rows, nanl, neig, &n);
-            if (c < best) {
-                best = c;
-                *pv = PROJ_AUTO[i];
-                nsl = n;
-            }
-        }
+        *pv = proj_auto<R>(rows, nanl, neig, &nsl);
         proj_tile<R>(*pv, &BM, &BN, &BK);
     }
     const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
@@ -1206,22 +1215,30 @@ struct Subspace {
 // LDS-staged kernels).
 constexpr int SUB_PROJ_V = 2, SUB_BACK_V = 2;
 
-// split-K partials of a^H b (na x nbc over mtxd rows) into part; returns the number of slices in *nsl
+// split-K partials of a^H b (na x nbc over mtxd rows) into part; returns the
+// number of slices in *nsl.  by_size: the projection's choice of shape and slices;
+// else shape SUB_PROJ_V in slices that make 256 blocks (Rayleigh-Ritz: its vectors'
+// phases follow the rounding of the Gram matrices).
 int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb, int nbc, int mtxd,
-                  DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0) {
-    constexpr int BM = direct_bm<double, SUB_PROJ_V>(), BN = direct_bn<double, SUB_PROJ_V>();
-    constexpr int BK = direct_bk<double, SUB_PROJ_V>();
+                  DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0, bool by_size = false) {
+    int BM, BN, BK, nsl = 1;
+    const int pv = by_size ? proj_auto<double>(mtxd, na, nbc, &nsl) : SUB_PROJ_V;
+    proj_tile<double>(pv, &BM, &BN, &BK);
     const int tm = (na + BM - 1) / BM, tn = (nbc + BN - 1) / BN;
     const int ksteps = (mtxd + BK - 1) / BK;
-    int nsl = std::max(1, std::min(ksteps, (256 + tm * tn - 1) / (tm * tn)));
+    if (!by_size) nsl = std::max(1, std::min(ksteps, (256 + tm * tn - 1) / (tm * tn)));
     // slices are whole K chunks of the kernel
     const int kslice = ((ksteps + nsl - 1) / nsl) * BK;
     nsl = (mtxd + kslice - 1) / kslice;
     int rc;
     if ((rc = part.reserve(16 * (size_t)nsl * na * nbc))) return rc;
-    hipLaunchKernelGGL((k_proj_direct<double, SUB_PROJ_V>), dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, st,
-                       (const cplx<double> *)a, lda, b, ldb, (cplx<double> *)part.p, mtxd, na, nbc, kslice,
-                       lower);
+#define CPW_PD(V)                                                                                                   \
+    if (pv == V)                                                                                                    \
+        hipLaunchKernelGGL((k_proj_direct<double, V>), dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, st,                \
+                           (const cplx<double> *)a, lda, b, ldb, (cplx<double> *)part.p, mtxd, na, nbc, kslice, lower);
+    CPW_PD(1) CPW_PD(SUB_PROJ_V)
+    CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
+#undef CPW_PD
     HIPCHK(hipGetLastError());
     *nsl_out = nsl;
     return CPWGPU_OK;
@@ -1291,6 +1308,19 @@ int jacobi(double2 *M, double2 *W, double2 *V, int n, int max_sweeps, double tol
     return CPWGPU_OK;
 }
 
+// l = the lower Cholesky factor of a (n <= SE_TRI_MAX) and dinv its reciprocal diagonal
+int cholesky_lds(const double2 *a, double2 *l, double *dinv, int n, int *dinfo, hipStream_t st) {
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_cholesky_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)se_lds_bytes(SE_TRI_MAX)));
+        attr = true;
+    }
+    hipLaunchKernelGGL(k_cholesky_lds, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, a, l, dinv, n, dinfo);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
+}
+
 // V = the generalised eigenvectors of (M, S), ascending, and their eigenvalues
 // in g_ss.eig; S, M, W are overwritten; dinfo[0]: failed Cholesky pivot (or 0),
 // dinfo[1]: Jacobi sweeps.
@@ -1301,8 +1331,6 @@ int small_eig(double2 *S, double2 *M, double2 *W, double2 *V, int n, int max_swe
     double *dinv = (double *)g_ss.dinv.p;
     static bool attr = false;
     if (!attr) {
-        HIPCHK(hipFuncSetAttribute((const void *)k_cholesky_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)se_lds_bytes(SE_TRI_MAX)));
         HIPCHK(hipFuncSetAttribute((const void *)k_back_cols<4>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    16 * (SE_BW + 1) * SE_MAX));
         HIPCHK(hipFuncSetAttribute((const void *)k_back_cols<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1310,8 +1338,7 @@ int small_eig(double2 *S, double2 *M, double2 *W, double2 *V, int n, int max_swe
         attr = true;
     }
     if (n <= SE_TRI_MAX) {
-        hipLaunchKernelGGL(k_cholesky_lds, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, (const double2 *)S, S, dinv, n,
-                           dinfo);
+        if ((rc = cholesky_lds(S, S, dinv, n, dinfo, st))) return rc;
     } else {
         hipLaunchKernelGGL(k_cholesky, dim3(1), dim3(SS_THREADS), 0, st, S, n, dinfo);
         hipLaunchKernelGGL(k_factor_dinv, dim3((n + 255) / 256), dim3(256), 0, st, (const double2 *)S, dinv, n);
@@ -1457,7 +1484,7 @@ constexpr unsigned long long DT_SEED = 0x243F6A8885A308D3ull;
 int gram(const double2 *a, long lda, int na, const double2 *b, long ldb, int nbc, int mtxd,
          const double *scale, double2 *out, hipStream_t st, int lower = 0) {
     int nsl, rc;
-    if ((rc = gram_partials(a, lda, na, b, ldb, nbc, mtxd, g_ss.part, &nsl, st, lower))) return rc;
+    if ((rc = gram_partials(a, lda, na, b, ldb, nbc, mtxd, g_ss.part, &nsl, st, lower, true))) return rc;
     launch_proj_reduce<double>((const cplx<double> *)g_ss.part.p, scale, (cplx<double> *)out, na,
                                nbc, nsl, st, lower);
     HIPCHK(hipGetLastError());
@@ -1467,16 +1494,46 @@ int gram(const double2 *a, long lda, int na, const double2 *b, long ldb, int nbc
 // y(:, 0:nc) = beta*y + x(:, 0:nk) c; c column-major (nk, nc) with ld nk; beta 0 or 1
 int rotate(const double2 *x, long ldx, int nk, const double2 *c, int nc, double2 *y, long ldy,
            int mtxd, int beta, hipStream_t st) {
-    constexpr int BI = back_bi<double, SUB_BACK_V>(), BN = back_bn<double, SUB_BACK_V>();
-    hipLaunchKernelGGL((k_back_direct<double, SUB_BACK_V>), dim3((mtxd + BI - 1) / BI, (nc + BN - 1) / BN),
-                       dim3(GEMM_THREADS), 0, st, (const cplx<double> *)x, ldx, (const cplx<double> *)c, y,
-                       ldy, mtxd, nk, nc, beta, (const double2 *)nullptr, 0L, (const double *)nullptr);
+    const int bv = back_shape64(mtxd, nc);
+#define CPW_BD(V)                                                                                                  \
+    if (bv == V)                                                                                                   \
+        hipLaunchKernelGGL((k_back_direct<double, V>), dim3((mtxd + back_bi<double, V>() - 1) / back_bi<double, V>(), \
+                                                            (nc + back_bn<double, V>() - 1) / back_bn<double, V>()), \
+                           dim3(GEMM_THREADS), 0, st, (const cplx<double> *)x, ldx, (const cplx<double> *)c, y,    \
+                           ldy, mtxd, nk, nc, beta, (const double2 *)nullptr, 0L, (const double *)nullptr);
+    CPW_BD(2) CPW_BD(BACK_BANDS + 1)
+#undef CPW_BD
     HIPCHK(hipGetLastError());
     return CPWGPU_OK;
 }
 
 inline dim3 dt_grid(int rows, int cols) {
     return dim3((unsigned)((rows + DT_THREADS - 1) / DT_THREADS), (unsigned)cols);
+}
+
+// Eigenpairs of the Hermitian n x n matrix m (lower triangle, n <= SE_DIAG_MAX):
+// eigenvalues ascending in w, eigenvectors in v, g_dt.info[1] nonzero if it failed.
+int subspace_eig(const double2 *m, double2 *v, double *w, int n, hipStream_t st) {
+    int rc;
+    constexpr int MAX_SWEEPS = 40;  // a matrix of random elements takes 8 to 10
+    const int np = (n + 1) & ~1, half = np / 2;
+    if ((rc = g_ss.rec.reserve(sizeof(double4) * (size_t)MAX_SWEEPS * (np - 1) * half)) ||
+        (rc = g_ss.pos.reserve(4 * (size_t)np + 64)) || (rc = g_ss.info.reserve(64)))
+        return rc;
+    static bool attr = false;
+    if (!attr) {
+        HIPCHK(hipFuncSetAttribute((const void *)k_jacobi_tri, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)se_lds_bytes(SE_DIAG_MAX)));
+        attr = true;
+    }
+    double4 *rec = (double4 *)g_ss.rec.p;
+    int *pos = (int *)g_ss.pos.p, *sweeps = (int *)g_ss.info.p + 1;
+    hipLaunchKernelGGL(k_jacobi_tri, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, m, rec, w, n, MAX_SWEEPS, 1e-13,
+                       pos, sweeps, (int *)g_dt.info.p + 1);
+    hipLaunchKernelGGL(k_jacobi_vectors, dim3((n + SE_VROWS - 1) / SE_VROWS), dim3(64), 0, st, (const double4 *)rec,
+                       (const int *)sweeps, (const int *)pos, v, n);
+    HIPCHK(hipGetLastError());
+    return CPWGPU_OK;
 }
 
 // Orthonormalises t(:, 0:m) (unit columns on entry) against the orthonormal
@@ -1506,6 +1563,7 @@ int orthonormalize(int mtxd, const double2 *x, long ldx, int nx, double2 *t, lon
         return rotate(x, ldx, nx, P, m, t, ldt, mtxd, 1, st);
     };
     const rocblas_double_complex one(1.0, 0.0);
+    double2 *const t0 = t;
     for (int pass = 0; pass < 2 && m > 0; pass++) {
         if (nx > 0) {
             if ((rc = project())) return rc;
@@ -1513,27 +1571,43 @@ int orthonormalize(int mtxd, const double2 *x, long ldx, int nx, double2 *t, lon
         }
         const int ld = m;
         if ((rc = gram(t, ldt, m, t, ldt, m, mtxd, nullptr, G, st, 1))) return rc;
-        HIPCHK(hipMemcpyAsync(G0, G, 16 * (size_t)ld * ld, hipMemcpyDeviceToDevice, st));
-        BLASCHK(rocsolver_zpotrf(g_blas, rocblas_fill_lower, m, (rocblas_double_complex *)G, ld, dinfo));
+        // the factor in LDS and t <- t L^-H as a product with the inverse (a block
+        // of 72: 60 + 20 + 35 us against 109 + 290 of zpotrf and ztrsm); rocSOLVER
+        // and rocBLAS for larger blocks and where columns are dropped
+        const bool small = m <= SE_TRI_MAX && ldt == mtxd;
         int info = 0;
+        if (small) {
+            if ((rc = g_ss.dinv.reserve(8 * (size_t)m)) || (rc = g_ss.tmp.reserve(16 * (size_t)mtxd * m))) return rc;
+            if ((rc = cholesky_lds(G, G0, (double *)g_ss.dinv.p, m, dinfo, st))) return rc;
+        } else {
+            HIPCHK(hipMemcpyAsync(G0, G, 16 * (size_t)ld * ld, hipMemcpyDeviceToDevice, st));
+            BLASCHK(rocsolver_zpotrf(g_blas, rocblas_fill_lower, m, (rocblas_double_complex *)G0, ld, dinfo));
+        }
+        // G0 holds the factor, and G the matrix (its lower triangle) unless zpotrf made it
+        std::vector<double> d(m);
+        if (pass == 0) {
+            hipLaunchKernelGGL(k_diag_sq, dim3((m + DT_THREADS - 1) / DT_THREADS), dim3(DT_THREADS), 0, st,
+                               (const double2 *)G0, (long)ld, m, (double *)g_dt.d.p);
+            HIPCHK(hipMemcpyAsync(d.data(), g_dt.d.p, 8 * (size_t)m, hipMemcpyDeviceToHost, st));
+        }
         HIPCHK(hipMemcpyAsync(&info, dinfo, sizeof info, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         if (info > 0) {
             // leading minor of order info not positive definite: keep the columns before it
             m = info - 1;
             if (m == 0) break;
-            HIPCHK(hipMemcpyAsync(G, G0, 16 * (size_t)ld * ld, hipMemcpyDeviceToDevice, st));
-            BLASCHK(rocsolver_zpotrf(g_blas, rocblas_fill_lower, m, (rocblas_double_complex *)G, ld, dinfo));
+            HIPCHK(hipMemcpyAsync(G0, G, 16 * (size_t)ld * ld, hipMemcpyDeviceToDevice, st));
+            BLASCHK(rocsolver_zpotrf(g_blas, rocblas_fill_lower, m, (rocblas_double_complex *)G0, ld, dinfo));
+            if (pass == 0) {
+                hipLaunchKernelGGL(k_diag_sq, dim3((m + DT_THREADS - 1) / DT_THREADS), dim3(DT_THREADS), 0, st,
+                                   (const double2 *)G0, (long)ld, m, (double *)g_dt.d.p);
+                HIPCHK(hipMemcpyAsync(d.data(), g_dt.d.p, 8 * (size_t)m, hipMemcpyDeviceToHost, st));
+            }
             HIPCHK(hipMemcpyAsync(&info, dinfo, sizeof info, hipMemcpyDeviceToHost, st));
             HIPCHK(hipStreamSynchronize(st));
             if (info != 0) return fail(CPWGPU_ERR_NOTPD, "Cholesky of a leading block failed (%d)", info);
         }
         if (pass == 0) {
-            std::vector<double> d(m);
-            hipLaunchKernelGGL(k_diag_sq, dim3((m + DT_THREADS - 1) / DT_THREADS), dim3(DT_THREADS), 0, st,
-                               (const double2 *)G, (long)ld, m, (double *)g_dt.d.p);
-            HIPCHK(hipMemcpyAsync(d.data(), g_dt.d.p, 8 * (size_t)m, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
             for (int k = 0; k < m; k++)
                 if (d[k] < DT_PIVOT) {
                     m = k;
@@ -1541,19 +1615,35 @@ int orthonormalize(int mtxd, const double2 *x, long ldx, int nx, double2 *t, lon
                 }
             if (m == 0) break;
         }
-        // t <- t L^-H
-        BLASCHK(rocblas_ztrsm(g_blas, rocblas_side_right, rocblas_fill_lower,
-                              rocblas_operation_conjugate_transpose, rocblas_diagonal_non_unit, mtxd, m,
-                              &one, (const rocblas_double_complex *)G, ld, (rocblas_double_complex *)t,
-                              (int)ldt));
+        if (small && m == ld) {
+            // G = L^-H, then the product into the other buffer
+            const auto inverse = [&](auto rows_per_lane) {
+                hipLaunchKernelGGL((k_solve_cols<decltype(rows_per_lane)::value, false, true>), dim3(m), dim3(64), 0, st,
+                                   (const double2 *)G0, (const double *)g_ss.dinv.p, (const double2 *)nullptr, G, m);
+            };
+            if (m <= 64) inverse(std::integral_constant<int, 1>{});
+            else if (m <= 128) inverse(std::integral_constant<int, 2>{});
+            else inverse(std::integral_constant<int, 4>{});
+            double2 *o = t == t0 ? (double2 *)g_ss.tmp.p : t0;
+            if ((rc = rotate(t, ldt, m, G, m, o, mtxd, mtxd, 0, st))) return rc;
+            t = o;
+        } else {
+            // t <- t L^-H
+            BLASCHK(rocblas_ztrsm(g_blas, rocblas_side_right, rocblas_fill_lower,
+                                  rocblas_operation_conjugate_transpose, rocblas_diagonal_non_unit, mtxd, m,
+                                  &one, (const rocblas_double_complex *)G0, ld, (rocblas_double_complex *)t,
+                                  (int)ldt));
+        }
     }
+    if (t != t0 && m > 0)
+        HIPCHK(hipMemcpyAsync(t0, t, 16 * (size_t)mtxd * m, hipMemcpyDeviceToDevice, st));
     *kept = m;
     return CPWGPU_OK;
 }
 
 // Rayleigh-Ritz on the orthonormal basis xa(:, 0:nt) with hxa = H xa (ld
 // mtxd): the lowest nk Ritz vectors go to xo and H times them to hxo (ld
-// mtxd); all nt Ritz values to g_dt.w (ascending), zheevd's info to
+// mtxd); all nt Ritz values to g_dt.w (ascending), the eigensolver's info to
 // g_dt.info[1].  When po is given and nt > nk, po receives the part of the
 // Ritz vectors from the columns beyond nk, xa(:, nk:nt) C(nk:nt, 0:nk): the
 // search directions of the next step.
@@ -1562,7 +1652,11 @@ int ritz_step(int mtxd, const double2 *xa, const double2 *hxa, int nt, int nk, d
     int rc;
     double2 *M = (double2 *)g_dt.m.p;
     if ((rc = gram(xa, mtxd, nt, hxa, mtxd, nt, mtxd, nullptr, M, st, 1))) return rc;
-    BLASCHK(rocsolver_zheevd(g_blas, rocblas_evect_original, rocblas_fill_lower, nt,
+    if (nt <= SE_DIAG_MAX) {
+        if ((rc = g_ss.v.reserve(16 * (size_t)nt * nt))) return rc;
+        if ((rc = subspace_eig(M, (double2 *)g_ss.v.p, (double *)g_dt.w.p, nt, st))) return rc;
+        M = (double2 *)g_ss.v.p;
+    } else BLASCHK(rocsolver_zheevd(g_blas, rocblas_evect_original, rocblas_fill_lower, nt,
                              (rocblas_double_complex *)M, nt, (double *)g_dt.w.p, (double *)g_dt.e.p,
                              (int *)g_dt.info.p + 1));
     if ((rc = rotate(xa, mtxd, nt, M, nk, xo, mtxd, mtxd, 0, st))) return rc;
@@ -1921,7 +2015,7 @@ int plan_ditsp(cpwgpu_plan_s *p, int prec, int icmax, int iguess, double epspsi,
         HIPCHK(hipMemcpyAsync(wv.data(), E, 8 * (size_t)nb, hipMemcpyDeviceToHost, st));
         HIPCHK(hipMemcpyAsync(&info, dinfo + 1, sizeof info, hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-        if (info) return fail(CPWGPU_ERR_HIP, "zheevd of the subspace failed (info %d)", info);
+        if (info) return fail(CPWGPU_ERR_HIP, "eigenproblem of the subspace failed (info %d)", info);
         iters = ic;
         xmax = *std::max_element(res.begin(), res.begin() + neig);
         if (trace)

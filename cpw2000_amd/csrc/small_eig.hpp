@@ -27,6 +27,7 @@ namespace cpwgpu {
 constexpr int SE_MAX = 256;      // largest n of the solves by columns
 constexpr int SE_TRI_MAX = 140;  // largest n whose lower triangle fits in LDS
 constexpr int SE_FULL_MAX = 96;  // largest n whose matrix fits in LDS
+constexpr int SE_DIAG_MAX = 128; // largest n of k_jacobi_tri (one lane per pair)
 constexpr int SE_THREADS = 1024;
 
 // a b and conj(a) b with the second product of each sum rounded first
@@ -99,12 +100,13 @@ __device__ __forceinline__ double lane_value(double x, int lane) {
 
 // One forward substitution per wavefront: column c of out = L^-1 in, with L
 // column-major in t and dinv its reciprocal diagonal.  in: column c of the matrix,
-// or with HERM row c conjugated.  Lane j holds rows j, j + 64, ... (RPL of
+// or with HERM row c conjugated; INVH: the identity, and out is L^-H (the column
+// stored as a conjugated row).  Lane j holds rows j, j + 64, ... (RPL of
 // them); a solved value goes to all lanes by readlane, so the chain has no
 // memory access: the columns of L are loaded SE_PRE ahead.  Each row subtracts its
 // terms in the order of the columns.
 constexpr int SE_PRE = 8;
-template <int RPL, bool HERM>
+template <int RPL, bool HERM, bool INVH = false>
 __global__ __launch_bounds__(64) void k_solve_cols(const double2 *__restrict__ t, const double *__restrict__ dinv,
                                                    const double2 *__restrict__ in, double2 *__restrict__ out, int n) {
     const int c = blockIdx.x, lane = threadIdx.x;
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(64) void k_solve_cols(const double2 *__restrict__ t
 #pragma unroll
     for (int q = 0; q < RPL; q++) {
         const int i = min(lane + 64 * q, n - 1);
-        s[q] = HERM ? zconj(in[c + (long)i * n]) : in[i + (long)c * n];
+        s[q] = INVH ? make_double2(i == c ? 1.0 : 0.0, 0.0) : HERM ? zconj(in[c + (long)i * n]) : in[i + (long)c * n];
         di[q] = dinv[i];
     }
     // column k of L at this lane's rows (clamped: rows not below k are not used)
@@ -148,7 +150,10 @@ __global__ __launch_bounds__(64) void k_solve_cols(const double2 *__restrict__ t
     }
 #pragma unroll
     for (int q = 0; q < RPL; q++)
-        if (lane + 64 * q < n) out[lane + 64 * q + (long)c * n] = s[q];
+        if (lane + 64 * q < n) {
+            if (INVH) out[c + (long)(lane + 64 * q) * n] = zconj(s[q]);
+            else out[lane + 64 * q + (long)c * n] = s[q];
+        }
 }
 
 // In place on v: v <- L^-H v.  Row i subtracts conj(L_ki) v_k for k = i + 1, i + 2,
@@ -390,14 +395,163 @@ __global__ __launch_bounds__(SE_THREADS) void k_jacobi_lds(const double2 *__rest
     if (tid == 0) *sweeps_out = sweep;
 }
 
-// Eigenvectors of k_jacobi_lds: v = J_1 J_2 ... with columns in the order of
+// Jacobi of the iterative diagonalisation's subspace matrix, n <= SE_DIAG_MAX: all
+// sweeps in one workgroup on the packed lower triangle in LDS (h: lower triangle,
+// column-major).  Each step of that iteration starts from Ritz vectors, so the
+// matrix comes nearly diagonal and few sweeps do.  A round is one chain of
+// latencies, so it is kept short: the rotation from three reciprocal square
+// roots (k_jacobi_lds, whose results the caller of a Rayleigh-Ritz step keeps to
+// the bit, takes a hypot, four divisions and two square roots), and with half of
+// the blocks gone by symmetry one to three blocks per thread.  Outputs as
+// k_jacobi_lds; info: 1 if max_sweeps did not do.  us at n = 72, from Ritz vectors, with the vectors: 318 on average (from 150), zheevd 1,600.
+__device__ __forceinline__ double fast_rsqrt(double x) {
+    double r = __builtin_amdgcn_rsq(x);  // refined by two Newton steps
+#pragma unroll
+    for (int i = 0; i < 2; i++) r = fma(0.5 * r, fma(-x * r, r, 1.0), r);
+    return r;
+}
+
+__global__ __launch_bounds__(SE_THREADS) void k_jacobi_tri(const double2 *__restrict__ h, double4 *__restrict__ rec,
+                                                           double *__restrict__ eig, int n, int max_sweeps, double tol,
+                                                           int *__restrict__ pos, int *__restrict__ sweeps_out,
+                                                           int *__restrict__ info) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    double2 *P = reinterpret_cast<double2 *>(smem_raw);
+    constexpr int HMAX = SE_DIAG_MAX / 2;
+    __shared__ double red[2][SE_THREADS / 64];
+    __shared__ Rotation rot[HMAX];
+    __shared__ int rp[HMAX], rq[HMAX];
+    static_assert(HMAX <= 64, "one lane per pair");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int np = (n + 1) & ~1, half = np / 2, nblk = half * (half + 1) / 2;
+    const auto get = [&](int i, int j) {
+        const double2 v = P[i >= j ? tri(i) + j : tri(j) + i];
+        return i >= j ? v : zconj(v);
+    };
+    const auto put = [&](int i, int j, double2 v) { P[i >= j ? tri(i) + j : tri(j) + i] = i >= j ? v : zconj(v); };
+    for (int c = wave; c < n; c += SE_THREADS / 64)
+        for (int r = c + lane; r < n; r += 64) {
+            const double2 v = h[r + (long)c * n];
+            P[tri(r) + c] = r == c ? make_double2(v.x, 0.0) : v;
+        }
+    // blocks (k, l), k >= l, of this thread: fixed over the rounds
+    constexpr int MAXB = (HMAX * (HMAX + 1) / 2 + SE_THREADS - 1) / SE_THREADS;
+    int bk[MAXB], bl[MAXB];
+#pragma unroll
+    for (int u = 0; u < MAXB; u++) {
+        const int t = tid + u * SE_THREADS;
+        int k = (int)((sqrtf(8.f * t + 1.f) - 1.f) * 0.5f);
+        if (tri(k) > t) k--;
+        if (tri(k + 1) <= t) k++;
+        bk[u] = k;
+        bl[u] = t - tri(k);
+    }
+    int sweep = 0;
+    for (; sweep < max_sweeps; sweep++) {
+        __syncthreads();
+        double off = 0.0, tot = 0.0;
+        for (int r = wave; r < n; r += SE_THREADS / 64)
+            for (int c = lane; c <= r; c += 64) {
+                const double2 x = P[tri(r) + c];
+                const double m = fma(x.x, x.x, x.y * x.y);
+                if (c < r) off += 2.0 * m;
+                tot += c < r ? 2.0 * m : m;
+            }
+        for (int s = 1; s < 64; s <<= 1) {
+            off += __shfl_xor(off, s);
+            tot += __shfl_xor(tot, s);
+        }
+        if (lane == 0) {
+            red[0][wave] = off;
+            red[1][wave] = tot;
+        }
+        __syncthreads();
+        off = tot = 0.0;
+        for (int w = 0; w < SE_THREADS / 64; w++) {
+            off += red[0][w];
+            tot += red[1][w];
+        }
+        if (jacobi_done(off, tot, tol)) break;
+        const double thr = jacobi_threshold(tot, tol, n), thr2 = fmax(thr * thr, 1e-280);  // squares stay normal
+        for (int round = 0; round < np - 1; round++) {
+            if (tid < half) {
+                int p, q;
+                rr_pair(tid, round, np, p, q);
+                Rotation r{1.0, 0.0, make_double2(1.0, 0.0)};
+                if (q < n) {
+                    const double app = P[tri(p) + p].x, aqq = P[tri(q) + q].x;
+                    const double2 apq = zconj(P[tri(q) + p]);  // q > p
+                    const double g2 = fma(apq.x, apq.x, apq.y * apq.y);
+                    if (g2 > thr2) {
+                        const double d = aqq - app;
+                        const double rg = fast_rsqrt(g2), rh = fast_rsqrt(fma(d, d, 4.0 * g2));
+                        const double c2 = fma(0.5 * fabs(d), rh, 0.5), rc = fast_rsqrt(c2);
+                        r.u = make_double2(apq.x * rg, -apq.y * rg);
+                        r.c = c2 * rc;
+                        r.s = (d >= 0.0 ? g2 : -g2) * rg * rh * rc;
+                    }
+                }
+                rot[tid] = r;
+                rp[tid] = p;
+                rq[tid] = q;
+                rec[((long)sweep * (np - 1) + round) * half + tid] = make_double4(r.c, r.s, r.u.x, r.u.y);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < MAXB; u++) {
+                if (tid + u * SE_THREADS >= nblk) break;
+                const int k = bk[u], l = bl[u];
+                const Rotation rk = rot[k], rl = rot[l];
+                if (rk.s == 0.0 && rl.s == 0.0) continue;  // two identities
+                const int pk = rp[k], qk = rq[k], pl = rp[l], ql = rq[l];
+                const bool kq = qk < n, lq = ql < n;  // the dummy index has no row
+                const double2 z = make_double2(0.0, 0.0);
+                double2 a00 = get(pk, pl), a01 = lq ? get(pk, ql) : z, a10 = kq ? get(qk, pl) : z,
+                        a11 = kq && lq ? get(qk, ql) : z;
+                rotate_rows(rk, a00, a10);
+                rotate_rows(rk, a01, a11);
+                rotate_cols(rl, a00, a01);
+                rotate_cols(rl, a10, a11);
+                if (k == l) {  // the annihilated pair: real diagonal, one off-diagonal element
+                    put(pk, pk, make_double2(a00.x, 0.0));
+                    if (kq) {
+                        put(qk, qk, make_double2(a11.x, 0.0));
+                        put(qk, pk, z);
+                    }
+                } else {
+                    put(pk, pl, a00);
+                    if (lq) put(pk, ql, a01);
+                    if (kq) put(qk, pl, a10);
+                    if (kq && lq) put(qk, ql, a11);
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int i = tid; i < n; i += SE_THREADS) {
+        const double e = P[tri(i) + i].x;
+        int r = 0;
+        for (int j = 0; j < n; j++) {
+            const double f = P[tri(j) + j].x;
+            r += (f < e) || (f == e && j < i);
+        }
+        pos[i] = r;
+        eig[r] = e;
+    }
+    if (tid == 0) {
+        *sweeps_out = sweep;
+        *info = sweep == max_sweeps;
+    }
+}
+
+// Eigenvectors of k_jacobi_lds and k_jacobi_tri: v = J_1 J_2 ... with columns in the order of
 // pos.  A row of v depends on no other: SE_VROWS rows per wavefront, in LDS, all
 // rotations of a round at once, no block barrier; the next round's rotations are
 // loaded while this one's are applied.
 constexpr int SE_VROWS = 2;
 __global__ __launch_bounds__(64) void k_jacobi_vectors(const double4 *__restrict__ rec, const int *__restrict__ sweeps,
                                                        const int *__restrict__ pos, double2 *__restrict__ v, int n) {
-    __shared__ double2 row[SE_VROWS][SE_FULL_MAX + 1];  // + the dummy index of an odd n
+    __shared__ double2 row[SE_VROWS][SE_DIAG_MAX + 1];  // + the dummy index of an odd n
     const int lane = threadIdx.x, i0 = blockIdx.x * SE_VROWS;
     const int np = (n + 1) & ~1, half = np / 2;
     for (int j = lane; j < np; j += 64)
