@@ -571,8 +571,8 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         cplx<R> *pt = part;
 #define CPW_PD(V)                                                                                                     \
     if (pv == V)                                                                                                      \
-        launch_timed(CPWGPU_K_PROJ, (k_proj_direct<R, V>), grid, dim3(GEMM_THREADS), 0, s, anl, lda, ps, ldp, pt, rows, \
-                     nanl, neig, kslice, 0);
+        launch_batchable<ProjDirect<R, V>>(CPWGPU_K_PROJ, (k_proj_direct<R, V>), grid, dim3(GEMM_THREADS), 0, s, anl,    \
+                                           lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
         CPW_PD(1) CPW_PD(2) CPW_PD(3) CPW_PD(4)
         CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
 #undef CPW_PD
@@ -588,7 +588,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         // launch_proj_reduce's launch, with the measurement hook
         const long tot = (long)nanl * neig;
         if (tot > 0)
-            launch_timed(CPWGPU_K_PROJ_REDUCE, k_proj_reduce<R>, dim3((unsigned)((tot + RED_OUT - 1) / RED_OUT)),
+            launch_batchable<ProjReduce<R>>(CPWGPU_K_PROJ_REDUCE, k_proj_reduce<R>, dim3((unsigned)((tot + RED_OUT - 1) / RED_OUT)),
                          dim3(RED_OUT * RED_GRP), 0, s, (const cplx<R> *)part, pv_.xnl, dhd, nanl, neig, nsl, 0);
     }
     if (phase != NL_PROJ) {
@@ -600,7 +600,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         const double *ek = kin ? (const double *)p->ekpg.p : nullptr;
 #define CPW_BD(V)                                                                                  \
     if (bv == V)                                                                                   \
-        launch_timed(CPWGPU_K_BACK, (k_back_direct<R, V>),                                                  \
+        launch_batchable<BackDirect<R, V>>(CPWGPU_K_BACK, (k_back_direct<R, V>),                                                  \
                            dim3((rows + back_bi<R, V>() - 1) / back_bi<R, V>(),                  \
                                 (neig + back_bn<R, V>() - 1) / back_bn<R, V>()),                   \
                            dim3(GEMM_THREADS), 0, s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta, kp,   \
@@ -610,7 +610,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
 #undef CPW_BD
 #define CPW_BL(NT)                                                                                            \
     if (bv == BACK_BANDS + NT)                                                                                \
-        launch_timed(CPWGPU_K_BACK, (k_back<R, GemmCfg<R>::KC / 2, NT>),                                      \
+        launch_batchable<BackLds<R, GemmCfg<R>::KC / 2, NT>>(CPWGPU_K_BACK, (k_back<R, GemmCfg<R>::KC / 2, NT>),                                      \
                      dim3((rows + BP_BI - 1) / BP_BI, (neig + 16 * NT - 1) / (16 * NT)), dim3(GEMM_THREADS), 0, \
                      s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta, kp, ldp, ek);
         if constexpr (sizeof(R) == 4) { CPW_BL(1) CPW_BL(2) CPW_BL(3) }
@@ -2918,11 +2918,110 @@ PlanState plan_state(const cpwgpu_plan_s *p) {
 }
 }  // namespace
 
+namespace {
+// k-points of a graph whose applies are launched together, step by step
+// (k_batch): they take the same kernels, and share nothing.
+struct BatchGroup {
+    std::vector<int> ks;
+    size_t blocks = 0;  // of the step with the most
+};
+
+// Small kernels cost what a launch costs; kernels that fill the GPU by themselves
+// gain nothing, and the columns of several k-points leave the caches between the
+// steps.  So k-points whose largest step has at most BATCH_POINT blocks join groups
+// of at most BATCH_BLOCKS.  us per graph launch, one k-point after the other / in
+// groups: 8 of a primitive cell, 16 bands 176 / 53; 6 of 36^3, 20 bands 190 / 82
+// (4,096 blocks a group: 104); 10 of 36^3, 40 bands 366 / 178 (8,192 a group: 207);
+// 4 of 36 x 36 x 72, 40 bands (2,880 blocks each) 231 / 160; 4 of 72^3, 16 bands 449 /
+// 402, 64 bands (4,608 blocks each) 1,064 / 1,099.
+constexpr size_t BATCH_POINT = 4096, BATCH_BLOCKS = 16384;
+
+// true if no k-point reads or writes what another writes, workspaces included
+bool independent(int nk, const cpwgpu_plan_t *plans, const int *neig, const double *const *psi, const long *ldp,
+                 double *const *hpsi, const long *ldh) {
+    using Span = std::pair<const double *, const double *>;
+    const auto span = [&](const double *p, long ld, int k) { return Span(p, p + 2 * ld * neig[k]); };
+    const std::less<const double *> lt;
+    const auto meet = [&](Span a, Span b) { return lt(a.first, b.second) && lt(b.first, a.second); };
+    for (int k = 0; k < nk; k++) {
+        if (neig[k] == 0) continue;
+        const Span out = span(hpsi[k], ldh[k], k);
+        for (int j = 0; j < nk; j++)
+            if (j != k && neig[j] > 0 &&
+                (plans[j] == plans[k] || meet(out, span(hpsi[j], ldh[j], j)) || meet(out, span(psi[j], ldp[j], j))))
+                return false;
+    }
+    return true;
+}
+
+// The recorded k-points in groups, in order of their first member.
+std::vector<BatchGroup> batch_groups(const std::vector<Recorder> &recs) {
+    const auto same = [](const Recorder &a, const Recorder &b) {
+        if (a.steps.size() != b.steps.size()) return false;
+        for (size_t i = 0; i < a.steps.size(); i++)
+            if (a.steps[i].fn != b.steps[i].fn || a.steps[i].threads != b.steps[i].threads) return false;
+        return true;
+    };
+    std::vector<BatchGroup> groups;
+    for (size_t k = 0; k < recs.size(); k++) {
+        if (!recs[k].ok || recs[k].steps.empty()) continue;
+        size_t most = 0;
+        for (const BatchStep &t : recs[k].steps) most = std::max(most, (size_t)t.grid.x * t.grid.y * t.grid.z + 7);
+        if (most > BATCH_POINT) continue;
+        BatchGroup *to = nullptr;
+        for (BatchGroup &g : groups)
+            if (!to && (int)g.ks.size() < BATCH_MAX && g.blocks + most <= BATCH_BLOCKS && same(recs[g.ks[0]], recs[k])) to = &g;
+        if (!to) {
+            groups.emplace_back();
+            to = &groups.back();
+        }
+        to->ks.push_back((int)k);
+        to->blocks += most;
+    }
+    return groups;
+}
+
+// The launches of one group on stream s; its tables are at tab (host) and dev,
+// from byte off on, which this advances.  launch false: only fills the tables.
+int batch_group_steps(const std::vector<Recorder> &recs, const BatchGroup &g, std::vector<char> &tab, const char *dev,
+                      size_t &off, bool launch, hipStream_t s) {
+    const auto place = [&](size_t n) {
+        const size_t at = (off + 255) & ~(size_t)255;
+        off = at + n;
+        if (tab.size() < off) tab.resize(off);
+        return at;
+    };
+    const int n = (int)g.ks.size();
+    for (size_t i = 0; i < recs[g.ks[0]].steps.size(); i++) {
+        const BatchStep &lead = recs[g.ks[0]].steps[i];
+        const size_t one = lead.args.size(), at_dims = place(sizeof(BatchDim) * n), at_args = place(one * n);
+        int first = 0;
+        size_t shmem = 0;
+        for (int m = 0; m < n; m++) {
+            const BatchStep &t = recs[g.ks[m]].steps[i];
+            const BatchDim d{first, (int)t.grid.x, (int)t.grid.y, (int)t.grid.z};
+            memcpy(tab.data() + at_dims + sizeof d * m, &d, sizeof d);
+            memcpy(tab.data() + at_args + one * m, t.args.data(), one);
+            first += (d.gx * d.gy * d.gz + 7) & ~7;
+            shmem = std::max(shmem, t.shmem);
+        }
+        if (!launch) continue;
+        const char *dims = dev + at_dims, *packs = dev + at_args;
+        int count = n;
+        void *args[3] = {&dims, &packs, &count};
+        HIPCHK(hipFuncSetAttribute(lead.fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem));
+        HIPCHK(hipLaunchKernel(lead.fn, dim3((unsigned)first), dim3(lead.threads), args, shmem, s));
+    }
+    return CPWGPU_OK;
+}
+}  // namespace
+
 struct cpwgpu_graph_s {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int prec = CPWGPU_PREC_FP64;
     std::vector<PlanState> state;  // per k-point, at capture
+    DevBuf tab;                    // arguments of the batched launches
 };
 
 extern "C" {
@@ -2940,37 +3039,58 @@ int cpwgpu_graph_create(cpwgpu_graph_t *graph, int nk, const cpwgpu_plan_t *plan
     for (int k = 0; k < nk; k++)
         if (!plans[k] || neig[k] < 0 || ldp[k] < plans[k]->mtxd || ldh[k] < plans[k]->mtxd)
             return fail(CPWGPU_ERR_ARG, "bad arguments for k-point %d", k);
-    // the k-points in sequence, each apply overlapping its own non-local GEMMs
-    // with its FFT chain (a batched order that chains all GEMMs on the second
-    // stream measured no faster: the pairs already fill the GPU)
-    auto apply = [&](hipStream_t s) -> int {
-        for (int k = 0; k < nk; k++) {
-            if (neig[k] == 0) continue;
-            const int st2 = prec == CPWGPU_PREC_FP64
-                                ? apply_t<double>(plans[k], neig[k], psi[k], ldp[k], hpsi[k], ldh[k], s)
-                                : apply_t<float>(plans[k], neig[k], psi[k], ldp[k], hpsi[k], ldh[k], s);
-            if (st2) return st2;
-        }
-        return CPWGPU_OK;
+    const auto one = [&](int k, hipStream_t s) -> int {
+        if (neig[k] == 0) return CPWGPU_OK;
+        return prec == CPWGPU_PREC_FP64 ? apply_t<double>(plans[k], neig[k], psi[k], ldp[k], hpsi[k], ldh[k], s)
+                                        : apply_t<float>(plans[k], neig[k], psi[k], ldp[k], hpsi[k], ldh[k], s);
     };
     // eager pass: every buffer, attribute and FP32 projector copy exists before capture
     const bool prof = g_prof.on;
     g_prof.on = false;
-    if ((st = apply(g_stream))) { g_prof.on = prof; return st; }
+    for (int k = 0; k < nk && !st; k++) st = one(k, g_stream);
+    if (st) { g_prof.on = prof; return st; }
     HIPCHK(hipStreamSynchronize(g_stream));
-    hipStream_t cs = nullptr;
-    HIPCHK(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
+    // small k-points together, the others one after the other
+    std::vector<Recorder> recs(nk);
+    const int ix = prec == CPWGPU_PREC_FP32 ? 1 : 0;
+    if (independent(nk, plans, neig, psi, ldp, hpsi, ldh))
+        for (int k = 0; k < nk && !st; k++) {
+            if (g_overlap && plans[k]->sched_var[ix] > 0) continue;  // two streams
+            g_rec = &recs[k];
+            st = one(k, g_stream);
+            g_rec = nullptr;
+        }
+    if (st) { g_prof.on = prof; return st; }
+    std::vector<BatchGroup> groups = batch_groups(recs);
+    std::vector<char> batched(nk, 0), tab;
+    size_t off = 0;
+    for (const BatchGroup &g : groups)
+        if (g.ks.size() > 1) {
+            for (int k : g.ks) batched[k] = 1;
+            batch_group_steps(recs, g, tab, nullptr, off, false, nullptr);
+        }
     cpwgpu_graph_s *gr = new cpwgpu_graph_s();
-    hipError_t e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) st = apply(cs);
-    hipError_t e2 = e == hipSuccess ? hipStreamEndCapture(cs, &gr->graph) : e;
+    hipStream_t cs = nullptr;
+    hipError_t e = hipSuccess, e2 = hipSuccess;
+    if (!tab.empty() && !(st = gr->tab.reserve(tab.size())))
+        e = hipMemcpy(gr->tab.p, tab.data(), tab.size(), hipMemcpyHostToDevice);
+    if (!st && e == hipSuccess) e = hipStreamCreateWithFlags(&cs, hipStreamNonBlocking);
+    if (!st && e == hipSuccess && (e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal)) == hipSuccess) {
+        off = 0;
+        for (const BatchGroup &g : groups)
+            if (g.ks.size() > 1 && !st) st = batch_group_steps(recs, g, tab, (const char *)gr->tab.p, off, true, cs);
+        for (int k = 0; k < nk && !st; k++)
+            if (!batched[k]) st = one(k, cs);
+        e2 = hipStreamEndCapture(cs, &gr->graph);
+    }
     g_prof.on = prof;
     if (e == hipSuccess && e2 == hipSuccess && st == CPWGPU_OK)
         e2 = hipGraphInstantiate(&gr->exec, gr->graph, nullptr, nullptr, 0);
-    (void)hipStreamDestroy(cs);
+    if (cs) (void)hipStreamDestroy(cs);
     if (st != CPWGPU_OK || e != hipSuccess || e2 != hipSuccess) {
         if (gr->exec) (void)hipGraphExecDestroy(gr->exec);
         if (gr->graph) (void)hipGraphDestroy(gr->graph);
+        gr->tab.release();
         delete gr;
         if (st) return st;
         return fail(CPWGPU_ERR_HIP, "graph capture: %s", hipGetErrorString(e != hipSuccess ? e : e2));
@@ -3008,6 +3128,7 @@ int cpwgpu_graph_destroy(cpwgpu_graph_t graph) {
     hipDeviceSynchronize();
     if (graph->exec) HIPCHK(hipGraphExecDestroy(graph->exec));
     if (graph->graph) HIPCHK(hipGraphDestroy(graph->graph));
+    graph->tab.release();
     delete graph;
     return CPWGPU_OK;
 }

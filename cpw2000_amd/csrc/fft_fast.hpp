@@ -85,152 +85,167 @@ __device__ __forceinline__ void load_twiddles(cplx<R> *dst, const double2 *src, 
 // ---------------------------------------------------------------------------
 // psi(G) -> colbuf[band][z][col]: scatter + inverse FFT along z
 // ---------------------------------------------------------------------------
-template <typename R, int N3>
-__global__ __launch_bounds__(FT) void k_col_bwd_fast(
-    const double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__ colbuf,
-    const int *__restrict__ col_ptr, const int *__restrict__ ent_i, const int *__restrict__ ent_cz,
-    const double2 *__restrict__ tw3, FftGeom g, int ntiles, int nb) {
-    constexpr int CT = col_tile<N3>();
-    constexpr int LS = N3 + 1;
-    __shared__ cplx<R> tw[N3];
-    __shared__ cplx<R> lines[CT * LS];
-    int band, tile;
-    if (!xcd_band_tile(blockIdx.x, ntiles, nb, band, tile)) return;
-    const int c0 = tile * CT;
-    const int nc = min(CT, g.ncol - c0);
-    const double2 *pb = psi + (long)band * ldp;
-    const int e0 = col_ptr[c0], e1 = col_ptr[c0 + nc];
-    // The first CB_PRE sphere entries of each thread (index, then value: two
-    // dependent global round trips) are loaded before the twiddles and the
-    // clearing of the lines, which they overlap; each tile has at least one
-    // entry, so a clamped entry index is always valid.
-    constexpr int CB_PRE = 4;
-    int pcz[CB_PRE];
-    double2 pv[CB_PRE];
-    {
-        int pi[CB_PRE];
+template <typename R, int N3> struct ColBwdFast {
+    static constexpr int T = FT, W = 1;
+    static __device__ __forceinline__ void run(const Blk blk, const double2 *__restrict__ psi, long ldp, cplx<R>
+        *__restrict__ colbuf, const int *__restrict__ col_ptr, const int *__restrict__ ent_i, const int *__restrict__
+        ent_cz, const double2 *__restrict__ tw3, FftGeom g, int ntiles, int nb) {
+        constexpr int CT = col_tile<N3>();
+        constexpr int LS = N3 + 1;
+        __shared__ cplx<R> tw[N3];
+        __shared__ cplx<R> lines[CT * LS];
+        int band, tile;
+        if (!xcd_band_tile(blk.x, ntiles, nb, band, tile)) return;
+        const int c0 = tile * CT;
+        const int nc = min(CT, g.ncol - c0);
+        const double2 *pb = psi + (long)band * ldp;
+        const int e0 = col_ptr[c0], e1 = col_ptr[c0 + nc];
+        // The first CB_PRE sphere entries of each thread (index, then value: two
+        // dependent global round trips) are loaded before the twiddles and the
+        // clearing of the lines, which they overlap; each tile has at least one
+        // entry, so a clamped entry index is always valid.
+        constexpr int CB_PRE = 4;
+        int pcz[CB_PRE];
+        double2 pv[CB_PRE];
+        {
+            int pi[CB_PRE];
 #pragma unroll
-        for (int q = 0; q < CB_PRE; q++) {
-            const int e = e0 + (int)threadIdx.x + q * FT;
-            const int ec = e < e1 ? e : e0;
-            pcz[q] = ent_cz[ec];
-            pi[q] = ent_i[ec];
+            for (int q = 0; q < CB_PRE; q++) {
+                const int e = e0 + (int)threadIdx.x + q * FT;
+                const int ec = e < e1 ? e : e0;
+                pcz[q] = ent_cz[ec];
+                pi[q] = ent_i[ec];
+            }
+#pragma unroll
+            for (int q = 0; q < CB_PRE; q++) pv[q] = pb[pi[q]];
         }
+        load_twiddles(tw, tw3, N3);
+        for (int t = threadIdx.x; t < CT * LS; t += FT) lines[t] = mk<R>(0, 0);
+        __syncthreads();
 #pragma unroll
-        for (int q = 0; q < CB_PRE; q++) pv[q] = pb[pi[q]];
+        for (int q = 0; q < CB_PRE; q++)
+            if (e0 + (int)threadIdx.x + q * FT < e1)
+                lines[((pcz[q] >> 12) - c0) * LS + (pcz[q] & 0xfff)] = mk<R>((R)pv[q].x, (R)pv[q].y);
+        for (int e = e0 + (int)threadIdx.x + CB_PRE * FT; e < e1; e += FT) {
+            const int cz = ent_cz[e];
+            const double2 p = pb[ent_i[e]];
+            lines[((cz >> 12) - c0) * LS + (cz & 0xfff)] = mk<R>((R)p.x, (R)p.y);
+        }
+        __syncthreads();
+        line_fft<R, N3, +1>(lines, nc, LS, 1, tw);
+        cplx<R> *ob = colbuf + (long)band * N3 * g.ncolp + c0;
+        for (int t = threadIdx.x; t < N3 * CT; t += FT) {
+            const int z = t / CT, cc = t - z * CT;
+            if (cc < nc) ob[(long)z * g.ncolp + cc] = lines[cc * LS + z];
+        }
     }
-    load_twiddles(tw, tw3, N3);
-    for (int t = threadIdx.x; t < CT * LS; t += FT) lines[t] = mk<R>(0, 0);
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < CB_PRE; q++)
-        if (e0 + (int)threadIdx.x + q * FT < e1)
-            lines[((pcz[q] >> 12) - c0) * LS + (pcz[q] & 0xfff)] = mk<R>((R)pv[q].x, (R)pv[q].y);
-    for (int e = e0 + (int)threadIdx.x + CB_PRE * FT; e < e1; e += FT) {
-        const int cz = ent_cz[e];
-        const double2 p = pb[ent_i[e]];
-        lines[((cz >> 12) - c0) * LS + (cz & 0xfff)] = mk<R>((R)p.x, (R)p.y);
-    }
-    __syncthreads();
-    line_fft<R, N3, +1>(lines, nc, LS, 1, tw);
-    cplx<R> *ob = colbuf + (long)band * N3 * g.ncolp + c0;
-    for (int t = threadIdx.x; t < N3 * CT; t += FT) {
-        const int z = t / CT, cc = t - z * CT;
-        if (cc < nc) ob[(long)z * g.ncolp + cc] = lines[cc * LS + z];
-    }
+};
+template <typename R, int N3>
+__global__ __launch_bounds__(FT) void k_col_bwd_fast(const double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__
+    colbuf, const int *__restrict__ col_ptr, const int *__restrict__ ent_i, const int *__restrict__ ent_cz, const
+    double2 *__restrict__ tw3, FftGeom g, int ntiles, int nb) {
+    ColBwdFast<R, N3>::run(Blk::here(), psi, ldp, colbuf, col_ptr, ent_i, ent_cz, tw3, g, ntiles, nb);
 }
 
 // ---------------------------------------------------------------------------
 // colbuf -> forward FFT along z -> hpsi = local/N (+ ekpg psi) (+ hpsi)
 // ---------------------------------------------------------------------------
+template <typename R, int N3> struct ColFwdFast {
+    static constexpr int T = FT, W = 1;
+    static __device__ __forceinline__ void run(const Blk blk, const double2 *__restrict__ psi, long ldp, double2
+        *__restrict__ hpsi, long ldh, const cplx<R> *__restrict__ colbuf, const int *__restrict__ col_ptr, const int
+        *__restrict__ ent_i, const int *__restrict__ ent_cz, const double *__restrict__ ekpg, const double2
+        *__restrict__ tw3, FftGeom g, int ntiles, int nb, double inv_n, int mode) {
+        constexpr int CT = col_tile<N3>();
+        constexpr int LS = N3 + 1;
+        __shared__ cplx<R> tw[N3];
+        __shared__ cplx<R> lines[CT * LS];
+        int band, tile;
+        if (!xcd_band_tile(blk.x, ntiles, nb, band, tile)) return;
+        const int c0 = tile * CT;
+        const int nc = min(CT, g.ncol - c0);
+        load_twiddles(tw, tw3, N3);
+        const double2 *pb = psi + (long)band * ldp;
+        double2 *hb = hpsi + (long)band * ldh;
+        const int e0 = col_ptr[c0], e1 = col_ptr[c0 + nc];
+        // The first CF_PRE sphere entries of each thread: index, and the terms
+        // added to local/N (ekpg*psi and/or what hpsi already holds) are loaded
+        // before the transform, so their two dependent global round trips overlap it.
+        const bool kin = mode & COLF_KIN, acc = mode & COLF_ACC;
+        constexpr int CF_PRE = 4;
+        int pcz[CF_PRE], pi[CF_PRE];
+        double2 ph[CF_PRE];
+#pragma unroll
+        for (int q = 0; q < CF_PRE; q++) {
+            const int e = e0 + (int)threadIdx.x + q * FT;
+            const int ec = e < e1 ? e : e0;  // clamped: always a valid entry
+            pcz[q] = ent_cz[ec];
+            pi[q] = ent_i[ec];
+        }
+#pragma unroll
+        for (int q = 0; q < CF_PRE; q++) {
+            ph[q] = acc ? hb[pi[q]] : make_double2(0.0, 0.0);
+            if (kin) {
+                const double2 p = pb[pi[q]];
+                const double ek = ekpg[pi[q]];
+                ph[q].x += ek * p.x;
+                ph[q].y += ek * p.y;
+            }
+        }
+        // the tile's columns into the lines: every load of a thread issued before
+        // the first LDS store, so the round trips overlap (loads at clamped,
+        // valid positions; only the positions that exist are stored)
+        const cplx<R> *ib = colbuf + (long)band * N3 * g.ncolp + c0;
+        constexpr int NPT = (N3 * CT + FT - 1) / FT;
+        cplx<R> cv[NPT];
+#pragma unroll
+        for (int u = 0; u < NPT; u++) {
+            const int t = min((int)threadIdx.x + u * FT, N3 * CT - 1);
+            const int z = t / CT, cc = t - z * CT;
+            cv[u] = ib[(long)z * g.ncolp + min(cc, nc - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < NPT; u++) {
+            const int t = (int)threadIdx.x + u * FT;
+            const int z = t / CT, cc = t - z * CT;
+            if (t < N3 * CT && cc < nc) lines[cc * LS + z] = cv[u];
+        }
+        __syncthreads();
+        line_fft<R, N3, -1>(lines, nc, LS, 1, tw);
+        // hpsi = local/N + ekpg psi (+ the non-local term already in hpsi)
+#pragma unroll
+        for (int q = 0; q < CF_PRE; q++) {
+            if (e0 + (int)threadIdx.x + q * FT < e1) {
+                const cplx<R> v = lines[((pcz[q] >> 12) - c0) * LS + (pcz[q] & 0xfff)];
+                hb[pi[q]] = make_double2((double)v.x * inv_n + ph[q].x, (double)v.y * inv_n + ph[q].y);
+            }
+        }
+        for (int e = e0 + threadIdx.x + CF_PRE * FT; e < e1; e += FT) {
+            const int cz = ent_cz[e];
+            const int i = ent_i[e];
+            const cplx<R> v = lines[((cz >> 12) - c0) * LS + (cz & 0xfff)];
+            double2 h = make_double2((double)v.x * inv_n, (double)v.y * inv_n);
+            if (kin) {
+                const double2 p = pb[i];
+                const double ek = ekpg[i];
+                h.x += ek * p.x;
+                h.y += ek * p.y;
+            }
+            if (acc) {
+                const double2 o = hb[i];
+                h.x += o.x;
+                h.y += o.y;
+            }
+            hb[i] = h;
+        }
+    }
+};
 template <typename R, int N3>
-__global__ __launch_bounds__(FT) void k_col_fwd_fast(
-    const double2 *__restrict__ psi, long ldp, double2 *__restrict__ hpsi, long ldh,
-    const cplx<R> *__restrict__ colbuf, const int *__restrict__ col_ptr,
-    const int *__restrict__ ent_i, const int *__restrict__ ent_cz, const double *__restrict__ ekpg,
-    const double2 *__restrict__ tw3, FftGeom g, int ntiles, int nb, double inv_n, int mode) {
-    constexpr int CT = col_tile<N3>();
-    constexpr int LS = N3 + 1;
-    __shared__ cplx<R> tw[N3];
-    __shared__ cplx<R> lines[CT * LS];
-    int band, tile;
-    if (!xcd_band_tile(blockIdx.x, ntiles, nb, band, tile)) return;
-    const int c0 = tile * CT;
-    const int nc = min(CT, g.ncol - c0);
-    load_twiddles(tw, tw3, N3);
-    const double2 *pb = psi + (long)band * ldp;
-    double2 *hb = hpsi + (long)band * ldh;
-    const int e0 = col_ptr[c0], e1 = col_ptr[c0 + nc];
-    // The first CF_PRE sphere entries of each thread: index, and the terms
-    // added to local/N (ekpg*psi and/or what hpsi already holds) are loaded
-    // before the transform, so their two dependent global round trips overlap it.
-    const bool kin = mode & COLF_KIN, acc = mode & COLF_ACC;
-    constexpr int CF_PRE = 4;
-    int pcz[CF_PRE], pi[CF_PRE];
-    double2 ph[CF_PRE];
-#pragma unroll
-    for (int q = 0; q < CF_PRE; q++) {
-        const int e = e0 + (int)threadIdx.x + q * FT;
-        const int ec = e < e1 ? e : e0;  // clamped: always a valid entry
-        pcz[q] = ent_cz[ec];
-        pi[q] = ent_i[ec];
-    }
-#pragma unroll
-    for (int q = 0; q < CF_PRE; q++) {
-        ph[q] = acc ? hb[pi[q]] : make_double2(0.0, 0.0);
-        if (kin) {
-            const double2 p = pb[pi[q]];
-            const double ek = ekpg[pi[q]];
-            ph[q].x += ek * p.x;
-            ph[q].y += ek * p.y;
-        }
-    }
-    // the tile's columns into the lines: every load of a thread issued before
-    // the first LDS store, so the round trips overlap (loads at clamped,
-    // valid positions; only the positions that exist are stored)
-    const cplx<R> *ib = colbuf + (long)band * N3 * g.ncolp + c0;
-    constexpr int NPT = (N3 * CT + FT - 1) / FT;
-    cplx<R> cv[NPT];
-#pragma unroll
-    for (int u = 0; u < NPT; u++) {
-        const int t = min((int)threadIdx.x + u * FT, N3 * CT - 1);
-        const int z = t / CT, cc = t - z * CT;
-        cv[u] = ib[(long)z * g.ncolp + min(cc, nc - 1)];
-    }
-#pragma unroll
-    for (int u = 0; u < NPT; u++) {
-        const int t = (int)threadIdx.x + u * FT;
-        const int z = t / CT, cc = t - z * CT;
-        if (t < N3 * CT && cc < nc) lines[cc * LS + z] = cv[u];
-    }
-    __syncthreads();
-    line_fft<R, N3, -1>(lines, nc, LS, 1, tw);
-    // hpsi = local/N + ekpg psi (+ the non-local term already in hpsi)
-#pragma unroll
-    for (int q = 0; q < CF_PRE; q++) {
-        if (e0 + (int)threadIdx.x + q * FT < e1) {
-            const cplx<R> v = lines[((pcz[q] >> 12) - c0) * LS + (pcz[q] & 0xfff)];
-            hb[pi[q]] = make_double2((double)v.x * inv_n + ph[q].x, (double)v.y * inv_n + ph[q].y);
-        }
-    }
-    for (int e = e0 + threadIdx.x + CF_PRE * FT; e < e1; e += FT) {
-        const int cz = ent_cz[e];
-        const int i = ent_i[e];
-        const cplx<R> v = lines[((cz >> 12) - c0) * LS + (cz & 0xfff)];
-        double2 h = make_double2((double)v.x * inv_n, (double)v.y * inv_n);
-        if (kin) {
-            const double2 p = pb[i];
-            const double ek = ekpg[i];
-            h.x += ek * p.x;
-            h.y += ek * p.y;
-        }
-        if (acc) {
-            const double2 o = hb[i];
-            h.x += o.x;
-            h.y += o.y;
-        }
-        hb[i] = h;
-    }
+__global__ __launch_bounds__(FT) void k_col_fwd_fast(const double2 *__restrict__ psi, long ldp, double2 *__restrict__
+    hpsi, long ldh, const cplx<R> *__restrict__ colbuf, const int *__restrict__ col_ptr, const int *__restrict__
+    ent_i, const int *__restrict__ ent_cz, const double *__restrict__ ekpg, const double2 *__restrict__ tw3, FftGeom
+    g, int ntiles, int nb, double inv_n, int mode) {
+    ColFwdFast<R, N3>::run(Blk::here(), psi, ldp, hpsi, ldh, colbuf, col_ptr, ent_i, ent_cz, ekpg, tw3, g, ntiles, nb, inv_n, mode);
 }
 
 // ---------------------------------------------------------------------------

@@ -24,6 +24,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include "batch.hpp"
 #include <stdint.h>
 
 #include "fft_core.hpp"

@@ -322,140 +322,144 @@ __device__ __forceinline__ void scatter_plane(cplx<R> *__restrict__ cb, const cp
 // ---------------------------------------------------------------------------
 template <int N> constexpr int pr_sub_stride() { return N / 2 + 3; }
 
+template <typename R, int N, int GX, int GY, int P, int T_, int W_, bool YW, bool PR, int SC> struct PlaneReg {
+    static constexpr int T = T_, W = W_;
+    static __device__ __forceinline__ void run(const Blk blk, cplx<R> *__restrict__ colbuf, const int *__restrict__
+        col_uy, const R *__restrict__ vr, const double2 *__restrict__ twg, FftGeom g, int nb, int S_arg) {
+        static_assert(N % GX == 0 && N % GY == 0 && T % 64 == 0, "bad plane shape");
+        constexpr int MX = N / GX, MY = N / GY;
+        const int S = SC ? SC : S_arg;
+        // slots that can hold box points (all of them unless PR)
+        constexpr u64mask XB = PR ? box_slots(N, GX, MX, N / 4) : full_mask(MX);
+        constexpr u64mask YB = PR ? box_slots(N, GY, MY, N / 4) : full_mask(MY);
+        extern __shared__ __align__(16) unsigned char smem_raw[];
+        cplx<R> *twN = reinterpret_cast<cplx<R> *>(smem_raw);  // [N]
+        cplx<R> *sub = twN + N;                                 // [P][N][S]
+        const int n3 = g.n[2];
+        const int z = blk.x % n3;
+        const int b0 = (blk.x / n3) * P;
+        const int np = min(P, nb - b0);  // planes of this block that exist
+        const int nx = g.nx, kd1 = g.kd[0], ushift = N - nx, xhi = N - kd1;
+        const int tid = threadIdx.x;
+
+        // the first GPRE z-column values of each thread (first plane) are loaded
+        // before the twiddles and the clearing of the sub-plane, which they
+        // overlap (clamped: the kernel runs only with g.ncol >= 1); four named
+        // values, not an array, so that FP64 keeps them in registers too
+        constexpr int GPRE = 4, NPRE = GPRE;
+        struct Pre { int uy; cplx<R> v; };
+        const cplx<R> *cb0 = colbuf + ((long)b0 * n3 + z) * g.ncolp;
+        const auto pre = [&](int u) {
+            const int c = min(tid + u * T, g.ncol - 1);
+            return Pre{col_uy[c], cb0[c]};
+        };
+        const Pre q0 = pre(0), q1 = pre(1), q2 = pre(2), q3 = pre(3);
+        load_twiddles(twN, twg, N);
+        for (int q = tid; q < P * N * S; q += T) sub[q] = mk<R>(0, 0);
+        __syncthreads();
+        const auto put = [&](int u, const Pre &q) {
+            if (tid + u * T < g.ncol) sub[(q.uy >> 16) * S + (q.uy & 0xffff)] = q.v;
+        };
+        put(0, q0);
+        put(1, q1);
+        put(2, q2);
+        put(3, q3);
+        for (int p = 0; p < np; p++)
+            gather_plane<R, T>(sub + p * N * S, colbuf + ((long)(b0 + p) * n3 + z) * g.ncolp, col_uy, g.ncol, S,
+                               p == 0 ? NPRE * T : 0);
+        __syncthreads();
+
+        if constexpr (YW) {
+            for (int p = 0; p < P; p++) line_fft_wave<R, N, +1, T>(sub + p * N * S, nx, 1, S, twN);
+        } else {  // inverse y on the P * nx box lines
+            const Lanes<R, GY> L;
+            const int ntask = P * nx;
+            for (int task = tid / GY; task < ntask; task += T / GY) {
+                const int p = task / nx, u = task - p * nx;
+                cplx<R> *col = sub + p * N * S + u;
+                cplx<R> v[MY];
+#pragma unroll
+                for (int j = 0; j < MY; j++)
+                    if (has_bit(YB, j)) v[j] = col[(L.g + GY * j) * S];
+                line_dif<+1, GY, MY, R, YB>(v, L, twN);
+#pragma unroll
+                for (int k = 0; k < MY; k++) col[(k + MY * L.k2) * S] = v[k];
+            }
+        }
+        __syncthreads();
+
+        {  // rows: inverse x, V(r), forward x
+            const Lanes<R, GX> L;
+            const int ntask = P * N;
+            // the lane twiddles of every row: in FP64, read once into registers
+            // where they fit (up to 9 per lane; all loads in flight together),
+            // else read from LDS as each transform uses them.  (FP64 blocks are
+            // held to 3 per CU by LDS anyway; in FP32 the 16 extra registers cost
+            // a wave per SIMD and measured 5% slower.)
+            constexpr bool HOIST = sizeof(R) == 8 && MX <= 9;
+            cplx<R> twx[MX];
+            if constexpr (HOIST) {
+#pragma unroll
+                for (int k = 1; k < MX; k++) twx[k] = twN[L.g * k];
+            }
+            const auto tw = [&]() {
+                if constexpr (HOIST) return TwRegs<R, MX>{twx};
+                else return TwLds<R>{twN, L.g};
+            }();
+            for (int task = tid / GX; task < ntask; task += T / GX) {
+                const int p = task / N, y = task - p * N;
+                cplx<R> *row = sub + (p * N + y) * S;
+                cplx<R> v[MX];
+                // x = g + GX j: box columns, or the zero column nx for the gap
+#pragma unroll
+                for (int j = 0; j < MX; j++) {
+                    const int x = L.g + GX * j;
+                    if (has_bit(XB, j)) v[j] = row[x <= kd1 ? x : x >= xhi ? x - ushift : nx];
+                }
+                // (with bfly_t the odd positions carry negated values between the two)
+                line_dif_tw<+1, GX, MX, R, XB, true>(v, L, tw);
+                const R *vy = vr + ((long)z * g.n[1] + y) * g.id + MX * L.k2;
+#pragma unroll
+                for (int k = 0; k < MX; k++) v[k] = scale(v[k], vy[k]);
+                line_dit_tw<-1, GX, MX, R, XB, true>(v, L, tw);
+                // gap columns go to the trash column nx + 1
+#pragma unroll
+                for (int m = 0; m < MX; m++) {
+                    const int x = L.g + GX * m;
+                    if (has_bit(XB, m)) row[x <= kd1 ? x : x >= xhi ? x - ushift : nx + 1] = v[m];
+                }
+            }
+        }
+        __syncthreads();
+
+        if constexpr (YW) {
+            for (int p = 0; p < P; p++) line_fft_wave<R, N, -1, T>(sub + p * N * S, nx, 1, S, twN);
+        } else {  // forward y
+            const Lanes<R, GY> L;
+            const int ntask = P * nx;
+            for (int task = tid / GY; task < ntask; task += T / GY) {
+                const int p = task / nx, u = task - p * nx;
+                cplx<R> *col = sub + p * N * S + u;
+                cplx<R> v[MY];
+#pragma unroll
+                for (int k = 0; k < MY; k++) v[k] = col[(k + MY * L.k2) * S];
+                line_dit<-1, GY, MY, R, YB>(v, L, twN);
+                // rows outside the y box are not gathered back
+#pragma unroll
+                for (int m = 0; m < MY; m++)
+                    if (has_bit(YB, m)) col[(L.g + GY * m) * S] = v[m];
+            }
+        }
+        __syncthreads();
+        // scatter back, the map entries of four columns per thread loaded together
+        for (int p = 0; p < np; p++)
+            scatter_plane<R, T>(colbuf + ((long)(b0 + p) * n3 + z) * g.ncolp, sub + p * N * S, col_uy, g.ncol, S);
+    }
+};
 template <typename R, int N, int GX, int GY, int P, int T, int W, bool YW = false, bool PR = false, int SC = 0>
-__global__ __launch_bounds__(T, W) void k_plane_reg(cplx<R> *__restrict__ colbuf,
-                                                 const int *__restrict__ col_uy,
-                                                 const R *__restrict__ vr,
-                                                 const double2 *__restrict__ twg, FftGeom g,
-                                                 int nb, int S_arg) {
-    static_assert(N % GX == 0 && N % GY == 0 && T % 64 == 0, "bad plane shape");
-    constexpr int MX = N / GX, MY = N / GY;
-    const int S = SC ? SC : S_arg;
-    // slots that can hold box points (all of them unless PR)
-    constexpr u64mask XB = PR ? box_slots(N, GX, MX, N / 4) : full_mask(MX);
-    constexpr u64mask YB = PR ? box_slots(N, GY, MY, N / 4) : full_mask(MY);
-    extern __shared__ __align__(16) unsigned char smem_raw[];
-    cplx<R> *twN = reinterpret_cast<cplx<R> *>(smem_raw);  // [N]
-    cplx<R> *sub = twN + N;                                 // [P][N][S]
-    const int n3 = g.n[2];
-    const int z = blockIdx.x % n3;
-    const int b0 = (blockIdx.x / n3) * P;
-    const int np = min(P, nb - b0);  // planes of this block that exist
-    const int nx = g.nx, kd1 = g.kd[0], ushift = N - nx, xhi = N - kd1;
-    const int tid = threadIdx.x;
-
-    // the first GPRE z-column values of each thread (first plane) are loaded
-    // before the twiddles and the clearing of the sub-plane, which they
-    // overlap (clamped: the kernel runs only with g.ncol >= 1); four named
-    // values, not an array, so that FP64 keeps them in registers too
-    constexpr int GPRE = 4, NPRE = GPRE;
-    struct Pre { int uy; cplx<R> v; };
-    const cplx<R> *cb0 = colbuf + ((long)b0 * n3 + z) * g.ncolp;
-    const auto pre = [&](int u) {
-        const int c = min(tid + u * T, g.ncol - 1);
-        return Pre{col_uy[c], cb0[c]};
-    };
-    const Pre q0 = pre(0), q1 = pre(1), q2 = pre(2), q3 = pre(3);
-    load_twiddles(twN, twg, N);
-    for (int q = tid; q < P * N * S; q += T) sub[q] = mk<R>(0, 0);
-    __syncthreads();
-    const auto put = [&](int u, const Pre &q) {
-        if (tid + u * T < g.ncol) sub[(q.uy >> 16) * S + (q.uy & 0xffff)] = q.v;
-    };
-    put(0, q0);
-    put(1, q1);
-    put(2, q2);
-    put(3, q3);
-    for (int p = 0; p < np; p++)
-        gather_plane<R, T>(sub + p * N * S, colbuf + ((long)(b0 + p) * n3 + z) * g.ncolp, col_uy, g.ncol, S,
-                           p == 0 ? NPRE * T : 0);
-    __syncthreads();
-
-    if constexpr (YW) {
-        for (int p = 0; p < P; p++) line_fft_wave<R, N, +1, T>(sub + p * N * S, nx, 1, S, twN);
-    } else {  // inverse y on the P * nx box lines
-        const Lanes<R, GY> L;
-        const int ntask = P * nx;
-        for (int task = tid / GY; task < ntask; task += T / GY) {
-            const int p = task / nx, u = task - p * nx;
-            cplx<R> *col = sub + p * N * S + u;
-            cplx<R> v[MY];
-#pragma unroll
-            for (int j = 0; j < MY; j++)
-                if (has_bit(YB, j)) v[j] = col[(L.g + GY * j) * S];
-            line_dif<+1, GY, MY, R, YB>(v, L, twN);
-#pragma unroll
-            for (int k = 0; k < MY; k++) col[(k + MY * L.k2) * S] = v[k];
-        }
-    }
-    __syncthreads();
-
-    {  // rows: inverse x, V(r), forward x
-        const Lanes<R, GX> L;
-        const int ntask = P * N;
-        // the lane twiddles of every row: in FP64, read once into registers
-        // where they fit (up to 9 per lane; all loads in flight together),
-        // else read from LDS as each transform uses them.  (FP64 blocks are
-        // held to 3 per CU by LDS anyway; in FP32 the 16 extra registers cost
-        // a wave per SIMD and measured 5% slower.)
-        constexpr bool HOIST = sizeof(R) == 8 && MX <= 9;
-        cplx<R> twx[MX];
-        if constexpr (HOIST) {
-#pragma unroll
-            for (int k = 1; k < MX; k++) twx[k] = twN[L.g * k];
-        }
-        const auto tw = [&]() {
-            if constexpr (HOIST) return TwRegs<R, MX>{twx};
-            else return TwLds<R>{twN, L.g};
-        }();
-        for (int task = tid / GX; task < ntask; task += T / GX) {
-            const int p = task / N, y = task - p * N;
-            cplx<R> *row = sub + (p * N + y) * S;
-            cplx<R> v[MX];
-            // x = g + GX j: box columns, or the zero column nx for the gap
-#pragma unroll
-            for (int j = 0; j < MX; j++) {
-                const int x = L.g + GX * j;
-                if (has_bit(XB, j)) v[j] = row[x <= kd1 ? x : x >= xhi ? x - ushift : nx];
-            }
-            // (with bfly_t the odd positions carry negated values between the two)
-            line_dif_tw<+1, GX, MX, R, XB, true>(v, L, tw);
-            const R *vy = vr + ((long)z * g.n[1] + y) * g.id + MX * L.k2;
-#pragma unroll
-            for (int k = 0; k < MX; k++) v[k] = scale(v[k], vy[k]);
-            line_dit_tw<-1, GX, MX, R, XB, true>(v, L, tw);
-            // gap columns go to the trash column nx + 1
-#pragma unroll
-            for (int m = 0; m < MX; m++) {
-                const int x = L.g + GX * m;
-                if (has_bit(XB, m)) row[x <= kd1 ? x : x >= xhi ? x - ushift : nx + 1] = v[m];
-            }
-        }
-    }
-    __syncthreads();
-
-    if constexpr (YW) {
-        for (int p = 0; p < P; p++) line_fft_wave<R, N, -1, T>(sub + p * N * S, nx, 1, S, twN);
-    } else {  // forward y
-        const Lanes<R, GY> L;
-        const int ntask = P * nx;
-        for (int task = tid / GY; task < ntask; task += T / GY) {
-            const int p = task / nx, u = task - p * nx;
-            cplx<R> *col = sub + p * N * S + u;
-            cplx<R> v[MY];
-#pragma unroll
-            for (int k = 0; k < MY; k++) v[k] = col[(k + MY * L.k2) * S];
-            line_dit<-1, GY, MY, R, YB>(v, L, twN);
-            // rows outside the y box are not gathered back
-#pragma unroll
-            for (int m = 0; m < MY; m++)
-                if (has_bit(YB, m)) col[(L.g + GY * m) * S] = v[m];
-        }
-    }
-    __syncthreads();
-    // scatter back, the map entries of four columns per thread loaded together
-    for (int p = 0; p < np; p++)
-        scatter_plane<R, T>(colbuf + ((long)(b0 + p) * n3 + z) * g.ncolp, sub + p * N * S, col_uy, g.ncol, S);
+__global__ __launch_bounds__(T, W) void k_plane_reg(cplx<R> *__restrict__ colbuf, const int *__restrict__ col_uy,
+    const R *__restrict__ vr, const double2 *__restrict__ twg, FftGeom g, int nb, int S_arg) {
+    PlaneReg<R, N, GX, GY, P, T, W, YW, PR, SC>::run(Blk::here(), colbuf, col_uy, vr, twg, g, nb, S_arg);
 }
 
 // LDS bytes of k_plane_reg

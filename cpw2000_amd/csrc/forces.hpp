@@ -241,7 +241,7 @@ __global__ __launch_bounds__(GEMM_THREADS, 2) void k_force_phi(
     __shared__ double red[4][PHI_BA][3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 15, lg = lane >> 4;
-    const Tile3 tl = gemm_tile_yfirst();
+    const Tile3 tl = gemm_tile_yfirst(Blk::here());
     const int i0 = tl.x * PHI_BI + wave * 16 * IT;
     const int a0 = tl.y * PHI_BA;
     const cplx<double> *pcol[IT];

@@ -101,6 +101,10 @@ inline Prof g_prof;
 // recorded around it, which would idle the stream between the kernels.
 template <typename... Args, typename F = void (*)(Args...)>
 void launch_timed(int k, F f, dim3 grid, dim3 block, size_t shmem, hipStream_t s, Args... args) {
+    if (g_rec) {  // a kernel that cannot be batched
+        g_rec->ok = false;
+        return;
+    }
     if (g_prof.on && (g_prof.mask >> k & 1u)) {
         hipEvent_t a = g_prof.get(), b = a ? g_prof.get() : nullptr;
         if (a && b) {
@@ -111,6 +115,20 @@ void launch_timed(int k, F f, dim3 grid, dim3 block, size_t shmem, hipStream_t s
         if (a) g_prof.pool.push_back(a);
     }
     hipLaunchKernelGGL(f, grid, block, shmem, s, args...);
+}
+
+// The same for kernel f whose body is K::run: recorded for a batch when a
+// recorder is set.
+template <class K, typename... Args, typename F = void (*)(Args...)>
+void launch_batchable(int k, F f, dim3 grid, dim3 block, size_t shmem, hipStream_t s, Args... args) {
+    if (g_rec) {
+        const auto p = make_pack(args...);
+        static_assert(std::is_trivially_copyable<decltype(p)>::value, "arguments are copied to the device");
+        const char *b = reinterpret_cast<const char *>(&p);
+        g_rec->steps.push_back({(const void *)k_batch<K, Args...>, grid, block.x, shmem, {b, b + sizeof p}});
+        return;
+    }
+    launch_timed(k, f, grid, block, shmem, s, args...);
 }
 
 }  // namespace cpwgpu

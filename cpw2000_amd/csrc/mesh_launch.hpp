@@ -14,11 +14,11 @@ int launch_col_fast(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int s
     const int ntiles = (g.ncol + CT - 1) / CT;
     const dim3 grid(8 * ((a.nb + 7) / 8) * ntiles);
     if (stage == ST_COL_BWD) {
-        launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, colbuf,
+        launch_batchable<ColBwdFast<R, N>>(CPWGPU_K_COL_BWD, (k_col_bwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, colbuf,
                            (const int *)p->col_ptr.p, (const int *)p->ent_i.p,
                            (const int *)p->ent_cz.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb);
     } else {
-        launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, a.hpsi, a.ldh,
+        launch_batchable<ColFwdFast<R, N>>(CPWGPU_K_COL_FWD, (k_col_fwd_fast<R, N>), grid, dim3(FT), 0, s, a.psi, a.ldp, a.hpsi, a.ldh,
                            (const cplx<R> *)colbuf, (const int *)p->col_ptr.p,
                            (const int *)p->ent_i.p, (const int *)p->ent_cz.p,
                            (const double *)p->ekpg.p, (const double2 *)p->tw[2].p, g, ntiles, a.nb,
@@ -62,7 +62,7 @@ int launch_plane_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, cons
         const FftGeom &g = p->g;
         if (PR && !prune_fits(g))
             return fail(CPWGPU_ERR_MODE, "plane variant %d needs the sphere box inside N/4", V);
-        const auto go = [&](auto kernel, int S, bool &attr) -> int {
+        const auto go = [&](auto kernel, auto body, int S, bool &attr) -> int {
             const size_t dyn = plane_reg_lds<R, N, P>(S);
             if (dyn > 160 * 1024)
                 return fail(CPWGPU_ERR_SIZE, "plane variant %d: %zu bytes of LDS", V, dyn);
@@ -70,24 +70,34 @@ int launch_plane_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, cons
                 HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
                 attr = true;
             }
-            launch_timed(CPWGPU_K_PLANE, kernel, dim3(((a.nb + P - 1) / P) * g.n[2]), dim3(T), dyn, s, colbuf,
-                         (const int *)p->col_uy.p, vr, (const double2 *)p->tw[0].p, g, a.nb, S);
+            const dim3 grid(((a.nb + P - 1) / P) * g.n[2]);
+            const int *uy = (const int *)p->col_uy.p;
+            const double2 *tw = (const double2 *)p->tw[0].p;
+            if constexpr (std::is_void<typename decltype(body)::type>::value)
+                launch_timed(CPWGPU_K_PLANE, kernel, grid, dim3(T), dyn, s, colbuf, uy, vr, tw, g, a.nb, S);
+            else
+                launch_batchable<typename decltype(body)::type>(CPWGPU_K_PLANE, kernel, grid, dim3(T), dyn, s, colbuf, uy,
+                                                                vr, tw, g, a.nb, S);
             HIPCHK(hipGetLastError());
             return CPWGPU_OK;
         };
+        // body: the default shape of the length can be batched
+        struct None { using type = void; };
         const int S = reg_stride(g.nx);
         static bool attr_rt = false;
         if constexpr (PR) {
             constexpr int SC = pr_stride<R, N, V>();
             static bool attr_ct = false;
-            if (S <= SC) return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, SC>, SC, attr_ct);
+            struct Body { using type = PlaneReg<R, N, GX, GY, P, T, W, YW, PR, SC>; };
+            using B = typename std::conditional<V == plane_var_default<R, N>(), Body, None>::type;
+            if (S <= SC) return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, SC>, B{}, SC, attr_ct);
             // kd = N/4 exactly where the stride is N/2 + 1
             if constexpr (SC >= N / 2 + 3 || N % 4 != 0)
                 return fail(CPWGPU_ERR_MODE, "plane variant %d: %d box columns exceed its row stride", V, g.nx);
             else
-                return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, S, attr_rt);
+                return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, None{}, S, attr_rt);
         } else {
-            return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, S, attr_rt);
+            return go(k_plane_reg<R, N, GX, GY, P, T, W, YW, PR, 0>, None{}, S, attr_rt);
         }
     }
 }
@@ -126,14 +136,14 @@ int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int st
         const int *zm = (const int *)p->zmap.p;
         if (stage == ST_COL_BWD) {
             if (pr)
-                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
+                launch_batchable<ColBwdReg<R, N, G, true>>(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
                                    zm, tw3, g, ntiles, a.nb);
             else
                 launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
                                    zm, tw3, g, ntiles, a.nb);
         } else {
             if (pr)
-                launch_timed(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
+                launch_batchable<ColFwdReg<R, N, G, true>>(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,
                                    a.ldh, (const cplx<R> *)colbuf, zm, (const double *)p->ekpg.p, tw3, g, ntiles,
                                    a.nb, p->inv_n, a.mode);
             else

@@ -60,18 +60,18 @@ __device__ __forceinline__ int xcd_linear(int L, int T) {
 struct Tile3 {
     int x, y, z;
 };
-__device__ __forceinline__ Tile3 gemm_tile_xfirst() {
-    const int gx = gridDim.x, gy = gridDim.y;
-    const int L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-    const int j = xcd_linear(L, gx * gy * (int)gridDim.z);
+__device__ __forceinline__ Tile3 gemm_tile_xfirst(const Blk b) {
+    const int gx = b.gx, gy = b.gy;
+    const int L = b.x + gx * (b.y + gy * b.z);
+    const int j = xcd_linear(L, gx * gy * b.gz);
     const int r = j / gx;
     return {j - r * gx, r % gy, r / gy};
 }
 // The same for a 2-D grid with y fastest: the band tiles of one block of
 // plane waves (which read the same projector rows) run on one XCD.
-__device__ __forceinline__ Tile3 gemm_tile_yfirst() {
-    const int gx = gridDim.x, gy = gridDim.y;
-    const int j = xcd_linear(blockIdx.x + gx * blockIdx.y, gx * gy);
+__device__ __forceinline__ Tile3 gemm_tile_yfirst(const Blk b) {
+    const int gx = b.gx, gy = b.gy;
+    const int j = xcd_linear(b.x + gx * b.y, gx * gy);
     const int x = j / gy;
     return {x, j - x * gy, 0};
 }
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void k_proj(const cplx<R> *__restrict
     constexpr int LPB = BN * BK / GEMM_THREADS;   // (psi)
     __shared__ __align__(16) R sA[2][2][BM][KP];  // [buf][re/im][a][k]
     __shared__ __align__(16) R sB[2][2][BN][KP];  // [buf][re/im][n][k]
-    const Tile3 tl = gemm_tile_xfirst();
+    const Tile3 tl = gemm_tile_xfirst(Blk::here());
     const int a0 = tl.x * BM, n0 = tl.y * BN;
     // lower != 0: only the lower triangle (a >= n) of a Hermitian Gram matrix
     // is wanted; tiles wholly above the diagonal are skipped (whole block)
@@ -324,131 +324,139 @@ __device__ __forceinline__ void load_psi_tail(double2 (&dst)[KPL], const double2
     }
 }
 
-template <typename R, int V>
-__global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_direct(
-    const cplx<R> *__restrict__ anl, long lda, const double2 *__restrict__ psi, long ldp,
-    cplx<R> *__restrict__ part, int mtxd, int nanl, int neig, int kslice, int lower = 0) {
-    typedef typename MF<R>::v4 v4;
-    constexpr int WM = DirectCfg<R, V>::WM, WN = DirectCfg<R, V>::WN;
-    constexpr int KPL = DirectCfg<R, V>::KPL, KC = 4 * KPL;
-    constexpr int BM = direct_bm<R, V>(), BN = direct_bn<R, V>();
-    const Tile3 tl = gemm_tile_xfirst();
-    const int a0 = tl.x * BM, n0 = tl.y * BN;
-    // lower != 0: only the lower triangle (a >= n) of a Hermitian Gram matrix;
-    // tiles wholly above the diagonal are skipped (the reduction zeroes them)
-    if (lower && a0 + BM <= n0) return;
-    const int kb = tl.z * kslice, ke = min(mtxd, kb + kslice);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int GM = DirectCfg<R, V>::GM;
-    const int wm = wave % GM, wn = wave / GM;
-    const int lr = lane & 15, lg = lane >> 4;
-    const cplx<R> *arow[WM];
+template <typename R, int V> struct ProjDirect {
+    static constexpr int T = GEMM_THREADS, W = (DirectCfg<R, V>::W);
+    static __device__ __forceinline__ void run(const Blk blk, const cplx<R> *__restrict__ anl, long lda, const
+        double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__ part, int mtxd, int nanl, int neig, int kslice,
+        int lower) {
+        typedef typename MF<R>::v4 v4;
+        constexpr int WM = DirectCfg<R, V>::WM, WN = DirectCfg<R, V>::WN;
+        constexpr int KPL = DirectCfg<R, V>::KPL, KC = 4 * KPL;
+        constexpr int BM = direct_bm<R, V>(), BN = direct_bn<R, V>();
+        const Tile3 tl = gemm_tile_xfirst(blk);
+        const int a0 = tl.x * BM, n0 = tl.y * BN;
+        // lower != 0: only the lower triangle (a >= n) of a Hermitian Gram matrix;
+        // tiles wholly above the diagonal are skipped (the reduction zeroes them)
+        if (lower && a0 + BM <= n0) return;
+        const int kb = tl.z * kslice, ke = min(mtxd, kb + kslice);
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        constexpr int GM = DirectCfg<R, V>::GM;
+        const int wm = wave % GM, wn = wave / GM;
+        const int lr = lane & 15, lg = lane >> 4;
+        const cplx<R> *arow[WM];
 #pragma unroll
-    for (int t = 0; t < WM; t++) {
-        const int a = a0 + wm * WM * 16 + t * 16 + lr;
-        arow[t] = anl + (long)min(a, nanl - 1) * lda;
-    }
-    const double2 *bcol[WN];
-#pragma unroll
-    for (int t = 0; t < WN; t++) {
-        const int n = n0 + wn * WN * 16 + t * 16 + lr;
-        bcol[t] = psi + (long)min(n, neig - 1) * ldp;
-    }
-    v4 P1[WM][WN], P2[WM][WN], P3[WM][WN];
-#pragma unroll
-    for (int i = 0; i < WM; i++)
-#pragma unroll
-        for (int j = 0; j < WN; j++) {
-            P1[i][j] = v4{0, 0, 0, 0};
-            P2[i][j] = v4{0, 0, 0, 0};
-            P3[i][j] = v4{0, 0, 0, 0};
+        for (int t = 0; t < WM; t++) {
+            const int a = a0 + wm * WM * 16 + t * 16 + lr;
+            arow[t] = anl + (long)min(a, nanl - 1) * lda;
         }
-    constexpr int D = DirectCfg<R, V>::D;
-    cplx<R> ra[D][WM][KPL];
-    double2 rb[D][WN][KPL];
-    // tail: the last, partial chunk of the slice
-    auto load = [&](cplx<R>(&ra_)[WM][KPL], double2(&rb_)[WN][KPL], int k0, bool tail) {
-        const int i0 = k0 + lg * KPL;
-        if (!tail) {
+        const double2 *bcol[WN];
 #pragma unroll
-            for (int t = 0; t < WM; t++) load_row_full<R, KPL>(ra_[t], arow[t], i0);
-#pragma unroll
-            for (int t = 0; t < WN; t++) load_psi_full<KPL>(rb_[t], bcol[t], i0);
-        } else {
-#pragma unroll
-            for (int t = 0; t < WM; t++) load_row_tail<R, KPL>(ra_[t], arow[t], i0, mtxd);
-#pragma unroll
-            for (int t = 0; t < WN; t++) load_psi_tail<KPL>(rb_[t], bcol[t], i0, ke, mtxd);
+        for (int t = 0; t < WN; t++) {
+            const int n = n0 + wn * WN * 16 + t * 16 + lr;
+            bcol[t] = psi + (long)min(n, neig - 1) * ldp;
         }
-    };
-    auto compute = [&](const cplx<R>(&ra_)[WM][KPL], const double2(&rb_)[WN][KPL]) {
+        v4 P1[WM][WN], P2[WM][WN], P3[WM][WN];
 #pragma unroll
-        for (int u = 0; u < KPL; u++) {
-            R ar[WM], ai[WM], as[WM], br[WN], bi[WN], bs[WN];
+        for (int i = 0; i < WM; i++)
 #pragma unroll
-            for (int t = 0; t < WM; t++) {
-                ar[t] = ra_[t][u].x;
-                ai[t] = ra_[t][u].y;
-                as[t] = ar[t] - ai[t];
+            for (int j = 0; j < WN; j++) {
+                P1[i][j] = v4{0, 0, 0, 0};
+                P2[i][j] = v4{0, 0, 0, 0};
+                P3[i][j] = v4{0, 0, 0, 0};
             }
+        constexpr int D = DirectCfg<R, V>::D;
+        cplx<R> ra[D][WM][KPL];
+        double2 rb[D][WN][KPL];
+        // tail: the last, partial chunk of the slice
+        auto load = [&](cplx<R>(&ra_)[WM][KPL], double2(&rb_)[WN][KPL], int k0, bool tail) {
+            const int i0 = k0 + lg * KPL;
+            if (!tail) {
 #pragma unroll
-            for (int t = 0; t < WN; t++) {
-                br[t] = (R)rb_[t][u].x;
-                bi[t] = (R)rb_[t][u].y;
-                bs[t] = br[t] + bi[t];
+                for (int t = 0; t < WM; t++) load_row_full<R, KPL>(ra_[t], arow[t], i0);
+#pragma unroll
+                for (int t = 0; t < WN; t++) load_psi_full<KPL>(rb_[t], bcol[t], i0);
+            } else {
+#pragma unroll
+                for (int t = 0; t < WM; t++) load_row_tail<R, KPL>(ra_[t], arow[t], i0, mtxd);
+#pragma unroll
+                for (int t = 0; t < WN; t++) load_psi_tail<KPL>(rb_[t], bcol[t], i0, ke, mtxd);
             }
+        };
+        auto compute = [&](const cplx<R>(&ra_)[WM][KPL], const double2(&rb_)[WN][KPL]) {
 #pragma unroll
-            for (int mi = 0; mi < WM; mi++)
+            for (int u = 0; u < KPL; u++) {
+                R ar[WM], ai[WM], as[WM], br[WN], bi[WN], bs[WN];
 #pragma unroll
-                for (int ni = 0; ni < WN; ni++) {
-                    P1[mi][ni] = MF<R>::mma(ar[mi], br[ni], P1[mi][ni]);
-                    P2[mi][ni] = MF<R>::mma(ai[mi], bi[ni], P2[mi][ni]);
-                    P3[mi][ni] = MF<R>::mma(as[mi], bs[ni], P3[mi][ni]);
+                for (int t = 0; t < WM; t++) {
+                    ar[t] = ra_[t][u].x;
+                    ai[t] = ra_[t][u].y;
+                    as[t] = ar[t] - ai[t];
                 }
-        }
-    };
-    // Full chunks through a ring of D register buffers, D per trip: chunk
-    // c + D - 1 is loaded while chunk c is multiplied, unconditionally (at
-    // the last full chunk again when there is none: a valid address whose
-    // values go unused), so that the loop body is one straight block and each
-    // chunk's loads have D - 1 chunks of MFMAs to arrive.  The scheduling barrier
-    // keeps the loads above those MFMAs: without it the compiler sinks them to
-    // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122).  Then the partial
-    // chunk, if any.  Chunks are accumulated in K order for any D.
-    const int nfull = max(0, ke - kb) / KC;
-    if (nfull > 0) {
 #pragma unroll
-        for (int j = 0; j < D - 1; j++) load(ra[j], rb[j], kb + min(j, nfull - 1) * KC, false);
-        int c = 0;
-        for (; c + D <= nfull; c += D) {
+                for (int t = 0; t < WN; t++) {
+                    br[t] = (R)rb_[t][u].x;
+                    bi[t] = (R)rb_[t][u].y;
+                    bs[t] = br[t] + bi[t];
+                }
 #pragma unroll
-            for (int j = 0; j < D; j++) {
-                load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
-                __builtin_amdgcn_sched_barrier(0);
-                compute(ra[j], rb[j]);
+                for (int mi = 0; mi < WM; mi++)
+#pragma unroll
+                    for (int ni = 0; ni < WN; ni++) {
+                        P1[mi][ni] = MF<R>::mma(ar[mi], br[ni], P1[mi][ni]);
+                        P2[mi][ni] = MF<R>::mma(ai[mi], bi[ni], P2[mi][ni]);
+                        P3[mi][ni] = MF<R>::mma(as[mi], bs[ni], P3[mi][ni]);
+                    }
             }
-        }
+        };
+        // Full chunks through a ring of D register buffers, D per trip: chunk
+        // c + D - 1 is loaded while chunk c is multiplied, unconditionally (at
+        // the last full chunk again when there is none: a valid address whose
+        // values go unused), so that the loop body is one straight block and each
+        // chunk's loads have D - 1 chunks of MFMAs to arrive.  The scheduling barrier
+        // keeps the loads above those MFMAs: without it the compiler sinks them to
+        // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122).  Then the partial
+        // chunk, if any.  Chunks are accumulated in K order for any D.
+        const int nfull = max(0, ke - kb) / KC;
+        if (nfull > 0) {
 #pragma unroll
-        for (int j = 0; j < D - 1; j++)
-            if (c + j < nfull) compute(ra[j], rb[j]);
-    }
-    if (kb + nfull * KC < ke) {
-        load(ra[0], rb[0], kb + nfull * KC, true);
-        compute(ra[0], rb[0]);
-    }
-    cplx<R> *ps = part + (long)tl.z * neig * nanl;
+            for (int j = 0; j < D - 1; j++) load(ra[j], rb[j], kb + min(j, nfull - 1) * KC, false);
+            int c = 0;
+            for (; c + D <= nfull; c += D) {
 #pragma unroll
-    for (int mi = 0; mi < WM; mi++)
-#pragma unroll
-        for (int ni = 0; ni < WN; ni++) {
-            const int n = n0 + wn * WN * 16 + ni * 16 + lr;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int a = a0 + wm * WM * 16 + mi * 16 + MF<R>::row(lg, r);
-                const R p1 = P1[mi][ni][r], p2 = P2[mi][ni][r], p3 = P3[mi][ni][r];
-                if (a < nanl && n < neig) ps[(long)n * nanl + a] = mk<R>(p1 + p2, p3 - p1 + p2);
+                for (int j = 0; j < D; j++) {
+                    load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
+                    __builtin_amdgcn_sched_barrier(0);
+                    compute(ra[j], rb[j]);
+                }
             }
+#pragma unroll
+            for (int j = 0; j < D - 1; j++)
+                if (c + j < nfull) compute(ra[j], rb[j]);
         }
+        if (kb + nfull * KC < ke) {
+            load(ra[0], rb[0], kb + nfull * KC, true);
+            compute(ra[0], rb[0]);
+        }
+        cplx<R> *ps = part + (long)tl.z * neig * nanl;
+#pragma unroll
+        for (int mi = 0; mi < WM; mi++)
+#pragma unroll
+            for (int ni = 0; ni < WN; ni++) {
+                const int n = n0 + wn * WN * 16 + ni * 16 + lr;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int a = a0 + wm * WM * 16 + mi * 16 + MF<R>::row(lg, r);
+                    const R p1 = P1[mi][ni][r], p2 = P2[mi][ni][r], p3 = P3[mi][ni][r];
+                    if (a < nanl && n < neig) ps[(long)n * nanl + a] = mk<R>(p1 + p2, p3 - p1 + p2);
+                }
+            }
+    }
+};
+template <typename R, int V>
+__global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_direct(const cplx<R> *__restrict__ anl,
+    long lda, const double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__ part, int mtxd, int nanl, int neig,
+    int kslice, int lower = 0) {
+    ProjDirect<R, V>::run(Blk::here(), anl, lda, psi, ldp, part, mtxd, nanl, neig, kslice, lower);
 }
 
 // dhd[n][a] = xnlkb[a] * sum_s part[s][n][a]   (fixed summation order: deterministic)
@@ -456,46 +464,50 @@ __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_dir
 // slices g, g+4, ... into four independent partial sums (16 loads in flight
 // per thread), then the groups are combined through LDS in group order.
 constexpr int RED_OUT = 64, RED_GRP = 4;
+template <typename R> struct ProjReduce {
+    static constexpr int T = RED_OUT * RED_GRP, W = 1;
+    static __device__ __forceinline__ void run(const Blk blk, const cplx<R> *__restrict__ part, const double
+        *__restrict__ xnl, cplx<R> *__restrict__ dhd, int nanl, int neig, int nslice, int lower) {
+        __shared__ cplx<R> red[RED_GRP][RED_OUT];
+        const int o = threadIdx.x % RED_OUT, grp = threadIdx.x / RED_OUT;
+        const long tot = (long)nanl * neig;
+        const long t = (long)blk.x * RED_OUT + o;
+        const long tc = t < tot ? t : tot - 1;  // clamped, always a valid address
+        R sr[4] = {0, 0, 0, 0}, si[4] = {0, 0, 0, 0};
+        int s = grp;
+        for (; s + 3 * RED_GRP < nslice; s += 4 * RED_GRP) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const cplx<R> v = part[(long)(s + u * RED_GRP) * tot + tc];
+                sr[u] += v.x;
+                si[u] += v.y;
+            }
+        }
+        for (; s < nslice; s += RED_GRP) {
+            const cplx<R> v = part[(long)s * tot + tc];
+            sr[0] += v.x;
+            si[0] += v.y;
+        }
+        red[grp][o] = mk<R>((sr[0] + sr[1]) + (sr[2] + sr[3]), (si[0] + si[1]) + (si[2] + si[3]));
+        __syncthreads();
+        if (grp == 0 && t < tot) {
+            R r = 0, i = 0;
+#pragma unroll
+            for (int g2 = 0; g2 < RED_GRP; g2++) {
+                r += red[g2][o].x;
+                i += red[g2][o].y;
+            }
+            const R x = xnl ? (R)xnl[t % nanl] : (R)1;  // no scaling for plain Gram matrices
+            // lower: the strict upper triangle (partials of skipped tiles) is zero
+            const bool up = lower && (t % nanl) < (t / nanl);
+            dhd[t] = up ? mk<R>((R)0, (R)0) : mk<R>(x * r, x * i);
+        }
+    }
+};
 template <typename R>
-__global__ __launch_bounds__(RED_OUT * RED_GRP) void k_proj_reduce(const cplx<R> *__restrict__ part,
-                                                                  const double *__restrict__ xnl,
-                                                                  cplx<R> *__restrict__ dhd,
-                                                                  int nanl, int neig, int nslice,
-                                                                  int lower = 0) {
-    __shared__ cplx<R> red[RED_GRP][RED_OUT];
-    const int o = threadIdx.x % RED_OUT, grp = threadIdx.x / RED_OUT;
-    const long tot = (long)nanl * neig;
-    const long t = (long)blockIdx.x * RED_OUT + o;
-    const long tc = t < tot ? t : tot - 1;  // clamped, always a valid address
-    R sr[4] = {0, 0, 0, 0}, si[4] = {0, 0, 0, 0};
-    int s = grp;
-    for (; s + 3 * RED_GRP < nslice; s += 4 * RED_GRP) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const cplx<R> v = part[(long)(s + u * RED_GRP) * tot + tc];
-            sr[u] += v.x;
-            si[u] += v.y;
-        }
-    }
-    for (; s < nslice; s += RED_GRP) {
-        const cplx<R> v = part[(long)s * tot + tc];
-        sr[0] += v.x;
-        si[0] += v.y;
-    }
-    red[grp][o] = mk<R>((sr[0] + sr[1]) + (sr[2] + sr[3]), (si[0] + si[1]) + (si[2] + si[3]));
-    __syncthreads();
-    if (grp == 0 && t < tot) {
-        R r = 0, i = 0;
-#pragma unroll
-        for (int g2 = 0; g2 < RED_GRP; g2++) {
-            r += red[g2][o].x;
-            i += red[g2][o].y;
-        }
-        const R x = xnl ? (R)xnl[t % nanl] : (R)1;  // no scaling for plain Gram matrices
-        // lower: the strict upper triangle (partials of skipped tiles) is zero
-        const bool up = lower && (t % nanl) < (t / nanl);
-        dhd[t] = up ? mk<R>((R)0, (R)0) : mk<R>(x * r, x * i);
-    }
+__global__ __launch_bounds__(RED_OUT * RED_GRP) void k_proj_reduce(const cplx<R> *__restrict__ part, const double
+    *__restrict__ xnl, cplx<R> *__restrict__ dhd, int nanl, int neig, int nslice, int lower = 0) {
+    ProjReduce<R>::run(Blk::here(), part, xnl, dhd, nanl, neig, nslice, lower);
 }
 
 // Launches k_proj_reduce over nanl * neig outputs (nothing to do when empty).
@@ -524,133 +536,137 @@ constexpr int BP_BN = 64;  // bands per block
 // KCX: projectors per LDS chunk (variant 0 uses GemmCfg<R>::KC; half of it
 // keeps fewer values in flight per lane, for more waves per SIMD)
 // NT: tiles of 16 bands per block
-template <typename R, int KCX = GemmCfg<R>::KC, int NT = BP_BN / 16>
-__global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict__ anl, long lda,
-                                                       const cplx<R> *__restrict__ dhd,
-                                                       double2 *__restrict__ hpsi, long ldh,
-                                                       int mtxd, int nanl, int neig, int beta,
-                                                       const double2 *__restrict__ kpsi = nullptr,
-                                                       long ldk = 0,
-                                                       const double *__restrict__ ekpg = nullptr) {
-    typedef typename MF<R>::v4 v4;
-    // LDS rows padded by 16 bytes: an odd number of 16-byte units per row
-    constexpr int KC = KCX, KCP = KCX + 16 / (int)sizeof(R);
-    static_assert((KCP * sizeof(R) / 16) % 2 == 1 && KC % 16 == 0, "bad k_back chunk");
-    constexpr int KPL = KC / 4;             // projectors per lane group per chunk
-    constexpr int BN = 16 * NT;
-    constexpr int DPT = BN * KC / GEMM_THREADS;  // dhd values a thread stages
-    __shared__ __align__(16) R sD[3][BN][KCP];   // re, im, re+im
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lr = lane & 15, lg = lane >> 4;
-    const Tile3 tl = gemm_tile_yfirst();
-    const int i = tl.x * BP_BI + wave * 16 + lr;
-    const int n0 = tl.y * BN;
-    v4 P1[NT], P2[NT], P3[NT];
+template <typename R, int KCX, int NT> struct BackLds {
+    static constexpr int T = GEMM_THREADS, W = 1;
+    static __device__ __forceinline__ void run(const Blk blk, const cplx<R> *__restrict__ anl, long lda, const
+        cplx<R> *__restrict__ dhd, double2 *__restrict__ hpsi, long ldh, int mtxd, int nanl, int neig, int beta,
+        const double2 *__restrict__ kpsi, long ldk, const double *__restrict__ ekpg) {
+        typedef typename MF<R>::v4 v4;
+        // LDS rows padded by 16 bytes: an odd number of 16-byte units per row
+        constexpr int KC = KCX, KCP = KCX + 16 / (int)sizeof(R);
+        static_assert((KCP * sizeof(R) / 16) % 2 == 1 && KC % 16 == 0, "bad k_back chunk");
+        constexpr int KPL = KC / 4;             // projectors per lane group per chunk
+        constexpr int BN = 16 * NT;
+        constexpr int DPT = BN * KC / GEMM_THREADS;  // dhd values a thread stages
+        __shared__ __align__(16) R sD[3][BN][KCP];   // re, im, re+im
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int lr = lane & 15, lg = lane >> 4;
+        const Tile3 tl = gemm_tile_yfirst(blk);
+        const int i = tl.x * BP_BI + wave * 16 + lr;
+        const int n0 = tl.y * BN;
+        v4 P1[NT], P2[NT], P3[NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        P1[t] = v4{0, 0, 0, 0};
-        P2[t] = v4{0, 0, 0, 0};
-        P3[t] = v4{0, 0, 0, 0};
-    }
-    // staging of dhd: value q of a thread is projector tid % KC of band row
-    // tid / KC + q * (256 / KC)
-    constexpr int RPQ = GEMM_THREADS / KC;
-    static_assert(GEMM_THREADS % KC == 0 && BN % RPQ == 0, "bad k_back staging");
-    const int srow = threadIdx.x / KC, soff = threadIdx.x % KC;
-    cplx<R> rd[DPT];
-    // rows beyond the matrix (bands n >= neig, plane waves i >= mtxd) are
-    // read at clamped addresses and only reach outputs that are not stored;
-    // full chunks issue plain loads (first used after the current chunk's
-    // MFMAs), the projector tail is clamped with dhd zero-masked
-    const auto dat = [&](int q, int a) { return (long)min(n0 + srow + q * RPQ, neig - 1) * nanl + a; };
-    auto dload = [&](int ka) {
-        if (ka + KC <= nanl) {  // the same for the whole block
+        for (int t = 0; t < NT; t++) {
+            P1[t] = v4{0, 0, 0, 0};
+            P2[t] = v4{0, 0, 0, 0};
+            P3[t] = v4{0, 0, 0, 0};
+        }
+        // staging of dhd: value q of a thread is projector tid % KC of band row
+        // tid / KC + q * (256 / KC)
+        constexpr int RPQ = GEMM_THREADS / KC;
+        static_assert(GEMM_THREADS % KC == 0 && BN % RPQ == 0, "bad k_back staging");
+        const int srow = threadIdx.x / KC, soff = threadIdx.x % KC;
+        cplx<R> rd[DPT];
+        // rows beyond the matrix (bands n >= neig, plane waves i >= mtxd) are
+        // read at clamped addresses and only reach outputs that are not stored;
+        // full chunks issue plain loads (first used after the current chunk's
+        // MFMAs), the projector tail is clamped with dhd zero-masked
+        const auto dat = [&](int q, int a) { return (long)min(n0 + srow + q * RPQ, neig - 1) * nanl + a; };
+        auto dload = [&](int ka) {
+            if (ka + KC <= nanl) {  // the same for the whole block
 #pragma unroll
-            for (int q = 0; q < DPT; q++) rd[q] = dhd[dat(q, ka + soff)];
-        } else {
+                for (int q = 0; q < DPT; q++) rd[q] = dhd[dat(q, ka + soff)];
+            } else {
+#pragma unroll
+                for (int q = 0; q < DPT; q++) {
+                    const int a = ka + soff;
+                    const cplx<R> v = dhd[dat(q, min(a, nanl - 1))];
+                    rd[q] = mk<R>(a < nanl ? v.x : (R)0, a < nanl ? v.y : (R)0);
+                }
+            }
+        };
+        cplx<R> av[KPL];
+        const cplx<R> *acol = anl + min(i, mtxd - 1);
+        auto aload = [&](int ka) {
+            if (ka + KC <= nanl) {
+#pragma unroll
+                for (int u = 0; u < KPL; u++) av[u] = acol[(long)(ka + lg * KPL + u) * lda];
+            } else {
+#pragma unroll
+                for (int u = 0; u < KPL; u++) av[u] = acol[(long)min(ka + lg * KPL + u, nanl - 1) * lda];
+            }
+        };
+        dload(0);
+        aload(0);
+        for (int ka = 0; ka < nanl; ka += KC) {
 #pragma unroll
             for (int q = 0; q < DPT; q++) {
-                const int a = ka + soff;
-                const cplx<R> v = dhd[dat(q, min(a, nanl - 1))];
-                rd[q] = mk<R>(a < nanl ? v.x : (R)0, a < nanl ? v.y : (R)0);
+                sD[0][srow + q * RPQ][soff] = rd[q].x;
+                sD[1][srow + q * RPQ][soff] = rd[q].y;
+                sD[2][srow + q * RPQ][soff] = rd[q].x + rd[q].y;
             }
-        }
-    };
-    cplx<R> av[KPL];
-    const cplx<R> *acol = anl + min(i, mtxd - 1);
-    auto aload = [&](int ka) {
-        if (ka + KC <= nanl) {
-#pragma unroll
-            for (int u = 0; u < KPL; u++) av[u] = acol[(long)(ka + lg * KPL + u) * lda];
-        } else {
-#pragma unroll
-            for (int u = 0; u < KPL; u++) av[u] = acol[(long)min(ka + lg * KPL + u, nanl - 1) * lda];
-        }
-    };
-    dload(0);
-    aload(0);
-    for (int ka = 0; ka < nanl; ka += KC) {
-#pragma unroll
-        for (int q = 0; q < DPT; q++) {
-            sD[0][srow + q * RPQ][soff] = rd[q].x;
-            sD[1][srow + q * RPQ][soff] = rd[q].y;
-            sD[2][srow + q * RPQ][soff] = rd[q].x + rd[q].y;
-        }
-        __syncthreads();
-        R cr[KPL], ci[KPL], cs[KPL];
-#pragma unroll
-        for (int u = 0; u < KPL; u++) {
-            cr[u] = av[u].x;
-            ci[u] = av[u].y;
-            cs[u] = av[u].x + av[u].y;
-        }
-        if (ka + KC < nanl) {
-            dload(ka + KC);
-            aload(ka + KC);
-        }
-#pragma unroll
-        for (int ni = 0; ni < NT; ni++) {
-            R dr[KPL], di[KPL], ds[KPL];
+            __syncthreads();
+            R cr[KPL], ci[KPL], cs[KPL];
 #pragma unroll
             for (int u = 0; u < KPL; u++) {
-                dr[u] = sD[0][ni * 16 + lr][lg * KPL + u];
-                di[u] = sD[1][ni * 16 + lr][lg * KPL + u];
-                ds[u] = sD[2][ni * 16 + lr][lg * KPL + u];
+                cr[u] = av[u].x;
+                ci[u] = av[u].y;
+                cs[u] = av[u].x + av[u].y;
+            }
+            if (ka + KC < nanl) {
+                dload(ka + KC);
+                aload(ka + KC);
             }
 #pragma unroll
-            for (int u = 0; u < KPL; u++) {
-                P1[ni] = MF<R>::mma(dr[u], cr[u], P1[ni]);
-                P2[ni] = MF<R>::mma(di[u], ci[u], P2[ni]);
-                P3[ni] = MF<R>::mma(ds[u], cs[u], P3[ni]);
+            for (int ni = 0; ni < NT; ni++) {
+                R dr[KPL], di[KPL], ds[KPL];
+#pragma unroll
+                for (int u = 0; u < KPL; u++) {
+                    dr[u] = sD[0][ni * 16 + lr][lg * KPL + u];
+                    di[u] = sD[1][ni * 16 + lr][lg * KPL + u];
+                    ds[u] = sD[2][ni * 16 + lr][lg * KPL + u];
+                }
+#pragma unroll
+                for (int u = 0; u < KPL; u++) {
+                    P1[ni] = MF<R>::mma(dr[u], cr[u], P1[ni]);
+                    P2[ni] = MF<R>::mma(di[u], ci[u], P2[ni]);
+                    P3[ni] = MF<R>::mma(ds[u], cs[u], P3[ni]);
+                }
             }
+            __syncthreads();
         }
-        __syncthreads();
-    }
-    if (i < mtxd) {
-        // the kinetic term in FP64 (coalesced rows of psi) and the term already
-        // in hpsi: the loads of four outputs issued together (at clamped rows:
-        // a row beyond neig is loaded and not used), then their stores
-        const double ek = kpsi ? ekpg[i] : 0.0;
+        if (i < mtxd) {
+            // the kinetic term in FP64 (coalesced rows of psi) and the term already
+            // in hpsi: the loads of four outputs issued together (at clamped rows:
+            // a row beyond neig is loaded and not used), then their stores
+            const double ek = kpsi ? ekpg[i] : 0.0;
 #pragma unroll
-        for (int ni = 0; ni < NT; ni++) {
-            double2 kp[4], ho[4];
+            for (int ni = 0; ni < NT; ni++) {
+                double2 kp[4], ho[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const long nc = min(n0 + ni * 16 + MF<R>::row(lg, r), neig - 1);
-                kp[r] = kpsi ? kpsi[nc * ldk + i] : make_double2(0.0, 0.0);
-                ho[r] = beta ? hpsi[nc * ldh + i] : make_double2(0.0, 0.0);
-            }
+                for (int r = 0; r < 4; r++) {
+                    const long nc = min(n0 + ni * 16 + MF<R>::row(lg, r), neig - 1);
+                    kp[r] = kpsi ? kpsi[nc * ldk + i] : make_double2(0.0, 0.0);
+                    ho[r] = beta ? hpsi[nc * ldh + i] : make_double2(0.0, 0.0);
+                }
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int n = n0 + ni * 16 + MF<R>::row(lg, r);
-                if (n < neig) {
-                    const R p1 = P1[ni][r], p2 = P2[ni][r], p3 = P3[ni][r];
-                    hpsi[(long)n * ldh + i] = make_double2((double)(p1 - p2) + ek * kp[r].x + ho[r].x,
-                                                           (double)(p3 - p1 - p2) + ek * kp[r].y + ho[r].y);
+                for (int r = 0; r < 4; r++) {
+                    const int n = n0 + ni * 16 + MF<R>::row(lg, r);
+                    if (n < neig) {
+                        const R p1 = P1[ni][r], p2 = P2[ni][r], p3 = P3[ni][r];
+                        hpsi[(long)n * ldh + i] = make_double2((double)(p1 - p2) + ek * kp[r].x + ho[r].x,
+                                                               (double)(p3 - p1 - p2) + ek * kp[r].y + ho[r].y);
+                    }
                 }
             }
         }
     }
+};
+template <typename R, int KCX = GemmCfg<R>::KC, int NT = BP_BN / 16>
+__global__ __launch_bounds__(GEMM_THREADS) void k_back(const cplx<R> *__restrict__ anl, long lda, const cplx<R>
+    *__restrict__ dhd, double2 *__restrict__ hpsi, long ldh, int mtxd, int nanl, int neig, int beta, const double2
+    *__restrict__ kpsi = nullptr, long ldk = 0, const double *__restrict__ ekpg = nullptr) {
+    BackLds<R, KCX, NT>::run(Blk::here(), anl, lda, dhd, hpsi, ldh, mtxd, nanl, neig, beta, kpsi, ldk, ekpg);
 }
 
 // ---------------------------------------------------------------------------
@@ -680,142 +696,149 @@ template <> struct BackDirectCfg<double, 3> { static constexpr int NT = 2, IT = 
 template <typename R, int V> constexpr int back_bi() { return 4 * 16 * BackDirectCfg<R, V>::IT; }
 template <typename R, int V> constexpr int back_bn() { return 16 * BackDirectCfg<R, V>::NT; }
 
-template <typename R, int V>
-__global__ __launch_bounds__(GEMM_THREADS, (BackDirectCfg<R, V>::W)) void k_back_direct(
-    const cplx<R> *__restrict__ anl, long lda, const cplx<R> *__restrict__ dhd,
-    double2 *__restrict__ hpsi, long ldh, int mtxd, int nanl, int neig, int beta,
-    const double2 *__restrict__ kpsi, long ldk, const double *__restrict__ ekpg) {
-    typedef typename MF<R>::v4 v4;
-    constexpr int NT = BackDirectCfg<R, V>::NT, IT = BackDirectCfg<R, V>::IT;
-    constexpr int KPL = BackDirectCfg<R, V>::KPL, KC = 4 * KPL;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lr = lane & 15, lg = lane >> 4;
-    const Tile3 tl = gemm_tile_yfirst();
-    const int i0 = tl.x * back_bi<R, V>() + wave * 16 * IT;
-    const int n0 = tl.y * back_bn<R, V>();
-    // projector values of this lane's plane waves (column i of anlga^T) and
-    // dhd rows (bands) of its NT row tiles, at clamped addresses: a clamped
-    // row only reaches outputs that are not stored (see load_row_full)
-    bool iok[IT];
-    const cplx<R> *acol[IT];
-#pragma unroll
-    for (int q = 0; q < IT; q++) {
-        const int i = i0 + q * 16 + lr;
-        iok[q] = i < mtxd;
-        acol[q] = anl + min(i, mtxd - 1);
-    }
-    const cplx<R> *drow[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) drow[t] = dhd + (long)min(n0 + t * 16 + lr, neig - 1) * nanl;
-    v4 P1[NT][IT], P2[NT][IT], P3[NT][IT];
-#pragma unroll
-    for (int t = 0; t < NT; t++)
+template <typename R, int V> struct BackDirect {
+    static constexpr int T = GEMM_THREADS, W = (BackDirectCfg<R, V>::W);
+    static __device__ __forceinline__ void run(const Blk blk, const cplx<R> *__restrict__ anl, long lda, const
+        cplx<R> *__restrict__ dhd, double2 *__restrict__ hpsi, long ldh, int mtxd, int nanl, int neig, int beta,
+        const double2 *__restrict__ kpsi, long ldk, const double *__restrict__ ekpg) {
+        typedef typename MF<R>::v4 v4;
+        constexpr int NT = BackDirectCfg<R, V>::NT, IT = BackDirectCfg<R, V>::IT;
+        constexpr int KPL = BackDirectCfg<R, V>::KPL, KC = 4 * KPL;
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int lr = lane & 15, lg = lane >> 4;
+        const Tile3 tl = gemm_tile_yfirst(blk);
+        const int i0 = tl.x * back_bi<R, V>() + wave * 16 * IT;
+        const int n0 = tl.y * back_bn<R, V>();
+        // projector values of this lane's plane waves (column i of anlga^T) and
+        // dhd rows (bands) of its NT row tiles, at clamped addresses: a clamped
+        // row only reaches outputs that are not stored (see load_row_full)
+        bool iok[IT];
+        const cplx<R> *acol[IT];
 #pragma unroll
         for (int q = 0; q < IT; q++) {
-            P1[t][q] = v4{0, 0, 0, 0};
-            P2[t][q] = v4{0, 0, 0, 0};
-            P3[t][q] = v4{0, 0, 0, 0};
+            const int i = i0 + q * 16 + lr;
+            iok[q] = i < mtxd;
+            acol[q] = anl + min(i, mtxd - 1);
         }
-    constexpr int D = BackDirectCfg<R, V>::D;
-    cplx<R> dv[D][NT][KPL], av[D][IT][KPL];
-    // full chunks: plain loads; the projector tail: clamped, dhd zero-masked
-    auto load = [&](cplx<R>(&d)[NT][KPL], cplx<R>(&a_)[IT][KPL], int ka, bool tail) {
-        if (!tail) {
+        const cplx<R> *drow[NT];
 #pragma unroll
-            for (int u = 0; u < KPL; u++) {
-                const int a = ka + lg * KPL + u;
+        for (int t = 0; t < NT; t++) drow[t] = dhd + (long)min(n0 + t * 16 + lr, neig - 1) * nanl;
+        v4 P1[NT][IT], P2[NT][IT], P3[NT][IT];
 #pragma unroll
-                for (int t = 0; t < NT; t++) d[t][u] = drow[t][a];
-#pragma unroll
-                for (int q = 0; q < IT; q++) a_[q][u] = acol[q][(long)a * lda];
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < KPL; u++) {
-                const int a = ka + lg * KPL + u;
-                const int acl = min(a, nanl - 1);
-                const bool aok = a < nanl;
-#pragma unroll
-                for (int t = 0; t < NT; t++) {
-                    const cplx<R> v = drow[t][acl];
-                    d[t][u] = mk<R>(aok ? v.x : (R)0, aok ? v.y : (R)0);
-                }
-#pragma unroll
-                for (int q = 0; q < IT; q++) a_[q][u] = acol[q][(long)acl * lda];
-            }
-        }
-    };
-    auto compute = [&](const cplx<R>(&d)[NT][KPL], const cplx<R>(&a_)[IT][KPL]) {
-#pragma unroll
-        for (int u = 0; u < KPL; u++) {
-            R cr[IT], ci[IT], cs[IT];
+        for (int t = 0; t < NT; t++)
 #pragma unroll
             for (int q = 0; q < IT; q++) {
-                cr[q] = a_[q][u].x;
-                ci[q] = a_[q][u].y;
-                cs[q] = a_[q][u].x + a_[q][u].y;
+                P1[t][q] = v4{0, 0, 0, 0};
+                P2[t][q] = v4{0, 0, 0, 0};
+                P3[t][q] = v4{0, 0, 0, 0};
             }
+        constexpr int D = BackDirectCfg<R, V>::D;
+        cplx<R> dv[D][NT][KPL], av[D][IT][KPL];
+        // full chunks: plain loads; the projector tail: clamped, dhd zero-masked
+        auto load = [&](cplx<R>(&d)[NT][KPL], cplx<R>(&a_)[IT][KPL], int ka, bool tail) {
+            if (!tail) {
 #pragma unroll
-            for (int t = 0; t < NT; t++) {
-                const R ds = d[t][u].x + d[t][u].y;
+                for (int u = 0; u < KPL; u++) {
+                    const int a = ka + lg * KPL + u;
+#pragma unroll
+                    for (int t = 0; t < NT; t++) d[t][u] = drow[t][a];
+#pragma unroll
+                    for (int q = 0; q < IT; q++) a_[q][u] = acol[q][(long)a * lda];
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < KPL; u++) {
+                    const int a = ka + lg * KPL + u;
+                    const int acl = min(a, nanl - 1);
+                    const bool aok = a < nanl;
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        const cplx<R> v = drow[t][acl];
+                        d[t][u] = mk<R>(aok ? v.x : (R)0, aok ? v.y : (R)0);
+                    }
+#pragma unroll
+                    for (int q = 0; q < IT; q++) a_[q][u] = acol[q][(long)acl * lda];
+                }
+            }
+        };
+        auto compute = [&](const cplx<R>(&d)[NT][KPL], const cplx<R>(&a_)[IT][KPL]) {
+#pragma unroll
+            for (int u = 0; u < KPL; u++) {
+                R cr[IT], ci[IT], cs[IT];
 #pragma unroll
                 for (int q = 0; q < IT; q++) {
-                    P1[t][q] = MF<R>::mma(d[t][u].x, cr[q], P1[t][q]);
-                    P2[t][q] = MF<R>::mma(d[t][u].y, ci[q], P2[t][q]);
-                    P3[t][q] = MF<R>::mma(ds, cs[q], P3[t][q]);
+                    cr[q] = a_[q][u].x;
+                    ci[q] = a_[q][u].y;
+                    cs[q] = a_[q][u].x + a_[q][u].y;
+                }
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const R ds = d[t][u].x + d[t][u].y;
+#pragma unroll
+                    for (int q = 0; q < IT; q++) {
+                        P1[t][q] = MF<R>::mma(d[t][u].x, cr[q], P1[t][q]);
+                        P2[t][q] = MF<R>::mma(d[t][u].y, ci[q], P2[t][q]);
+                        P3[t][q] = MF<R>::mma(ds, cs[q], P3[t][q]);
+                    }
+                }
+            }
+        };
+        // full chunks through a ring of D register buffers with unconditional
+        // (clamped) prefetch, as in k_proj_direct, then the partial chunk
+        const int nfull = nanl / KC;
+        if (nfull > 0) {
+#pragma unroll
+            for (int j = 0; j < D - 1; j++) load(dv[j], av[j], min(j, nfull - 1) * KC, false);
+            int c = 0;
+            for (; c + D <= nfull; c += D) {
+#pragma unroll
+                for (int j = 0; j < D; j++) {
+                    load(dv[(j + D - 1) % D], av[(j + D - 1) % D], min(c + j + D - 1, nfull - 1) * KC, false);
+                    __builtin_amdgcn_sched_barrier(0);  // as in k_proj_direct
+                    compute(dv[j], av[j]);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < D - 1; j++)
+                if (c + j < nfull) compute(dv[j], av[j]);
+        }
+        if (nfull * KC < nanl) {
+            load(dv[0], av[0], nfull * KC, true);
+            compute(dv[0], av[0]);
+        }
+#pragma unroll
+        for (int q = 0; q < IT; q++) {
+            if (!iok[q]) continue;
+            const int i = i0 + q * 16 + lr;
+            // as in k_back: the loads of four outputs issued together, then the stores
+            const double ek = kpsi ? ekpg[i] : 0.0;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                double2 kp[4], ho[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const long nc = min(n0 + t * 16 + MF<R>::row(lg, r), neig - 1);
+                    kp[r] = kpsi ? kpsi[nc * ldk + i] : make_double2(0.0, 0.0);
+                    ho[r] = beta ? hpsi[nc * ldh + i] : make_double2(0.0, 0.0);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int n = n0 + t * 16 + MF<R>::row(lg, r);
+                    if (n < neig) {
+                        const R p1 = P1[t][q][r], p2 = P2[t][q][r], p3 = P3[t][q][r];
+                        hpsi[(long)n * ldh + i] = make_double2((double)(p1 - p2) + ek * kp[r].x + ho[r].x,
+                                                               (double)(p3 - p1 - p2) + ek * kp[r].y + ho[r].y);
+                    }
                 }
             }
         }
-    };
-    // full chunks through a ring of D register buffers with unconditional
-    // (clamped) prefetch, as in k_proj_direct, then the partial chunk
-    const int nfull = nanl / KC;
-    if (nfull > 0) {
-#pragma unroll
-        for (int j = 0; j < D - 1; j++) load(dv[j], av[j], min(j, nfull - 1) * KC, false);
-        int c = 0;
-        for (; c + D <= nfull; c += D) {
-#pragma unroll
-            for (int j = 0; j < D; j++) {
-                load(dv[(j + D - 1) % D], av[(j + D - 1) % D], min(c + j + D - 1, nfull - 1) * KC, false);
-                __builtin_amdgcn_sched_barrier(0);  // as in k_proj_direct
-                compute(dv[j], av[j]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < D - 1; j++)
-            if (c + j < nfull) compute(dv[j], av[j]);
     }
-    if (nfull * KC < nanl) {
-        load(dv[0], av[0], nfull * KC, true);
-        compute(dv[0], av[0]);
-    }
-#pragma unroll
-    for (int q = 0; q < IT; q++) {
-        if (!iok[q]) continue;
-        const int i = i0 + q * 16 + lr;
-        // as in k_back: the loads of four outputs issued together, then the stores
-        const double ek = kpsi ? ekpg[i] : 0.0;
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            double2 kp[4], ho[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const long nc = min(n0 + t * 16 + MF<R>::row(lg, r), neig - 1);
-                kp[r] = kpsi ? kpsi[nc * ldk + i] : make_double2(0.0, 0.0);
-                ho[r] = beta ? hpsi[nc * ldh + i] : make_double2(0.0, 0.0);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int n = n0 + t * 16 + MF<R>::row(lg, r);
-                if (n < neig) {
-                    const R p1 = P1[t][q][r], p2 = P2[t][q][r], p3 = P3[t][q][r];
-                    hpsi[(long)n * ldh + i] = make_double2((double)(p1 - p2) + ek * kp[r].x + ho[r].x,
-                                                           (double)(p3 - p1 - p2) + ek * kp[r].y + ho[r].y);
-                }
-            }
-        }
-    }
+};
+template <typename R, int V>
+__global__ __launch_bounds__(GEMM_THREADS, (BackDirectCfg<R, V>::W)) void k_back_direct(const cplx<R> *__restrict__
+    anl, long lda, const cplx<R> *__restrict__ dhd, double2 *__restrict__ hpsi, long ldh, int mtxd, int nanl, int
+    neig, int beta, const double2 *__restrict__ kpsi, long ldk, const double *__restrict__ ekpg) {
+    BackDirect<R, V>::run(Blk::here(), anl, lda, dhd, hpsi, ldh, mtxd, nanl, neig, beta, kpsi, ldk, ekpg);
 }
 
 // FP64 -> FP32 copy of the projectors (FP32-mixed mode)
