@@ -27,6 +27,7 @@
 #include "subspace.hpp"
 #include "small_eig.hpp"
 #include "forces.hpp"
+#include "host_copy.hpp"
 #include "ditsp.hpp"
 #include "spin.hpp"
 #include "proj_kb.hpp"
@@ -784,14 +785,18 @@ int set_potential(cpwgpu_plan_s *p, const double *vscr, int mxdscr) {
     if ((st = upload(p->v64, vscr, p->ntot))) return st;
     {
         // V(G=0): mean over the n1*n2*n3 points (x beyond n1 is padding when id > n1)
-        double s = 0.0;
+        // in eight sums (one chain of additions took 0.4 ms at 72^3)
+        double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         const int n1 = p->g.n[0], n2 = p->g.n[1], n3 = p->g.n[2], id = p->g.id;
         for (int k3 = 0; k3 < n3; k3++)
             for (int k2 = 0; k2 < n2; k2++) {
                 const double *row = vscr + ((size_t)k3 * n2 + k2) * id;
-                for (int k1 = 0; k1 < n1; k1++) s += row[k1];
+                int k1 = 0;
+                for (; k1 + 8 <= n1; k1 += 8)
+                    for (int u = 0; u < 8; u++) s[u] += row[k1 + u];
+                for (; k1 < n1; k1++) s[0] += row[k1];
             }
-        p->v0 = s / ((double)n1 * n2 * n3);
+        p->v0 = (((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]))) / ((double)n1 * n2 * n3);
     }
     if ((st = p->v32.reserve(sizeof(float) * p->ntot))) return st;
     hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((p->ntot + 255) / 256)), dim3(256), 0, g_stream,
@@ -846,9 +851,11 @@ int set_projectors_host(cpwgpu_plan_s *p, const double *anlga, const double *xnl
     if (nanl < 0) return fail(CPWGPU_ERR_ARG, "nanl = %d", nanl);
     if (nanl > 0 && (!anlga || !xnlkb)) return fail(CPWGPU_ERR_ARG, "null projector array");
     return replace_projectors(p, nanl, [&](double2 *anl, long lda) -> int {
-        if (p->mtxd > 0)
-            HIPCHK(hipMemcpy2DAsync(anl, 16 * (size_t)lda, anlga, 16 * (size_t)mxddim, 16 * (size_t)p->mtxd, nanl,
-                                    hipMemcpyHostToDevice, g_stream));
+        if (p->mtxd > 0) {
+            const int rc = copy_in(anl, 16 * (size_t)lda, anlga, 16 * (size_t)mxddim, 16 * (size_t)p->mtxd,
+                                   nanl, g_stream);
+            if (rc) return rc;
+        }
         return upload(p->xnl, xnlkb, nanl);
     });
 }
@@ -1016,9 +1023,7 @@ int set_projectors_spin_host(cpwgpu_plan_s *p, const double *anlsp, const double
     const long slda = std::max(1, 2 * p->mtxd);
     st = p->sanl64.reserve(16 * (size_t)slda * nanlsp);
     if (!st && p->mtxd > 0) {
-        const hipError_t e = hipMemcpy2DAsync(p->sanl64.p, 16 * (size_t)slda, anlsp, 16 * (size_t)(2 * (size_t)mxddim),
-                                              16 * (size_t)(2 * p->mtxd), nanlsp, hipMemcpyHostToDevice, g_stream);
-        if (e != hipSuccess) st = fail(CPWGPU_ERR_HIP, "projector copy: %s", hipGetErrorString(e));
+        st = copy_in(p->sanl64.p, 16 * (size_t)slda, anlsp, 32 * (size_t)mxddim, 32 * (size_t)p->mtxd, nanlsp, g_stream);
     }
     if (!st) st = upload(p->sxnl, xnlkbsp, nanlsp);
     p->snanl = st ? 0 : nanlsp;
@@ -2649,6 +2654,7 @@ int cpwgpu_finalize(void) {
     g_drop.hs.release();
     g_drop.hd.release();
     g_drop.c8.release();
+    g_hc.release();
     g_spin_tmp.release();
     g_kb_tab.release(); g_kb_types.release(); g_kb_atoms.release(); g_kb_gw.release(); g_kb_out.release();
     if (g_blas) {
@@ -2805,8 +2811,8 @@ int cpwgpu_proj_nl_kb_c16(const double *rkpt, const int *mtxd, const int *isort,
         (st = g_kb_out.reserve(16 * (size_t)m * na)) ||
         (st = kb_build(s, (const double *)g_kb_gw.p, m, (double2 *)g_kb_out.p, m)))
         return st;
-    HIPCHK(hipMemcpy2DAsync(anlga, 16 * (size_t)*mxddim, g_kb_out.p, 16 * (size_t)m, 16 * (size_t)m, na,
-                            hipMemcpyDeviceToHost, g_stream));
+    if ((st = copy_out(anlga, 16 * (size_t)*mxddim, g_kb_out.p, 16 * (size_t)m, 16 * (size_t)m, na,
+                 g_stream))) return st;
     HIPCHK(hipStreamSynchronize(g_stream));
     return CPWGPU_OK;
 }
@@ -3306,15 +3312,13 @@ int cpwgpu_hk_psi_c16(const int *mtxd, const int *neig, const double *psi, doubl
     const size_t colb = 16 * (size_t)(*mtxd);
     if ((st = g_drop.psi.reserve(colb * *neig))) return st;
     if ((st = g_drop.hpsi.reserve(colb * *neig))) return st;
-    HIPCHK(hipMemcpy2DAsync(g_drop.psi.p, colb, psi, 16 * (size_t)*mxddim, colb, *neig,
-                            hipMemcpyHostToDevice, g_stream));
+    if ((st = copy_in(g_drop.psi.p, colb, psi, 16 * (size_t)*mxddim, colb, *neig, g_stream))) return st;
     const double *dpsi = (const double *)g_drop.psi.p;
     double *dhpsi = (double *)g_drop.hpsi.p;
     st = g_prec == CPWGPU_PREC_FP32 ? apply_t<float>(p, *neig, dpsi, *mtxd, dhpsi, *mtxd, g_stream)
                                     : apply_t<double>(p, *neig, dpsi, *mtxd, dhpsi, *mtxd, g_stream);
     if (st) return st;
-    HIPCHK(hipMemcpy2DAsync(hpsi, 16 * (size_t)*mxddim, g_drop.hpsi.p, colb, colb, *neig,
-                            hipMemcpyDeviceToHost, g_stream));
+    if ((st = copy_out(hpsi, 16 * (size_t)*mxddim, g_drop.hpsi.p, colb, colb, *neig, g_stream))) return st;
     HIPCHK(hipStreamSynchronize(g_stream));
     return CPWGPU_OK;
 }
@@ -3363,15 +3367,13 @@ int cpwgpu_hk_psi_allk_c16(const int *nrk, const int *mtxd_allk, const int *nban
                                       xnlkb_allk ? xnlkb_allk + k * ma : nullptr, nanl, *mxddim)))
             return st;
         const size_t colb = 16 * (size_t)mtxd, off = 2 * k * md * mb;  // doubles
-        HIPCHK(hipMemcpy2DAsync(g_allk.psi.p, colb, psi_allk + off, 16 * md, colb, nb, hipMemcpyHostToDevice,
-                                g_stream));
+        if ((st = copy_in(g_allk.psi.p, colb, psi_allk + off, 16 * md, colb, nb, g_stream))) return st;
         const double *dpsi = (const double *)g_allk.psi.p;
         double *dhpsi = (double *)g_allk.hpsi.p;
         st = g_prec == CPWGPU_PREC_FP32 ? apply_t<float>(p, nb, dpsi, mtxd, dhpsi, mtxd, g_stream)
                                         : apply_t<double>(p, nb, dpsi, mtxd, dhpsi, mtxd, g_stream);
         if (st) return st;
-        HIPCHK(hipMemcpy2DAsync(hpsi_allk + off, 16 * md, g_allk.hpsi.p, colb, colb, nb, hipMemcpyDeviceToHost,
-                                g_stream));
+        if ((st = copy_out(hpsi_allk + off, 16 * md, g_allk.hpsi.p, colb, colb, nb, g_stream))) return st;
     }
     HIPCHK(hipStreamSynchronize(g_stream));
     return CPWGPU_OK;
@@ -3444,16 +3446,14 @@ int cpwgpu_hk_psi_spin_c16(const int *mtxd, const int *neig, const double *psi_s
     const size_t colb = 32 * (size_t)(*mtxd);  // two components
     if ((st = g_drop.psi.reserve(colb * *neig))) return st;
     if ((st = g_drop.hpsi.reserve(colb * *neig))) return st;
-    HIPCHK(hipMemcpy2DAsync(g_drop.psi.p, colb, psi_sp, 32 * (size_t)*mxddim, colb, *neig, hipMemcpyHostToDevice,
-                            g_stream));
+    if ((st = copy_in(g_drop.psi.p, colb, psi_sp, 32 * (size_t)*mxddim, colb, *neig, g_stream))) return st;
     const double2 *dpsi = (const double2 *)g_drop.psi.p;
     double2 *dhpsi = (double2 *)g_drop.hpsi.p;
     const long ld = 2L * *mtxd;
     st = g_prec == CPWGPU_PREC_FP32 ? apply_spin<float>(p, *neig, dpsi, ld, dhpsi, ld, g_stream)
                                     : apply_spin<double>(p, *neig, dpsi, ld, dhpsi, ld, g_stream);
     if (st) return st;
-    HIPCHK(hipMemcpy2DAsync(hpsi_sp, 32 * (size_t)*mxddim, g_drop.hpsi.p, colb, colb, *neig, hipMemcpyDeviceToHost,
-                            g_stream));
+    if ((st = copy_out(hpsi_sp, 32 * (size_t)*mxddim, g_drop.hpsi.p, colb, colb, *neig, g_stream))) return st;
     HIPCHK(hipStreamSynchronize(g_stream));
     return CPWGPU_OK;
 }
@@ -3496,14 +3496,15 @@ int cpwgpu_hk_psi_c8(const int *mtxd, const int *neig, const float *psi, float *
     std::vector<double> x(xnlkb ? xnlkb : (const float *)nullptr, xnlkb ? xnlkb + na : (const float *)nullptr);
     if (na > 0 && (!anlga || !xnlkb)) return fail(CPWGPU_ERR_ARG, "null projector array");
     st = replace_projectors(p, na, [&](double2 *anl, long lda) -> int {
-        HIPCHK(hipMemcpy2DAsync(g_drop.c8.p, c8b, anlga, 8 * (size_t)*mxddim, c8b, na, hipMemcpyHostToDevice, g_stream));
+        const int rc = copy_in(g_drop.c8.p, c8b, anlga, 8 * (size_t)*mxddim, c8b, na, g_stream);
+        if (rc) return rc;
         hipLaunchKernelGGL(k_to_c128, grid((long)m * na), dim3(256), 0, g_stream, (const cplx<float> *)g_drop.c8.p,
                            (long)m, anl, lda, m, na);
         HIPCHK(hipGetLastError());
         return upload(p->xnl, x.data(), na);
     });
     if (st) return st;
-    HIPCHK(hipMemcpy2DAsync(g_drop.c8.p, c8b, psi, 8 * (size_t)*mxddim, c8b, n, hipMemcpyHostToDevice, g_stream));
+    if ((st = copy_in(g_drop.c8.p, c8b, psi, 8 * (size_t)*mxddim, c8b, n, g_stream))) return st;
     hipLaunchKernelGGL(k_to_c128, grid((long)m * n), dim3(256), 0, g_stream, (const cplx<float> *)g_drop.c8.p,
                        (long)m, (double2 *)g_drop.psi.p, (long)m, m, n);
     HIPCHK(hipGetLastError());
@@ -3511,7 +3512,7 @@ int cpwgpu_hk_psi_c8(const int *mtxd, const int *neig, const float *psi, float *
     hipLaunchKernelGGL(k_to_c64, grid((long)m * n), dim3(256), 0, g_stream, (const double2 *)g_drop.hpsi.p,
                        (long)m, (cplx<float> *)g_drop.c8.p, (long)m, m, n);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpy2DAsync(hpsi, 8 * (size_t)*mxddim, g_drop.c8.p, c8b, c8b, n, hipMemcpyDeviceToHost, g_stream));
+    if ((st = copy_out(hpsi, 8 * (size_t)*mxddim, g_drop.c8.p, c8b, c8b, n, g_stream))) return st;
     HIPCHK(hipStreamSynchronize(g_stream));
     return CPWGPU_OK;
 }
@@ -3577,18 +3578,17 @@ int cpwgpu_ditsp_c16(const int *ipr, int *ifail, const int *icmax, const int *ig
         (st = g_drop.hs.reserve(16 * (size_t)ms * ms)) || (st = g_drop.hd.reserve(8 * (size_t)m)))
         return st;
     if (*iguess == 1)
-        HIPCHK(hipMemcpy2DAsync(g_drop.psi.p, colb, psi, 16 * (size_t)*mxddim, colb, n, hipMemcpyHostToDevice,
-                                g_stream));
-    HIPCHK(hipMemcpy2DAsync(g_drop.hs.p, 16 * (size_t)ms, hamsm, 16 * (size_t)*mxdsml, 16 * (size_t)ms, ms,
-                            hipMemcpyHostToDevice, g_stream));
+        if ((st = copy_in(g_drop.psi.p, colb, psi, 16 * (size_t)*mxddim, colb, n, g_stream))) return st;
+    if ((st = copy_in(g_drop.hs.p, 16 * (size_t)ms, hamsm, 16 * (size_t)*mxdsml, 16 * (size_t)ms, ms,
+                 g_stream))) return st;
     HIPCHK(hipMemcpyAsync(g_drop.hd.p, hdiag, 8 * (size_t)m, hipMemcpyHostToDevice, g_stream));
     int stats[5] = {0, 0, 0, 0, -1};
     double2 *dpsi = (double2 *)g_drop.psi.p, *dhpsi = (double2 *)g_drop.hpsi.p;
     if ((st = plan_ditsp(p, g_prec, *icmax, *iguess, *epspsi, n, ms, (const double2 *)g_drop.hs.p, ms,
                          (const double *)g_drop.hd.p, dpsi, m, dhpsi, m, ei, ifail, stats, g_stream)))
         return st;
-    HIPCHK(hipMemcpy2DAsync(psi, 16 * (size_t)*mxddim, dpsi, colb, colb, n, hipMemcpyDeviceToHost, g_stream));
-    HIPCHK(hipMemcpy2DAsync(hpsi, 16 * (size_t)*mxddim, dhpsi, colb, colb, n, hipMemcpyDeviceToHost, g_stream));
+    if ((st = copy_out(psi, 16 * (size_t)*mxddim, dpsi, colb, colb, n, g_stream))) return st;
+    if ((st = copy_out(hpsi, 16 * (size_t)*mxddim, dhpsi, colb, colb, n, g_stream))) return st;
     HIPCHK(hipStreamSynchronize(g_stream));
     // messages of Src/ditsp/ditsp_c16.f90:386-419
     if (ms >= m) {

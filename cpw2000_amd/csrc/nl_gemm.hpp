@@ -414,7 +414,8 @@ template <typename R, int V> struct ProjDirect {
         // values go unused), so that the loop body is one straight block and each
         // chunk's loads have D - 1 chunks of MFMAs to arrive.  The scheduling barrier
         // keeps the loads above those MFMAs: without it the compiler sinks them to
-        // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122).  Then the partial
+        // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122; in FP64 also a barrier
+        // after them: 80,852 x 864 x 512 3,790 -> 3,620 us).  Then the partial
         // chunk, if any.  Chunks are accumulated in K order for any D.
         const int nfull = max(0, ke - kb) / KC;
         if (nfull > 0) {
@@ -427,6 +428,7 @@ template <typename R, int V> struct ProjDirect {
                     load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
                     __builtin_amdgcn_sched_barrier(0);
                     compute(ra[j], rb[j]);
+                        if (sizeof(R) == 8) __builtin_amdgcn_sched_barrier(0);
                 }
             }
 #pragma unroll
