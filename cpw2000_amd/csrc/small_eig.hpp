@@ -10,7 +10,7 @@
 // (solves, no barrier), and for larger Jacobi matrices one launch per round with
 // the matrix spread over the compute units (one memory round trip a round).
 // us at n = 128, one workgroup in global memory before / now: Cholesky 382 / 184,
-// solves 2263 / 82, Jacobi 28,275 / 4,700 (1,016 rounds of 4.5), back-substitution
+// solves 2263 / 82, Jacobi 28,275 / 3,900 (1,016 rounds of 3.7), back-substitution
 // 871 / 300; n = 64, the whole step 4,492 / 1,709.
 //
 // Every value is computed by the same operations in the same order whatever the
@@ -255,23 +255,20 @@ struct Rotation {
     double2 u;
 };
 
-// rotation that annihilates apq of the pair with diagonal app, aqq; identity for |apq| <= thr
+// rotation that annihilates apq of the pair with diagonal app, aqq; identity for
+// |apq| <= thr.  No branch: a wavefront has lanes of both kinds, and the values of
+// an identity's chain (infinite or NaN for apq = 0) are not taken.
 __device__ __forceinline__ Rotation jacobi_rotation(double app, double aqq, double2 apq, double thr) {
-    Rotation r{1.0, 0.0, make_double2(1.0, 0.0)};
     // |apq| without squaring: once the element has decayed below ~1e-154,
     // apq.x^2 + apq.y^2 is denormal and keeps only a few digits, |u| drifts from
     // 1 and the phase factor would rescale row and column q
     const double g = hypot(apq.x, apq.y);
-    if (g > thr) {
-        const double zeta = (aqq - app) / (2.0 * g);
-        const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(fma(zeta, zeta, 1.0)));
-        if (t != 0.0) {  // a zero angle is the identity: no phase either
-            r.u = make_double2(apq.x / g, -apq.y / g);  // exp(-i phi)
-            r.c = 1.0 / sqrt(fma(t, t, 1.0));
-            r.s = t * r.c;
-        }
-    }
-    return r;
+    const double zeta = (aqq - app) / (2.0 * g);
+    const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(fma(zeta, zeta, 1.0)));
+    const bool on = g > thr && t != 0.0;  // a zero angle is the identity: no phase either
+    const double c = 1.0 / sqrt(fma(t, t, 1.0));
+    const double ux = apq.x / g, uy = -apq.y / g;  // exp(-i phi)
+    return Rotation{on ? c : 1.0, on ? t * c : 0.0, make_double2(on ? ux : 1.0, on ? uy : 0.0)};
 }
 
 // (p, q) -> (c p - s t, s p + c t)
@@ -618,29 +615,45 @@ __global__ __launch_bounds__(SE_THREADS) void k_jacobi_check(const double2 *__re
 // elements for their rotations), a wavefront per l and its lanes the k; the
 // others rotate the columns of v in place, a wavefront per pair and its lanes the
 // rows.  Rotations are recomputed where they are used: a round is one trip to
-// memory and one chain of square roots and divisions, with no barrier.
+// memory and one chain of square roots and divisions, with no barrier.  So all
+// loads go out together, and a wavefront that holds pair l among its own k takes
+// that rotation from its lane (n <= 128: always).  us per round at n = 128: 4.4 with
+// the threshold awaited first and both rotations computed, 3.7 so.
 __global__ __launch_bounds__(256) void k_jacobi_round(const double2 *__restrict__ a, double2 *__restrict__ b,
                                                       double2 *__restrict__ v, int n, int round,
                                                       const JacobiCtl *__restrict__ ctl) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int np = (n + 1) & ~1, half = np / 2, nl4 = (half + 3) / 4;
     const double thr = ctl->thr;
-    if (ctl->stop) return;
-    const auto pair_rotation = [&](int p, int q) {
-        if (q >= n) return Rotation{1.0, 0.0, make_double2(1.0, 0.0)};
-        return jacobi_rotation(a[p + (long)p * n].x, a[q + (long)q * n].x, a[p + (long)q * n], thr);
+    const int stop = ctl->stop;
+    // rotation of the pair (p, q); elements of a pair with the dummy index n are not used
+    const auto pair_rotation = [&](int p, int q, double app, double aqq, double2 apq) {
+        const Rotation r = jacobi_rotation(app, aqq, apq, thr);
+        return q < n ? r : Rotation{1.0, 0.0, make_double2(1.0, 0.0)};
     };
+    const auto at = [&](int i, int j) { return a[min(i, n - 1) + (long)min(j, n - 1) * n]; };
     if ((int)blockIdx.y < nl4) {
-        const int k = blockIdx.x * 64 + lane, l = blockIdx.y * 4 + wave;
-        if (l >= half || k >= half) return;
+        const int k0 = blockIdx.x * 64, k = min(k0 + lane, half - 1), l = blockIdx.y * 4 + wave;
+        if (l >= half) return;
         int pk, qk, pl, ql;
         rr_pair(k, round, np, pk, qk);
         rr_pair(l, round, np, pl, ql);
         const bool kq = qk < n, lq = ql < n;  // the dummy index has no row
         const double2 z = make_double2(0.0, 0.0);
-        const long cp = (long)pl * n, cq = (long)ql * n;
-        double2 a00 = a[pk + cp], a01 = lq ? a[pk + cq] : z, a10 = kq ? a[qk + cp] : z, a11 = kq && lq ? a[qk + cq] : z;
-        const Rotation rk = pair_rotation(pk, qk), rl = pair_rotation(pl, ql);
+        double2 a00 = at(pk, pl), a01 = at(pk, ql), a10 = at(qk, pl), a11 = at(qk, ql);
+        const double kpp = at(pk, pk).x, kqq = at(qk, qk).x;
+        const double2 kpq = at(pk, qk);
+        Rotation rl;
+        const bool held = l >= k0 && l < k0 + 64;  // the same for the wavefront
+        if (!held) rl = pair_rotation(pl, ql, at(pl, pl).x, at(ql, ql).x, at(pl, ql));
+        if (stop) return;
+        const Rotation rk = pair_rotation(pk, qk, kpp, kqq, kpq);
+        if (held)
+            rl = Rotation{lane_value(rk.c, l - k0), lane_value(rk.s, l - k0),
+                          make_double2(lane_value(rk.u.x, l - k0), lane_value(rk.u.y, l - k0))};
+        if (!lq) a01 = z;
+        if (!kq) a10 = z;
+        if (!(kq && lq)) a11 = z;
         if (rk.s != 0.0) {
             rotate_rows(rk, a00, a10);
             rotate_rows(rk, a01, a11);
@@ -649,6 +662,8 @@ __global__ __launch_bounds__(256) void k_jacobi_round(const double2 *__restrict_
             rotate_cols(rl, a00, a01);
             rotate_cols(rl, a10, a11);
         }
+        if (k0 + lane >= half) return;
+        const long cp = (long)pl * n, cq = (long)ql * n;
         b[pk + cp] = a00;
         if (lq) b[pk + cq] = a01;
         if (kq) b[qk + cp] = a10;
@@ -659,9 +674,17 @@ __global__ __launch_bounds__(256) void k_jacobi_round(const double2 *__restrict_
         int p, q;
         rr_pair(k, round, np, p, q);
         if (q >= n) return;
-        const Rotation r = pair_rotation(p, q);
-        if (r.s == 0.0) return;
-        for (int i = blockIdx.x * 64 + lane; i < n; i += gridDim.x * 64)
+        const int i0 = blockIdx.x * 64 + lane, ic = min(i0, n - 1);
+        double2 vp = v[ic + (long)p * n], vq = v[ic + (long)q * n];
+        const Rotation r = pair_rotation(p, q, at(p, p).x, at(q, q).x, at(p, q));
+        if (stop || r.s == 0.0) return;
+        // the first rows were loaded with the rotation's elements
+        rotate_cols(r, vp, vq);
+        if (i0 < n) {
+            v[i0 + (long)p * n] = vp;
+            v[i0 + (long)q * n] = vq;
+        }
+        for (int i = i0 + gridDim.x * 64; i < n; i += gridDim.x * 64)
             rotate_cols(r, v[i + (long)p * n], v[i + (long)q * n]);
     }
 }
