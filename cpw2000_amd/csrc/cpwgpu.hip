@@ -404,10 +404,11 @@ template <typename R> void proj_tile(int pv, int *BM, int *BN, int *BK) {
 // the projectors once per 16 bands).  us, 128 x 32 / 64 x 16: 23,928 plane waves x
 // 256 projectors x 16 bands 30 / 22, x 40 57 / 47, x 72 82 / 75, x 100 84 / 101;
 // 7,550 x 128 x 20 18 / 8, x 100 21 / 23; 80,852 x 864 x 72 656 / 861.
-// FP32: LDS-staged with half chunks, 16, 32 or 48 bands per block: what pads least,
-// 6% per flop against the narrow one where more than 3 tiles of bands are full.
-// us at 64 / 48 / 32 / 16 bands per block: 23,928 x 256 x 16 37 / 29 / 22 / 15, x 72
-// 60 / 43 / 48 / 42, x 128 61 / 68 / 58 / 61, x 144 91 / 67 / 72 / 70.
+// FP32: LDS-staged with half chunks, 16, 32, 48 or 64 bands per block: what pads
+// least, 6% per flop against the narrow one where more than 3 tiles of bands are
+// full, 5% for the wide one from 8 tiles on.
+// us at 64 / 48 / 32 / 16 bands per block: 23,928 x 256 x 16 34 / 28 / 21 / 15, x 72
+// 60 / 43 / 48 / 42, x 128 55 / 70 / 58 / 61, x 144 91 / 67 / 72 / 70.
 int back_shape64(int rows, int neig) {
     const long big = ((long)(rows + 127) / 128 * ((neig + 31) / 32) + 255) / 256;
     const long small = ((long)(rows + 63) / 64 * ((neig + 15) / 16) + 255) / 256;
@@ -419,8 +420,8 @@ template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int nei
     if (sizeof(R) == 4) {
         const int t = (neig + 15) / 16;
         if (t <= 3) return BACK_BANDS + 1;
-        const double c1 = 1.06 * t, c2 = 2.0 * ((t + 1) / 2), c3 = 3.0 * ((t + 2) / 3);
-        return BACK_BANDS + (c1 < c2 && c1 < c3 ? 1 : c3 < c2 ? 3 : 2);
+        const double c[4] = {1.06 * t, 2.0 * ((t + 1) / 2), 3.0 * ((t + 2) / 3), t < 8 ? HUGE_VAL : 3.8 * ((t + 3) / 4)};
+        return BACK_BANDS + 1 + (int)(std::min_element(c, c + 4) - c);
     }
     return back_shape64(rows, neig);
 }
@@ -614,7 +615,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         launch_batchable<BackLds<R, GemmCfg<R>::KC / 2, NT>>(CPWGPU_K_BACK, (k_back<R, GemmCfg<R>::KC / 2, NT>),                                      \
                      dim3((rows + BP_BI - 1) / BP_BI, (neig + 16 * NT - 1) / (16 * NT)), dim3(GEMM_THREADS), 0, \
                      s, anl, lda, dh, hp, ldh, rows, nanl, neig, beta, kp, ldp, ek);
-        if constexpr (sizeof(R) == 4) { CPW_BL(1) CPW_BL(2) CPW_BL(3) }
+        if constexpr (sizeof(R) == 4) { CPW_BL(1) CPW_BL(2) CPW_BL(3) CPW_BL(4) }
 #undef CPW_BL
         if (bv == 0)
             launch_timed(CPWGPU_K_BACK, k_back<R>, dim3((rows + BP_BI - 1) / BP_BI, (neig + BP_BN - 1) / BP_BN),
@@ -1072,13 +1073,19 @@ int apply_spin(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, double2
     hipLaunchKernelGGL(k_spin_split, eg, dim3(SP_THREADS), 0, s, psi, ldp, mtxd, neig, sp);
     HIPCHK(hipGetLastError());
     const bool nl = p->snanl > 0;
-    if (nl) {
+    // FP64 on one stream, as apply_t; FP32 with the non-local term on the second one
+    // (us, two streams / one: FP64 64 bands 860 / 828, 20 bands 392 / 399, 6 bands
+    // 259 / 243; FP32 484 / 492, 205 / 227, 112 / 129)
+    const bool beside = nl && sizeof(R) == 4;
+    const double *dpsi = (const double *)psi;
+    double *dhpsi = (double *)hpsi;
+    if (nl && !beside) {
+        if ((st = nonlocal<R>(p, spin_proj(p), neig, dpsi, ldp, dhpsi, ldh, 1, false, s, nullptr, NL_PROJ))) return st;
+    } else if (nl) {
         if ((st = ensure_aux())) return st;
         HIPCHK(hipEventRecord(g_fork, s));
         HIPCHK(hipStreamWaitEvent(g_aux, g_fork, 0));
-        if ((st = nonlocal<R>(p, spin_proj(p), neig, (const double *)psi, ldp, (double *)hpsi, ldh, 0, false,
-                              g_aux)))
-            return st;
+        if ((st = nonlocal<R>(p, spin_proj(p), neig, dpsi, ldp, dhpsi, ldh, 0, false, g_aux))) return st;
         HIPCHK(hipEventRecord(g_join, g_aux));
     }
     const R *vr = sizeof(R) == 8 ? (const R *)p->vsp64.p : (const R *)p->vsp32.p;
@@ -1128,10 +1135,11 @@ int apply_spin(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, double2
     } else {
         // no z column (mtxd = 0 handled above): nothing local
     }
-    if (nl) HIPCHK(hipStreamWaitEvent(s, g_join, 0));
+    if (beside) HIPCHK(hipStreamWaitEvent(s, g_join, 0));
     hipLaunchKernelGGL(k_spin_merge, eg, dim3(SP_THREADS), 0, s, (const double2 *)sh, mtxd, neig, hpsi, ldh,
-                       nl ? 1 : 0);
+                       beside ? 1 : 0);
     HIPCHK(hipGetLastError());
+    if (nl && !beside) return nonlocal<R>(p, spin_proj(p), neig, dpsi, ldp, dhpsi, ldh, 1, false, s, nullptr, NL_BACK);
     return CPWGPU_OK;
 }
 

@@ -159,13 +159,15 @@ template <typename R, int N> constexpr int plane_var_default() {
 
 // register shape of the coupled two-component plane kernel: (x lanes, y
 // lanes, threads, waves per SIMD); both components' rows live in registers.
-// FP64: the two sub-planes (about 86 KB at 72) allow one block per CU, so the
-// block has 512 threads for 2 waves per SIMD (184 VGPRs fit that budget).
-template <typename R> struct SpinShape;
-template <> struct SpinShape<float> { static constexpr int GX = 8, GY = 8, T = 256, W = 3; };
-template <> struct SpinShape<double> { static constexpr int GX = 8, GY = 8, T = 512, W = 2; };
+// FP64: the two sub-planes (about 90 KB at 72) allow one block per CU, whose rows
+// are one round of tasks (8 N threads; with 512, 72 rows left 8 of them to a second
+// round); a box beyond N/4 needs the registers of 2 waves per SIMD.
+template <typename R, int N, bool CS> struct SpinShape {
+    static constexpr int GX = 8, GY = 8;
+    static constexpr int T = sizeof(R) == 4 ? 256 : CS ? 8 * N : 512, W = sizeof(R) == 4 || CS ? 3 : 2;
+};
 template <typename R, int N> constexpr bool spin_reg_ok() {
-    return reg_ok<R, N, SpinShape<R>::GX, SpinShape<R>::GY>();
+    return reg_ok<R, N, 8, 8>();
 }
 
 // Register shapes of the density pass: 8 lanes per line, den_threads() threads,

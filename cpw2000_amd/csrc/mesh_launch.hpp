@@ -174,33 +174,29 @@ int launch_plane(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, const R 
 template <typename R, int N>
 int launch_plane_spin_reg(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long vstride, int npair,
                           hipStream_t s) {
-    constexpr int GX = SpinShape<R>::GX, GY = SpinShape<R>::GY, T = SpinShape<R>::T, W = SpinShape<R>::W;
     if constexpr (!spin_reg_ok<R, N>()) {
         return fail(CPWGPU_ERR_MODE, "register two-component plane kernel is not built for N = %d", N);
     } else {
         const FftGeom &g = p->g;
-        // a box inside N/4: the compile-time row stride
-        const bool cs = prune_fits(g);
-        const int S = cs ? pr_sub_stride<N>() : reg_stride(g.nx);
-        const size_t dyn = sizeof(cplx<R>) * ((size_t)N + 2 * (size_t)N * S);
-        if (dyn > 160 * 1024)
-            return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
-        static bool attr = false;
-        if (!attr) {
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, false>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            HIPCHK(hipFuncSetAttribute((const void *)k_plane_spin_reg<R, N, GX, GY, T, W, true>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            attr = true;
-        }
-        if (cs)
-            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, true>), dim3(g.n[2] * npair), dim3(T), dyn, s,
-                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
-        else
-            launch_timed(CPWGPU_K_PLANE, (k_plane_spin_reg<R, N, GX, GY, T, W, false>), dim3(g.n[2] * npair), dim3(T), dyn, s,
-                               colbuf, (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
-        HIPCHK(hipGetLastError());
-        return CPWGPU_OK;
+        const auto go = [&](auto kernel, int S, int T, bool &attr) -> int {
+            const size_t dyn = sizeof(cplx<R>) * ((size_t)N + 2 * (size_t)N * S);
+            if (dyn > 160 * 1024)
+                return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
+            if (!attr) {
+                HIPCHK(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                attr = true;
+            }
+            launch_timed(CPWGPU_K_PLANE, kernel, dim3(g.n[2] * npair), dim3(T), dyn, s, colbuf,
+                         (const int *)p->col_uy.p, vr, vstride, (const double2 *)p->tw[0].p, g, npair, S);
+            HIPCHK(hipGetLastError());
+            return CPWGPU_OK;
+        };
+        static bool attr_p = false, attr_u = false;
+        using P = SpinShape<R, N, true>;
+        using U = SpinShape<R, N, false>;
+        // a box inside N/4: the pruned shape
+        if (prune_fits(g)) return go(k_plane_spin_reg<R, N, P::GX, P::GY, P::T, P::W, true>, pr_sub_stride<N>(), P::T, attr_p);
+        return go(k_plane_spin_reg<R, N, U::GX, U::GY, U::T, U::W, false>, reg_stride(g.nx), U::T, attr_u);
     }
 }
 

@@ -412,11 +412,14 @@ template <typename R, int V> struct ProjDirect {
         // c + D - 1 is loaded while chunk c is multiplied, unconditionally (at
         // the last full chunk again when there is none: a valid address whose
         // values go unused), so that the loop body is one straight block and each
-        // chunk's loads have D - 1 chunks of MFMAs to arrive.  The scheduling barrier
-        // keeps the loads above those MFMAs: without it the compiler sinks them to
-        // save registers (FP64 23,847 x 256 x 128: 90 us, sunk 122; in FP64 also a barrier
-        // after them: 80,852 x 864 x 512 3,790 -> 3,620 us).  Then the partial
-        // chunk, if any.  Chunks are accumulated in K order for any D.
+        // chunk's loads have D - 1 chunks of MFMAs to arrive.  The compiler
+        // would sink the loads below those MFMAs to save registers (FP64 23,847 x 256 x
+        // 128: 90 us, sunk 122), so they are kept apart: in FP64 by scheduling barriers on
+        // both sides of the MFMAs (80,852 x 864 x 512 3,620 us; 3,790 without the second),
+        // in FP32 by a branch it cannot see through (shape 2, 23,928 x 256 x 128: 54 us,
+        // with barriers 57).  Then the partial chunk, if any.  Chunks are accumulated in K order for any D.
+        int always = 1;
+        asm volatile("" : "+s"(always));
         const int nfull = max(0, ke - kb) / KC;
         if (nfull > 0) {
 #pragma unroll
@@ -426,9 +429,13 @@ template <typename R, int V> struct ProjDirect {
 #pragma unroll
                 for (int j = 0; j < D; j++) {
                     load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
-                    __builtin_amdgcn_sched_barrier(0);
-                    compute(ra[j], rb[j]);
-                        if (sizeof(R) == 8) __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (sizeof(R) == 8) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        compute(ra[j], rb[j]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    } else if (always) {
+                        compute(ra[j], rb[j]);
+                    }
                 }
             }
 #pragma unroll
@@ -563,26 +570,30 @@ template <typename R, int KCX, int NT> struct BackLds {
             P2[t] = v4{0, 0, 0, 0};
             P3[t] = v4{0, 0, 0, 0};
         }
-        // staging of dhd: value q of a thread is projector tid % KC of band row
-        // tid / KC + q * (256 / KC)
-        constexpr int RPQ = GEMM_THREADS / KC;
-        static_assert(GEMM_THREADS % KC == 0 && BN % RPQ == 0, "bad k_back staging");
-        const int srow = threadIdx.x / KC, soff = threadIdx.x % KC;
+        // staging of dhd: TPR threads per band row, each with VPT consecutive
+        // projectors; all rows in one pass (three of them for 48 rows), so that a
+        // thread's values follow from one address.  Chunks of 64: a whole row per
+        // wavefront (23,928 x 256 x 128 77 -> 61 us; with chunks of 32 that loses 12%)
+        constexpr int TPR = KC >= 64 ? KC : NT == 3 ? 16 : 16 / NT, RPP = GEMM_THREADS / TPR, VPT = KC / TPR;
+        static_assert(BN % RPP == 0 && KC % TPR == 0 && DPT == BN / RPP * VPT, "bad k_back staging");
+        const int srow = threadIdx.x / TPR, soff = threadIdx.x % TPR * VPT;
         cplx<R> rd[DPT];
         // rows beyond the matrix (bands n >= neig, plane waves i >= mtxd) are
         // read at clamped addresses and only reach outputs that are not stored;
         // full chunks issue plain loads (first used after the current chunk's
         // MFMAs), the projector tail is clamped with dhd zero-masked
-        const auto dat = [&](int q, int a) { return (long)min(n0 + srow + q * RPQ, neig - 1) * nanl + a; };
+        long dbase[BN / RPP];
+#pragma unroll
+        for (int w = 0; w < BN / RPP; w++) dbase[w] = (long)min(n0 + srow + w * RPP, neig - 1) * nanl;
         auto dload = [&](int ka) {
             if (ka + KC <= nanl) {  // the same for the whole block
 #pragma unroll
-                for (int q = 0; q < DPT; q++) rd[q] = dhd[dat(q, ka + soff)];
+                for (int q = 0; q < DPT; q++) rd[q] = dhd[dbase[q / VPT] + ka + soff + q % VPT];
             } else {
 #pragma unroll
                 for (int q = 0; q < DPT; q++) {
-                    const int a = ka + soff;
-                    const cplx<R> v = dhd[dat(q, min(a, nanl - 1))];
+                    const int a = ka + soff + q % VPT;
+                    const cplx<R> v = dhd[dbase[q / VPT] + min(a, nanl - 1)];
                     rd[q] = mk<R>(a < nanl ? v.x : (R)0, a < nanl ? v.y : (R)0);
                 }
             }
@@ -603,9 +614,9 @@ template <typename R, int KCX, int NT> struct BackLds {
         for (int ka = 0; ka < nanl; ka += KC) {
 #pragma unroll
             for (int q = 0; q < DPT; q++) {
-                sD[0][srow + q * RPQ][soff] = rd[q].x;
-                sD[1][srow + q * RPQ][soff] = rd[q].y;
-                sD[2][srow + q * RPQ][soff] = rd[q].x + rd[q].y;
+                sD[0][srow + q / VPT * RPP][soff + q % VPT] = rd[q].x;
+                sD[1][srow + q / VPT * RPP][soff + q % VPT] = rd[q].y;
+                sD[2][srow + q / VPT * RPP][soff + q % VPT] = rd[q].x + rd[q].y;
             }
             __syncthreads();
             R cr[KPL], ci[KPL], cs[KPL];

@@ -151,8 +151,13 @@ __global__ __launch_bounds__(FT) void k_plane_spin(cplx<R> *__restrict__ colbuf,
 // M consecutive x points of the two components and applies the 2x2 potential
 // there (vsp = [V1 + V2, V1 - V2, V3, V4], stride vstride), then both forward
 // transforms.  Grid: n3 * npair blocks of T threads, one (z, band pair) each.
-// CS: the sphere box lies inside N/4 (checked by the caller) and the row
-// stride is the compile-time pr_sub_stride<N>() instead of the argument.
+// CS: the sphere box lies inside N/4 (checked by the caller): the row stride is
+// the compile-time pr_sub_stride<N>(), the register slots that hold only x outside
+// the box are known zeros (as in k_plane_reg) and the y lines go through the
+// wave-exchanged LDS transform.  In FP64 the lane twiddles of the rows are held in
+// registers where there are few threads.  FP64 has one block per CU (90 KB at 72),
+// so its phases wait for each other: at 72, 64 band pairs, 352 us (368 unpruned with
+// 512 threads) of which the FP64 issue is about half.
 template <typename R, int N, int GX, int GY, int T, int W, bool CS = false>
 __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ colbuf,
                                                       const int *__restrict__ col_uy,
@@ -161,6 +166,7 @@ __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ c
                                                       int npair, int S_arg) {
     static_assert(N % GX == 0 && N % GY == 0 && T % 64 == 0, "bad plane shape");
     constexpr int MX = N / GX, MY = N / GY;
+    constexpr u64mask XB = CS ? box_slots(N, GX, MX, N / 4) : full_mask(MX);
     const int S = CS ? pr_sub_stride<N>() : S_arg;
     extern __shared__ __align__(16) unsigned char smem_raw[];
     cplx<R> *twN = reinterpret_cast<cplx<R> *>(smem_raw);  // [N]
@@ -170,17 +176,37 @@ __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ c
     const int nx = g.nx, kd1 = g.kd[0], ushift = N - nx, xhi = N - kd1;
     const int tid = threadIdx.x;
 
-    load_twiddles(twN, twg, N);
-    for (int q = tid; q < 2 * N * S; q += T) sub[q] = mk<R>(0, 0);
-    __syncthreads();
     cplx<R> *cb[2];
     cb[0] = colbuf + ((long)pair * n3 + z) * g.ncolp;
     cb[1] = colbuf + ((long)(pair + npair) * n3 + z) * g.ncolp;
-    gather_plane<R, T>(sub, cb[0], col_uy, g.ncol, S, 0);
-    gather_plane<R, T>(sub + N * S, cb[1], col_uy, g.ncol, S, 0);
+    // the first two z-column values of each thread and component, loaded before the
+    // sub-planes are cleared (clamped: ncol >= 1)
+    constexpr int NPRE = 2;
+    const int c0 = min(tid, g.ncol - 1), c1 = min(tid + T, g.ncol - 1);
+    const auto place = [&](int c) {
+        const int uy = col_uy[c];
+        return (uy >> 16) * S + (uy & 0xffff);
+    };
+    const int p0 = place(c0), p1 = place(c1);
+    typedef R V2 __attribute__((ext_vector_type(2)));  // structures go to scratch memory
+    const auto col = [](const cplx<R> *p) { return *reinterpret_cast<const V2 *>(p); };
+    const V2 u0 = col(cb[0] + c0), u1 = col(cb[0] + c1), d0 = col(cb[1] + c0), d1 = col(cb[1] + c1);
+    load_twiddles(twN, twg, N);
+    for (int q = tid; q < 2 * N * S; q += T) sub[q] = mk<R>(0, 0);
+    __syncthreads();
+    // (a clamped column is stored again with the same value)
+    sub[p0] = mk<R>(u0.x, u0.y);
+    sub[p1] = mk<R>(u1.x, u1.y);
+    sub[N * S + p0] = mk<R>(d0.x, d0.y);
+    sub[N * S + p1] = mk<R>(d1.x, d1.y);
+    gather_plane<R, T>(sub, cb[0], col_uy, g.ncol, S, NPRE * T);
+    gather_plane<R, T>(sub + N * S, cb[1], col_uy, g.ncol, S, NPRE * T);
     __syncthreads();
 
-    {  // inverse y on the 2 * nx box lines
+    if constexpr (CS) {
+        line_fft_wave<R, N, +1, T>(sub, nx, 1, S, twN);
+        line_fft_wave<R, N, +1, T>(sub + N * S, nx, 1, S, twN);
+    } else {  // inverse y on the 2 * nx box lines
         const Lanes<R, GY> L;
         for (int task = tid / GY; task < 2 * nx; task += T / GY) {
             const int p = task >= nx ? 1 : 0, u = task - p * nx;
@@ -197,6 +223,16 @@ __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ c
 
     {  // rows: inverse x of both components, the 2x2 potential, forward x
         const Lanes<R, GX> L;
+        constexpr bool HOIST = CS && sizeof(R) == 8 && MX <= 9 && T <= 512;
+        cplx<R> twx[MX];
+        if constexpr (HOIST) {
+#pragma unroll
+            for (int k = 1; k < MX; k++) twx[k] = twN[L.g * k];
+        }
+        const auto tw = [&]() {
+            if constexpr (HOIST) return TwRegs<R, MX>{twx};
+            else return TwLds<R>{twN, L.g};
+        }();
         for (int y = tid / GX; y < N; y += T / GX) {
             cplx<R> *ru = sub + y * S, *rd = sub + (N + y) * S;
             cplx<R> u[MX], d[MX];
@@ -204,14 +240,16 @@ __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ c
             for (int j = 0; j < MX; j++) {
                 const int x = L.g + GX * j;
                 const int o = x <= kd1 ? x : x >= xhi ? x - ushift : nx;
-                u[j] = ru[o];
-                d[j] = rd[o];
+                if (has_bit(XB, j)) {
+                    u[j] = ru[o];
+                    d[j] = rd[o];
+                }
             }
             // (with the one-instruction FP32 butterflies the odd positions of
             // both components carry negated values until the forward x: the
             // potential below is linear)
-            line_dif<+1, GX, MX, R, full_mask(MX), true>(u, L, twN);
-            line_dif<+1, GX, MX, R, full_mask(MX), true>(d, L, twN);
+            line_dif_tw<+1, GX, MX, R, XB, true>(u, L, tw);
+            line_dif_tw<+1, GX, MX, R, XB, true>(d, L, tw);
             const R *v0 = vsp + ((long)z * g.n[1] + y) * g.id + MX * L.k2;
 #pragma unroll
             for (int k = 0; k < MX; k++) {
@@ -220,20 +258,25 @@ __global__ __launch_bounds__(T, W) void k_plane_spin_reg(cplx<R> *__restrict__ c
                 u[k] = mk<R>(vu * a.x + vx * b.x + vy * b.y, vu * a.y + vx * b.y - vy * b.x);
                 d[k] = mk<R>(vd * b.x + vx * a.x - vy * a.y, vd * b.y + vx * a.y + vy * a.x);
             }
-            line_dit<-1, GX, MX, R, full_mask(MX), true>(u, L, twN);
-            line_dit<-1, GX, MX, R, full_mask(MX), true>(d, L, twN);
+            line_dit_tw<-1, GX, MX, R, XB, true>(u, L, tw);
+            line_dit_tw<-1, GX, MX, R, XB, true>(d, L, tw);
 #pragma unroll
             for (int m = 0; m < MX; m++) {
                 const int x = L.g + GX * m;
                 const int o = x <= kd1 ? x : x >= xhi ? x - ushift : nx + 1;
-                ru[o] = u[m];
-                rd[o] = d[m];
+                if (has_bit(XB, m)) {
+                    ru[o] = u[m];
+                    rd[o] = d[m];
+                }
             }
         }
     }
     __syncthreads();
 
-    {  // forward y
+    if constexpr (CS) {
+        line_fft_wave<R, N, -1, T>(sub, nx, 1, S, twN);
+        line_fft_wave<R, N, -1, T>(sub + N * S, nx, 1, S, twN);
+    } else {  // forward y
         const Lanes<R, GY> L;
         for (int task = tid / GY; task < 2 * nx; task += T / GY) {
             const int p = task >= nx ? 1 : 0, u = task - p * nx;
