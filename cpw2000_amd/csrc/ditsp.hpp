@@ -77,7 +77,15 @@ __global__ __launch_bounds__(DT_THREADS) void k_normalize_cols(double2 *__restri
     __shared__ double red[DT_THREADS];
     double2 *c = t + (long)blockIdx.x * ldt;
     double s = 0.0;
-    for (int i = threadIdx.x; i < mtxd; i += DT_THREADS) s += c[i].x * c[i].x + c[i].y * c[i].y;
+    constexpr int U = 8;  // rows in flight per thread, as in k_residual
+    for (int i0 = threadIdx.x; i0 < mtxd; i0 += U * DT_THREADS) {
+        double2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = c[min(i0 + u * DT_THREADS, mtxd - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * DT_THREADS < mtxd) s += v[u].x * v[u].x + v[u].y * v[u].y;
+    }
     red[threadIdx.x] = s;
     __syncthreads();
     for (int h = DT_THREADS / 2; h > 0; h >>= 1) {
@@ -86,7 +94,14 @@ __global__ __launch_bounds__(DT_THREADS) void k_normalize_cols(double2 *__restri
     }
     const double nrm = red[0];
     const double f = nrm > 0.0 ? 1.0 / sqrt(nrm) : 0.0;
-    for (int i = threadIdx.x; i < mtxd; i += DT_THREADS) c[i] = make_double2(f * c[i].x, f * c[i].y);
+    for (int i0 = threadIdx.x; i0 < mtxd; i0 += U * DT_THREADS) {
+        double2 v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = c[min(i0 + u * DT_THREADS, mtxd - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (i0 + u * DT_THREADS < mtxd) c[i0 + u * DT_THREADS] = make_double2(f * v[u].x, f * v[u].y);
+    }
 }
 
 // Deterministic random start vectors for columns [c0, c0 + ncols): uniform

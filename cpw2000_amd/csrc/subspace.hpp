@@ -149,10 +149,22 @@ __global__ __launch_bounds__(256) void k_residual(const double2 *__restrict__ ps
     const int n = blockIdx.x;
     const double e = eig[n];
     double s = 0.0;
-    for (int i = threadIdx.x; i < mtxd; i += blockDim.x) {
-        const double2 p = psi[(long)n * ldp + i], h = hpsi[(long)n * ldh + i];
-        const double rx = h.x - e * p.x, ry = h.y - e * p.y;
-        s += rx * rx + ry * ry;
+    // eight rows in flight per thread (clamped), added in order: a column is one
+    // block's, and a memory round trip per row took twice the time
+    constexpr int U = 8;
+    for (int i0 = threadIdx.x; i0 < mtxd; i0 += U * 256) {
+        double2 p[U], h[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = min(i0 + u * 256, mtxd - 1);
+            p[u] = psi[(long)n * ldp + i];
+            h[u] = hpsi[(long)n * ldh + i];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const double rx = h[u].x - e * p[u].x, ry = h[u].y - e * p[u].y;
+            if (i0 + u * 256 < mtxd) s += rx * rx + ry * ry;
+        }
     }
     red[threadIdx.x] = s;
     __syncthreads();
