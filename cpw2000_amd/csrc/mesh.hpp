@@ -55,6 +55,11 @@ template <typename R, int N> constexpr RegShapeT reg_shape(int v) {
         // one pruned shape: 9 in FP64, 10 in FP32
         if (v != (sizeof(R) == 8 ? 9 : 10)) return NO_SHAPE;
         const int w = sizeof(R) == 8 ? 3 : N % 8 == 0 ? 5 : 4;
+        // FP64: as many threads as one round of rows takes, by 4 lanes (us per H|psi>
+        // call against 256 threads by 8 (36: by 4) lanes: 32, 72 bands on 32 x 32 x 128
+        // 106 / 102; 36, 60 bands on 36 x 36 x 72 71 / 70; 40, 60 bands on 40^3 56 / 53)
+        if (sizeof(R) == 8 && N == 32) return RegShapeT{4, 4, 1, 128, 4, false, true};
+        if (sizeof(R) == 8 && (N == 36 || N == 40)) return RegShapeT{4, 4, 1, 192, w, true, true};
         return N == 18 ? RegShapeT{2, 2, 1, 64, 2, false, true}
              : N == 20 ? RegShapeT{4, 4, 1, 128, w, false, true}
              : N == 36 ? RegShapeT{4, 4, 1, 256, w, true, true}
