@@ -2490,9 +2490,23 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         if (t < best) { best = t; best_pv = v; }
     }
     p->plane_var[ix] = best_pv;
+    // Against the defaults by size as a whole: each choice above was made with the
+    // others as they stood, some of them from a single apply (216 atoms, 512 bands,
+    // FP64: chosen 15.7 ms, defaults 13.2).
+    if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 8, &best))) return st;
+    int *const choice[7] = {&p->plane_var[ix], &p->proj_var[ix], &p->back_var[ix], &p->splitk[ix],
+                            &p->kin_var[ix], &p->col_var[ix], &p->sched_var[ix]};
+    int tuned[7];
+    for (int i = 0; i < 7; i++) {
+        tuned[i] = *choice[i];
+        *choice[i] = -1;
+    }
+    if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 8, &t))) return st;
+    if (best < t)
+        for (int i = 0; i < 7; i++) *choice[i] = tuned[i];
     // leave hpsi holding H psi of the chosen configuration
     if ((st = cpwgpu_plan_apply(p, neig, psi, ldp, hpsi, ldh, prec, s))) return st;
-    tune_cache_store(key, best_pv, best_jv, best_bv, best_sk, best_kv, best_cv, best_sv);
+    tune_cache_store(key, *choice[0], *choice[1], *choice[2], *choice[3], *choice[4], *choice[5], *choice[6]);
     return CPWGPU_OK;
 }
 
