@@ -306,10 +306,11 @@ int cpwgpu_hk_psi_allk_c16(const int *nrk, const int *mtxd_allk, const int *nban
 typedef struct cpwgpu_graph_s *cpwgpu_graph_t;
 /* Records H|psi> for nk k-points (plans[k], neig[k] bands psi[k](ldp[k]) ->
  * hpsi[k](ldh[k]) on device, each k with its own plane-wave count) into one
- * HIP graph (each k-point's non-local GEMMs overlap its FFT chain, as in
- * cpwgpu_plan_apply).  The batch is applied once eagerly first (buffers,
- * kernel attributes), then captured; the device arrays must stay valid while
- * the graph exists, and the graph must be destroyed before its plans.
+ * HIP graph (small k-points that share nothing are launched together, step by
+ * step; the others one after the other, as cpwgpu_plan_apply).  The batch is
+ * applied once eagerly first (buffers, kernel attributes), then captured; the
+ * device arrays must stay valid while the graph exists, and the graph must be
+ * destroyed before its plans.
  * Replaces the k-loop of Src/cpw/cpw_scf.f90:488-544 around hk_psi_c16 for a
  * batch of k-points.
  * The graph reads the plans' potential and projectors where they live, so a
@@ -372,8 +373,9 @@ int cpwgpu_rayleigh_ritz(int mtxd, int nb, double *psi_dev, long ldp, double *hp
  *               vectors iterated (neig + buffer), mtxds used, iteration at
  *               which FP64 H took over (-1: FP64 throughout)
  * Up to max(8, neig/8) buffer vectors beyond neig are iterated and not
- * required to converge.  The small eigenproblems use rocSOLVER (zheevd,
- * zpotrf) and rocBLAS (ztrsm) on the calling stream.  Returns when done;
+ * required to converge.  The small matrix of the start, subspaces beyond 128
+ * vectors and blocks beyond 140 use rocSOLVER (zheevd, zpotrf) and rocBLAS
+ * (ztrsm) on the calling stream.  Returns when done;
  * not converging within icmax is reported in ifail, not as an error. */
 int cpwgpu_plan_ditsp(cpwgpu_plan_t plan, int prec, int icmax, int iguess, double epspsi, int neig,
                       int mtxds, const double *hamsm_dev, long ldhs, const double *hdiag_dev,
