@@ -1526,12 +1526,16 @@ inline dim3 dt_grid(int rows, int cols) {
 
 // Eigenpairs of the Hermitian n x n matrix m (lower triangle, n <= SE_DIAG_MAX):
 // eigenvalues ascending in w, eigenvectors in v, g_dt.info[1] nonzero if it failed.
+// The sweeps stop at 1e-14 |m|, which the two refinement steps take to rounding.
 int subspace_eig(const double2 *m, double2 *v, double *w, int n, hipStream_t st) {
     int rc;
     constexpr int MAX_SWEEPS = 40;  // a matrix of random elements takes 8 to 10
     const int np = (n + 1) & ~1, half = np / 2;
+    const size_t mat = 16 * (size_t)n * n;
     if ((rc = g_ss.rec.reserve(sizeof(double4) * (size_t)MAX_SWEEPS * (np - 1) * half)) ||
-        (rc = g_ss.pos.reserve(4 * (size_t)np + 64)) || (rc = g_ss.info.reserve(64)))
+        (rc = g_ss.pos.reserve(4 * (size_t)np + 64)) || (rc = g_ss.info.reserve(64)) ||
+        (rc = g_ss.eig.reserve(8 * (size_t)n)) || (rc = g_ss.s.reserve(mat)) || (rc = g_ss.m.reserve(mat)) ||
+        (rc = g_ss.w.reserve(mat)))
         return rc;
     static bool attr = false;
     if (!attr) {
@@ -1541,10 +1545,19 @@ int subspace_eig(const double2 *m, double2 *v, double *w, int n, hipStream_t st)
     }
     double4 *rec = (double4 *)g_ss.rec.p;
     int *pos = (int *)g_ss.pos.p, *sweeps = (int *)g_ss.info.p + 1;
-    hipLaunchKernelGGL(k_jacobi_tri, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, m, rec, w, n, MAX_SWEEPS, 1e-13,
+    hipLaunchKernelGGL(k_jacobi_tri, dim3(1), dim3(SE_THREADS), se_lds_bytes(n), st, m, rec, w, n, MAX_SWEEPS, 1e-14,
                        pos, sweeps, (int *)g_dt.info.p + 1);
     hipLaunchKernelGGL(k_jacobi_vectors, dim3((n + SE_VROWS - 1) / SE_VROWS), dim3(64), 0, st, (const double4 *)rec,
                        (const int *)sweeps, (const int *)pos, v, n);
+    const dim3 tiles((n + SE_RT - 1) / SE_RT, (n + SE_RT - 1) / SE_RT), block(SE_RT * SE_RT);
+    double2 *t = (double2 *)g_ss.m.p, *e = (double2 *)g_ss.w.p;
+    const auto refine = [&](const double2 *x, const double *wx, double2 *y, double *wy) {
+        hipLaunchKernelGGL(k_refine_product<true>, tiles, block, 0, st, m, x, t, n);
+        hipLaunchKernelGGL(k_refine_step, tiles, block, 0, st, x, (const double2 *)t, wx, e, wy, n);
+        hipLaunchKernelGGL(k_refine_product<false>, tiles, block, 0, st, x, (const double2 *)e, y, n);
+    };
+    refine(v, w, (double2 *)g_ss.s.p, (double *)g_ss.eig.p);
+    refine((const double2 *)g_ss.s.p, (const double *)g_ss.eig.p, v, w);
     HIPCHK(hipGetLastError());
     return CPWGPU_OK;
 }
