@@ -381,19 +381,19 @@ struct Work {
     bool lean = false;  // split-K partials of one round of blocks only (proj_shape)
 };
 
-// Block tile (BM x BN) and K granule of the projection kernel variant pv.
-template <typename R> void proj_tile(int pv, int *BM, int *BN, int *BK) {
-    *BM = proj_bm<R>();
-    *BN = proj_bn<R>();
-    *BK = GemmCfg<R>::BK;
-    if (pv == NPROJ_DIRECT + 1) {
-        *BM = 2 * proj_half_wm<R>() * 16;
-        *BN = 2 * proj_half_wn<R>() * 16;
-    }
-#define CPW_PD(V) if (pv == V) { *BM = direct_bm<R, V>(); *BN = direct_bn<R, V>(); *BK = direct_bk<R, V>(); }
+// Block tile (BM x BN), K granule and chains of accumulators (C, E: DirectCfg) of the
+// projection kernel variant pv.
+struct ProjTile {
+    int BM, BN, BK, C;
+    bool E;
+};
+template <typename R> ProjTile proj_tile(int pv) {
+#define CPW_PD(V) if (pv == V) return {direct_bm<R, V>(), direct_bn<R, V>(), direct_bk<R, V>(), DirectCfg<R, V>::C, DirectCfg<R, V>::E};
     CPW_PD(1) CPW_PD(2) CPW_PD(3) CPW_PD(4)
     CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
 #undef CPW_PD
+    if (pv == NPROJ_DIRECT + 1) return {2 * proj_half_wm<R>() * 16, 2 * proj_half_wn<R>() * 16, GemmCfg<R>::BK, 1, false};
+    return {proj_bm<R>(), proj_bn<R>(), GemmCfg<R>::BK, 1, false};
 }
 
 // Back-projection kernel for rows plane waves and neig bands.  FP64: direct with
@@ -439,12 +439,15 @@ template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int nei
 // Without a kernel set by the caller the same cost chooses it, among the direct
 // kernel with 64 (FP32 128) projectors x 64 bands per block and those 16, 32, 48
 // and 80 bands wide; slow is the time per flop of each relative to the first.  It
-// took the fastest at every size measured but three (within 7%): us, 64 wide /
-// chosen: FP64 23,928 x 256 x 16 41 / 26 (16 wide), x 72 90 / 68 (80), x 128 92 / 92;
-// 7,550 x 128 x 40 18 / 15 (16); 80,852 x 864 x 72 815 / 581 (80), x 144 1213 / 1062
-// (80); FP32 23,928 x 256 x 20 30 / 20 (32), x 72 49 / 43 (80); 7,550 x 128 x 128
-// 22 / 16 (16).
-// lean: as a target of 256 blocks, the smallest workspace.
+// took the fastest at every size measured but four (within 7%): us, 64 wide /
+// chosen: FP64 23,928 x 256 x 16 43 / 26 (16 wide), x 72 88 / 65 (80), x 128 91 / 91;
+// 7,550 x 128 x 40 11.2 / 12.0; 80,852 x 864 x 72 815 / 581 (80), x 144 1213 / 1062
+// (80); FP32 23,928 x 256 x 20 25 / 16 (32), x 72 47 / 38 (80); 7,550 x 128 x 128
+// 16 / 15 (16).
+// No choice makes the product less accurate than the LDS-staged kernel in 256 blocks
+// (chain_rows): the 64 (128) wide kernel empties its accumulators that often, the
+// narrow ones have several, and the others take more slices.
+// lean: the fewest slices, for the smallest workspace.
 template <typename R> struct ProjShapes;
 template <> struct ProjShapes<double> {
     static constexpr double slow[5] = {1.0, 1.65, 1.22, 1.39, 1.18};
@@ -454,19 +457,46 @@ template <> struct ProjShapes<float> {
 };
 constexpr int PROJ_AUTO[5] = {1, PROJ_BANDS + 1, PROJ_BANDS + 2, PROJ_BANDS + 3, PROJ_BANDS + 5};
 
-// estimated us of the projection with block tile BM x BN and K granule BK, and
-// its number of slices
-template <typename R> double proj_cost(int BM, int BN, int BK, double slow, int rows, int nanl, int neig, int *nsl) {
+// Rows of a slice when the product is cut into 256 blocks of bm x bn tiles, whole
+// chunks of bk: the longest sum that one accumulator is to hold.  <beta|psi> is off
+// by sqrt(1.6 + 0.185 L + 0.009 n) roundings (rms, in units of |beta||psi|/sqrt(rows),
+// FP32 and FP64, 729 to 23,928 rows) for n slices whose chains are L rows long, so
+// that fewer slices mean a less accurate product: 7,550 x 128 x 128 with 32 slices
+// of 240 rows 6.7, with 236 of 32 rows 3.2.
+int chain_rows(int rows, int nanl, int neig, int bm, int bn, int bk) {
+    const long tiles = (long)((nanl + bm - 1) / bm) * ((neig + bn - 1) / bn);
+    const long ksteps = (rows + bk - 1) / bk, n = std::max(1L, std::min(ksteps, (256 + tiles - 1) / tiles));
+    return (int)((ksteps + n - 1) / n) * bk;
+}
+
+// Chunks after which kernel tile t empties its accumulators so that a chain has at most
+// lmax rows: whole trips of its ring; none if it cannot.
+constexpr int NO_FLUSH = 1 << 30;
+int flush_chunks(const ProjTile &t, int lmax) {
+    const int n = lmax / t.BK / DIRECT_D * DIRECT_D;
+    return t.E && n > 0 ? n : NO_FLUSH;
+}
+
+// the fewest slices of whole chunks whose chains are at most lmax rows long
+long fewest_slices(const ProjTile &t, int rows, int lmax) {
+    if (flush_chunks(t, lmax) < NO_FLUSH) return 1;
+    const long ksteps = (rows + t.BK - 1) / t.BK, most = std::max(1L, (long)lmax * t.C / t.BK);
+    return std::max(1L, (ksteps + most - 1) / most);
+}
+
+// estimated us of the projection with block tile t, and its number of slices, whose
+// chains are at most lmax rows long
+template <typename R> double proj_cost(const ProjTile &t, double slow, int rows, int nanl, int neig, int lmax, int *nsl) {
     constexpr long CUS = 256;
-    const long tiles = (long)((nanl + BM - 1) / BM) * ((neig + BN - 1) / BN);
-    const long ksteps = (rows + BK - 1) / BK;
+    const long tiles = (long)((nanl + t.BM - 1) / t.BM) * ((neig + t.BN - 1) / t.BN);
+    const long ksteps = (rows + t.BK - 1) / t.BK, fewest = fewest_slices(t, rows, lmax);
     // us of one K step on one CU (6 of the 8 flops of a complex product, at
     // 0.7 of the matrix peak) and of one slice's partials
-    const double step = slow * 6.0 * BM * BN * BK / (sizeof(R) == 8 ? 2.1e5 : 4.2e5);
+    const double step = slow * 6.0 * t.BM * t.BN * t.BK / (sizeof(R) == 8 ? 2.1e5 : 4.2e5);
     const double per = 0.04 + 2.0 * sizeof(cplx<R>) * nanl * neig / 6e6;
     double best = HUGE_VAL;
     const auto consider = [&](long n) {
-        n = std::max(1L, std::min<long>(n, ksteps));
+        n = std::max(fewest, std::min<long>(n, ksteps));
         const long len = (ksteps + n - 1) / n;
         const double cost = (double)((tiles * n + CUS - 1) / CUS) * len * step + n * per;
         if (cost < best) {
@@ -481,13 +511,12 @@ template <typename R> double proj_cost(int BM, int BN, int BK, double slow, int 
 }
 
 // the cheapest of PROJ_AUTO and its number of slices
-template <typename R> int proj_auto(int rows, int nanl, int neig, int *nsl) {
+template <typename R> int proj_auto(int rows, int nanl, int neig, int lmax, int *nsl) {
     double best = HUGE_VAL;
     int pv = 1;
     for (int i = 0; i < 5; i++) {
-        int BM, BN, BK, n = 1;
-        proj_tile<R>(PROJ_AUTO[i], &BM, &BN, &BK);
-        const double c = proj_cost<R>(BM, BN, BK, ProjShapes<R>::slow[i], rows, nanl, neig, &n);
+        int n = 1;
+        const double c = proj_cost<R>(proj_tile<R>(PROJ_AUTO[i]), ProjShapes<R>::slow[i], rows, nanl, neig, lmax, &n);
         if (c < best) {
             best = c;
             pv = PROJ_AUTO[i];
@@ -498,24 +527,28 @@ template <typename R> int proj_auto(int rows, int nanl, int neig, int *nsl) {
 }
 
 template <typename R> void proj_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *pv, int *nsl_out,
-                                      int *kslice_out, bool lean = false) {
+                                      int *kslice_out, bool lean = false, int *chain = nullptr) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
-    const int set = p->proj_var[ix], target = p->splitk[ix] > 0 ? p->splitk[ix] : lean ? 256 : 0;
-    int BM, BN, BK, nsl = 1;
+    const int set = p->proj_var[ix], target = p->splitk[ix];
+    // chains as long as those of the LDS-staged kernel (or of the one that is set) in 256 blocks
+    const ProjTile ref = proj_tile<R>(set >= 0 && set < NPROJ_VAR ? set : 0);
+    const int lmax = chain_rows(rows, nanl, neig, ref.BM, ref.BN, ref.BK);
+    int nsl = 1;
     if (set >= 0) {
         *pv = set < NPROJ_VAR ? set : 0;
-        proj_tile<R>(*pv, &BM, &BN, &BK);
-        if (target <= 0) proj_cost<R>(BM, BN, BK, 1.0, rows, nanl, neig, &nsl);
+        if (target <= 0) proj_cost<R>(proj_tile<R>(*pv), 1.0, rows, nanl, neig, lmax, &nsl);
     } else {
-        *pv = proj_auto<R>(rows, nanl, neig, &nsl);
-        proj_tile<R>(*pv, &BM, &BN, &BK);
+        *pv = proj_auto<R>(rows, nanl, neig, lmax, &nsl);
     }
-    const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
-    const int ksteps = (rows + BK - 1) / BK;
+    const ProjTile t = proj_tile<R>(*pv);
+    const int tm = (nanl + t.BM - 1) / t.BM, tn = (neig + t.BN - 1) / t.BN;
+    const int ksteps = (rows + t.BK - 1) / t.BK;
     if (target > 0) nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
-    const int kslice = ((ksteps + nsl - 1) / nsl) * BK;
+    else if (lean) nsl = (int)fewest_slices(t, rows, lmax);
+    const int kslice = ((ksteps + nsl - 1) / nsl) * t.BK;
     *nsl_out = (rows + kslice - 1) / kslice;
     *kslice_out = kslice;
+    if (chain) *chain = flush_chunks(t, lmax);
 }
 
 // hpsi = beta*hpsi + sum_a beta_a xnlkb_a <beta_a|psi> (Src/cpw_lib/hk_psi_nl_c16.f90:82-96),
@@ -551,10 +584,10 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
         anl = (const cplx<R> *)pv_.anl32->p;
     }
     const long lda = sizeof(R) == 8 ? pv_.lda : *pv_.lda32;
-    int pv, nsl, kslice, BM, BN, BK;
-    proj_shape<R>(p, rows, nanl, neig, &pv, &nsl, &kslice, w && w->lean);
-    proj_tile<R>(pv, &BM, &BN, &BK);
-    const int tm = (nanl + BM - 1) / BM, tn = (neig + BN - 1) / BN;
+    int pv, nsl, kslice, chain;
+    proj_shape<R>(p, rows, nanl, neig, &pv, &nsl, &kslice, w && w->lean, &chain);
+    const ProjTile tile = proj_tile<R>(pv);
+    const int tm = (nanl + tile.BM - 1) / tile.BM, tn = (neig + tile.BN - 1) / tile.BN;
     cplx<R> *part, *dhd;
     if (w) {
         if (cs * (size_t)nsl * neig * nanl > w->part_n || cs * (size_t)neig * nanl > w->dhd_n)
@@ -574,7 +607,7 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
 #define CPW_PD(V)                                                                                                     \
     if (pv == V)                                                                                                      \
         launch_batchable<ProjDirect<R, V>>(CPWGPU_K_PROJ, (k_proj_direct<R, V>), grid, dim3(GEMM_THREADS), 0, s, anl,    \
-                                           lda, ps, ldp, pt, rows, nanl, neig, kslice, 0);
+                                           lda, ps, ldp, pt, rows, nanl, neig, kslice, 0, chain);
         CPW_PD(1) CPW_PD(2) CPW_PD(3) CPW_PD(4)
         CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
 #undef CPW_PD
@@ -1229,26 +1262,30 @@ struct Subspace {
 constexpr int SUB_PROJ_V = 2, SUB_BACK_V = 2;
 
 // split-K partials of a^H b (na x nbc over mtxd rows) into part; returns the
-// number of slices in *nsl.  by_size: the projection's choice of shape and slices;
-// else shape SUB_PROJ_V in slices that make 256 blocks (Rayleigh-Ritz: its vectors'
-// phases follow the rounding of the Gram matrices).
+// number of slices in *nsl.  by_size: the projection's choice of shape and slices, with
+// chains no longer than those of the other choice, shape SUB_PROJ_V in slices that make
+// 256 blocks (Rayleigh-Ritz: its vectors' phases follow the rounding of the Gram
+// matrices).
 int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb, int nbc, int mtxd,
                   DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0, bool by_size = false) {
-    int BM, BN, BK, nsl = 1;
-    const int pv = by_size ? proj_auto<double>(mtxd, na, nbc, &nsl) : SUB_PROJ_V;
-    proj_tile<double>(pv, &BM, &BN, &BK);
-    const int tm = (na + BM - 1) / BM, tn = (nbc + BN - 1) / BN;
-    const int ksteps = (mtxd + BK - 1) / BK;
+    int nsl = 1;
+    const ProjTile sub = proj_tile<double>(SUB_PROJ_V);
+    const int lmax = chain_rows(mtxd, na, nbc, sub.BM, sub.BN, sub.BK);
+    const int pv = by_size ? proj_auto<double>(mtxd, na, nbc, lmax, &nsl) : SUB_PROJ_V;
+    const ProjTile t = proj_tile<double>(pv);
+    const int tm = (na + t.BM - 1) / t.BM, tn = (nbc + t.BN - 1) / t.BN;
+    const int ksteps = (mtxd + t.BK - 1) / t.BK;
     if (!by_size) nsl = std::max(1, std::min(ksteps, (256 + tm * tn - 1) / (tm * tn)));
     // slices are whole K chunks of the kernel
-    const int kslice = ((ksteps + nsl - 1) / nsl) * BK;
+    const int kslice = ((ksteps + nsl - 1) / nsl) * t.BK;
     nsl = (mtxd + kslice - 1) / kslice;
     int rc;
     if ((rc = part.reserve(16 * (size_t)nsl * na * nbc))) return rc;
 #define CPW_PD(V)                                                                                                   \
     if (pv == V)                                                                                                    \
         hipLaunchKernelGGL((k_proj_direct<double, V>), dim3(tm, tn, nsl), dim3(GEMM_THREADS), 0, st,                \
-                           (const cplx<double> *)a, lda, b, ldb, (cplx<double> *)part.p, mtxd, na, nbc, kslice, lower);
+                           (const cplx<double> *)a, lda, b, ldb, (cplx<double> *)part.p, mtxd, na, nbc, kslice, lower,            \
+                           flush_chunks(t, lmax));
     CPW_PD(1) CPW_PD(SUB_PROJ_V)
     CPW_PD(PROJ_BANDS + 1) CPW_PD(PROJ_BANDS + 2) CPW_PD(PROJ_BANDS + 3) CPW_PD(PROJ_BANDS + 5)
 #undef CPW_PD

@@ -260,19 +260,27 @@ constexpr int DIRECT_D = 2;
 constexpr int NPROJ_DIRECT = 4;
 constexpr int PROJ_BANDS = 16;
 // (WM*16) x (WN*16) per wave, GM waves along the projectors and 4 / GM along the
-// bands.  PROJ_BANDS + WN: WN band tiles, four waves along the projectors
+// bands.  PROJ_BANDS + WN: WN band tiles, four waves along the projectors.
+// The matrix instruction rounds its accumulator after every row, so the error of a
+// product grows with the rows that one accumulator takes (its chain).  C: the rows of a
+// slice are dealt to C accumulators, which are added at its end.  E: the accumulators
+// are emptied into a second sum every `chain` chunks (64 registers where another set of
+// accumulators takes 96; a flush is 80 additions a lane, against 12 matrix instructions
+// a chunk).
 template <typename R, int V> struct DirectCfg {
     static constexpr int GM = 4, WM = sizeof(R) == 4 ? 2 : 1, WN = V - PROJ_BANDS, KPL = 2, W = 2, D = DIRECT_D;
+    static constexpr int C = WN == 1 ? 4 : WN <= 3 ? 2 : 1;
+    static constexpr bool E = false;
 };
 // (all compile without register spills on gfx950)
-template <> struct DirectCfg<float, 1> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<float, 2> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<float, 3> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 8, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<float, 4> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 1> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 2> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 1, D = DIRECT_D; };
-template <> struct DirectCfg<double, 3> { static constexpr int GM = 2, WM = 4, WN = 1, KPL = 2, W = 2, D = DIRECT_D; };
-template <> struct DirectCfg<double, 4> { static constexpr int GM = 2, WM = 2, WN = 1, KPL = 4, W = 2, D = DIRECT_D; };
+template <> struct DirectCfg<float, 1> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 2, W = 2, D = DIRECT_D, C = 1; static constexpr bool E = true; };
+template <> struct DirectCfg<float, 2> { static constexpr int GM = 2, WM = 4, WN = 2, KPL = 4, W = 1, D = DIRECT_D, C = 1; static constexpr bool E = false; };
+template <> struct DirectCfg<float, 3> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 8, W = 1, D = DIRECT_D, C = 1; static constexpr bool E = false; };
+template <> struct DirectCfg<float, 4> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 2, D = DIRECT_D, C = 1; static constexpr bool E = false; };
+template <> struct DirectCfg<double, 1> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 2, W = 2, D = DIRECT_D, C = 1; static constexpr bool E = true; };
+template <> struct DirectCfg<double, 2> { static constexpr int GM = 2, WM = 2, WN = 2, KPL = 4, W = 1, D = DIRECT_D, C = 1; static constexpr bool E = false; };
+template <> struct DirectCfg<double, 3> { static constexpr int GM = 2, WM = 4, WN = 1, KPL = 2, W = 2, D = DIRECT_D, C = 1; static constexpr bool E = false; };
+template <> struct DirectCfg<double, 4> { static constexpr int GM = 2, WM = 2, WN = 1, KPL = 4, W = 2, D = DIRECT_D, C = 1; static constexpr bool E = false; };
 template <typename R, int V> constexpr int direct_bm() { return DirectCfg<R, V>::GM * DirectCfg<R, V>::WM * 16; }
 template <typename R, int V> constexpr int direct_bn() { return 4 / DirectCfg<R, V>::GM * DirectCfg<R, V>::WN * 16; }
 template <typename R, int V> constexpr int direct_bk() { return 4 * DirectCfg<R, V>::KPL; }
@@ -328,7 +336,7 @@ template <typename R, int V> struct ProjDirect {
     static constexpr int T = GEMM_THREADS, W = (DirectCfg<R, V>::W);
     static __device__ __forceinline__ void run(const Blk blk, const cplx<R> *__restrict__ anl, long lda, const
         double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__ part, int mtxd, int nanl, int neig, int kslice,
-        int lower) {
+        int lower, int chain) {
         typedef typename MF<R>::v4 v4;
         constexpr int WM = DirectCfg<R, V>::WM, WN = DirectCfg<R, V>::WN;
         constexpr int KPL = DirectCfg<R, V>::KPL, KC = 4 * KPL;
@@ -355,15 +363,45 @@ template <typename R, int V> struct ProjDirect {
             const int n = n0 + wn * WN * 16 + t * 16 + lr;
             bcol[t] = psi + (long)min(n, neig - 1) * ldp;
         }
-        v4 P1[WM][WN], P2[WM][WN], P3[WM][WN];
+        constexpr int C = DirectCfg<R, V>::C;
+        static_assert(DirectCfg<R, V>::D * KPL % C == 0, "bad k_proj_direct chains");
+        v4 P1[C][WM][WN], P2[C][WM][WN], P3[C][WM][WN];
 #pragma unroll
-        for (int i = 0; i < WM; i++)
+        for (int q = 0; q < C; q++)
 #pragma unroll
-            for (int j = 0; j < WN; j++) {
-                P1[i][j] = v4{0, 0, 0, 0};
-                P2[i][j] = v4{0, 0, 0, 0};
-                P3[i][j] = v4{0, 0, 0, 0};
-            }
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++) {
+                    P1[q][i][j] = v4{0, 0, 0, 0};
+                    P2[q][i][j] = v4{0, 0, 0, 0};
+                    P3[q][i][j] = v4{0, 0, 0, 0};
+                }
+        // the chains of one product, pairwise
+        const auto total = [](const v4(&p)[C][WM][WN], int mi, int ni) {
+            if constexpr (C == 4) return (p[0][mi][ni] + p[1][mi][ni]) + (p[2][mi][ni] + p[3][mi][ni]);
+            else if constexpr (C == 2) return p[0][mi][ni] + p[1][mi][ni];
+            else return p[0][mi][ni];
+        };
+        constexpr bool E = DirectCfg<R, V>::E;
+        v4 re[WM][WN], im[WM][WN];  // the second sum
+        if constexpr (E) {
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++) re[i][j] = im[i][j] = v4{0, 0, 0, 0};
+        }
+        const auto flush = [&]() {
+#pragma unroll
+            for (int i = 0; i < WM; i++)
+#pragma unroll
+                for (int j = 0; j < WN; j++) {
+                    const v4 p1 = P1[0][i][j], p2 = P2[0][i][j], p3 = P3[0][i][j];
+                    re[i][j] += p1 + p2;
+                    im[i][j] += p3 - p1 + p2;
+                    P1[0][i][j] = P2[0][i][j] = P3[0][i][j] = v4{0, 0, 0, 0};
+                }
+        };
+        int next = chain;
         constexpr int D = DirectCfg<R, V>::D;
         cplx<R> ra[D][WM][KPL];
         double2 rb[D][WN][KPL];
@@ -382,9 +420,11 @@ template <typename R, int V> struct ProjDirect {
                 for (int t = 0; t < WN; t++) load_psi_tail<KPL>(rb_[t], bcol[t], i0, ke, mtxd);
             }
         };
-        auto compute = [&](const cplx<R>(&ra_)[WM][KPL], const double2(&rb_)[WN][KPL]) {
+        // buf: the chunk's place in the ring (a constant once unrolled)
+        auto compute = [&](const cplx<R>(&ra_)[WM][KPL], const double2(&rb_)[WN][KPL], int buf) {
 #pragma unroll
             for (int u = 0; u < KPL; u++) {
+                const int q = (buf * KPL + u) % C;
                 R ar[WM], ai[WM], as[WM], br[WN], bi[WN], bs[WN];
 #pragma unroll
                 for (int t = 0; t < WM; t++) {
@@ -402,9 +442,9 @@ template <typename R, int V> struct ProjDirect {
                 for (int mi = 0; mi < WM; mi++)
 #pragma unroll
                     for (int ni = 0; ni < WN; ni++) {
-                        P1[mi][ni] = MF<R>::mma(ar[mi], br[ni], P1[mi][ni]);
-                        P2[mi][ni] = MF<R>::mma(ai[mi], bi[ni], P2[mi][ni]);
-                        P3[mi][ni] = MF<R>::mma(as[mi], bs[ni], P3[mi][ni]);
+                        P1[q][mi][ni] = MF<R>::mma(ar[mi], br[ni], P1[q][mi][ni]);
+                        P2[q][mi][ni] = MF<R>::mma(ai[mi], bi[ni], P2[q][mi][ni]);
+                        P3[q][mi][ni] = MF<R>::mma(as[mi], bs[ni], P3[q][mi][ni]);
                     }
             }
         };
@@ -417,7 +457,7 @@ template <typename R, int V> struct ProjDirect {
         // 128: 90 us, sunk 122), so they are kept apart: in FP64 by scheduling barriers on
         // both sides of the MFMAs (80,852 x 864 x 512 3,620 us; 3,790 without the second),
         // in FP32 by a branch it cannot see through (shape 2, 23,928 x 256 x 128: 54 us,
-        // with barriers 57).  Then the partial chunk, if any.  Chunks are accumulated in K order for any D.
+        // with barriers 57).  Then the partial chunk, if any.  Each chain takes its rows in K order.
         int always = 1;
         asm volatile("" : "+s"(always));
         const int nfull = max(0, ke - kb) / KC;
@@ -426,25 +466,31 @@ template <typename R, int V> struct ProjDirect {
             for (int j = 0; j < D - 1; j++) load(ra[j], rb[j], kb + min(j, nfull - 1) * KC, false);
             int c = 0;
             for (; c + D <= nfull; c += D) {
+                if constexpr (E) {
+                    if (c >= next) {
+                        next += chain;
+                        flush();
+                    }
+                }
 #pragma unroll
                 for (int j = 0; j < D; j++) {
                     load(ra[(j + D - 1) % D], rb[(j + D - 1) % D], kb + min(c + j + D - 1, nfull - 1) * KC, false);
                     if constexpr (sizeof(R) == 8) {
                         __builtin_amdgcn_sched_barrier(0);
-                        compute(ra[j], rb[j]);
+                        compute(ra[j], rb[j], j);
                         __builtin_amdgcn_sched_barrier(0);
                     } else if (always) {
-                        compute(ra[j], rb[j]);
+                        compute(ra[j], rb[j], j);
                     }
                 }
             }
 #pragma unroll
             for (int j = 0; j < D - 1; j++)
-                if (c + j < nfull) compute(ra[j], rb[j]);
+                if (c + j < nfull) compute(ra[j], rb[j], j);
         }
         if (kb + nfull * KC < ke) {
             load(ra[0], rb[0], kb + nfull * KC, true);
-            compute(ra[0], rb[0]);
+            compute(ra[0], rb[0], 0);
         }
         cplx<R> *ps = part + (long)tl.z * neig * nanl;
 #pragma unroll
@@ -452,11 +498,16 @@ template <typename R, int V> struct ProjDirect {
 #pragma unroll
             for (int ni = 0; ni < WN; ni++) {
                 const int n = n0 + wn * WN * 16 + ni * 16 + lr;
+                const v4 p1 = total(P1, mi, ni), p2 = total(P2, mi, ni), p3 = total(P3, mi, ni);
+                v4 x = p1 + p2, y = p3 - p1 + p2;
+                if constexpr (E) {
+                    x += re[mi][ni];
+                    y += im[mi][ni];
+                }
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int a = a0 + wm * WM * 16 + mi * 16 + MF<R>::row(lg, r);
-                    const R p1 = P1[mi][ni][r], p2 = P2[mi][ni][r], p3 = P3[mi][ni][r];
-                    if (a < nanl && n < neig) ps[(long)n * nanl + a] = mk<R>(p1 + p2, p3 - p1 + p2);
+                    if (a < nanl && n < neig) ps[(long)n * nanl + a] = mk<R>(x[r], y[r]);
                 }
             }
     }
@@ -464,8 +515,8 @@ template <typename R, int V> struct ProjDirect {
 template <typename R, int V>
 __global__ __launch_bounds__(GEMM_THREADS, (DirectCfg<R, V>::W)) void k_proj_direct(const cplx<R> *__restrict__ anl,
     long lda, const double2 *__restrict__ psi, long ldp, cplx<R> *__restrict__ part, int mtxd, int nanl, int neig,
-    int kslice, int lower = 0) {
-    ProjDirect<R, V>::run(Blk::here(), anl, lda, psi, ldp, part, mtxd, nanl, neig, kslice, lower);
+    int kslice, int lower, int chain) {
+    ProjDirect<R, V>::run(Blk::here(), anl, lda, psi, ldp, part, mtxd, nanl, neig, kslice, lower, chain);
 }
 
 // dhd[n][a] = xnlkb[a] * sum_s part[s][n][a]   (fixed summation order: deterministic)
