@@ -262,22 +262,25 @@ template <typename R> int plane_var_resolve(const cpwgpu_plan_s *p, int v, bool 
     return v < 0 || !*ok ? def : v;
 }
 
-// Column kernel the next apply uses; *ok: whether v is usable (1, the register
-// lines, needs them built for n3).  Default: LDS lines in FP32 (inverse + forward
-// at 72, 128 bands: 24 + 50 us against 35 + 61); in FP64 register lines for the
-// forward columns (72: 62 against 65, 32x32x128, 72 bands: 15 against 19, 36, 20
-// bands: 5 against 8), for the inverse ones only up to 40 (36: 6.5 against 7.1;
-// 72: 38 against 37).  Choice 0 or 1 holds for both directions; the default is
-// reported for the forward one.
+// Column kernel the next apply uses; *ok: whether v is usable (1 needs the register
+// lines built for n3).  Default: LDS lines (0) in FP32 (inverse + forward at 72, 128
+// bands: 24 + 50 us against 35 + 61), register lines (1) in FP64 (forward, 72: 62
+// against 65, 32x32x128, 72 bands: 15 against 19, 36, 20 bands: 5 against 8), whose
+// inverse columns beyond 40 points still take the LDS lines (col_reg_inverse; 36: 6.5
+// against 7.1; 72: 38 against 37).
 template <typename R> int col_var_resolve(const cpwgpu_plan_s *p, int v, bool *ok, int stage = ST_COL_FWD) {
     const FftGeom &g = p->g;
-    bool built = false;
-#define CPW_CB(N) if (g.n[2] == N) built = col_reg_built<R, N>();
+    bool built = false, inverse = false;
+#define CPW_CB(N)                              \
+    if (g.n[2] == N) {                         \
+        built = col_reg_built<R, N>();         \
+        inverse = col_reg_inverse<R, N>();     \
+    }
     CPW_FAST_SIZES(CPW_CB)
 #undef CPW_CB
     if (ok) *ok = v <= 0 || (v == 1 && built);
-    if (v < 0) return built && sizeof(R) == 8 && (stage == ST_COL_FWD || g.n[2] <= 40) ? 1 : 0;
-    return v == 1 && built ? 1 : 0;
+    if (v < 0) v = sizeof(R) == 8;
+    return v == 1 && (stage == ST_COL_FWD ? built : inverse) ? 1 : 0;
 }
 
 // One stage of the local term: specialised kernels when the mesh allows,
@@ -414,9 +417,11 @@ int back_shape64(int rows, int neig) {
     const long small = ((long)(rows + 63) / 64 * ((neig + 15) / 16) + 255) / 256;
     return big <= 3 && 0.25 * 1.35 * small < big ? BACK_BANDS + 1 : 2;
 }
+// The number of this choice among the back-projection kernels (cpwgpu_plan_set_variant).
+template <typename R> constexpr int BACK_DEFAULT = sizeof(R) == 4 ? NBACK_DIRECT + 1 : 2;
 template <typename R> int back_variant(const cpwgpu_plan_s *p, int rows, int neig) {
-    const int ix = sizeof(R) == 4 ? 1 : 0;
-    if (p->back_var[ix] >= 0) return p->back_var[ix] < NBACK_VAR ? p->back_var[ix] : 0;
+    const int v = p->back_var[sizeof(R) == 4 ? 1 : 0];
+    if (v >= 0 && v != BACK_DEFAULT<R>) return v < NBACK_VAR ? v : 0;
     if (sizeof(R) == 4) {
         const int t = (neig + 15) / 16;
         if (t <= 3) return BACK_BANDS + 1;
@@ -455,18 +460,22 @@ template <> struct ProjShapes<double> {
 template <> struct ProjShapes<float> {
     static constexpr double slow[5] = {1.0, 1.72, 1.36, 1.13, 1.01};
 };
+// Numbers of the choice by size (cpwgpu_plan_set_variant): kernel 1 is the direct one with
+// the block that suits the bands, 256 blocks (the compute units) stand for whole rounds
+// of them.
+constexpr int PROJ_DEFAULT = 1, SPLITK_DEFAULT = 256;
 constexpr int PROJ_AUTO[5] = {1, PROJ_BANDS + 1, PROJ_BANDS + 2, PROJ_BANDS + 3, PROJ_BANDS + 5};
 
-// Rows of a slice when the product is cut into 256 blocks of bm x bn tiles, whole
-// chunks of bk: the longest sum that one accumulator is to hold.  <beta|psi> is off
+// Rows of a slice when the product is cut into that many blocks of tile t, whole
+// chunks: the longest sum that one accumulator is to hold.  <beta|psi> is off
 // by sqrt(1.6 + 0.185 L + 0.009 n) roundings (rms, in units of |beta||psi|/sqrt(rows),
 // FP32 and FP64, 729 to 23,928 rows) for n slices whose chains are L rows long, so
 // that fewer slices mean a less accurate product: 7,550 x 128 x 128 with 32 slices
 // of 240 rows 6.7, with 236 of 32 rows 3.2.
-int chain_rows(int rows, int nanl, int neig, int bm, int bn, int bk) {
-    const long tiles = (long)((nanl + bm - 1) / bm) * ((neig + bn - 1) / bn);
-    const long ksteps = (rows + bk - 1) / bk, n = std::max(1L, std::min(ksteps, (256 + tiles - 1) / tiles));
-    return (int)((ksteps + n - 1) / n) * bk;
+int chain_rows(const ProjTile &t, int rows, int nanl, int neig, int blocks) {
+    const long tiles = (long)((nanl + t.BM - 1) / t.BM) * ((neig + t.BN - 1) / t.BN);
+    const long ksteps = (rows + t.BK - 1) / t.BK, n = std::max(1L, std::min(ksteps, (blocks + tiles - 1) / tiles));
+    return (int)((ksteps + n - 1) / n) * t.BK;
 }
 
 // Chunks after which kernel tile t empties its accumulators so that a chain has at most
@@ -529,22 +538,24 @@ template <typename R> int proj_auto(int rows, int nanl, int neig, int lmax, int 
 template <typename R> void proj_shape(const cpwgpu_plan_s *p, int rows, int nanl, int neig, int *pv, int *nsl_out,
                                       int *kslice_out, bool lean = false, int *chain = nullptr) {
     const int ix = sizeof(R) == 4 ? 1 : 0;
-    const int set = p->proj_var[ix], target = p->splitk[ix];
-    // chains as long as those of the LDS-staged kernel (or of the one that is set) in 256 blocks
-    const ProjTile ref = proj_tile<R>(set >= 0 && set < NPROJ_VAR ? set : 0);
-    const int lmax = chain_rows(rows, nanl, neig, ref.BM, ref.BN, ref.BK);
+    const int set = p->proj_var[ix] >= 0 && p->proj_var[ix] < NPROJ_VAR ? p->proj_var[ix] : PROJ_DEFAULT;
+    const int target = p->splitk[ix] == SPLITK_DEFAULT ? 0 : p->splitk[ix];
+    // chains as long as those of the kernel that is set in that many blocks; by size, of the
+    // LDS-staged one in 256 (64 bands wide in the caller's number of blocks)
+    const ProjTile ref = proj_tile<R>(set != PROJ_DEFAULT ? set : target > 0 ? 1 : 0);
+    const int lmax = chain_rows(ref, rows, nanl, neig, target > 0 ? target : 256);
     int nsl = 1;
-    if (set >= 0) {
-        *pv = set < NPROJ_VAR ? set : 0;
-        if (target <= 0) proj_cost<R>(proj_tile<R>(*pv), 1.0, rows, nanl, neig, lmax, &nsl);
-    } else {
+    if (set == PROJ_DEFAULT) {
         *pv = proj_auto<R>(rows, nanl, neig, lmax, &nsl);
+    } else {
+        *pv = set;
+        if (target <= 0) proj_cost<R>(proj_tile<R>(set), 1.0, rows, nanl, neig, lmax, &nsl);
     }
     const ProjTile t = proj_tile<R>(*pv);
     const int tm = (nanl + t.BM - 1) / t.BM, tn = (neig + t.BN - 1) / t.BN;
     const int ksteps = (rows + t.BK - 1) / t.BK;
-    if (target > 0) nsl = std::max(1, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
-    else if (lean) nsl = (int)fewest_slices(t, rows, lmax);
+    if (target > 0 || lean) nsl = (int)fewest_slices(t, rows, lmax);
+    if (target > 0) nsl = std::max(nsl, std::min(ksteps, (target + tm * tn - 1) / (tm * tn)));
     const int kslice = ((ksteps + nsl - 1) / nsl) * t.BK;
     *nsl_out = (rows + kslice - 1) / kslice;
     *kslice_out = kslice;
@@ -1270,7 +1281,7 @@ int gram_partials(const double2 *a, long lda, int na, const double2 *b, long ldb
                   DevBuf &part, int *nsl_out, hipStream_t st, int lower = 0, bool by_size = false) {
     int nsl = 1;
     const ProjTile sub = proj_tile<double>(SUB_PROJ_V);
-    const int lmax = chain_rows(mtxd, na, nbc, sub.BM, sub.BN, sub.BK);
+    const int lmax = chain_rows(sub, mtxd, na, nbc, 256);
     const int pv = by_size ? proj_auto<double>(mtxd, na, nbc, lmax, &nsl) : SUB_PROJ_V;
     const ProjTile t = proj_tile<double>(pv);
     const int tm = (na + t.BM - 1) / t.BM, tn = (nbc + t.BN - 1) / t.BN;
@@ -2478,13 +2489,12 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         // projection kernel x split-K target
         const int cand[4] = {128, 256, 512, 1024};
         best = 3.4e38f;
-        for (int jv = -1; jv < NPROJ_VAR; jv++)
+        for (int jv = 0; jv < NPROJ_VAR; jv++)
             for (int c : cand) {
-                if (jv < 0 && c != cand[0]) continue;  // the default chooses its own split
                 p->proj_var[ix] = jv;
-                p->splitk[ix] = jv < 0 ? -1 : c;
+                p->splitk[ix] = c;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
-                if (t < best) { best = t; best_sk = p->splitk[ix]; best_jv = jv; }
+                if (t < best) { best = t; best_sk = c; best_jv = jv; }
             }
     }
     p->proj_var[ix] = best_jv;
@@ -2492,7 +2502,7 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
     int best_bv = 0;
     if (p->nanl > 0) {
         best = 3.4e38f;
-        for (int bv = -1; bv < NBACK_VAR; bv++) {
+        for (int bv = 0; bv < NBACK_VAR; bv++) {
             p->back_var[ix] = bv;
             if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
             if (t < best) { best = t; best_bv = bv; }
@@ -2518,7 +2528,7 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &best))) return st;
         for (int sv = 1; sv <= 2; sv++) {
             p->sched_var[ix] = sv;
-            for (int bv = -1; bv < NBACK_VAR; bv++) {
+            for (int bv = 0; bv < NBACK_VAR; bv++) {
                 p->back_var[ix] = bv;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t))) return st;
                 if (t < best) { best = t; best_sv = sv; best_bv = bv; }
@@ -2584,19 +2594,18 @@ int tune_spin(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         const int cand[4] = {128, 256, 512, 1024};
         int best_jv = 0, best_sk = -1;
         best = 3.4e38f;
-        for (int jv = -1; jv < NPROJ_VAR; jv++)
+        for (int jv = 0; jv < NPROJ_VAR; jv++)
             for (int c : cand) {
-                if (jv < 0 && c != cand[0]) continue;  // the default chooses its own split
                 p->proj_var[ix] = jv;
-                p->splitk[ix] = jv < 0 ? -1 : c;
+                p->splitk[ix] = c;
                 if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t, true))) return st;
-                if (t < best) { best = t; best_sk = p->splitk[ix]; best_jv = jv; }
+                if (t < best) { best = t; best_sk = c; best_jv = jv; }
             }
         p->proj_var[ix] = best_jv;
         p->splitk[ix] = best_sk;
         int best_bv = 0;
         best = 3.4e38f;
-        for (int bv = -1; bv < NBACK_VAR; bv++) {
+        for (int bv = 0; bv < NBACK_VAR; bv++) {
             p->back_var[ix] = bv;
             if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 5, &t, true))) return st;
             if (t < best) { best = t; best_bv = bv; }
@@ -3301,15 +3310,15 @@ int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value) 
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_SPLITK) {
-        *value = plan->splitk[ix] > 0 ? plan->splitk[ix] : 256;
+        *value = plan->splitk[ix] > 0 ? plan->splitk[ix] : SPLITK_DEFAULT;
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_PROJ) {
-        *value = plan->proj_var[ix] >= 0 ? std::min(plan->proj_var[ix], NPROJ_VAR - 1) : 1;
+        *value = plan->proj_var[ix] >= 0 ? plan->proj_var[ix] : PROJ_DEFAULT;
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_BACK) {
-        *value = plan->back_var[ix] >= 0 ? std::min(plan->back_var[ix], NBACK_VAR - 1) : ix ? NBACK_DIRECT + 1 : 2;
+        *value = plan->back_var[ix] >= 0 ? plan->back_var[ix] : ix ? BACK_DEFAULT<float> : BACK_DEFAULT<double>;
         return CPWGPU_OK;
     }
     if (what == CPWGPU_TUNE_KIN) {

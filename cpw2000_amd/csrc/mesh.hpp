@@ -137,6 +137,10 @@ template <typename R, int N> constexpr int col_reg_g() {
     return reg_ok<R, N, 8, 8>() ? 8 : reg_ok<R, N, 4, 4>() ? 4 : 0;
 }
 template <typename R, int N> constexpr bool col_reg_built() { return col_reg_g<R, N>() > 0; }
+// whether the register lines serve the inverse columns too
+template <typename R, int N> constexpr bool col_reg_inverse() {
+    return col_reg_built<R, N>() && (sizeof(R) == 4 || N <= 40);
+}
 // the sphere box inside |z| <= N3/4: the pruned register column kernels
 inline bool col_prune_fits(const FftGeom &g) { return 4 * g.kd[2] <= g.n[2]; }
 

@@ -135,12 +135,16 @@ int launch_col_reg(cpwgpu_plan_s *p, const LocalArgs &a, cplx<R> *colbuf, int st
         const double2 *tw3 = (const double2 *)p->tw[2].p;
         const int *zm = (const int *)p->zmap.p;
         if (stage == ST_COL_BWD) {
-            if (pr)
-                launch_batchable<ColBwdReg<R, N, G, true>>(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
-                                   zm, tw3, g, ntiles, a.nb);
-            else
-                launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
-                                   zm, tw3, g, ntiles, a.nb);
+            if constexpr (col_reg_inverse<R, N>()) {
+                if (pr)
+                    launch_batchable<ColBwdReg<R, N, G, true>>(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
+                                       zm, tw3, g, ntiles, a.nb);
+                else
+                    launch_timed(CPWGPU_K_COL_BWD, (k_col_bwd_reg<R, N, G, false>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, colbuf,
+                                       zm, tw3, g, ntiles, a.nb);
+            } else {
+                return fail(CPWGPU_ERR_MODE, "register inverse column kernels are not built for N = %d", N);
+            }
         } else {
             if (pr)
                 launch_batchable<ColFwdReg<R, N, G, true>>(CPWGPU_K_COL_FWD, (k_col_fwd_reg<R, N, G, true>), grid, dim3(COLR_T), 0, s, a.psi, a.ldp, a.hpsi,

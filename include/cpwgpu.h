@@ -219,18 +219,19 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
  *                       lies inside N/4).  On meshes outside the fully
  *                       specialised set 0 = the generic kernel
  *   CPWGPU_TUNE_SPLITK  target number of blocks of the split-K projection
- *                       GEMM (64..4096); -1 = default (whole rounds of the
- *                       compute units; reported as 256)
+ *                       GEMM (64..4096); 256, the number of compute units,
+ *                       stands for whole rounds of them, as many as are
+ *                       cheapest; -1 = default (256)
  *   CPWGPU_TUNE_PROJ    kernel of the projection GEMM: 0 = LDS-staged tiles,
- *                       1..4 = direct register loads in four tile shapes,
- *                       5 = LDS-staged with half the wave tile;
- *                       -1 = default (by size; reported for wide blocks of
- *                       bands)
+ *                       1..4 = direct register loads in four tile shapes (1:
+ *                       the block that suits the number of bands), 5 =
+ *                       LDS-staged with half the wave tile; -1 = default (1)
  *   CPWGPU_TUNE_BACK    kernel of the back-projection GEMM: 0 = LDS-staged D,
- *                       1..3 = direct register loads in three tile shapes,
- *                       4 = LDS-staged with half-size projector chunks;
- *                       -1 = default (by size; reported for wide blocks of
- *                       bands)
+ *                       1..3 = direct register loads in three tile shapes (2,
+ *                       FP64: also a smaller block where few bands leave the
+ *                       GPU idle), 4 = LDS-staged with half-size projector
+ *                       chunks (FP32: 16 to 64 bands per block, by their
+ *                       number); -1 = default (FP64 2, FP32 4)
  *   CPWGPU_TUNE_KIN     where ekpg*psi is added when projectors are set: 0 = in
  *                       the back-projection epilogue, 1 = in the gather of the
  *                       forward column kernel (moves work between the two
@@ -241,8 +242,9 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
  *                       where built, else 0)
  *   CPWGPU_TUNE_COL     z-column kernels: 0 = LDS two-pass lines, 1 =
  *                       register-resident lines (built where a column fits in
- *                       the registers of 8 or 4 lanes); -1 = default (FP64 1
- *                       where built, else 0)
+ *                       the registers of 8 or 4 lanes; in FP64 the inverse
+ *                       columns of more than 40 points stay with the LDS
+ *                       lines); -1 = default (FP64 1 where built, else 0)
  *   CPWGPU_TUNE_SCHED   stream schedule: 0 = everything on the caller's stream
  *                       (projection, D scaling, local term written, back-
  *                       projection added to it); with overlap on, 1 = the projection and D scaling
@@ -260,7 +262,8 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
 #define CPWGPU_TUNE_COL 6
 #define CPWGPU_TUNE_SCHED 7
 int cpwgpu_plan_set_variant(cpwgpu_plan_t plan, int prec, int what, int value);
-/* Current choice (the value used by the next apply, defaults resolved). */
+/* Current choice (the value used by the next apply, defaults resolved): setting it on
+ * a plan of the same k-point runs the same kernels. */
 int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value);
 /* Autotuner: times cpwgpu_plan_apply for every plane variant built for the
  * mesh, then both projection kernels with a few split-K targets, then both
