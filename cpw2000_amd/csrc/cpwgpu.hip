@@ -2399,8 +2399,7 @@ void tune_cache_store(const TuneKey &k, int plane, int proj, int back, int split
     std::fclose(f);
 }
 
-// median-free timing: the best of `reps` applies (two-component ones with
-// spin) after one warm-up
+// the best of `reps` applies (two-component ones with spin) after one warm-up
 int time_apply(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hpsi, long ldh,
                int prec, hipStream_t s, int reps, float *best, bool spin = false) {
     auto apply = [&]() {
@@ -2430,6 +2429,31 @@ int time_apply(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, a, b));
         *best = std::min(*best, ms / BATCH);
+    }
+    hipEventDestroy(a);
+    hipEventDestroy(b);
+    return st;
+}
+
+// ms per apply in a loop of at least 20 ms without a wait, after a quarter as many untimed
+int time_loop(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *hpsi, long ldh, int prec, hipStream_t s,
+              float *ms) {
+    float one = 0.f;
+    int st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 1, &one);
+    if (st) return st;
+    const int n = std::max(4, std::min(2000, (int)(20.f / std::max(one, 1e-3f)) + 1)), lead = (n + 3) / 4;
+    hipEvent_t a, b;
+    HIPCHK(hipEventCreate(&a));
+    HIPCHK(hipEventCreate(&b));
+    for (int i = 0; i < lead + n && !st; i++) {
+        if (i == lead) HIPCHK(hipEventRecord(a, s));
+        st = cpwgpu_plan_apply(p, neig, psi, ldp, hpsi, ldh, prec, s);
+    }
+    if (!st) {
+        HIPCHK(hipEventRecord(b, s));
+        HIPCHK(hipEventSynchronize(b));
+        HIPCHK(hipEventElapsedTime(ms, a, b));
+        *ms /= n;
     }
     hipEventDestroy(a);
     hipEventDestroy(b);
@@ -2550,19 +2574,22 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         if (t < best) { best = t; best_pv = v; }
     }
     p->plane_var[ix] = best_pv;
-    // Against the defaults by size as a whole: each choice above was made with the
-    // others as they stood, some of them from a single apply (216 atoms, 512 bands,
-    // FP64: chosen 15.7 ms, defaults 13.2).
-    if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 8, &best))) return st;
+    // Against the defaults by size as a whole, in turn: each choice above was made with
+    // the others as they stood, and from a few applies with a wait after each, while a
+    // caller's loop pays the time that the clocks settle to (216 atoms, 512 bands, FP64:
+    // a choice of 12.6 ms by single applies takes 15.4 in a loop, the defaults 13.2).
     int *const choice[7] = {&p->plane_var[ix], &p->proj_var[ix], &p->back_var[ix], &p->splitk[ix],
                             &p->kin_var[ix], &p->col_var[ix], &p->sched_var[ix]};
     int tuned[7];
-    for (int i = 0; i < 7; i++) {
-        tuned[i] = *choice[i];
-        *choice[i] = -1;
-    }
-    if ((st = time_apply(p, neig, psi, ldp, hpsi, ldh, prec, s, 8, &t))) return st;
-    if (best < t)
+    for (int i = 0; i < 7; i++) tuned[i] = *choice[i];
+    double sum[2] = {0.0, 0.0};
+    for (int round = 0; round < 5; round++)
+        for (int def = 0; def < 2; def++) {
+            for (int i = 0; i < 7; i++) *choice[i] = def ? -1 : tuned[i];
+            if ((st = time_loop(p, neig, psi, ldp, hpsi, ldh, prec, s, &t))) return st;
+            sum[def] += t;
+        }
+    if (sum[0] < sum[1])
         for (int i = 0; i < 7; i++) *choice[i] = tuned[i];
     // leave hpsi holding H psi of the chosen configuration
     if ((st = cpwgpu_plan_apply(p, neig, psi, ldp, hpsi, ldh, prec, s))) return st;
