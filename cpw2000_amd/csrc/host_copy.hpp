@@ -20,8 +20,22 @@ constexpr int HC_LANES = 8;                    // threads, the caller's own amon
 constexpr size_t HC_CHUNK = 2ull << 20;        // bytes per pinned piece; two per lane
 constexpr size_t HC_MIN = 4ull << 20;          // smaller copies go to the runtime
 
-// Pinned pieces, kept from the first large copy to cpwgpu_finalize (32 MB).  Used
-// under the library's lock, by one copy at a time.
+// The library's device is the current one while this lives; the caller's is again
+// afterwards.
+struct OnDevice {
+    int before = 0;
+    hipError_t err;
+    OnDevice() {
+        err = hipGetDevice(&before);
+        if (err == hipSuccess && before != g_device) err = hipSetDevice(g_device);
+    }
+    ~OnDevice() {
+        if (before != g_device) (void)hipSetDevice(before);
+    }
+};
+
+// Pinned pieces, kept from the first large copy to cpwgpu_finalize or a copy for
+// another device (32 MB).  Used under the library's lock, by one copy at a time.
 struct HostCopy {
     struct Lane {
         char *pin[2] = {nullptr, nullptr};
@@ -30,10 +44,13 @@ struct HostCopy {
     } lane[HC_LANES];
     int lanes = 0;      // those that have their pieces
     bool tried = false;
+    int device = 0;     // of the events
 
     void init() {
+        if (tried && device != g_device) release();
         if (tried) return;
         tried = true;
+        device = g_device;
         const int want = std::max(1, std::min<int>(HC_LANES, (int)std::thread::hardware_concurrency()));
         for (; lanes < want; lanes++)
             for (int i = 0; i < 2; i++)
@@ -74,6 +91,8 @@ template <bool GATHER> inline void copy_piece(char *buf, char *a, size_t ld, siz
 template <bool IN>
 int host_copy_2d(void *dev, size_t ldd, void *host, size_t ldh, size_t width, size_t cols, hipStream_t s) {
     const size_t total = width * cols;
+    OnDevice on;
+    if (on.err != hipSuccess) return fail(CPWGPU_ERR_HIP, "device %d: %s", g_device, hipGetErrorString(on.err));
     if (total >= HC_MIN) g_hc.init();
     if (total < HC_MIN || g_hc.lanes == 0) {
         if (IN) HIPCHK(hipMemcpy2DAsync(dev, ldd, host, ldh, width, cols, hipMemcpyHostToDevice, s));
