@@ -2792,6 +2792,13 @@ int cpwgpu_finalize(void) {
 
 const char *cpwgpu_last_error(void) { return g_err.c_str(); }
 
+int cpwgpu_host_copy_lanes(int *lanes) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (!lanes) return fail(CPWGPU_ERR_ARG, "null argument");
+    *lanes = g_hc.lanes;
+    return CPWGPU_OK;
+}
+
 int cpwgpu_set_ditsp_method(int method) {
     if (method != CPWGPU_DITSP_BLOCK && method != CPWGPU_DITSP_CHEB)
         return fail(CPWGPU_ERR_MODE, "diagonalisation method %d", method);

@@ -43,22 +43,24 @@ struct HostCopy {
         bool used[2] = {false, false};
     } lane[HC_LANES];
     int lanes = 0;      // those that have their pieces
-    bool tried = false;
     int device = 0;     // of the events
 
+    // the lanes that are missing: also those that could not be had at an earlier copy
     void init() {
-        if (tried && device != g_device) release();
-        if (tried) return;
-        tried = true;
+        if (device != g_device) release();
         device = g_device;
         const int want = std::max(1, std::min<int>(HC_LANES, (int)std::thread::hardware_concurrency()));
         for (; lanes < want; lanes++)
-            for (int i = 0; i < 2; i++)
-                if (hipHostMalloc((void **)&lane[lanes].pin[i], HC_CHUNK, hipHostMallocDefault) != hipSuccess ||
-                    hipEventCreateWithFlags(&lane[lanes].ev[i], hipEventDisableTiming) != hipSuccess) {
+            for (int i = 0; i < 2; i++) {
+                Lane &l = lane[lanes];
+                if (!l.pin[i] && hipHostMalloc((void **)&l.pin[i], HC_CHUNK, hipHostMallocDefault) != hipSuccess)
+                    l.pin[i] = nullptr;
+                if (!l.ev[i] && hipEventCreateWithFlags(&l.ev[i], hipEventDisableTiming) != hipSuccess) l.ev[i] = nullptr;
+                if (!l.pin[i] || !l.ev[i]) {
                     (void)hipGetLastError();
                     return;
                 }
+            }
     }
     void release() {
         for (Lane &l : lane)
@@ -69,7 +71,6 @@ struct HostCopy {
                 l = i ? Lane{} : l;
             }
         lanes = 0;
-        tried = false;
     }
 };
 inline HostCopy g_hc;

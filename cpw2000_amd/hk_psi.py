@@ -52,6 +52,7 @@ EXPORTS = (
     "cpwgpu_hk_psi_spin_c16", "cpwgpu_plan_set_potential_spin", "cpwgpu_plan_set_projectors_spin",
     "cpwgpu_plan_apply_spin", "cpwgpu_hk_psi_c8", "cpwgpu_hk_psi_allk_c16",
     "cpwgpu_proj_nl_kb_c16", "cpwgpu_plan_build_projectors_kb", "cpwgpu_plan_apply_noalloc",
+    "cpwgpu_host_copy_lanes",
 )
 
 # tunables of a plan (CPWGPU_TUNE_* in include/cpwgpu.h)
@@ -109,6 +110,7 @@ def lib():
         L.cpwgpu_plan_apply.argtypes = [vp, C.c_int, dp, C.c_long, dp, C.c_long, C.c_int, vp]
         L.cpwgpu_plan_apply_noalloc.argtypes = [vp, C.c_int, dp, C.c_long, dp, C.c_long, C.c_int, vp]
         L.cpwgpu_plan_info.argtypes = [vp, ip]
+        L.cpwgpu_host_copy_lanes.argtypes = [ip]
         L.cpwgpu_profile.argtypes = [C.c_int, C.c_uint]
         L.cpwgpu_rayleigh_ritz.argtypes = [C.c_int, C.c_int, dp, C.c_long, dp, C.c_long, C.c_int,
                                            dp, dp, vp]
@@ -349,6 +351,13 @@ def hk_psi_c16_dict(d, psi=None, hpsi=None, neig=None):
                       np.asfortranarray(d["anlga"], np.complex128), np.asfortranarray(d["xnlkb"]),
                       d["nanl"], d["mxddim"], max(psi.shape[1], 1), max(d["mxdanl"], 1),
                       d["mxdgve"], d["mxdscr"])
+
+
+def host_copy_lanes():
+    """Threads of the last large host-array copy (cpwgpu_host_copy_lanes); 0: by the runtime."""
+    out = C.c_int(0)
+    _check(lib().cpwgpu_host_copy_lanes(C.byref(out)))
+    return out.value
 
 
 def profile(on, kernels=None):

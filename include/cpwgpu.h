@@ -54,6 +54,10 @@ int cpwgpu_init(int device);
 int cpwgpu_finalize(void);
 /* Message describing the last error of the calling thread ("" if none). */
 const char *cpwgpu_last_error(void);
+/* Threads that copied the last large host matrix (4 MB or more) through pinned
+ * memory; 0: none was copied yet, or pinned memory was not to be had and the
+ * runtime copied it (the next large copy tries again). */
+int cpwgpu_host_copy_lanes(int *lanes);
 /* Precision of cpwgpu_hk_psi_c16 (CPWGPU_PREC_*); default FP64. */
 int cpwgpu_set_precision(int prec);
 /* 1 (default): the non-local GEMMs run on a second stream beside the FFT

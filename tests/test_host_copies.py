@@ -28,3 +28,23 @@ p.set_projectors(big["anlga"], big["xnlkb"], 700)
 fake.hipGetDevice(C.byref(dev))
 assert dev.value == 1, dev.value
 """)
+
+
+def test_pinned_memory_that_comes_later():
+    out = run("""
+print(hk.host_copy_lanes())
+d, p = small()
+big = small(700, seed=1)[0]
+have = hk.host_copy_lanes()
+hk._check(hk.lib().cpwgpu_finalize())
+_, p = small()
+for refused in (100, 3, 0):   # allocations that fail: all, all but a lane's first, none
+    fake.fake_fail_host_malloc(refused)
+    p.set_projectors(big["anlga"], big["xnlkb"], 700)
+    print(hk.host_copy_lanes())
+    fake.fake_fail_host_malloc(0)
+print(have)
+""").split()
+    none, refused, few, later, full = (int(v) for v in out)
+    assert none == 0 and refused == 0 and full > 0
+    assert few == 0 and later == full
