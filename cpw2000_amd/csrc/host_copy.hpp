@@ -6,6 +6,8 @@
 // one chunk runs beside the host copy of the next.
 // 128 bands and 256 projectors of the 64-atom cell (147 MB in, 49 MB out), the whole
 // call: 10,600 us through the runtime, 5,950 so (4,300 of it the DMA and the kernels).
+// With other threads on every CPU (a BLAS's workers spin for 0.1 s after a call) the
+// copies wait for them: 10-12 ms.
 #pragma once
 
 #include "host.hpp"
