@@ -2225,11 +2225,14 @@ int plan_density(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const
     return CPWGPU_OK;
 }
 
-int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const double *occ_h,
-                int natom, const double *rat, const double *avec, const int *proj_atom, int nq,
-                const int *qv, int nspec, const int *species, const double *fq, double *force,
-                double *enl, hipStream_t s) {
+// on the library stream, like the uploads: they read the host arrays until the
+// synchronisation at the end, or that of plan_forces after an error
+int forces_on_stream(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const double *occ_h,
+                     int natom, const double *rat, const double *avec, const int *proj_atom, int nq,
+                     const int *qv, int nspec, const int *species, const double *fq, double *force,
+                     double *enl) {
     const FftGeom &g = p->g;
+    const hipStream_t s = g_stream;
     if (!full_sizes(g)) return fail(CPWGPU_ERR_SIZE, "forces need a mesh with a two-pass split");
     int rc;
     const int nanl = p->nanl;
@@ -2256,8 +2259,6 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
         if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
         occ = (const double *)g_fw.occ.p;
     }
-    // the uploads go through the library stream; the host arrays are read until
-    // the synchronisation at the end
     // local part ------------------------------------------------------------
     if (nq > 0) {
         const int W1 = 2 * Q1 + 1, W2 = 2 * Q2 + 1;
@@ -2266,7 +2267,6 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
             (rc = upload(g_fw.qv, qv, 3 * (size_t)nq)) || (rc = upload(g_fw.fq, fq, (size_t)nq * nspec)) ||
             (rc = upload(g_fw.rat, rat, 3 * (size_t)natom)) || (rc = upload(g_fw.species, species, (size_t)natom)))
             return rc;
-        if (s != g_stream) HIPCHK(hipStreamSynchronize(g_stream));
         int ngrp;
         if ((rc = density_planes(p, neig, psi, ldp, occ, &ngrp, s))) return rc;
         hipLaunchKernelGGL(k_rho_x, dim3(g.n[2], (g.n[1] + RHO_RY - 1) / RHO_RY), dim3(256),
@@ -2290,7 +2290,6 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
         if ((rc = g_fw.coef.reserve(16 * (size_t)mat)) || (rc = g_fw.phi.reserve(24 * (size_t)nblk * nanl)) ||
             (rc = upload(g_fw.patom, proj_atom, (size_t)nanl)))
             return rc;
-        if (s != g_stream) HIPCHK(hipStreamSynchronize(g_stream));
         // <beta|psi> without the strengths
         ProjView pv = scalar_proj(p);
         pv.xnl = nullptr;
@@ -2340,6 +2339,15 @@ int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const 
         }
     if (enl) *enl = e_nl;
     return CPWGPU_OK;
+}
+
+int plan_forces(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const double *occ, int natom,
+                const double *rat, const double *avec, const int *proj_atom, int nq, const int *qv, int nspec,
+                const int *species, const double *fq, double *force, double *enl) {
+    const int rc = forces_on_stream(p, neig, psi, ldp, occ, natom, rat, avec, proj_atom, nq, qv, nspec, species, fq,
+                                    force, enl);
+    if (rc) (void)hipStreamSynchronize(g_stream);  // nothing reads the caller's arrays any more
+    return rc;
 }
 
 }  // namespace
@@ -3000,7 +3008,7 @@ int cpwgpu_plan_forces(cpwgpu_plan_t plan, int neig, const double *psi_dev, long
     int st = ensure_stream();
     if (st) return st;
     return plan_forces(plan, neig, (const double2 *)psi_dev, ldp, occ, natom, rat, avec, proj_atom, nq, qv,
-                       nspec, species, fq, force, enl, g_stream);
+                       nspec, species, fq, force, enl);
 }
 
 }  // extern "C"
