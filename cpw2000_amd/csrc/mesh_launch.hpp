@@ -198,9 +198,14 @@ int launch_plane_spin_reg(cpwgpu_plan_s *p, cplx<R> *colbuf, const R *vr, long v
         static bool attr_p = false, attr_u = false;
         using P = SpinShape<R, N, true>;
         using U = SpinShape<R, N, false>;
-        // a box inside N/4: the pruned shape
-        if (prune_fits(g)) return go(k_plane_spin_reg<R, N, P::GX, P::GY, P::T, P::W, true>, pr_sub_stride<N>(), P::T, attr_p);
-        return go(k_plane_spin_reg<R, N, U::GX, U::GY, U::T, U::W, false>, reg_stride(g.nx), U::T, attr_u);
+        // a box inside N/4: the pruned shape.  Its row stride holds every such box: where
+        // two planes of it do not fit (128 in FP64), those of a wider box do not either
+        if constexpr (sizeof(cplx<R>) * ((size_t)N + 2 * (size_t)N * pr_sub_stride<N>()) > 160 * 1024)
+            return fail(CPWGPU_ERR_SIZE, "two-component plane of %d x %d does not fit in LDS", N, N);
+        else if (prune_fits(g))
+            return go(k_plane_spin_reg<R, N, P::GX, P::GY, P::T, P::W, true>, pr_sub_stride<N>(), P::T, attr_p);
+        else
+            return go(k_plane_spin_reg<R, N, U::GX, U::GY, U::T, U::W, false>, reg_stride(g.nx), U::T, attr_u);
     }
 }
 
