@@ -3151,6 +3151,7 @@ struct cpwgpu_graph_s {
     int prec = CPWGPU_PREC_FP64;
     std::vector<PlanState> state;  // per k-point, at capture
     DevBuf tab;                    // arguments of the batched launches
+    int groups = 0, grouped = 0;   // groups launched together, k-points in them
 };
 
 extern "C" {
@@ -3199,6 +3200,11 @@ int cpwgpu_graph_create(cpwgpu_graph_t *graph, int nk, const cpwgpu_plan_t *plan
             batch_group_steps(recs, g, tab, nullptr, off, false, nullptr);
         }
     cpwgpu_graph_s *gr = new cpwgpu_graph_s();
+    for (const BatchGroup &g : groups)
+        if (g.ks.size() > 1) {
+            gr->groups++;
+            gr->grouped += (int)g.ks.size();
+        }
     hipStream_t cs = nullptr;
     hipError_t e = hipSuccess, e2 = hipSuccess;
     if (!tab.empty() && !(st = gr->tab.reserve(tab.size())))
@@ -3249,6 +3255,14 @@ int cpwgpu_graph_launch(cpwgpu_graph_t graph, void *stream) {
         }
     }
     HIPCHK(hipGraphLaunch(graph->exec, (hipStream_t)stream));
+    return CPWGPU_OK;
+}
+
+int cpwgpu_graph_info(cpwgpu_graph_t graph, int *out) {
+    if (!graph || !out) return fail(CPWGPU_ERR_ARG, "null argument");
+    out[0] = (int)graph->state.size();
+    out[1] = graph->groups;
+    out[2] = graph->grouped;
     return CPWGPU_OK;
 }
 

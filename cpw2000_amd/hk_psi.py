@@ -52,7 +52,7 @@ EXPORTS = (
     "cpwgpu_hk_psi_spin_c16", "cpwgpu_plan_set_potential_spin", "cpwgpu_plan_set_projectors_spin",
     "cpwgpu_plan_apply_spin", "cpwgpu_hk_psi_c8", "cpwgpu_hk_psi_allk_c16",
     "cpwgpu_proj_nl_kb_c16", "cpwgpu_plan_build_projectors_kb", "cpwgpu_plan_apply_noalloc",
-    "cpwgpu_host_copy_lanes",
+    "cpwgpu_host_copy_lanes", "cpwgpu_graph_info",
 )
 
 # tunables of a plan (CPWGPU_TUNE_* in include/cpwgpu.h)
@@ -118,6 +118,7 @@ def lib():
                                          vp, C.c_int, vp, dp, dp, dp]
         L.cpwgpu_graph_create.argtypes = [C.POINTER(vp), C.c_int, vp, vp, vp, vp, vp, vp, C.c_int]
         L.cpwgpu_graph_launch.argtypes = [vp, vp]
+        L.cpwgpu_graph_info.argtypes = [vp, ip]
         L.cpwgpu_graph_destroy.argtypes = [vp]
         L.cpwgpu_plan_set_variant.argtypes = [vp, C.c_int, C.c_int, C.c_int]
         L.cpwgpu_plan_get_variant.argtypes = [vp, C.c_int, C.c_int, ip]
@@ -685,6 +686,12 @@ class Graph:
         if stream is None:
             stream = torch.cuda.current_stream().cuda_stream
         _check(lib().cpwgpu_graph_launch(self._h, C.c_void_p(stream)))
+
+    def info(self):
+        """{"points", "groups", "grouped"}: k-points, groups launched together, k-points in groups."""
+        out = (C.c_int * 3)()
+        _check(lib().cpwgpu_graph_info(self._h, out))
+        return dict(zip(("points", "groups", "grouped"), list(out)))
 
     def close(self):
         if self._h:

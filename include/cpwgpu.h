@@ -333,6 +333,8 @@ int cpwgpu_graph_create(cpwgpu_graph_t *graph, int nk, const cpwgpu_plan_t *plan
  * cannot follow: another projector count, or a plan workspace reallocated by
  * a larger apply since the capture; create the graph again then. */
 int cpwgpu_graph_launch(cpwgpu_graph_t graph, void *stream);
+/* out[0..2] = k-points, groups of k-points launched together, k-points in groups. */
+int cpwgpu_graph_info(cpwgpu_graph_t graph, int *out);
 int cpwgpu_graph_destroy(cpwgpu_graph_t graph);
 
 /* ---- FP64 subspace step ----------------------------------------------------- */
