@@ -2365,8 +2365,10 @@ struct TuneKey {
     }
 };
 
-// one line per key: prec n1 n2 n3 nx ncol nanl neig | plane proj back splitk kin col sched
-// (lines without the last fields, kin, col and sched, read them as -1)
+// one line per key: prec n1 n2 n3 nx ncol nanl neig | plane proj back splitk kin col
+// sched | version.  Lines of another version, or of none, hold choices made among other
+// kernels under the same numbers (schedule 0 used two streams) and are passed over.
+constexpr int TUNE_CACHE_VERSION = 2;
 bool tune_cache_lookup(const TuneKey &k, int *plane, int *proj, int *back, int *splitk, int *kin, int *col,
                        int *sched) {
     const char *path = std::getenv("CPWGPU_TUNE_CACHE");
@@ -2377,18 +2379,18 @@ bool tune_cache_lookup(const TuneKey &k, int *plane, int *proj, int *back, int *
     bool found = false;
     while (std::fgets(line, sizeof line, f)) {
         TuneKey r;
-        int pv, jv, bv, sk, kv = -1, cv = -1, sv = -1;
-        const int n = std::sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d", &r.prec, &r.n1, &r.n2,
-                                  &r.n3, &r.nx, &r.ncol, &r.nanl, &r.neig, &pv, &jv, &bv, &sk, &kv, &cv, &sv);
-        if (n < 12) continue;
+        int pv, jv, bv, sk, kv, cv, sv, version;
+        const int n = std::sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d", &r.prec, &r.n1, &r.n2,
+                                  &r.n3, &r.nx, &r.ncol, &r.nanl, &r.neig, &pv, &jv, &bv, &sk, &kv, &cv, &sv, &version);
+        if (n != 16 || version != TUNE_CACHE_VERSION) continue;
         if (r == k) {  // the last entry for a key wins
             *plane = pv;
             *proj = jv;
             *back = bv;
             *splitk = sk;
-            *kin = n >= 13 ? kv : -1;
-            *col = n >= 14 ? cv : -1;
-            *sched = n >= 15 ? sv : -1;
+            *kin = kv;
+            *col = cv;
+            *sched = sv;
             found = true;
         }
     }
@@ -2402,8 +2404,8 @@ void tune_cache_store(const TuneKey &k, int plane, int proj, int back, int split
     if (!path || !*path) return;
     FILE *f = std::fopen(path, "a");
     if (!f) return;
-    std::fprintf(f, "%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d\n", k.prec, k.n1, k.n2, k.n3, k.nx, k.ncol,
-                 k.nanl, k.neig, plane, proj, back, splitk, kin, col, sched);
+    std::fprintf(f, "%d %d %d %d %d %d %d %d %d %d %d %d %d %d %d %d\n", k.prec, k.n1, k.n2, k.n3, k.nx, k.ncol,
+                 k.nanl, k.neig, plane, proj, back, splitk, kin, col, sched, TUNE_CACHE_VERSION);
     std::fclose(f);
 }
 

@@ -275,7 +275,8 @@ int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value);
  * keeps the fastest in the plan.  hpsi_dev is overwritten with H psi.
  * If the environment variable CPWGPU_TUNE_CACHE names a file, choices are
  * read from it for meshes already tuned (no timing) and appended after
- * tuning; the key is (precision, n1, n2, n3, nx, ncol, nanl, neig). */
+ * tuning; the key is (precision, n1, n2, n3, nx, ncol, nanl, neig).  Lines that
+ * a library with other kernels behind the numbers wrote are passed over. */
 int cpwgpu_plan_tune(cpwgpu_plan_t plan, int neig, const double *psi_dev, long ldp, double *hpsi_dev,
                      long ldh, int prec, void *stream);
 /* Autotuner of the two-component path (cpwgpu_plan_apply_spin arguments; the
