@@ -2712,7 +2712,8 @@ int apply_noalloc_t(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, dou
                     noalloc_need<R>(p, 1, true), NOALLOC_SCRATCH);
     // the last chunk has to fit as well: its kernel may cut more slices
     const auto fits_any = [&](int nb) { return nb == 0 || fits(nb, false) || fits(nb, true); };
-    int nbc = neig;
+    // (not from neig: each try costs the choice of a projection shape)
+    int nbc = (int)std::max<size_t>(1, std::min<size_t>(neig, NOALLOC_SCRATCH / (sizeof(cplx<R>) * p->g.n[2] * p->g.ncolp)));
     while (nbc > 1 && !(fits_any(nbc) && fits_any(neig % nbc))) nbc--;
     for (int b0 = 0; b0 < neig; b0 += nbc) {
         const int nb = std::min(nbc, neig - b0);
