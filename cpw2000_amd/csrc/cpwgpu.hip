@@ -2781,11 +2781,15 @@ int cpwgpu_finalize(void) {
         rocblas_destroy_handle(g_blas);
         g_blas = nullptr;
     }
-    for (DevBuf *b : {&g_dt.xa, &g_dt.hxa, &g_dt.xb, &g_dt.hxb, &g_dt.pb, &g_dt.cpk, &g_dt.hd, &g_dt.m,
-                      &g_dt.g, &g_dt.g0,
-                      &g_dt.pm, &g_dt.w, &g_dt.e, &g_dt.info, &g_dt.res, &g_dt.act, &g_dt.d, &g_dt.mones,
-                      &g_dt.eall, &g_fw.rhor, &g_fw.t1, &g_fw.t2, &g_fw.coef, &g_fw.phi})
+    for (DevBuf *b : {&g_dt.xa, &g_dt.hxa, &g_dt.xb, &g_dt.hxb, &g_dt.pb, &g_dt.cpk, &g_dt.hd, &g_dt.m, &g_dt.g,
+                      &g_dt.g0, &g_dt.pm, &g_dt.w, &g_dt.e, &g_dt.info, &g_dt.res, &g_dt.act, &g_dt.d, &g_dt.mones,
+                      &g_dt.eall, &g_fw.t1, &g_fw.t2, &g_fw.rho, &g_fw.qv, &g_fw.fq, &g_fw.rat, &g_fw.species,
+                      &g_fw.patom, &g_fw.occ, &g_fw.out, &g_fw.coef, &g_fw.phi, &g_fw.rhor, &g_ss.s, &g_ss.m, &g_ss.w,
+                      &g_ss.v, &g_ss.part, &g_ss.pos, &g_ss.info, &g_ss.eig, &g_ss.res, &g_ss.tmp, &g_ss.rec,
+                      &g_ss.dinv, &g_ss.jac, &g_ss.ctl})
         b->release();
+    if (g_ss.stop) HIPCHK(hipHostFree(g_ss.stop));
+    g_ss.stop = nullptr;
     if (g_aux) {
         HIPCHK(hipStreamSynchronize(g_aux));
         HIPCHK(hipStreamDestroy(g_aux));

@@ -190,7 +190,7 @@ struct cpwgpu_plan_s {
     bool sanl32_valid = false;
     DevBuf spsi, shpsi;
     ~cpwgpu_plan_s() {
-        col_ptr.release(); col_uy.release(); ent_i.release(); ent_cz.release(); ekpg.release();
+        col_ptr.release(); col_uy.release(); ent_i.release(); ent_cz.release(); ekpg.release(); zmap.release();
         for (auto &t : tw) t.release();
         v64.release(); v32.release(); anl64.release(); anl32.release(); xnl.release();
         colbuf.release(); part.release(); dhd.release(); gw.release();

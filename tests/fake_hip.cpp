@@ -25,7 +25,7 @@ int ndev = 1;
 thread_local int cur = 0;
 thread_local std::vector<Config> configs;
 double clock_us = 0.0;
-long since_sync = 0, fail_host_malloc = 0;
+long since_sync = 0, fail_host_malloc = 0, live = 0;
 std::map<const void *, std::string> names;
 std::map<const void *, size_t> vars;
 std::map<const void *, void *> var_mem;
@@ -61,6 +61,7 @@ void fake_fail_host_malloc(long n) { fail_host_malloc = n; }  // the next n allo
 void fake_cost(const char *part, double first, double later, long after) { costs.push_back({part, first, later, after}); }
 void fake_clear() { std::lock_guard<std::recursive_mutex> lk(mu); text.clear(); }
 const char *fake_log() { return text.c_str(); }
+long fake_live() { return live; }  // allocations, device and pinned, not given back
 
 // ---- the runtime ---------------------------------------------------------------
 hipError_t hipGetDeviceCount(int *n) { *n = ndev; return hipSuccess; }
@@ -69,15 +70,26 @@ hipError_t hipSetDevice(int d) { if (d < 0 || d >= ndev) return hipErrorInvalidD
 hipError_t hipDeviceSynchronize() { synced("device sync"); return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "fake error"; }
-hipError_t hipMalloc(void **p, size_t n) { *p = calloc(1, n ? n : 1); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
+    *p = calloc(1, n ? n : 1);
+    live += *p != nullptr;
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipFree(void *p) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
+    live -= p != nullptr;
+    free(p);
+    return hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     std::lock_guard<std::recursive_mutex> lk(mu);
     if (fail_host_malloc > 0) { fail_host_malloc--; return hipErrorOutOfMemory; }
     *p = malloc(n);
+    live++;
     return hipSuccess;
 }
-hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(new Stream{cur}); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { synced("stream sync"); return hipSuccess; }

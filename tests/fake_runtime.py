@@ -18,6 +18,7 @@ fake = C.CDLL({fake!r}, mode=C.RTLD_GLOBAL)
 fake.fake_log.restype = C.c_char_p
 fake.fake_cost.argtypes = [C.c_char_p, C.c_double, C.c_double, C.c_long]
 fake.fake_fail_host_malloc.argtypes = [C.c_long]
+fake.fake_live.restype = C.c_long
 import numpy as np
 from cpw2000_amd import hk_psi as hk, synth
 
