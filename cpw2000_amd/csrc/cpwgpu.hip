@@ -2590,10 +2590,19 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
     // a choice of 12.6 ms by single applies takes 15.4 in a loop, the defaults 13.2).
     int *const choice[7] = {&p->plane_var[ix], &p->proj_var[ix], &p->back_var[ix], &p->splitk[ix],
                             &p->kin_var[ix], &p->col_var[ix], &p->sched_var[ix]};
+    constexpr int what[7] = {CPWGPU_TUNE_PLANE, CPWGPU_TUNE_PROJ, CPWGPU_TUNE_BACK, CPWGPU_TUNE_SPLITK,
+                             CPWGPU_TUNE_KIN, CPWGPU_TUNE_COL, CPWGPU_TUNE_SCHED};
     int tuned[7];
-    for (int i = 0; i < 7; i++) tuned[i] = *choice[i];
+    bool same = true;
+    for (int i = 0; i < 7; i++) {
+        int def = -1;
+        tuned[i] = *choice[i];
+        *choice[i] = -1;
+        cpwgpu_plan_get_variant(p, prec, what[i], &def);
+        same = same && def == tuned[i];
+    }
     double sum[2] = {0.0, 0.0};
-    for (int round = 0; round < 5; round++)
+    for (int round = 0; round < 5 && !same; round++)
         for (int def = 0; def < 2; def++) {
             for (int i = 0; i < 7; i++) *choice[i] = def ? -1 : tuned[i];
             if ((st = time_loop(p, neig, psi, ldp, hpsi, ldh, prec, s, &t))) return st;
