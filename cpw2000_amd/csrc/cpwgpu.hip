@@ -675,8 +675,8 @@ int nonlocal(cpwgpu_plan_s *p, const ProjView &pv_, int neig, const double *psi,
     return CPWGPU_OK;
 }
 
-// second stream and fork/join events: the projector GEMMs (matrix cores) run
-// beside the FFT kernels (LDS / HBM)
+// second stream and fork/join events of the schedules that run projector GEMMs beside
+// FFT kernels (1, 2 and the FP32 two-component product)
 hipStream_t g_aux = nullptr;
 hipEvent_t g_fork = nullptr, g_join = nullptr;
 
@@ -2543,7 +2543,7 @@ int tune_plan(cpwgpu_plan_s *p, int neig, const double *psi, long ldp, double *h
         }
     }
     p->back_var[ix] = best_bv;
-    // where the kinetic term goes: it moves work between the two streams
+    // where the kinetic term goes: gather or back-projection
     int best_kv = 0;
     if (p->nanl > 0) {
         best = 3.4e38f;

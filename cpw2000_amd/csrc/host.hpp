@@ -162,13 +162,12 @@ struct cpwgpu_plan_s {
     // stream schedule: 0 (default) one stream; 1 the projection beside the
     // local term; 2 the inverse columns and planes beside the non-local term
     int sched_var[2] = {-1, -1};
-    // split-K target blocks of the projection GEMM per precision (-1 = 256)
+    // split-K target blocks of the projection GEMM per precision (-1 and
+    // SPLITK_DEFAULT: whole rounds of the compute units)
     int splitk[2] = {-1, -1};
-    // projection GEMM kernel per precision: 0 LDS-staged k_proj, 1 k_proj_direct
-    // (-1 = default)
+    // projection and back-projection GEMM kernel per precision (-1 and
+    // PROJ_DEFAULT, BACK_DEFAULT: by size)
     int proj_var[2] = {-1, -1};
-    // back-projection GEMM kernel per precision: 0 LDS-staged k_back, 1
-    // k_back_direct (-1 = default)
     int back_var[2] = {-1, -1};
     // where the kinetic term ekpg*psi is added when the non-local term is on:
     // 0 the back-projection epilogue, 1 the gather of the forward column kernel

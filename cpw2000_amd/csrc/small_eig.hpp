@@ -400,7 +400,8 @@ __global__ __launch_bounds__(SE_THREADS) void k_jacobi_lds(const double2 *__rest
 // roots (k_jacobi_lds, whose results the caller of a Rayleigh-Ritz step keeps to
 // the bit, takes a hypot, four divisions and two square roots), and with half of
 // the blocks gone by symmetry one to three blocks per thread.  Outputs as
-// k_jacobi_lds; info: 1 if max_sweeps did not do.  us at n = 72, from Ritz vectors, with the vectors: 318 on average (from 150), zheevd 1,600.
+// k_jacobi_lds; info: 1 if max_sweeps did not do.  us at n = 72, from Ritz vectors: 292 on
+// average (from 172), with the vectors 359, with the refinement below 403, zheevd 1,600.
 __device__ __forceinline__ double fast_rsqrt(double x) {
     double r = __builtin_amdgcn_rsq(x);  // refined by two Newton steps
 #pragma unroll
@@ -591,7 +592,7 @@ __global__ __launch_bounds__(64) void k_jacobi_vectors(const double4 *__restrict
 // Two steps (the second takes away the K^2 of the first) at 17 to 127 columns: v
 // orthonormal to 1e-15, A v = v w to 4e-16 |A|, close pairs included.
 // Three products of n <= 128 per step, one 16 x 16 tile per block: bound by
-// their launches.  Block iteration on the 64-atom cell, 42 vectors, 76 steps: vectors
+// their launches (7.8 + 7.3 + 6.9 us at 72).  Block iteration on the 64-atom cell, 42 vectors, 76 steps: vectors
 // orthonormal to 2.6e-15 (without the refinement 4e-13, with zheevd 4e-14), 222 ms (217,
 // 269).
 constexpr int SE_RT = 16;

@@ -162,8 +162,8 @@ def set_ditsp_method(method):
 
 
 def set_overlap(on):
-    """Non-local GEMMs on a second stream beside the FFT kernels (default) or
-    every kernel in sequence on the caller's stream."""
+    """Whether a set or tuned schedule may use a second stream (default), or every
+    kernel runs in sequence on the caller's stream (as the default schedule has it)."""
     _check(lib().cpwgpu_set_overlap(1 if on else 0))
 
 
@@ -440,17 +440,19 @@ class Plan:
         """Kernel choice for a precision: what = TUNE_PLANE (plane-stage kernel,
         0 .. NPLANE_VAR-1 as listed at NPLANE_VAR, -1 default), TUNE_PROJ
         (projection GEMM, 0 LDS-staged, 1..4 direct-load shapes, 5 LDS-staged
-        with half-size wave tiles), TUNE_BACK (back-projection GEMM, 0
-        LDS-staged, 1..3 direct-load shapes, 4 LDS-staged with half-size chunks),
-        TUNE_SPLITK (projection GEMM split-K target blocks, -1 default),
-        TUNE_KIN (kinetic term in the back-projection epilogue 0 or in the
+        with half-size wave tiles; 1, the default, takes the block that suits the
+        bands), TUNE_BACK (back-projection GEMM, 0 LDS-staged, 1..3 direct-load
+        shapes, 4 LDS-staged with half-size chunks; 2 in FP64 and 4 in FP32, the
+        defaults, by the number of bands), TUNE_SPLITK (projection GEMM split-K
+        target blocks; 256, the default, stands for whole rounds of the compute
+        units), TUNE_KIN (kinetic term in the back-projection epilogue 0 or in the
         column gather 1), TUNE_SPIN (plane kernel of apply_spin with nsp = 4:
         0 LDS two-pass, 1 register lines where built, -1 default), TUNE_COL
-        (z-column kernels: 0 LDS two-pass, 1 register lines where built) or
-        TUNE_SCHED (stream schedule: 0 the whole non-local term beside the
-        local one, 1 projection beside it and back-projection after it, 2 the
-        non-local term on the caller's stream with the column and plane
-        kernels beside it)."""
+        (z-column kernels: 0 LDS two-pass, 1 register lines where built, the
+        default in FP64) or TUNE_SCHED (stream schedule: 0, the default, one
+        stream; 1 the projection beside the local term and the back-projection
+        after it; 2 the non-local term on the caller's stream with the column and
+        plane kernels beside it).  -1: the default."""
         _check(lib().cpwgpu_plan_set_variant(self._h, int(prec), int(what), int(value)))
 
     def get_variant(self, prec, what):
@@ -461,7 +463,7 @@ class Plan:
     def tune(self, psi_t, hpsi_t, prec=PREC_FP32, stream=None):
         """Autotune the plan's kernels on these device arrays (hpsi_t receives
         H psi); returns the choice {"plane", "proj", "back", "splitk", "kin", "col",
-        "sched"}."""
+        "sched"}, which set_variant takes on another plan of the k-point."""
         import torch
 
         neig = psi_t.shape[0]

@@ -60,9 +60,10 @@ const char *cpwgpu_last_error(void);
 int cpwgpu_host_copy_lanes(int *lanes);
 /* Precision of cpwgpu_hk_psi_c16 (CPWGPU_PREC_*); default FP64. */
 int cpwgpu_set_precision(int prec);
-/* 1 (default): the non-local GEMMs run on a second stream beside the FFT
- * kernels (fork/join with events on the caller's stream); 0: every kernel on
- * the caller's stream, one after the other.  Same work and result. */
+/* 1 (default): where a stream schedule with two streams is set or tuned
+ * (CPWGPU_TUNE_SCHED 1 or 2), part of the kernels run on a second stream (fork/
+ * join with events on the caller's stream); 0: every kernel on the caller's
+ * stream, as the default schedule has it.  Same work and result. */
 int cpwgpu_set_overlap(int on);
 /* Iteration of cpwgpu_plan_ditsp / cpwgpu_ditsp_c16 (no counterpart in the
  * reference, whose Src/ditsp/ditsp_c16_loop.f90 relaxes band by band):
@@ -238,8 +239,7 @@ int cpwgpu_plan_info(cpwgpu_plan_t plan, int *out);
  *                       number); -1 = default (FP64 2, FP32 4)
  *   CPWGPU_TUNE_KIN     where ekpg*psi is added when projectors are set: 0 = in
  *                       the back-projection epilogue, 1 = in the gather of the
- *                       forward column kernel (moves work between the two
- *                       streams); -1 = default (0)
+ *                       forward column kernel; -1 = default (0)
  *   CPWGPU_TUNE_SPIN    plane kernel of cpwgpu_plan_apply_spin with nsp = 4: 0 =
  *                       LDS two-pass lines, 1 = register-resident lines (built
  *                       when 8 divides the mesh length); -1 = default (1
@@ -269,10 +269,12 @@ int cpwgpu_plan_set_variant(cpwgpu_plan_t plan, int prec, int what, int value);
 /* Current choice (the value used by the next apply, defaults resolved): setting it on
  * a plan of the same k-point runs the same kernels. */
 int cpwgpu_plan_get_variant(cpwgpu_plan_t plan, int prec, int what, int *value);
-/* Autotuner: times cpwgpu_plan_apply for every plane variant built for the
- * mesh, then both projection kernels with a few split-K targets, then both
- * back-projection kernels, on the caller's arrays (neig bands, stream), and
- * keeps the fastest in the plan.  hpsi_dev is overwritten with H psi.
+/* Autotuner: times cpwgpu_plan_apply on the caller's arrays (neig bands, stream)
+ * for the column kernels, every plane variant built for the mesh, the projection
+ * kernels with a few split-K targets, the back-projection kernels, the place of the
+ * kinetic term and the stream schedules, one after the other; then the whole choice
+ * against the defaults in loops of applies, and keeps the faster in the plan.
+ * hpsi_dev is overwritten with H psi.
  * If the environment variable CPWGPU_TUNE_CACHE names a file, choices are
  * read from it for meshes already tuned (no timing) and appended after
  * tuning; the key is (precision, n1, n2, n3, nx, ncol, nanl, neig).  Lines that
