@@ -2213,9 +2213,15 @@ int plan_density(cpwgpu_plan_s *p, int neig, const double2 *psi, long ldp, const
     int rc, ngrp;
     const double *occ = nullptr;
     if (occ_h) {
-        if ((rc = upload(g_fw.occ, occ_h, (size_t)neig))) return rc;
+        if ((rc = g_fw.occ.reserve(8 * (size_t)neig))) return rc;
         occ = (const double *)g_fw.occ.p;
-        HIPCHK(hipStreamSynchronize(g_stream));  // the upload went through the library stream
+        for (int b0 = 0; b0 < neig; b0 += OCC_ARGS) {
+            OccArgs a;
+            const int n = std::min(OCC_ARGS, neig - b0);
+            std::copy(occ_h + b0, occ_h + b0 + n, a.v);
+            hipLaunchKernelGGL(k_put_occ, dim3(1), dim3(OCC_ARGS), 0, s, a, n, (double *)g_fw.occ.p + b0);
+        }
+        HIPCHK(hipGetLastError());
     }
     if ((rc = density_planes(p, neig, psi, ldp, occ, &ngrp, s))) return rc;
     const long tot = (long)g.id * g.n[1] * g.n[2];

@@ -28,6 +28,17 @@
 
 namespace cpwgpu {
 
+// Occupations travel as kernel arguments, OCC_ARGS at a time: in the order of the
+// caller's stream, so that a call does not overwrite those that the call before it
+// still reads, and with no wait for a copy from the caller's array.
+constexpr int OCC_ARGS = 256;
+struct OccArgs {
+    double v[OCC_ARGS];
+};
+__global__ __launch_bounds__(OCC_ARGS) void k_put_occ(const OccArgs a, int n, double *__restrict__ out) {
+    if ((int)threadIdx.x < n) out[threadIdx.x] = a.v[threadIdx.x];
+}
+
 // sum over band groups of p[grp * step] in group order, eight loads in flight
 // (clamped; one after the other they cost a memory round trip each)
 __device__ __forceinline__ double sum_groups(const double *__restrict__ p, long step, int ngrp) {
