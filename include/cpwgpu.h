@@ -419,7 +419,9 @@ int cpwgpu_ditsp_c16(const int *ipr, int *ifail, const int *icmax, const int *ig
  * rhomsh).  psi_dev (ldp, neig) device complex128; occ host (neig) or NULL
  * (= 1); rho_dev device double in the vscr layout rho[(k3*n2 + k2)*id + k1]
  * (id*n2*n3 values, zero for k1 >= n1).  The mesh must be one of the
- * specialised sizes.  Enqueued on stream. */
+ * specialised sizes.  Enqueued on stream; occ is read before the call returns.
+ * Calls in a row on one stream need no wait between them; the work buffers are
+ * shared, so calls on different streams have to be ordered by the caller. */
 int cpwgpu_plan_density(cpwgpu_plan_t plan, int neig, const double *psi_dev, long ldp, const double *occ,
                         double *rho_dev, void *stream);
 
